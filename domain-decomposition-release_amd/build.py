@@ -33,12 +33,16 @@ COMMON = [
     "-I", os.path.join(ROOT, "include"), "-I", CSRC,
     "-Wall", "-Wno-unused-function", "-Wno-unused-variable", "-Wno-unused-command-line-argument",
 ]
-SOURCES = ["kernels.hip", "engine.cpp"]
+# kernels.hip once per family of kernels (DDX_PART), so that they compile in parallel
+PARTS = 9
+SOURCES = [("kernels.hip", p) for p in range(PARTS)] + [("engine.cpp", None)]
 
 
-def _compile(src):
-    obj = os.path.join(OBJ_DIR, os.path.splitext(src)[0] + ".o")
-    lang = ["-x", "hip"]
+def _compile(job):
+    src, part = job
+    stem = os.path.splitext(src)[0]
+    obj = os.path.join(OBJ_DIR, stem + ("" if part is None else f"_{part}") + ".o")
+    lang = ["-x", "hip"] + ([] if part is None else [f"-DDDX_PART={part}"])
     cmd = [HIPCC] + COMMON + lang + ["-c", os.path.join(CSRC, src), "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
@@ -46,7 +50,7 @@ def _compile(src):
     return obj
 
 
-def build(jobs=2, verbose=True):
+def build(jobs=8, verbose=True):
     os.makedirs(OBJ_DIR, exist_ok=True)
     os.makedirs(OUT_DIR, exist_ok=True)
     with ThreadPoolExecutor(max_workers=jobs) as ex:
@@ -98,7 +102,7 @@ def build_host(verbose=True, tool_only=False):
 
 if __name__ == "__main__":
     ap = argparse.ArgumentParser()
-    ap.add_argument("--jobs", type=int, default=2)
+    ap.add_argument("--jobs", type=int, default=8)
     a = ap.parse_args()
     try:
         build(a.jobs)

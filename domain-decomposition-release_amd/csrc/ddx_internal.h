@@ -11,6 +11,18 @@ constexpr int NF = 19;
 enum : int { VX = 0, VY, VZ, SXX, SYY, SZZ, SXY, SXZ, SYZ, SAU, VXP, VYP, VZP, UX, UY, UZ, VXRT, VYRT, VZRT };
 enum : int { PURE_FORWARD = 0, RTM_FORWARD = 1, RTM_BACKWARD = 2, RTM_REVERSE = 3, FWI = 4 };
 constexpr int kModes = 5;
+// Tap n of the staggered first derivative of half order `half`
+// (GEO/jarvis_device_geometry_bones.hpp:29-49, cu_cal_diff_coeff); 0 past it.
+constexpr float fd_tap(int half, int n) {
+  if (n >= half) return 0.f;
+  double a1 = 1, a2 = 1, a3 = 1;
+  for (int i = 0; i < half; i++) {
+    if (i != n) a1 = a1 * (2 * i + 1) * (2 * i + 1);
+    if (i < n) a2 = a2 * ((2 * n + 1) * (2 * n + 1) - (2 * i + 1) * (2 * i + 1));
+    if (i > n) a3 = a3 * ((2 * i + 1) * (2 * i + 1) - (2 * n + 1) * (2 * n + 1));
+  }
+  return (float)((n & 1 ? -a1 : a1) / ((2 * n + 1) * a2 * a3));
+}
 // Wavefield storage formats (fields, CPML memory variables, VOWR store): FP32,
 // or 16-bit codes of the value times a power-of-two scale per field class.
 enum : int { STORE_F32 = 0, STORE_F16 = 1, STORE_BF16 = 2, STORE_BFP16 = 3 };
@@ -50,48 +62,25 @@ inline int pml_blocks(int ni, int nj, int nk, int cz) {
   return pml_plane_tiles(ni, nj, cz) * ((nk + p - 1) / p);
 }
 
-// Pack on store: the kernels that update a subdomain's boundary layers also
-// write each updated value into the ghost layers of the neighbour that
-// receives it, so no separate CMM exchange pass reads the layers again.
-// Side order top, bottom, front, back, right, left (z lo, z hi, y lo, y hi,
-// x lo, x hi); a cell at local extended coordinate c along the side's axis
-// is sent when c < w (lo sides) or c >= en - w (hi sides), w the width the
-// receiver takes for the field (table H1), and lands at the receiver's
-// coordinate c + shift (the other two coordinates are equal on both sides).
-struct MirrorSide {
-  char *base;   // receiver's field 0 at its local extended (0,0,0), bytes; nullptr: no neighbour
-  long fpitch;  // elements between the receiver's fields
-  long sy, sz;  // receiver's strides
-  int shift;
-  int w[10];    // width sent per field id VX .. SAU (0: not sent)
-};
-struct MirrorDesc {
-  MirrorSide s[6];
-  int en[3];  // the sender's local extended size
-};
-
-// One subdomain's physical region (gridphy), in the subdomain's storage.
-// Field pointers address local extended cell (0,0,0); strides sy, sz in
-// elements; ghost cells toward neighbours live at negative / past-the-end
-// local coordinates.  Field elements are of the context's storage format.
+// One physical region (gridphy) of the whole grid, all subdomains of the
+// decomposition in it.  Field pointers address extended cell (0,0,0);
+// strides sy, sz in elements.  Field elements are of the context's storage
+// format.
 struct PhyDesc {
   void *f[NF];
   const float *dtr;  // dt / rho, per cell
   const float *lam;
   const float *mu;
   long sy, sz;
-  int ox, oy, oz;    // gridphy origin in local extended coordinates
+  int ox, oy, oz;    // gridphy origin in extended coordinates
   int nx, ny, nz;    // gridphy size
-  int gx, gy, gz;    // offset of this gridphy inside the global gridphy
-  int gnx, gny, gnz; // the global gridphy (VOWR variable order of the backward mode)
   int R;             // VOWR ring width
   int tiles_x, tiles_y;
   float dt;          // time step (FWI accumulators)
-  const MirrorDesc *mir;  // pack on store (z-blocked bricks); nullptr: none
   int blk0;
 };
 
-// One CPML slab of one subdomain (the reference's top/bottom, front/back,
+// One CPML slab of the whole grid (the reference's top/bottom, front/back,
 // right/left PML frames, BASE/fdtd3d_base_6_pml_meat.hpp:29-93).
 struct SlabDesc {
   void *f[NF];
@@ -99,12 +88,11 @@ struct SlabDesc {
   const float *lam;
   const float *mu;
   long sy, sz;
-  int i0, j0, k0, ni, nj, nk;        // box in local extended coordinates
+  int i0, j0, k0, ni, nj, nk;        // box in extended coordinates
   int axes;                          // damped axes: 1 x, 2 y, 4 z
   int xlo, xhi, ylo, yhi, zlo, zhi;  // a cell is in an axis' damping range iff c < lo || c >= hi
   void *psi;                         // [6 * naxes][ncell] memory variables (storage format)
   const float *coef;                 // [4 * naxes][ncell]: a, b, a_half, b_half per axis
-  const MirrorDesc *mir;             // pack on store; nullptr: none
   int blk0;
 };
 
@@ -126,42 +114,13 @@ struct PmlOrder {
   int grid = 0;                      // 8 x the largest xn
 };
 
-// Blocks of the CMM copy of one link: boxes at most kHaloNarrow cells long
-// in x (the x-face links, 3-4 cells) take one cell per thread, longer boxes
-// one row per wavefront (4 per block).
-constexpr int kHaloNarrow = 8;
-inline int halo_blocks(int ni, int nj, int nk) {
-  const long rows = (long)nj * nk;
-  return ni <= kHaloNarrow ? (int)((rows * ni + kBlock - 1) / kBlock)
-                           : (int)((rows + kBlock / 64 - 1) / (kBlock / 64));
-}
-
-// One CMM halo link of one field: the sender's boundary layers copied
-// straight into the receiver's ghost layers (both subdomains live on the
-// same device, so the contiguous message block of the reference's MPI
-// exchange is not needed).  Same box size on both sides, x fastest.
-struct HaloDesc {
-  const void *src;
-  void *dst;
-  long ssy, ssz, dsy, dsz;
-  int si, sj, sk;  // box origin in the sender's local coordinates
-  int di, dj, dk;  // box origin in the receiver's local coordinates (ghosts)
-  int ni, nj, nk;
-  int blk0;
-};
-
 // One box copied between a field and a contiguous buffer (the VOWR boundary
 // store).
 struct CopyDesc {
   void *field;
   long sy, sz;
   int i0, j0, k0, ni, nj, nk;
-  // element (i, j, k) of the box is buffer element buf_off + (bi + i) +
-  // bni * ((bj + j) + bnj * (bk + k)): the box is the sub-box at (bi, bj, bk)
-  // of a bni x bnj x .. buffer box (a ring box's part that lies in a
-  // neighbour's ghost layers); bi = bj = bk = 0, bni = ni, bnj = nj for a
-  // whole box
-  int bi, bj, bk, bni, bnj;
+  // the box is buffer elements buf_off .. , x fastest
   long buf_off;
   int cls;   // field class (0 velocity, 1 stress): the scale of a converting copy
   int fid;   // ring field index (0..9): the per-slice scale of a converting copy
@@ -228,15 +187,13 @@ struct MemberIO {
 // fmt: storage format; the 16-bit formats fold their scale ratios into
 // `sign` (velocity: sv/ss), `dt` (stress: ss/sv) and `rv` (CPML velocity:
 // sv/ss); ss, sv, inv_sv: the class scales themselves.
-void set_fd_table(const float tab[5][4]);
-// block order of the z-blocked bricks: 0 contiguous per XCD, g > 0 groups of g
-void set_brick_group(int g);
 // The physical-region launchers return false, launching nothing, when no
-// kernel exists for the brick shape, storage format and mode.
+// kernel exists for the brick shape, storage format and mode.  grp: block
+// order of the z-blocked bricks (0 contiguous per XCD, else groups of grp).
 bool launch_vel_phy(const Tiling &t, int mode, int fmt, const PhyDesc *d, const int *starts, int n, int nblk,
-                    float dx, float dy, float dz, float sign, int gnx, int gny, int gnz, int R, hipStream_t st);
+                    float dx, float dy, float dz, float sign, int grp, hipStream_t st);
 bool launch_stress_phy(const Tiling &t, int mode, int fmt, const PhyDesc *d, const int *starts, int n, int nblk,
-                       float dx, float dy, float dz, float dt, int gnx, int gny, int gnz, int R, hipStream_t st);
+                       float dx, float dy, float dz, float dt, int grp, hipStream_t st);
 // grp: blocks per XCD group of the group-interleaved block order (0: launch order)
 // ord (nullable): the XCD-partitioned block order of the table; without it
 // (or with ord->pieces null) the blocks follow the table's own order.
@@ -247,7 +204,6 @@ void launch_stress_pml(int cz, int with_sau, int fmt, const SlabDesc *d, const i
 // dir +1: field -> buffer (VOWR save); -1: buffer -> field (VOWR inject);
 // esz: element size in bytes (4 or 2)
 void launch_copy(int dir, int esz, const CopyDesc *d, const int *starts, int n, int nblk, void *buf, hipStream_t st);
-void launch_halo(int esz, const HaloDesc *d, const int *starts, int n, int nblk, hipStream_t st);
 // Converting copy between FP32 fields and a 16-bit buffer (fmt FP16 or
 // BF16): saved values are scaled by sc[cls] and rounded; injected ones
 // widened and scaled by 1 / sc[cls].

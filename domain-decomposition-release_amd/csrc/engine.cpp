@@ -3,13 +3,16 @@
 // CPML coefficients, CMM halo and VOWR descriptor tables, the time-loop
 // drivers and the C ABI declared in include/ddx.h.
 //
-// Device layout.  Each subdomain stores every field on its local extended
-// grid (gridext) plus 4 ghost layers on each side that faces a neighbour
-// subdomain; x is fastest and the x pitch is padded so that each row of the
-// physical region starts on a 128-byte boundary.  Ghost layers are filled by
-// the CMM exchange after every half step: one kernel per batch copies every
-// neighbour's boundary layers straight into the receiver's ghosts (the
-// contiguous message block of an MPI exchange is not needed on one device).
+// Device layout.  Every field is one array over the global extended grid
+// (gridext), x fastest, the x pitch padded so that each row of the physical
+// region starts on a 128-byte boundary.  A subdomain of the decomposition is
+// a window of those arrays: its ghost layers are its neighbours' own cells,
+// so every ghost is current as soon as its owner is updated, no halo is
+// copied, and one physical-region descriptor and six CPML slabs cover all
+// subdomains.  (Measured against subdomains with storage of their own, whose
+// ghosts were copied after every half step: the 256x256x200 RTM shot of 50
+// steps on 2x2x1 subdomains 181.8 -> 160.8 ms, 8 copies of 33 us per step of
+// it; a 141x97x75 one on 3x2x1 83.0 -> 63.5 ms.)
 #include <algorithm>
 #include <atomic>
 #include <climits>
@@ -57,17 +60,17 @@ static int gap_num(float l, float r, float d) {
   return nr - nl;
 }
 
-struct Geom {
+struct Geom {  // a subdomain: its place in the decomposition and in the global arrays
   int rank;
   int ci[3];            // index of the subdomain in the decomposition
   int pn[3], poff[3];   // gridphy size and offset inside the global gridphy
   int en[3];            // local gridext size
   int mlo[3], mhi[3];   // margins (pml_num on global sides, 0 toward neighbours)
   int nlo[3], nhi[3];   // neighbour ranks (-1: global boundary)
-  int glo[3], ghi[3];   // ghost widths
-  int pad_x;
+  // storage, in elements: strides, the position of the extended cell (0,0,0)
+  // inside a field, a field's size and the distance between fields
   long sy, sz, nstore, origin;
-  long fpitch;          // distance between consecutive fields of a subdomain (>= nstore)
+  long fpitch;
   float lphy[3], rphy[3], lext[3], rext[3];
   long ext_goff[3];     // offset of local gridext inside the global gridext
 };
@@ -106,8 +109,6 @@ static bool make_geom(const ddx_desc &d, int rank, Geom &g, std::string &err) {
     g.en[a] = pn + g.mlo[a] + g.mhi[a];
     g.lext[a] = -(float)g.mlo[a] * dd[a] + g.lphy[a];
     g.rext[a] = g.lext[a] + (float)(g.en[a] - 1) * dd[a];
-    g.glo[a] = g.nlo[a] >= 0 ? 4 : 0;
-    g.ghi[a] = g.nhi[a] >= 0 ? 4 : 0;
     g.ext_goff[a] = (long)g.poff[a] + m - g.mlo[a];
     if (pn < 8) { err = "subdomain too thin (needs >= 8 physical cells per axis)"; return false; }
   }
@@ -117,16 +118,36 @@ static bool make_geom(const ddx_desc &d, int rank, Geom &g, std::string &err) {
     err = "subdomain gridphy too large (more than 2^30 cells); use a finer decomposition";
     return false;
   }
-  // storage: align the first physical x cell of every row to 32 floats
-  g.pad_x = g.glo[0] + ((32 - (g.glo[0] + g.mlo[0]) % 32) % 32);
+  // storage of the whole grid; the first physical x cell of every row is
+  // aligned to 32 elements
+  const int pad_x = (32 - m % 32) % 32;
   // (+2: the paired bricks read up to 5 cells past an odd-width gridphy row)
-  const long wx = g.pad_x + g.en[0] + g.ghi[0] + 2;
+  const long wx = pad_x + (gn[0] + 2 * m) + 2;
   g.sy = (wx + 31) / 32 * 32;
-  g.sz = g.sy * (g.glo[1] + g.en[1] + g.ghi[1]);
-  g.nstore = g.sz * (g.glo[2] + g.en[2] + g.ghi[2]);
+  g.sz = g.sy * (gn[1] + 2 * m);
+  g.nstore = g.sz * (gn[2] + 2 * m);
   g.fpitch = g.nstore + kFieldPad;
-  g.origin = g.pad_x + g.sy * g.glo[1] + g.sz * g.glo[2];
+  g.origin = pad_x + g.ext_goff[0] + g.sy * g.ext_goff[1] + g.sz * g.ext_goff[2];
   return true;
+}
+
+// The whole grid as one region: what the stencil kernels sweep.  (pn and en
+// are the global sizes; the subdomains above carry their own.)  Not limited
+// to 2^30 cells: the bricks index cells in 64 bits.
+static Geom whole_grid(const ddx_desc &d, const Geom &any) {
+  Geom g = any;
+  const int gn[3] = {d.nx, d.ny, d.nz};
+  for (int a = 0; a < 3; a++) {
+    g.ci[a] = 0;
+    g.pn[a] = gn[a];
+    g.poff[a] = 0;
+    g.en[a] = gn[a] + 2 * d.pml_num;
+    g.mlo[a] = g.mhi[a] = d.pml_num;
+    g.nlo[a] = g.nhi[a] = -1;
+  }
+  g.origin -= g.ext_goff[0] + g.sy * g.ext_goff[1] + g.sz * g.ext_goff[2];
+  for (int a = 0; a < 3; a++) g.ext_goff[a] = 0;
+  return g;
 }
 
 // Widths of the CMM halo each subdomain receives, per field and side
@@ -165,18 +186,8 @@ static int ring_w(int f, int side, int R) {
 // Store order of the fields in a VOWR slice (elasticWaveRecon::initialize).
 static const int kRingFields[10] = {VX, VY, VZ, SXX, SYY, SZZ, SAU, SXY, SXZ, SYZ};
 
-// GEO/jarvis_device_geometry_bones.hpp:29-49 (cu_cal_diff_coeff).
 static void fd_coef(int half, float *out) {
-  for (int n = 0; n < half; n++) {
-    double a1 = 1, a2 = 1, a3 = 1;
-    for (int i = 0; i < half; i++) {
-      if (i != n) a1 = a1 * (2 * i + 1) * (2 * i + 1);
-      if (i < n) a2 = a2 * ((2 * n + 1) * (2 * n + 1) - (2 * i + 1) * (2 * i + 1));
-      if (i > n) a3 = a3 * ((2 * i + 1) * (2 * i + 1) - (2 * n + 1) * (2 * n + 1));
-    }
-    a1 = a1 * std::pow(-1.0, n);
-    out[n] = (float)(a1 / ((2 * n + 1) * a2 * a3));
-  }
+  for (int n = 0; n < half; n++) out[n] = fd_tap(half, n);
 }
 
 // CPML/fdtd3d_cpml_mpi_1_host_meat.hpp:147-620: damping profile of local
@@ -236,7 +247,6 @@ struct PhyTables {  // physical-region tables of one brick shape and model, per 
 };
 
 struct Slab {
-  int sub;
   int i0, j0, k0, ni, nj, nk, axes;
   int xlo, xhi, ylo, yhi, zlo, zhi;
   long ncell;
@@ -282,9 +292,9 @@ struct ddx_ctx {
   bool set_overlap = false;
   bool ring_oob = false;  // a boundary-store copy asked for a slice outside the store (none launched)
   int nsub = 0;
-  std::vector<Geom> g;
+  std::vector<Geom> g;  // the subdomains (windows of the global arrays)
+  Geom all;             // the whole grid
   int gext[3];
-  float fd[5][4];
   // Brick shape of the physical-region kernels per mode (index = mode),
   // the fastest of a sweep on MI355X for the 2x2x1 256x256x200 RTM shot:
   // deep z columns where the register budget allows, shallower ones for the
@@ -296,7 +306,7 @@ struct ddx_ctx {
   std::vector<void *> allocs;
   std::vector<size_t> alloc_bytes;  // size of each allocation in allocs
   double dev_bytes = 0;
-  std::vector<char *> wave[2];   // per subdomain: NF fields, fpitch elements apart
+  char *wave[2] = {nullptr, nullptr};  // NF fields, fpitch elements apart
   // storage format of wavefields, memory variables and the VOWR store, its
   // element size, and the log2 scales of the field classes (0 velocity,
   // 1 stress) with whether the caller fixed them
@@ -312,31 +322,25 @@ struct ddx_ctx {
   bool rlg_user[2] = {false, false};
   float wmax = 0.f;                  // wavelet peak |w|
   float vp_min = 0.f, rhovp = 0.f;   // model: minimum vp, mean rho * vp
-  // per model (0: modelling, 1: migration) and subdomain: dtr, lam, mu (fpitch apart)
-  std::vector<float *> model[2];
+  // per model (0: modelling, 1: migration): dtr, lam, mu (fpitch apart)
+  float *model[2] = {nullptr, nullptr};
   bool have_mig = false;         // RTM passes use model 1
   bool have_model = false, have_wavelet = false, have_geometry = false;
   float *wavelet = nullptr;
   std::vector<Slab> slabs;
   std::vector<PhyTables> phy_cache;  // physical-region tables per brick shape
+  int brick_group = kBrickGroup;     // XCD group size of the bricks' block order
   int pml_cz = 1;                    // planes per thread of the CPML kernels (1, 2, 4, 8)
   int pml_group = 32;                // XCD group size of the CPML block order (0: launch order)
   int pml_order = 0;                 // 1: the XCD-partitioned CPML block order (PmlOrder); 0: pml_group
   DevTable<SlabDesc> pml[2][2];  // [model][set]
-  // CMM halo links: [set][batch] batch 0 vel, 1 stress, 2 stress + sau
-  DevTable<HaloDesc> halo[2][3];
-  // exchange mode (ddx_set_exchange): 0 a direct copy of every link into the
-  // receiver's ghosts; 1 the CMM message blocks: every sender side packs the
-  // boundary layers of the batch's fields into one contiguous block (fields
-  // in push order), which the receiver unpacks into its ghosts
-  // 2: pack on store -- the kernels that update boundary layers write the
-  // receivers' ghosts themselves (MirrorDesc; needs DDX_MIRROR=1 at
-  // creation, and is then the default); a half step whose physical-region
-  // kernel has no such stores (the one-plane and LDS-tiled kernels) is
-  // followed by the mode-0 copy
+  // exchange mode (ddx_set_exchange): 0 and 2 need no copy, since a
+  // subdomain's ghosts are its neighbours' cells; 1 runs the CMM message
+  // blocks: every sender side packs the boundary layers of the batch's
+  // fields into one contiguous block (fields in push order), which the
+  // receiver unpacks into its ghosts
   int exch_mode = 0;
-  bool have_mirror = false;              // mirror tables exist (DDX_MIRROR=1 at creation)
-  MirrorDesc *d_mir[2] = {nullptr, nullptr};  // [set][subdomain]
+  bool have_mirror = false;  // mode 2 may be selected (DDX_MIRROR=1 at creation, and a neighbour)
   DevTable<CopyDesc> cmm_pack[2][3], cmm_unpack[2][3];  // [set][batch], built on first use of mode 1
   char *cmm_block[2][3] = {};                           // the blocks of a set and batch, link after link
   // snapshots of one field of set 0 during ddx_rtm_shot (gridphy of every
@@ -507,8 +511,12 @@ static int upload_pml_order(ddx_ctx *c, DevTable<SlabDesc> &t, const std::vector
   return DDX_OK;
 }
 
+// Extended cell (0,0,0) of subdomain s, or (fall) of the whole grid.
 static inline void *fptr(ddx_ctx *c, int set, int s, int f) {
-  return c->wave[set][s] + ((long)f * c->g[s].fpitch + c->g[s].origin) * c->esz;
+  return c->wave[set] + ((long)f * c->g[s].fpitch + c->g[s].origin) * c->esz;
+}
+static inline void *fall(ddx_ctx *c, int set, int f) {
+  return c->wave[set] + ((long)f * c->all.fpitch + c->all.origin) * c->esz;
 }
 static float scale_of(const ddx_ctx *c, int cls) { return std::ldexp(1.0f, c->lg[cls]); }
 // class of a field: 0 velocity, 1 stress, -1 FP32-only (FWI accumulators)
@@ -629,6 +637,12 @@ extern "C" int ddx_create(const ddx_desc *desc, ddx_ctx **out) {
       return DDX_EINVAL;
     }
   }
+  c->all = whole_grid(d, c->g[0]);
+  {  // exchange mode 2 is offered, and the default, with DDX_MIRROR=1 and a neighbour
+    const char *e = getenv("DDX_MIRROR");
+    c->have_mirror = c->nsub > 1 && e && atoi(e) == 1;
+    if (c->have_mirror) c->exch_mode = 2;
+  }
   hipError_t he = hipSetDevice(d.device);
   if (he == hipSuccess) he = hipStreamCreateWithFlags(&c->st, hipStreamNonBlocking);
   if (const char *e = getenv("DDX_PML_OVERLAP")) c->pml_overlap = atoi(e) != 0;
@@ -648,11 +662,6 @@ extern "C" int ddx_create(const ddx_desc *desc, ddx_ctx **out) {
     delete c;
     return DDX_EHIP;
   }
-  for (int h = 0; h <= 4; h++) {
-    for (int r = 0; r < 4; r++) c->fd[h][r] = 0.f;
-    if (h > 0) fd_coef(h, c->fd[h]);
-  }
-  set_fd_table(c->fd);
   // CPML work split, for sweeps (FP32 storage): 1, 2, 4, 8 planes per thread
   // with cached taps, or kPmlTiled + 2, 4, 8 (18, 20, 24) for LDS plane tiles
   if (const char *e = getenv("DDX_PML_CZ")) {
@@ -666,10 +675,9 @@ extern "C" int ddx_create(const ddx_desc *desc, ddx_ctx **out) {
   }
   // 1: the XCD-partitioned order (measured: 17% less CPML traffic, 4% slower), for sweeps
   if (const char *e = getenv("DDX_PML_ORDER")) c->pml_order = atoi(e) != 0;
-  {  // XCD group size of the brick blocks (process-wide); DDX_BRICK_GROUP for sweeps
-    const char *e = getenv("DDX_BRICK_GROUP");
-    const int v = e ? atoi(e) : kBrickGroup;
-    set_brick_group(v >= 0 && v <= 65536 ? v : kBrickGroup);
+  if (const char *e = getenv("DDX_BRICK_GROUP")) {  // XCD group size of the brick blocks, for sweeps
+    const int v = atoi(e);
+    if (v >= 0 && v <= 65536) c->brick_group = v;
   }
   if (const char *e = getenv("DDX_TILING")) {  // "TXxTYxCYxKZ[xFORM]", for tile sweeps
     Tiling t{0, 0, 0, 0};
@@ -711,92 +719,32 @@ extern "C" const char *ddx_last_error(const ddx_ctx *c) {
   return c ? c->err.c_str() : g_create_error.c_str();
 }
 
-// The pack-on-store tables (MirrorDesc) of every subdomain of a set: for each
-// side with a neighbour, the neighbour's storage and the widths it takes
-// per field (table H1, the receiver's opposite side).  Built only when
-// DDX_MIRROR=1 at creation: the stores into the neighbours' ghosts sit in
-// the bricks' plane loops, whose loads of the next plane may then not pass
-// them (the compiler cannot rule out aliasing), and the bricks ran 1.6-2x
-// slower than the copy exchange saves (measured on the 256x256x200 RTM
-// shot: velocity 208 -> 341 us, stress 216 -> 421 us per launch).
-static int build_mirrors(ddx_ctx *c) {
-  const char *e = getenv("DDX_MIRROR");
-  bool any_nb = false;
-  for (int s = 0; s < c->nsub; s++)
-    for (int a = 0; a < 3; a++) any_nb |= c->g[s].nlo[a] >= 0 || c->g[s].nhi[a] >= 0;
-  c->have_mirror = any_nb && e && atoi(e) == 1;
-  if (!c->have_mirror) return DDX_OK;
-  for (int set = 0; set < 2; set++) {
-    std::vector<MirrorDesc> h(c->nsub);
-    for (int s = 0; s < c->nsub; s++) {
-      const Geom &g = c->g[s];
-      MirrorDesc &m = h[s];
-      memset(&m, 0, sizeof m);
-      for (int a = 0; a < 3; a++) m.en[a] = g.en[a];
-      for (int side = 0; side < 6; side++) {
-        const int a = kSideAxis[side], hi = kSideHi[side];
-        const int r = hi ? g.nhi[a] : g.nlo[a];
-        if (r < 0) continue;
-        const Geom &gr = c->g[r];
-        MirrorSide &ms = m.s[side];
-        ms.base = (char *)fptr(c, set, r, 0);
-        ms.fpitch = gr.fpitch;
-        ms.sy = gr.sy;
-        ms.sz = gr.sz;
-        ms.shift = hi ? -g.en[a] : gr.en[a];
-        for (int f = 0; f < 10; f++) ms.w[f] = kHaloW[f][side ^ 1];
-      }
-    }
-    if (int rc = dalloc(c, (void **)&c->d_mir[set], sizeof(MirrorDesc) * h.size())) return rc;
-    HIPCHECK(c, hipMemcpyAsync(c->d_mir[set], h.data(), sizeof(MirrorDesc) * h.size(), hipMemcpyHostToDevice, c->st));
-    HIPCHECK(c, hipStreamSynchronize(c->st));
-  }
-  c->exch_mode = 2;
-  return DDX_OK;
-}
-static const MirrorDesc *mirror_of(const ddx_ctx *c, int set, int s) {
-  if (!c->have_mirror) return nullptr;
-  for (int a = 0; a < 3; a++)
-    if (c->g[s].nlo[a] >= 0 || c->g[s].nhi[a] >= 0) return c->d_mir[set] + s;
-  return nullptr;
-}
-
 // Physical-region descriptor tables for one brick shape (one per set); only
 // the first-block indices depend on the shape.  Built once per shape.
 static int build_phy_tables(ddx_ctx *c, const Tiling &t, int model, PhyTables &out) {
   out.t = t;
   out.model = model;
   for (int set = 0; set < 2; set++) {
-    std::vector<PhyDesc> h;
-    std::vector<int> st;
-    int blk = 0;
-    double cells = 0;
-    for (int s = 0; s < c->nsub; s++) {
-      const Geom &g = c->g[s];
-      PhyDesc p;
-      p.dt = c->d.dt;
-      for (int f = 0; f < NF; f++) p.f[f] = fptr(c, set, s, f);
-      p.dtr = c->model[model][s] + g.origin;
-      p.lam = c->model[model][s] + g.fpitch + g.origin;
-      p.mu = c->model[model][s] + 2 * g.fpitch + g.origin;
-      p.sy = g.sy; p.sz = g.sz;
-      p.ox = g.mlo[0]; p.oy = g.mlo[1]; p.oz = g.mlo[2];
-      p.nx = g.pn[0]; p.ny = g.pn[1]; p.nz = g.pn[2];
-      p.gx = g.poff[0]; p.gy = g.poff[1]; p.gz = g.poff[2];
-      p.gnx = c->d.nx; p.gny = c->d.ny; p.gnz = c->d.nz;
-      p.R = c->d.rec_width;
-      p.tiles_x = (g.pn[0] + kTileX - 1) / kTileX;
-      p.tiles_y = (g.pn[1] + kTileY - 1) / kTileY;
-      p.mir = mirror_of(c, set, s);
-      p.blk0 = blk;
-      st.push_back(blk);
-      blk += t.kz > 0 ? tiling_blocks(t, g.pn[0], g.pn[1], g.pn[2]) : p.tiles_x * p.tiles_y * g.pn[2];
-      cells += (double)g.pn[0] * g.pn[1] * g.pn[2];
-      h.push_back(p);
-    }
-    int rc = upload_table(c, out.set[set], h, st, blk);
+    const Geom &g = c->all;
+    PhyDesc p;
+    p.dt = c->d.dt;
+    for (int f = 0; f < NF; f++) p.f[f] = fall(c, set, f);
+    p.dtr = c->model[model] + g.origin;
+    p.lam = c->model[model] + g.fpitch + g.origin;
+    p.mu = c->model[model] + 2 * g.fpitch + g.origin;
+    p.sy = g.sy; p.sz = g.sz;
+    p.ox = g.mlo[0]; p.oy = g.mlo[1]; p.oz = g.mlo[2];
+    p.nx = g.pn[0]; p.ny = g.pn[1]; p.nz = g.pn[2];
+    p.R = c->d.rec_width;
+    p.tiles_x = (g.pn[0] + kTileX - 1) / kTileX;
+    p.tiles_y = (g.pn[1] + kTileY - 1) / kTileY;
+    p.blk0 = 0;
+    std::vector<PhyDesc> h(1, p);
+    const int blk =
+        t.kz > 0 ? tiling_blocks(t, g.pn[0], g.pn[1], g.pn[2]) : p.tiles_x * p.tiles_y * g.pn[2];
+    int rc = upload_table(c, out.set[set], h, std::vector<int>(1, 0), blk);
     if (rc) return rc;
-    out.set[set].cells = cells;
+    out.set[set].cells = (double)g.pn[0] * g.pn[1] * g.pn[2];
   }
   return DDX_OK;
 }
@@ -835,73 +783,18 @@ static int prepare_phy_tables(ddx_ctx *c, int model) {
 static int model_for(const ddx_ctx *c, int mode) { return (rtm_mode(mode) && c->have_mig) ? 1 : 0; }
 
 // Descriptor tables that do not depend on the model: wavefield storage,
-// physical-region tiles, CMM halo links, VOWR rings, imaging.
+// physical-region tiles, VOWR rings, imaging.
 static int build_tables(ddx_ctx *c) {
   int rc;
   const int S = c->nsub;
   for (int set = 0; set < 2; set++) {
-    c->wave[set].resize(S);
-    for (int s = 0; s < S; s++) {
-      rc = dalloc(c, (void **)&c->wave[set][s], (size_t)c->esz * NF * c->g[s].fpitch);
-      if (rc) return rc;
-    }
-  }
-  c->model[0].resize(S);
-  for (int s = 0; s < S; s++) {
-    rc = dalloc(c, (void **)&c->model[0][s], sizeof(float) * 3 * c->g[s].fpitch);
+    rc = dalloc(c, (void **)&c->wave[set], (size_t)c->esz * NF * c->all.fpitch);
     if (rc) return rc;
   }
-  if ((rc = build_mirrors(c))) return rc;
+  rc = dalloc(c, (void **)&c->model[0], sizeof(float) * 3 * c->all.fpitch);
+  if (rc) return rc;
   rc = prepare_phy_tables(c, 0);
   if (rc) return rc;
-  // CMM halo links: for every receiver subdomain and side with a neighbour,
-  // the neighbour's boundary layers of each field of the batch, in the
-  // reference's push order (vx, vy, vz | sxx, syy, szz, sxy, sxz, syz, sau).
-  static const int kBatch[3][8] = {{VX, VY, VZ, -1}, {SXX, SYY, SZZ, SXY, SXZ, SYZ, -1},
-                                   {SXX, SYY, SZZ, SXY, SXZ, SYZ, SAU, -1}};
-  for (int batch = 0; batch < 3; batch++) {
-    for (int set = 0; set < 2; set++) {
-      std::vector<HaloDesc> hh;
-      std::vector<int> st;
-      int blk = 0;
-      long cnt_all = 0;
-      for (int r = 0; r < S; r++) {
-        const Geom &gr = c->g[r];
-        for (int side = 0; side < 6; side++) {
-          const int a = kSideAxis[side], hi = kSideHi[side];
-          const int nb = hi ? gr.nhi[a] : gr.nlo[a];
-          if (nb < 0) continue;
-          const Geom &gs = c->g[nb];
-          for (int q = 0; kBatch[batch][q] >= 0; q++) {
-            const int f = kBatch[batch][q];
-            const int w = kHaloW[f][side];
-            if (w <= 0) continue;
-            int lo_r[3] = {0, 0, 0}, lo_s[3] = {0, 0, 0}, n[3] = {gr.en[0], gr.en[1], gr.en[2]};
-            n[a] = w;
-            if (hi) { lo_r[a] = gr.en[a]; lo_s[a] = 0; }
-            else { lo_r[a] = -w; lo_s[a] = gs.en[a] - w; }
-            HaloDesc h;
-            h.src = fptr(c, set, nb, f);
-            h.ssy = gs.sy; h.ssz = gs.sz;
-            h.si = lo_s[0]; h.sj = lo_s[1]; h.sk = lo_s[2];
-            h.dst = fptr(c, set, r, f);
-            h.dsy = gr.sy; h.dsz = gr.sz;
-            h.di = lo_r[0]; h.dj = lo_r[1]; h.dk = lo_r[2];
-            h.ni = n[0]; h.nj = n[1]; h.nk = n[2];
-            h.blk0 = blk;
-            st.push_back(blk);
-            const long cnt = (long)n[0] * n[1] * n[2];
-            blk += halo_blocks(n[0], n[1], n[2]);
-            cnt_all += cnt;
-            hh.push_back(h);
-          }
-        }
-      }
-      rc = upload_table(c, c->halo[set][batch], hh, st, blk);
-      if (rc) return rc;
-      c->halo[set][batch].bytes = 2.0 * c->esz * cnt_all;  // one read and one write per element
-    }
-  }
   // VOWR rings on the global sides of each subdomain's gridphy
   // (OP/jarvis_1_mpicu_halo_store_operator_meat.hpp:122-135, stored only on
   // sides without a neighbour, :137-217).
@@ -929,8 +822,6 @@ static int build_tables(ddx_ctx *c) {
           p.i0 = lo[0]; p.j0 = lo[1]; p.k0 = lo[2];
           p.ni = n[0]; p.nj = n[1]; p.nk = n[2];
           p.buf_off = off;
-          p.bi = p.bj = p.bk = 0;
-          p.bni = p.ni; p.bnj = p.nj;
           p.cls = f <= VZ ? 0 : 1;
           p.fid = fi;
           long cnt = (long)n[0] * n[1] * n[2];
@@ -941,35 +832,6 @@ static int build_tables(ddx_ctx *c) {
             blk[t] += (int)((cnt + kBlock - 1) / kBlock);
             h[t].push_back(p);
           }
-          // pack on store: the injection also writes the part of the ring
-          // box that lies in a send band of another axis into that
-          // receiver's ghost layers
-          for (int side2 = 0; c->have_mirror && side2 < 6; side2++) {
-            const int a2 = kSideAxis[side2], hi2 = kSideHi[side2];
-            const int r = hi2 ? g.nhi[a2] : g.nlo[a2];
-            const int w2 = kHaloW[f][side2 ^ 1];
-            if (r < 0 || a2 == a || w2 <= 0) continue;
-            const int b0 = hi2 ? g.en[a2] - w2 : 0, b1 = hi2 ? g.en[a2] : w2;
-            const int c0 = std::max(lo[a2], b0), c1 = std::min(lo[a2] + n[a2], b1);
-            if (c1 <= c0) continue;
-            const Geom &gr = c->g[r];
-            CopyDesc m = p;
-            int mlo[3] = {lo[0], lo[1], lo[2]}, mn[3] = {n[0], n[1], n[2]}, sub[3] = {0, 0, 0};
-            mlo[a2] = c0;
-            mn[a2] = c1 - c0;
-            sub[a2] = c0 - lo[a2];
-            mlo[a2] += hi2 ? -g.en[a2] : gr.en[a2];
-            m.field = fptr(c, 0, r, f);
-            m.sy = gr.sy; m.sz = gr.sz;
-            m.i0 = mlo[0]; m.j0 = mlo[1]; m.k0 = mlo[2];
-            m.ni = mn[0]; m.nj = mn[1]; m.nk = mn[2];
-            m.bi = sub[0]; m.bj = sub[1]; m.bk = sub[2];
-            m.bni = n[0]; m.bnj = n[1];
-            m.blk0 = blk[which];
-            st[which].push_back(blk[which]);
-            blk[which] += (int)(((long)mn[0] * mn[1] * mn[2] + kBlock - 1) / kBlock);
-            h[which].push_back(m);
-          }
           // a block floating point store starts every box on a run
           off += c->ring_fmt == STORE_BFP16 ? (cnt + kRingBlock - 1) / kRingBlock * kRingBlock : cnt;
         }
@@ -977,14 +839,6 @@ static int build_tables(ddx_ctx *c) {
     }
     c->ring_slice = off;
     c->ring_runs = (off + kRingBlock - 1) / kRingBlock;
-    // the block-scaled save takes a run as kRingBlock consecutive lanes: its
-    // table must hold whole boxes starting on runs
-    if (c->ring_fmt == STORE_BFP16)
-      for (const CopyDesc &p : h[0])
-        if (p.buf_off % kRingBlock || p.bi || p.bj || p.bk || p.bni != p.ni || p.bnj != p.nj) {
-          c->err = "internal: a VOWR save box is not a whole box on a run";
-          return DDX_EINVAL;
-        }
     for (int t = 0; t < 3; t++) {
       rc = upload_table(c, c->ring[t], h[t], st[t], blk[t]);
       if (rc) return rc;
@@ -1122,15 +976,14 @@ static int load_model(ddx_ctx *c, int which, const float *vp, const float *vs, c
   // free old slab storage is kept (slabs are rebuilt only once)
   const bool first = c->slabs.empty();
   bool too_big = false;
-  for (int s = 0; s < c->nsub; s++) {
-    const Geom &g = c->g[s];
+  {
+    const Geom &g = c->all;
     std::vector<float> host((size_t)3 * g.fpitch, 0.f);
     std::vector<float> evp((size_t)g.en[0] * g.en[1] * g.en[2]);
     parallel_for(g.en[2], [&](int k) {
       for (int j = 0; j < g.en[1]; j++)
         for (int i = 0; i < g.en[0]; i++) {
-          const long gi = i + g.ext_goff[0], gj = j + g.ext_goff[1], gk = k + g.ext_goff[2];
-          const float p = phy_at(vp, gi, gj, gk), q = phy_at(vs, gi, gj, gk), r = phy_at(rho, gi, gj, gk);
+          const float p = phy_at(vp, i, j, k), q = phy_at(vs, i, j, k), r = phy_at(rho, i, j, k);
           const long o = g.origin + i + g.sy * j + g.sz * k;
           host[o] = d.dt / r;                                   // dt / rho
           host[g.fpitch + o] = r * (p * p - 2.0f * q * q);      // lambda
@@ -1138,37 +991,37 @@ static int load_model(ddx_ctx *c, int which, const float *vp, const float *vs, c
           evp[(size_t)i + (size_t)g.en[0] * ((size_t)j + (size_t)g.en[1] * k)] = p;
         }
     });
-    HIPCHECK(c, hipMemcpyAsync(c->model[which][s], host.data(), sizeof(float) * host.size(), hipMemcpyHostToDevice,
+    HIPCHECK(c, hipMemcpyAsync(c->model[which], host.data(), sizeof(float) * host.size(), hipMemcpyHostToDevice,
                                c->st));
     HIPCHECK(c, hipStreamSynchronize(c->st));
     // CPML slabs (BASE/fdtd3d_base_6_pml_meat.hpp:29-93; sub_pad :213-223)
     if (first) {
       auto add = [&](int i0, int i1, int j0, int j1, int k0, int k1, int axes) {
-        if (i1 <= i0 || j1 <= j0 || k1 <= k0) return;
+        // the CPML kernels index a slab in 32 bits: larger ones are cut along z
+        const long plane = (long)(i1 - i0) * (j1 - j0), most = INT_MAX - kBlock;
+        if (plane > most) { too_big = true; return; }
+        const int step = (int)std::min<long>(k1 - k0, most / plane);
+        for (int kb = k0; kb < k1; kb += step) {
         Slab sl;
-        sl.sub = s;
-        sl.i0 = i0; sl.j0 = j0; sl.k0 = k0;
-        sl.ni = i1 - i0; sl.nj = j1 - j0; sl.nk = k1 - k0;
+        sl.i0 = i0; sl.j0 = j0; sl.k0 = kb;
+        sl.ni = i1 - i0; sl.nj = j1 - j0; sl.nk = std::min(step, k1 - kb);
         sl.axes = axes;
-        sl.xlo = g.mlo[0] > 0 ? g.mlo[0] : INT_MIN;
-        sl.xhi = g.mhi[0] > 0 ? g.en[0] - g.mhi[0] : INT_MAX;
-        sl.ylo = g.mlo[1] > 0 ? g.mlo[1] : INT_MIN;
-        sl.yhi = g.mhi[1] > 0 ? g.en[1] - g.mhi[1] : INT_MAX;
-        sl.zlo = g.mlo[2] > 0 ? g.mlo[2] : INT_MIN;
-        sl.zhi = g.mhi[2] > 0 ? g.en[2] - g.mhi[2] : INT_MAX;
-        sl.ncell = (long)sl.ni * sl.nj * sl.nk;
-        if (sl.ncell > INT_MAX - kBlock) too_big = true;  // the CPML kernels index slabs in 32 bits
+        sl.xlo = g.mlo[0]; sl.xhi = g.en[0] - g.mhi[0];
+        sl.ylo = g.mlo[1]; sl.yhi = g.en[1] - g.mhi[1];
+        sl.zlo = g.mlo[2]; sl.zhi = g.en[2] - g.mhi[2];
+        sl.ncell = plane * sl.nk;
         c->slabs.push_back(sl);
+        }
       };
       for_each_slab(g, add);
       if (too_big) {
-        c->err = "a CPML slab holds more than 2^31 cells";
+        c->slabs.clear();
+        c->err = "a CPML slab plane holds more than 2^31 cells";
         return DDX_EINVAL;
       }
     }
-    // coefficients of this subdomain's slabs
+    // coefficients of the slabs
     for (auto &sl : c->slabs) {
-      if (sl.sub != s) continue;
       const int naxes = __builtin_popcount(sl.axes);
       if (!sl.coef[which]) {
         int rc = dalloc(c, (void **)&sl.coef[which], sizeof(float) * 4 * naxes * sl.ncell);
@@ -1219,19 +1072,18 @@ static int load_model(ddx_ctx *c, int which, const float *vp, const float *vs, c
       int blk = 0;
       double cells = 0, psi_cells = 0;
       for (auto &sl : c->slabs) {
-        const Geom &g = c->g[sl.sub];
+        const Geom &g = c->all;
         SlabDesc p;
-        for (int f = 0; f < NF; f++) p.f[f] = fptr(c, set, sl.sub, f);
-        p.dtr = c->model[which][sl.sub] + g.origin;
-        p.lam = c->model[which][sl.sub] + g.fpitch + g.origin;
-        p.mu = c->model[which][sl.sub] + 2 * g.fpitch + g.origin;
+        for (int f = 0; f < NF; f++) p.f[f] = fall(c, set, f);
+        p.dtr = c->model[which] + g.origin;
+        p.lam = c->model[which] + g.fpitch + g.origin;
+        p.mu = c->model[which] + 2 * g.fpitch + g.origin;
         p.sy = g.sy; p.sz = g.sz;
         p.i0 = sl.i0; p.j0 = sl.j0; p.k0 = sl.k0; p.ni = sl.ni; p.nj = sl.nj; p.nk = sl.nk;
         p.axes = sl.axes;
         p.xlo = sl.xlo; p.xhi = sl.xhi; p.ylo = sl.ylo; p.yhi = sl.yhi; p.zlo = sl.zlo; p.zhi = sl.zhi;
         p.psi = sl.psi[set];
         p.coef = sl.coef[which];
-        p.mir = mirror_of(c, set, sl.sub);
         p.blk0 = blk;
         st.push_back(blk);
         blk += pml_blocks(sl.ni, sl.nj, sl.nk, c->pml_cz);
@@ -1345,13 +1197,8 @@ extern "C" int ddx_set_migration_model(ddx_ctx *c, const float *vp, const float 
     return DDX_ESTATE;
   }
   HIPCHECK(c, hipStreamSynchronize(c->st));
-  if (c->model[1].empty()) {
-    c->model[1].resize(c->nsub);
-    for (int s = 0; s < c->nsub; s++) {
-      int rc = dalloc(c, (void **)&c->model[1][s], sizeof(float) * 3 * c->g[s].fpitch);
-      if (rc) return rc;
-    }
-  }
+  if (!c->model[1])
+    if (int rc = dalloc(c, (void **)&c->model[1], sizeof(float) * 3 * c->all.fpitch)) return rc;
   int rc = load_model(c, 1, vp, vs, rho);
   if (rc) return rc;
   rc = prepare_phy_tables(c, 1);
@@ -1488,7 +1335,6 @@ static int build_cmm(ddx_ctx *c) {
             else { lo_s[a] = 0; lo_r[a] = gr.en[a]; }
             CopyDesc p{};
             p.ni = n[0]; p.nj = n[1]; p.nk = n[2];
-            p.bni = n[0]; p.bnj = n[1];
             p.buf_off = off;
             p.cls = f <= VZ ? 0 : 1;
             p.fid = 0;
@@ -1518,40 +1364,22 @@ static int build_cmm(ddx_ctx *c) {
   return DDX_OK;
 }
 
-// The CMM exchange of one batch of one set on stream st (exchange mode 0:
-// one direct copy per link; 1: pack into the message blocks, then unpack).
+// The CMM exchange of one batch of one set on stream st.  Nothing to move in
+// modes 0 and 2: a subdomain's ghosts are its neighbours' cells.  Mode 1
+// packs every boundary layer into the message blocks and unpacks them into
+// the ghosts (the cells they came from: the values do not change).
 static void exchange_on(ddx_ctx *c, int set, int batch, hipStream_t st) {
-  if (c->exch_mode == 1) {
-    const DevTable<CopyDesc> &p = c->cmm_pack[set][batch], &u = c->cmm_unpack[set][batch];
-    if (p.nblk == 0) return;
-    ProfScope ps(c, 4, p.bytes + u.bytes, st);
-    launch_copy(+1, c->esz, p.d, p.starts, p.n, p.nblk, c->cmm_block[set][batch], st);
-    launch_copy(-1, c->esz, u.d, u.starts, u.n, u.nblk, c->cmm_block[set][batch], st);
-    return;
-  }
-  const DevTable<HaloDesc> &h = c->halo[set][batch];
-  if (h.nblk == 0) return;
-  ProfScope ps(c, 4, h.bytes, st);
-  launch_halo(c->esz, h.d, h.starts, h.n, h.nblk, st);
+  if (c->exch_mode != 1) return;
+  const DevTable<CopyDesc> &p = c->cmm_pack[set][batch], &u = c->cmm_unpack[set][batch];
+  if (p.nblk == 0) return;
+  ProfScope ps(c, 4, p.bytes + u.bytes, st);
+  launch_copy(+1, c->esz, p.d, p.starts, p.n, p.nblk, c->cmm_block[set][batch], st);
+  launch_copy(-1, c->esz, u.d, u.starts, u.n, u.nblk, c->cmm_block[set][batch], st);
 }
 
 static int exchange(ddx_ctx *c, int set, int batch) {
   exchange_on(c, set, batch, c->st);
   return DDX_OK;
-}
-
-// Whether a half step whose physical-region kernel ran with brick shape t
-// has written the receivers' ghosts itself (pack on store): exchange mode
-// 2 and a z-blocked brick (the one-plane kernels, kz = 0, and the LDS-tiled
-// kernels, cy = 0, have no such stores).  The CPML kernels and the VOWR
-// injection always store into the ghosts when the mirror tables exist.
-static bool packed_on_store(const ddx_ctx *c, const Tiling &t) {
-  return c->exch_mode == 2 && c->have_mirror && t.kz > 0 && t.cy > 0;
-}
-// The exchange that follows a half step of brick shape t: nothing after a
-// packed store, else the copy of mode 0 or 1.
-static void exchange_after(ddx_ctx *c, int set, int batch, const Tiling &t, hipStream_t st) {
-  if (!packed_on_store(c, t)) exchange_on(c, set, batch, st);
 }
 
 // Algorithmic bytes per gridphy cell.  Velocity: 6 stress reads + 3 RMW of
@@ -1589,12 +1417,12 @@ static int phy_launch(ddx_ctx *c, int kernel, int set, int mode, const Tiling &t
     const float sign = mode == RTM_BACKWARD ? -1.f : 1.f;
     ProfScope ps(c, 0, phy_vel_bytes(c, mode) * ph.cells);
     launched = launch_vel_phy(t, mode, c->fmt, ph.d, ph.starts, ph.n, ph.nblk, c->d.dx, c->d.dy, c->d.dz,
-                              sign * ratio_vs(c), c->d.nx, c->d.ny, c->d.nz, c->d.rec_width, c->st);
+                              sign * ratio_vs(c), c->brick_group, c->st);
   } else {
     const float dt = mode == RTM_BACKWARD ? -c->d.dt : c->d.dt;
     ProfScope ps(c, 1, phy_stress_bytes(c, mode) * ph.cells);
     launched = launch_stress_phy(t, mode, c->fmt, ph.d, ph.starts, ph.n, ph.nblk, c->d.dx, c->d.dy, c->d.dz,
-                                 dt * ratio_sv(c), c->d.nx, c->d.ny, c->d.nz, c->d.rec_width, c->st);
+                                 dt * ratio_sv(c), c->brick_group, c->st);
   }
   if (!launched) {
     c->err = "no physical-region kernel for this brick shape, storage format and mode";
@@ -1662,14 +1490,14 @@ static int stress_update(ddx_ctx *c, int set, int mode) {
 static int vel_half(ddx_ctx *c, int set, int mode) {
   int rc = vel_update(c, set, mode);
   if (rc) return rc;
-  exchange_after(c, set, 0, c->tiling_vel[mode], c->st);
+  exchange_on(c, set, 0, c->st);
   return DDX_OK;
 }
 static int stress_half(ddx_ctx *c, int set, int mode) {
   int rc = stress_update(c, set, mode);
   if (rc) return rc;
   const bool sau = mode == RTM_BACKWARD || mode == RTM_REVERSE;
-  exchange_after(c, set, sau ? 2 : 1, c->tiling_stress[mode], c->st);
+  exchange_on(c, set, sau ? 2 : 1, c->st);
   return DDX_OK;
 }
 extern "C" int ddx_step_vel(ddx_ctx *c, int set, int mode) { return vel_half(c, set, mode); }
@@ -1732,8 +1560,7 @@ extern "C" int ddx_source(ddx_ctx *c, int set, int ishot, int it, int sign) {
 
 extern "C" int ddx_reset_wave(ddx_ctx *c, int set) {
   if (!c || set < 0 || set > 1) return DDX_EINVAL;
-  for (int s = 0; s < c->nsub; s++)
-    HIPCHECK(c, hipMemsetAsync(c->wave[set][s], 0, (size_t)c->esz * NF * c->g[s].fpitch, c->st));
+  HIPCHECK(c, hipMemsetAsync(c->wave[set], 0, (size_t)c->esz * NF * c->all.fpitch, c->st));
   for (auto &sl : c->slabs)
     if (sl.psi[set])
       HIPCHECK(c, hipMemsetAsync(sl.psi[set], 0, (size_t)c->esz * 6 * __builtin_popcount(sl.axes) * sl.ncell, c->st));
@@ -1947,14 +1774,14 @@ struct BatchMember {
 
 // What members of one fused launch must share.
 struct BatchKey {
-  int device = 0, fmt = 0, lg0 = 0, lg1 = 0, pml_cz = 1, pml_group = 0, pml_order = 1;
+  int device = 0, fmt = 0, lg0 = 0, lg1 = 0, pml_cz = 1, pml_group = 0, pml_order = 1, brick_group = 0;
   float dt = 0.f, dx = 0.f, dy = 0.f, dz = 0.f;
   Tiling tv{0, 0, 0, 0}, ts{0, 0, 0, 0};
 };
 static BatchKey batch_key(const ddx_ctx *c) {
   BatchKey k;
   k.device = c->d.device; k.fmt = c->fmt; k.lg0 = c->lg[0]; k.lg1 = c->lg[1];
-  k.pml_cz = c->pml_cz; k.pml_group = c->pml_group; k.pml_order = c->pml_order;
+  k.pml_cz = c->pml_cz; k.pml_group = c->pml_group; k.pml_order = c->pml_order; k.brick_group = c->brick_group;
   k.dt = c->d.dt; k.dx = c->d.dx; k.dy = c->d.dy; k.dz = c->d.dz;
   k.tv = c->tiling_vel[PURE_FORWARD];
   k.ts = c->tiling_stress[PURE_FORWARD];
@@ -2069,29 +1896,22 @@ static hipError_t fuse_members(const std::vector<BatchMember> &ms, FusedSet &f) 
   return e;
 }
 
-// the exchange of a batch member after a fused half step of brick shape t
-static void halo_on(ddx_ctx *c, int set, int batch, const Tiling &t, hipStream_t st) {
-  exchange_after(c, set, batch, t, st);
-}
-
 // One modelling time step of every member (each at its own time index, the
 // batch step gs minus its join step), in the order of model_step.
 static bool fused_step(const BatchKey &k, const FusedSet &f, const std::vector<BatchMember> &ms, int gs,
                        hipStream_t st, const int *gsp = nullptr) {
   const float rvs = std::ldexp(1.0f, k.lg0 - k.lg1), rsv = std::ldexp(1.0f, k.lg1 - k.lg0);
-  if (!launch_vel_phy(k.tv, PURE_FORWARD, k.fmt, f.v.d, f.v.starts, f.v.n, f.v.nblk, k.dx, k.dy, k.dz, rvs, 0, 0, 0,
-                      0, st))
+  if (!launch_vel_phy(k.tv, PURE_FORWARD, k.fmt, f.v.d, f.v.starts, f.v.n, f.v.nblk, k.dx, k.dy, k.dz, rvs, k.brick_group, st))
     return false;
   launch_vel_pml(k.pml_cz, k.fmt, f.p.d, f.p.starts, f.p.n, f.p.nblk, k.dx, k.dy, k.dz, rvs, k.pml_group,
                  k.pml_order ? &f.p.ord : nullptr, st);
-  for (const BatchMember &m : ms) halo_on(m.c, 0, 0, k.tv, st);
+  for (const BatchMember &m : ms) exchange_on(m.c, 0, 0, st);
   launch_source_batch(k.fmt, f.io.d, f.io.n, gs, gsp, st);
-  if (!launch_stress_phy(k.ts, PURE_FORWARD, k.fmt, f.s.d, f.s.starts, f.s.n, f.s.nblk, k.dx, k.dy, k.dz, k.dt * rsv,
-                         0, 0, 0, 0, st))
+  if (!launch_stress_phy(k.ts, PURE_FORWARD, k.fmt, f.s.d, f.s.starts, f.s.n, f.s.nblk, k.dx, k.dy, k.dz, k.dt * rsv, k.brick_group, st))
     return false;
   launch_stress_pml(k.pml_cz, 0, k.fmt, f.p.d, f.p.starts, f.p.n, f.p.nblk, k.dx, k.dy, k.dz, k.dt * rsv,
                     k.pml_group, k.pml_order ? &f.p.ord : nullptr, st);
-  for (const BatchMember &m : ms) halo_on(m.c, 0, 1, k.ts, st);
+  for (const BatchMember &m : ms) exchange_on(m.c, 0, 1, st);
   launch_recv_batch(k.fmt, f.io.d, f.io.starts, f.io.n, f.io.nblk, gs, gsp, st);
   return true;
 }
@@ -2408,19 +2228,18 @@ static bool rtm_fused_forward(const BatchKey &k, const ddx_ctx *c0, const RtmTab
                               const std::vector<ddx_ctx *> &cs, const std::vector<int> &its, int gs, hipStream_t st) {
   const int F = RTM_FORWARD;
   const float rvs = std::ldexp(1.0f, k.lg0 - k.lg1), rsv = std::ldexp(1.0f, k.lg1 - k.lg0);
-  if (!launch_vel_phy(c0->tiling_vel[F], F, k.fmt, T.fv.d, T.fv.starts, T.fv.n, T.fv.nblk, k.dx, k.dy, k.dz, rvs, 0,
-                      0, 0, 0, st))
+  if (!launch_vel_phy(c0->tiling_vel[F], F, k.fmt, T.fv.d, T.fv.starts, T.fv.n, T.fv.nblk, k.dx, k.dy, k.dz, rvs, k.brick_group, st))
     return false;
   launch_vel_pml(k.pml_cz, k.fmt, T.fp.d, T.fp.starts, T.fp.n, T.fp.nblk, k.dx, k.dy, k.dz, rvs, k.pml_group,
                  k.pml_order ? &T.fp.ord : nullptr, st);
-  for (ddx_ctx *c : cs) halo_on(c, 0, 0, c0->tiling_vel[F], st);
+  for (ddx_ctx *c : cs) exchange_on(c, 0, 0, st);
   launch_source_batch(k.fmt, T.src.d, T.src.n, gs, nullptr, st, 1.f);
   if (!launch_stress_phy(c0->tiling_stress[F], F, k.fmt, T.fs.d, T.fs.starts, T.fs.n, T.fs.nblk, k.dx, k.dy, k.dz,
-                         k.dt * rsv, 0, 0, 0, 0, st))
+                         k.dt * rsv, k.brick_group, st))
     return false;
   launch_stress_pml(k.pml_cz, 1, k.fmt, T.fp.d, T.fp.starts, T.fp.n, T.fp.nblk, k.dx, k.dy, k.dz, k.dt * rsv,
                     k.pml_group, k.pml_order ? &T.fp.ord : nullptr, st);
-  for (ddx_ctx *c : cs) halo_on(c, 0, 1, c0->tiling_stress[F], st);
+  for (ddx_ctx *c : cs) exchange_on(c, 0, 1, st);
   // each member saves slices 0 .. its own ntime - 2 (members of a
   // continuous batch may differ in ntime)
   for (size_t q = 0; q < cs.size(); q++)
@@ -2436,31 +2255,29 @@ static bool rtm_fused_reverse(const BatchKey &k, const ddx_ctx *c0, const RtmTab
   const float rvs = std::ldexp(1.0f, k.lg0 - k.lg1), rsv = std::ldexp(1.0f, k.lg1 - k.lg0);
   const float dx = k.dx, dy = k.dy, dz = k.dz, dt = k.dt;
   auto vel = [&](const FusedTable<PhyDesc> &t, int mode, float sign) {
-    return launch_vel_phy(c0->tiling_vel[mode], mode, k.fmt, t.d, t.starts, t.n, t.nblk, dx, dy, dz, sign * rvs, 0,
-                          0, 0, 0, st);
+    return launch_vel_phy(c0->tiling_vel[mode], mode, k.fmt, t.d, t.starts, t.n, t.nblk, dx, dy, dz, sign * rvs, k.brick_group, st);
   };
   auto stress = [&](const FusedTable<PhyDesc> &t, int mode, float d) {
-    return launch_stress_phy(c0->tiling_stress[mode], mode, k.fmt, t.d, t.starts, t.n, t.nblk, dx, dy, dz, d * rsv,
-                             0, 0, 0, 0, st);
+    return launch_stress_phy(c0->tiling_stress[mode], mode, k.fmt, t.d, t.starts, t.n, t.nblk, dx, dy, dz, d * rsv, k.brick_group, st);
   };
   launch_source_batch(k.fmt, T.src.d, T.src.n, gs, nullptr, st, -1.f);
   launch_inject_batch(k.fmt, T.inj.d, T.inj.starts, T.inj.n, T.inj.nblk, gs, st);
   if (!stress(T.bs, B, -dt)) return false;
   for (size_t q = 0; q < cs.size(); q++)
     if (its[q] >= 1) ring(cs[q], -1, 2, its[q] - 1, st);
-  for (ddx_ctx *c : cs) halo_on(c, 0, 2, c0->tiling_stress[B], st);
+  for (ddx_ctx *c : cs) exchange_on(c, 0, 2, st);
   if (!vel(T.rv, R, 1.f)) return false;
   launch_vel_pml(k.pml_cz, k.fmt, T.rp.d, T.rp.starts, T.rp.n, T.rp.nblk, dx, dy, dz, rvs, k.pml_group,
                  k.pml_order ? &T.rp.ord : nullptr, st);
-  for (ddx_ctx *c : cs) halo_on(c, 1, 0, c0->tiling_vel[R], st);
+  for (ddx_ctx *c : cs) exchange_on(c, 1, 0, st);
   if (!vel(T.bv, B, -1.f)) return false;
   for (size_t q = 0; q < cs.size(); q++)
     if (its[q] >= 1) ring(cs[q], -1, 1, its[q] - 1, st);
-  for (ddx_ctx *c : cs) halo_on(c, 0, 0, c0->tiling_vel[B], st);
+  for (ddx_ctx *c : cs) exchange_on(c, 0, 0, st);
   if (!stress(T.rs, R, dt)) return false;
   launch_stress_pml(k.pml_cz, 1, k.fmt, T.rp.d, T.rp.starts, T.rp.n, T.rp.nblk, dx, dy, dz, dt * rsv, k.pml_group,
                     k.pml_order ? &T.rp.ord : nullptr, st);
-  for (ddx_ctx *c : cs) halo_on(c, 1, 2, c0->tiling_stress[R], st);
+  for (ddx_ctx *c : cs) exchange_on(c, 1, 2, st);
   launch_image(c0->d.image_fp64, k.fmt, T.img.d, T.img.starts, T.img.n, T.img.nblk, 1.0f / std::ldexp(1.0f, k.lg0),
                st);
   return true;
@@ -2985,8 +2802,6 @@ extern "C" int ddx_set_snapshots(ddx_ctx *c, int field, int every) {
       p.i0 = g.mlo[0]; p.j0 = g.mlo[1]; p.k0 = g.mlo[2];
       p.ni = g.pn[0]; p.nj = g.pn[1]; p.nk = g.pn[2];
       p.buf_off = off;
-      p.bi = p.bj = p.bk = 0;
-      p.bni = p.ni; p.bnj = p.nj;
       p.cls = field <= VZ ? 0 : 1;
       p.fid = 0;
       p.blk0 = blk;
@@ -3073,10 +2888,10 @@ static int rtm_reverse_step(ddx_ctx *c, int ishot, int it) {
     if ((rc = ddx_source(c, 0, ishot, it, -1))) return rc;
     if ((rc = stress_update(c, 0, RTM_BACKWARD))) return rc;
     if (it - 1 >= 0) ring(c, -1, 2, it - 1);
-    exchange_after(c, 0, 2, c->tiling_stress[RTM_BACKWARD], c->st);
+    exchange_on(c, 0, 2, c->st);
     if ((rc = vel_update(c, 0, RTM_BACKWARD))) return rc;
     if (it - 1 >= 0) ring(c, -1, 1, it - 1);
-    exchange_after(c, 0, 0, c->tiling_vel[RTM_BACKWARD], c->st);
+    exchange_on(c, 0, 0, c->st);
     HIPCHECK(c, hipStreamWaitEvent(main_st, c->ev_rev_join, 0));
   } else {
     if ((rc = ddx_source(c, 0, ishot, it, -1))) return rc;
@@ -3085,11 +2900,11 @@ static int rtm_reverse_step(ddx_ctx *c, int ishot, int it) {
     // backward stress, ring inject of step it-1, then the halo exchange
     if ((rc = stress_update(c, 0, RTM_BACKWARD))) return rc;
     if (it - 1 >= 0) ring(c, -1, 2, it - 1);
-    exchange_after(c, 0, 2, c->tiling_stress[RTM_BACKWARD], c->st);
+    exchange_on(c, 0, 2, c->st);
     if ((rc = vel_half(c, 1, RTM_REVERSE))) return rc;
     if ((rc = vel_update(c, 0, RTM_BACKWARD))) return rc;
     if (it - 1 >= 0) ring(c, -1, 1, it - 1);
-    exchange_after(c, 0, 0, c->tiling_vel[RTM_BACKWARD], c->st);
+    exchange_on(c, 0, 0, c->st);
     if ((rc = stress_half(c, 1, RTM_REVERSE))) return rc;
   }
   {
@@ -3191,10 +3006,8 @@ extern "C" int ddx_check_finite(ddx_ctx *c, int *finite) {
   if (!c || !finite) return DDX_EINVAL;
   HIPCHECK(c, hipMemsetAsync(c->d_flag, 0, sizeof(int), c->st));
   for (int set = 0; set < 2; set++)
-    for (int s = 0; s < c->nsub; s++)
-      for (int f = VX; f <= VZ; f++)
-        launch_nonfinite(c->fmt, c->wave[set][s] + (long)f * c->g[s].fpitch * c->esz, c->g[s].nstore, c->d_flag,
-                         c->st);
+    for (int f = VX; f <= VZ; f++)
+      launch_nonfinite(c->fmt, c->wave[set] + (long)f * c->all.fpitch * c->esz, c->all.nstore, c->d_flag, c->st);
   int h = 0;
   HIPCHECK(c, hipMemcpyAsync(&h, c->d_flag, sizeof(int), hipMemcpyDeviceToHost, c->st));
   HIPCHECK(c, hipStreamSynchronize(c->st));
@@ -3243,31 +3056,22 @@ static int field_io(ddx_ctx *c, int set, int field, float *out, const float *in)
   if (!c || set < 0 || set > 1 || field < 0 || field >= NF) return DDX_EINVAL;
   const int cls = field_class(field);
   const float sc = cls >= 0 ? scale_of(c, cls) : 1.0f, inv = 1.0f / sc;
-  const long GX = c->gext[0], GY = c->gext[1];
-  if (out) std::fill(out, out + GX * GY * (long)c->gext[2], 0.f);
-  for (int s = 0; s < c->nsub; s++) {
-    const Geom &g = c->g[s];
-    std::vector<char> h((size_t)g.nstore * c->esz);
-    char *base = c->wave[set][s] + (long)field * g.fpitch * c->esz;
-    HIPCHECK(c, hipMemcpyAsync(h.data(), base, h.size(), hipMemcpyDeviceToHost, c->st));
-    HIPCHECK(c, hipStreamSynchronize(c->st));
-    for (int k = 0; k < g.en[2]; k++)
-      for (int j = 0; j < g.en[1]; j++)
-        for (int i = 0; i < g.en[0]; i++) {
-          const long o = g.origin + i + g.sy * j + g.sz * k;
-          const long q = (i + g.ext_goff[0]) + GX * ((j + g.ext_goff[1]) + GY * (k + g.ext_goff[2]));
-          if (out) out[q] = load_elem(c, h.data(), o, inv);
-          else store_elem(c, h.data(), o, in[q], sc);
-        }
-    if (in) {
-      HIPCHECK(c, hipMemcpyAsync(base, h.data(), h.size(), hipMemcpyHostToDevice, c->st));
-      HIPCHECK(c, hipStreamSynchronize(c->st));
+  const Geom &g = c->all;
+  std::vector<char> h((size_t)g.nstore * c->esz);
+  char *base = c->wave[set] + (long)field * g.fpitch * c->esz;
+  HIPCHECK(c, hipMemcpyAsync(h.data(), base, h.size(), hipMemcpyDeviceToHost, c->st));
+  HIPCHECK(c, hipStreamSynchronize(c->st));
+  long q = 0;
+  for (int k = 0; k < g.en[2]; k++)
+    for (int j = 0; j < g.en[1]; j++) {
+      const long o = g.origin + g.sy * j + g.sz * k;
+      for (int i = 0; i < g.en[0]; i++, q++) {
+        if (out) out[q] = load_elem(c, h.data(), o + i, inv);
+        else store_elem(c, h.data(), o + i, in[q], sc);
+      }
     }
-  }
-  // ghosts follow the owners
   if (in) {
-    const int batch = field <= VZ ? 0 : (field == SAU ? 2 : 1);
-    exchange(c, set, batch);
+    HIPCHECK(c, hipMemcpyAsync(base, h.data(), h.size(), hipMemcpyHostToDevice, c->st));
     HIPCHECK(c, hipStreamSynchronize(c->st));
   }
   return DDX_OK;
@@ -3320,7 +3124,7 @@ extern "C" int ddx_set_tiling_mode(ddx_ctx *c, int kernel, int mode, int tx, int
   HIPCHECK(c, hipStreamSynchronize(c->st));
   (kernel == 0 ? c->tiling_vel : c->tiling_stress)[mode] = t;
   for (int m = 0; m < 2; m++)
-    if (!c->model[m].empty() && !phy_tables(c, t, m)) return DDX_EHIP;
+    if (c->model[m] && !phy_tables(c, t, m)) return DDX_EHIP;
   return DDX_OK;
 }
 
@@ -3329,8 +3133,8 @@ extern "C" int ddx_set_tiling_mode(ddx_ctx *c, int kernel, int mode, int tx, int
 // propagation mode, time `reps` launches of every z-blocked shape of the
 // context's storage format (one-cell and paired bricks) with HIP events on
 // the context stream, and keep the fastest.  Results are cached per process
-// by storage format, decomposition and subdomain size bucket (each gridphy
-// axis rounded up to 32 cells), so contexts of similar size reuse them.  The
+// by storage format and grid size bucket (each gridphy axis rounded up to 32
+// cells), so contexts of similar size reuse them.  The
 // timing launches run on the current wavefields; both sets are reset
 // afterwards.
 static std::mutex g_tune_mu;
@@ -3338,10 +3142,9 @@ static std::map<std::string, Tiling> g_tune_cache;
 
 static std::string tune_key(const ddx_ctx *c, int kernel, int mode) {
   char b[160];
-  int big[3] = {0, 0, 0};
-  for (const Geom &g : c->g)
-    for (int a = 0; a < 3; a++) big[a] = std::max(big[a], (g.pn[a] + 31) / 32 * 32);
-  snprintf(b, sizeof b, "f%d k%d m%d n%d R%d b%dx%dx%d mig%d", c->fmt, kernel, mode, c->nsub,
+  int big[3];
+  for (int a = 0; a < 3; a++) big[a] = (c->all.pn[a] + 31) / 32 * 32;
+  snprintf(b, sizeof b, "f%d k%d m%d R%d b%dx%dx%d mig%d", c->fmt, kernel, mode,
            mode == RTM_BACKWARD ? c->d.rec_width : 0, big[0], big[1], big[2], (int)model_for(c, mode));
   return b;
 }
@@ -3424,7 +3227,7 @@ extern "C" int ddx_set_brick(ddx_ctx *c, int kernel, int mode, int tx, int ty, i
   HIPCHECK(c, hipStreamSynchronize(c->st));
   (kernel == 0 ? c->tiling_vel : c->tiling_stress)[mode] = t;
   for (int m = 0; m < 2; m++)
-    if (!c->model[m].empty() && !phy_tables(c, t, m)) return DDX_EHIP;
+    if (c->model[m] && !phy_tables(c, t, m)) return DDX_EHIP;
   return DDX_OK;
 }
 
@@ -3539,13 +3342,16 @@ extern "C" int ddx_estimate_bytes(const ddx_desc *d, int nrec, int nshot, int rt
     Geom g;
     std::string err;
     if (!make_geom(*d, r, g, err)) return DDX_EINVAL;
-    b += (2.0 * NF * fsz + 4.0 * 3.0 * models) * (double)g.fpitch;
     b += 9.0 * esz * (double)g.pn[0] * g.pn[1] * g.pn[2];
-    for_each_slab(g, [&](int i0, int i1, int j0, int j1, int k0, int k1, int axes) {
-      if (i1 <= i0 || j1 <= j0 || k1 <= k0) return;
-      const double ncell = (double)(i1 - i0) * (j1 - j0) * (k1 - k0);
-      b += ncell * __builtin_popcount(axes) * (4.0 * 4.0 * models + 12.0 * fsz);  // coefficients + 2 sets of psi
-    });
+    if (r == 0) {  // shared by all subdomains
+      const Geom w = whole_grid(*d, g);
+      b += (2.0 * NF * fsz + 4.0 * 3.0 * models) * (double)w.fpitch;
+      for_each_slab(w, [&](int i0, int i1, int j0, int j1, int k0, int k1, int axes) {
+        if (i1 <= i0 || j1 <= j0 || k1 <= k0) return;
+        const double ncell = (double)(i1 - i0) * (j1 - j0) * (k1 - k0);
+        b += ncell * __builtin_popcount(axes) * (4.0 * 4.0 * models + 12.0 * fsz);  // coefficients + 2 sets of psi
+      });
+    }
     if (rtm) {
       long ring = 0;
       for (int fi = 0; fi < 10; fi++)

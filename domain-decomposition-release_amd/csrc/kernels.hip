@@ -1,7 +1,7 @@
 // HIP kernels of the elastic FDTD / RTM engine, written for gfx950 (MI355X).
 //
 // All kernels are HBM-bound stencils or copies; none uses MFMA.  Every launch
-// covers all subdomains (or all slabs / halo boxes) of a context at once
+// covers the whole grid (or all slabs, or all boxes) of a context at once
 // through a descriptor table, so a time step costs a handful of launches
 // regardless of the decomposition.  Blocks map to descriptors by a binary
 // search over the descriptors' first-block indices.
@@ -9,6 +9,9 @@
 // Arithmetic follows the reference's operation order (see each kernel's
 // citation) and the library is compiled with -ffp-contract=off, so one FP32
 // rounding happens per source-level operation, as in the CPU oracle.
+//
+// The file is compiled once per kPart (build.py, -DDDX_PART=n): each part
+// instantiates the kernels of one family, so the parts build in parallel.
 #include "ddx_internal.h"
 
 #include <algorithm>
@@ -20,11 +23,9 @@ namespace ddx {
 // Coefficients of half order h (rows 1..4), zero-padded to 4 taps.  Row 4 is
 // phy_dc, rows R..4 are phy_dc_list (UTIL/.jarvis_2_geometry/
 // jarvis_device_geometry_bones.hpp:29-71); row 2 is pml_dc.
-__constant__ float c_fd[5][4];
-
-void set_fd_table(const float tab[5][4]) {
-  (void)hipMemcpyToSymbol(HIP_SYMBOL(c_fd), tab, sizeof(float) * 20);
-}
+#define DDX_FD_ROW(h) {fd_tap(h, 0), fd_tap(h, 1), fd_tap(h, 2), fd_tap(h, 3)}
+static __constant__ const float c_fd[5][4] = {DDX_FD_ROW(0), DDX_FD_ROW(1), DDX_FD_ROW(2), DDX_FD_ROW(3),
+                                              DDX_FD_ROW(4)};
 
 __device__ __forceinline__ int find_desc(const int *__restrict__ starts, int n, int b) {
   int lo = 0, hi = n - 1;
@@ -62,14 +63,12 @@ __device__ __forceinline__ int xcd_group_remap(int b, int nblk, int g) {
   return ((i / g) * 8 + x) * g + (i % g);
 }
 
-// Block order of the z-blocked bricks: 0 one contiguous chunk per XCD
-// (xcd_remap), g > 0 groups of g blocks dealt round-robin (the engine sets
-// 8: measured 1-3.5% faster than contiguous chunks on the 256x256x200 RTM
-// shot, every group size from 1 to 16 within 1% of each other).
-__constant__ int c_brick_group;
-void set_brick_group(int g) { (void)hipMemcpyToSymbol(HIP_SYMBOL(c_brick_group), &g, sizeof(int)); }
-__device__ __forceinline__ int brick_block(int b, int nblk) {
-  return c_brick_group > 0 ? xcd_group_remap(b, nblk, c_brick_group) : xcd_remap(b, nblk);
+// Block order of the z-blocked bricks: grp = 0 one contiguous chunk per XCD
+// (xcd_remap), grp > 0 groups of grp blocks dealt round-robin (the engine
+// passes 8: measured 1-3.5% faster than contiguous chunks on the 256x256x200
+// RTM shot, every group size from 1 to 16 within 1% of each other).
+__device__ __forceinline__ int brick_block(int b, int nblk, int grp) {
+  return grp > 0 ? xcd_group_remap(b, nblk, grp) : xcd_remap(b, nblk);
 }
 
 // Field pointers reach the kernels through descriptor tables in global
@@ -140,7 +139,7 @@ __device__ __forceinline__ void add_to(GT *p, long i, float v) {
 // imaging inputs and images) go through non-temporal loads and stores, so
 // they do not push the stencil halos of neighbouring bricks out of L2.  Same
 // arithmetic as `p[i] += v`.  (Measured: 2-4% faster bricks, imaging
-// 259 -> 174 us per launch; slower in the CPML kernels and the halo copy,
+// 259 -> 174 us per launch; slower in the CPML kernels,
 // which keep ordinary accesses.)
 template <typename GT>
 __device__ __forceinline__ void rmw_add(GT *p, long i, float v) {
@@ -156,61 +155,6 @@ __device__ __forceinline__ void rmw_add_t(GT *p, long i, T v) {
   const T old = __builtin_nontemporal_load(p + i);
   __builtin_nontemporal_store(old + v, p + i);
 }
-
-// ---------------------------------------------------------------------------
-// Pack on store (MirrorDesc): after a kernel stores an exchanged field at a
-// cell with local extended coordinates e, the same value goes into the
-// ghost layers of every receiver that takes the cell.  Subdomains are at
-// least 8 cells wide and halos at most 4, so a cell can be sent across at
-// most one side per axis: mir_cell finds that candidate side per axis once
-// per cell, and mir_put checks the field's width and stores.
-// ---------------------------------------------------------------------------
-struct MirCell {
-  const MirrorDesc *M;
-  int e[3];
-  int sd[3];  // candidate side per axis (x: 4 lo / 5 hi, y: 2 / 3, z: 0 / 1), -1: none
-  bool any;
-};
-__device__ __forceinline__ MirCell mir_cell(const MirrorDesc *__restrict__ M, int ex, int ey, int ez) {
-  MirCell m;
-  m.M = M;
-  m.e[0] = ex; m.e[1] = ey; m.e[2] = ez;
-  m.any = false;
-#pragma unroll
-  for (int a = 0; a < 3; a++) {
-    const int lo = 4 - 2 * a, c = m.e[a];
-    int sd = -1;
-    if (c < 4 && M->s[lo].base) sd = lo;
-    else if (c >= M->en[a] - 4 && M->s[lo + 1].base) sd = lo + 1;
-    m.sd[a] = sd;
-    m.any |= sd >= 0;
-  }
-  return m;
-}
-template <typename GT>
-__device__ __forceinline__ void mir_put(const MirCell &m, int f, float v) {
-#pragma unroll
-  for (int a = 0; a < 3; a++) {
-    const int sd = m.sd[a];
-    if (sd < 0) continue;
-    const MirrorSide &s = m.M->s[sd];
-    const int c = m.e[a], w = s.w[f];
-    if ((sd & 1) ? (c < m.M->en[a] - w) : (c >= w)) continue;
-    const int r0 = m.e[0] + (a == 0 ? s.shift : 0);
-    const int r1 = m.e[1] + (a == 1 ? s.shift : 0);
-    const int r2 = m.e[2] + (a == 2 ? s.shift : 0);
-    GT *p = (GT *)(void *)s.base;
-    stq(p, (long)f * s.fpitch + r0 + s.sy * r1 + s.sz * r2, v);
-  }
-}
-// the two cells of a pair (the second only when it is in gridphy)
-template <typename GT>
-__device__ __forceinline__ void mir_pair(const MirCell &ma, const MirCell &mb, bool both, int f, float va,
-                                         float vb) {
-  if (ma.any) mir_put<GT>(ma, f, va);
-  if (both && mb.any) mir_put<GT>(mb, f, vb);
-}
-
 
 // Forward-staggered: sum_r c[r] (f[i+(r+1)s] - f[i-r s]); backward-staggered:
 // sum_r c[r] (f[i+r s] - f[i-(r+1)s]); accumulated from r = 0 upward
@@ -280,10 +224,9 @@ __device__ __forceinline__ Coef4 coef_row(int h) {
 template <int MODE>
 __global__ __launch_bounds__(kBlock) void k_vel_phy(const PhyDesc *__restrict__ descs,
                                                     const int *__restrict__ starts, int n, float dx, float dy,
-                                                    float dz, float sign, int gnx, int gny, int gnz, int R) {
+                                                    float dz, float sign) {
   const int b = xcd_remap(blockIdx.x, gridDim.x);
   const PhyDesc &D = descs[find_desc(starts, n, b)];
-  gnx = D.gnx; gny = D.gny; gnz = D.gnz; R = D.R;  // per descriptor: fused batches mix grids
   const int t = b - D.blk0;
   const int tiles = D.tiles_x * D.tiles_y;
   const int k = t / tiles;
@@ -298,9 +241,9 @@ __global__ __launch_bounds__(kBlock) void k_vel_phy(const PhyDesc *__restrict__ 
 
   Coef4 cx, cy, cz;
   if (MODE == RTM_BACKWARD) {
-    cx = coef_row(vowr_order(D.gx + i, gnx, R));
-    cy = coef_row(vowr_order(D.gy + j, gny, R));
-    cz = coef_row(vowr_order(D.gz + k, gnz, R));
+    cx = coef_row(vowr_order(i, D.nx, D.R));
+    cy = coef_row(vowr_order(j, D.ny, D.R));
+    cz = coef_row(vowr_order(k, D.nz, D.R));
   } else {
     cx = coef_row(4);
     cy = cx;
@@ -342,11 +285,9 @@ __global__ __launch_bounds__(kBlock) void k_vel_phy(const PhyDesc *__restrict__ 
 template <int MODE>
 __global__ __launch_bounds__(kBlock) void k_stress_phy(const PhyDesc *__restrict__ descs,
                                                        const int *__restrict__ starts, int n, float dx,
-                                                       float dy, float dz, float dt, int gnx, int gny, int gnz,
-                                                       int R) {
+                                                       float dy, float dz, float dt) {
   const int b = xcd_remap(blockIdx.x, gridDim.x);
   const PhyDesc &D = descs[find_desc(starts, n, b)];
-  gnx = D.gnx; gny = D.gny; gnz = D.gnz; R = D.R;  // per descriptor: fused batches mix grids
   const int t = b - D.blk0;
   const int tiles = D.tiles_x * D.tiles_y;
   const int k = t / tiles;
@@ -361,9 +302,9 @@ __global__ __launch_bounds__(kBlock) void k_stress_phy(const PhyDesc *__restrict
 
   Coef4 cx, cy, cz;
   if (MODE == RTM_BACKWARD) {
-    cx = coef_row(vowr_order(D.gx + i, gnx, R));
-    cy = coef_row(vowr_order(D.gy + j, gny, R));
-    cz = coef_row(vowr_order(D.gz + k, gnz, R));
+    cx = coef_row(vowr_order(i, D.nx, D.R));
+    cy = coef_row(vowr_order(j, D.ny, D.R));
+    cz = coef_row(vowr_order(k, D.nz, D.R));
   } else {
     cx = coef_row(4);
     cy = cx;
@@ -503,7 +444,7 @@ __device__ __forceinline__ float ld_halo(const GT *p, const XLane &xl, long id_h
 // neighbouring lanes (tx = 64); `live`: the lane's cell is in gridphy.
 template <int MODE, int TX, int TY, int CY, int CZ, class S, bool XL = false>
 __device__ __forceinline__ void vel_zb_body(const PhyDesc &D, int i, int j0, int k0, float dx, float dy, float dz,
-                                            float sign, int gnx, int gny, int gnz, int R, bool live = true) {
+                                            float sign, bool live = true) {
   typedef typename GPtr<S>::T gT;
   const long sy = D.sy, sz = D.sz;
   const XLane xl = xlane(i, D.nx);
@@ -524,12 +465,12 @@ __device__ __forceinline__ void vel_zb_body(const PhyDesc &D, int i, int j0, int
   const gfloat *__restrict__ fdtr = G(D.dtr);
   constexpr bool P = (MODE == RTM_BACKWARD || MODE == RTM_REVERSE);
   const Coef4 c4 = coef_row(4);
-  const Coef4 cx = MODE == RTM_BACKWARD ? coef_row(vowr_order(D.gx + i, gnx, R)) : c4;
+  const Coef4 cx = MODE == RTM_BACKWARD ? coef_row(vowr_order(i, D.nx, D.R)) : c4;
 #pragma unroll
   for (int q = 0; q < CY; q++) {
     const int j = j0 + q * TY;
     if (j >= D.ny) continue;
-    const Coef4 cy = MODE == RTM_BACKWARD ? coef_row(vowr_order(D.gy + j, gny, R)) : c4;
+    const Coef4 cy = MODE == RTM_BACKWARD ? coef_row(vowr_order(j, D.ny, D.R)) : c4;
     const long base = (long)(D.ox + ic) + sy * (D.oy + j) + sz * (D.oz + k0);
     const long hbase = base + (xl.hx - ic);
     float zzz[CZ + 7], zxz[CZ + 7], zyz[CZ + 7], zsa[P ? CZ + 7 : 1];
@@ -541,7 +482,7 @@ __device__ __forceinline__ void vel_zb_body(const PhyDesc &D, int i, int j0, int
     for (int kk = 0; kk < CZ; kk++) {
       const int k = k0 + kk;
       if (k >= D.nz) break;
-      const Coef4 cz = MODE == RTM_BACKWARD ? coef_row(vowr_order(D.gz + k, gnz, R)) : c4;
+      const Coef4 cz = MODE == RTM_BACKWARD ? coef_row(vowr_order(k, D.nz, D.R)) : c4;
       const long id = base + (long)kk * sz;
       // the updated cells are read before the stencil taps (see stress_zb_body)
       const float ovx = ld_stream(fvx, id), ovy = ld_stream(fvy, id), ovz = ld_stream(fvz, id);
@@ -613,10 +554,6 @@ __device__ __forceinline__ void vel_zb_body(const PhyDesc &D, int i, int j0, int
         __builtin_nontemporal_store(dt * ix, G(D.f[VXRT]) + id);
         __builtin_nontemporal_store(dt * iy, G(D.f[VYRT]) + id);
         __builtin_nontemporal_store(dt * iz, G(D.f[VZRT]) + id);
-        if (D.mir) {
-          const MirCell m = mir_cell(D.mir, D.ox + i, D.oy + j, D.oz + k);
-          if (m.any) { mir_put<gT>(m, VX, nvx); mir_put<gT>(m, VY, nvy); mir_put<gT>(m, VZ, nvz); }
-        }
       } else {
         const float nvx = ovx + (a * sxx_x + bb * sxy_y + c * sxz_z);
         const float nvy = ovy + (a * syx_x + bb * syy_y + c * syz_z);
@@ -624,10 +561,6 @@ __device__ __forceinline__ void vel_zb_body(const PhyDesc &D, int i, int j0, int
         st_stream(fvx, id, nvx);
         st_stream(fvy, id, nvy);
         st_stream(fvz, id, nvz);
-        if (D.mir) {
-          const MirCell m = mir_cell(D.mir, D.ox + i, D.oy + j, D.oz + k);
-          if (m.any) { mir_put<gT>(m, VX, nvx); mir_put<gT>(m, VY, nvy); mir_put<gT>(m, VZ, nvz); }
-        }
       }
       if constexpr (P) {
         st_stream(fvxp, id, ovxp + a * sx);
@@ -641,7 +574,7 @@ __device__ __forceinline__ void vel_zb_body(const PhyDesc &D, int i, int j0, int
 // `dt` carries the stress-over-velocity scale ratio of the 16-bit formats.
 template <int MODE, int TX, int TY, int CY, int CZ, class S, bool XL = false>
 __device__ __forceinline__ void stress_zb_body(const PhyDesc &D, int i, int j0, int k0, float dx, float dy,
-                                               float dz, float dt, int gnx, int gny, int gnz, int R,
+                                               float dz, float dt,
                                                bool live = true) {
   typedef typename GPtr<S>::T gT;
   const long sy = D.sy, sz = D.sz;
@@ -661,12 +594,12 @@ __device__ __forceinline__ void stress_zb_body(const PhyDesc &D, int i, int j0, 
   const gfloat *__restrict__ fmu = G(D.mu);
   const float a = dt / dx, bb = dt / dy, c = dt / dz;
   const Coef4 c4 = coef_row(4);
-  const Coef4 cx = MODE == RTM_BACKWARD ? coef_row(vowr_order(D.gx + i, gnx, R)) : c4;
+  const Coef4 cx = MODE == RTM_BACKWARD ? coef_row(vowr_order(i, D.nx, D.R)) : c4;
 #pragma unroll
   for (int q = 0; q < CY; q++) {
     const int j = j0 + q * TY;
     if (j >= D.ny) continue;
-    const Coef4 cy = MODE == RTM_BACKWARD ? coef_row(vowr_order(D.gy + j, gny, R)) : c4;
+    const Coef4 cy = MODE == RTM_BACKWARD ? coef_row(vowr_order(j, D.ny, D.R)) : c4;
     const long base = (long)(D.ox + ic) + sy * (D.oy + j) + sz * (D.oz + k0);
     const long hbase = base + (xl.hx - ic);
     float zx[CZ + 7], zy[CZ + 7], zz[CZ + 7];
@@ -677,7 +610,7 @@ __device__ __forceinline__ void stress_zb_body(const PhyDesc &D, int i, int j0, 
     for (int kk = 0; kk < CZ; kk++) {
       const int k = k0 + kk;
       if (k >= D.nz) break;
-      const Coef4 cz = MODE == RTM_BACKWARD ? coef_row(vowr_order(D.gz + k, gnz, R)) : c4;
+      const Coef4 cz = MODE == RTM_BACKWARD ? coef_row(vowr_order(k, D.nz, D.R)) : c4;
       const long id = base + (long)kk * sz;
       // the updated cells are read before the stencil taps: on this target
       // the memory counter also tracks stores, so a read issued after a
@@ -731,14 +664,6 @@ __device__ __forceinline__ void stress_zb_body(const PhyDesc &D, int i, int j0, 
       st_stream(fsxz, id, nxz);
       st_stream(fsyz, id, nyz);
       if constexpr (rtm_mode(MODE)) st_stream(fsau, id, nau);
-      if (D.mir) {
-        const MirCell m = mir_cell(D.mir, D.ox + i, D.oy + j, D.oz + k);
-        if (m.any) {
-          mir_put<gT>(m, SXX, nxx); mir_put<gT>(m, SYY, nyy); mir_put<gT>(m, SZZ, nzz);
-          mir_put<gT>(m, SXY, nxy); mir_put<gT>(m, SXZ, nxz); mir_put<gT>(m, SYZ, nyz);
-          if constexpr (rtm_mode(MODE)) mir_put<gT>(m, SAU, nau);
-        }
-      }
     }
   }
 }
@@ -748,8 +673,8 @@ __device__ __forceinline__ void stress_zb_body(const PhyDesc &D, int i, int j0, 
 // gridphy boundary (vowr_order gives 4 for d >= 3, and always for R = 4).
 // Block-uniform, so interior bricks run the constant-coefficient code.
 template <int TX, int TY, int CY, int CZ>
-__device__ __forceinline__ bool brick_full_order(const PhyDesc &D, int t, int gnx, int gny, int gnz, int R) {
-  if (R >= 4) return true;
+__device__ __forceinline__ bool brick_full_order(const PhyDesc &D, int t) {
+  if (D.R >= 4) return true;
   const int tiles_x = (D.nx + TX - 1) / TX;
   const int tiles_y = (D.ny + TY * CY - 1) / (TY * CY);
   const int per = tiles_x * tiles_y;
@@ -757,10 +682,10 @@ __device__ __forceinline__ bool brick_full_order(const PhyDesc &D, int t, int gn
   const int rem = t - zc * per;
   const int ty = rem / tiles_x;
   const int tx = rem - ty * tiles_x;
-  const int x0 = D.gx + tx * TX, x1 = D.gx + min(tx * TX + TX, D.nx) - 1;
-  const int y0 = D.gy + ty * TY * CY, y1 = D.gy + min((ty + 1) * TY * CY, D.ny) - 1;
-  const int z0 = D.gz + zc * CZ, z1 = D.gz + min(zc * CZ + CZ, D.nz) - 1;
-  return x0 >= 3 && x1 <= gnx - 4 && y0 >= 3 && y1 <= gny - 4 && z0 >= 3 && z1 <= gnz - 4;
+  const int x0 = tx * TX, x1 = min(tx * TX + TX, D.nx) - 1;
+  const int y0 = ty * TY * CY, y1 = min((ty + 1) * TY * CY, D.ny) - 1;
+  const int z0 = zc * CZ, z1 = min(zc * CZ + CZ, D.nz) - 1;
+  return x0 >= 3 && x1 <= D.nx - 4 && y0 >= 3 && y1 <= D.ny - 4 && z0 >= 3 && z1 <= D.nz - 4;
 }
 
 // Extra attributes of the brick kernels (occupancy experiments), empty by default.
@@ -774,37 +699,34 @@ __device__ __forceinline__ bool brick_full_order(const PhyDesc &D, int t, int gn
 template <int MODE, int TX, int TY, int CY, int CZ, class S, bool XL = false>
 __global__ __launch_bounds__(TX *TY) DDX_BRICK_ATTR void k_vel_phy_zb(const PhyDesc *__restrict__ descs,
                                                        const int *__restrict__ starts, int n, float dx, float dy,
-                                                       float dz, float sign, int gnx, int gny, int gnz, int R) {
+                                                       float dz, float sign, int grp) {
   static_assert(!XL || TX == 64, "lane-exchange bricks need one wavefront per x row");
-  const int b = brick_block(blockIdx.x, gridDim.x);
+  const int b = brick_block(blockIdx.x, gridDim.x, grp);
   const PhyDesc &D = descs[find_desc(starts, n, b)];
-  gnx = D.gnx; gny = D.gny; gnz = D.gnz; R = D.R;  // per descriptor: fused batches mix grids
   int i, j0, k0;
   const bool live = zbrick<TX, TY, CY, CZ>(D, b - D.blk0, i, j0, k0);
   if (!XL && !live) return;
   // backward mode and reverse mode differ only in the coefficient rows
-  if (MODE == RTM_BACKWARD && brick_full_order<TX, TY, CY, CZ>(D, b - D.blk0, gnx, gny, gnz, R))
-    vel_zb_body<RTM_REVERSE, TX, TY, CY, CZ, S, XL>(D, i, j0, k0, dx, dy, dz, sign, gnx, gny, gnz, R, live);
+  if (MODE == RTM_BACKWARD && brick_full_order<TX, TY, CY, CZ>(D, b - D.blk0))
+    vel_zb_body<RTM_REVERSE, TX, TY, CY, CZ, S, XL>(D, i, j0, k0, dx, dy, dz, sign, live);
   else
-    vel_zb_body<MODE, TX, TY, CY, CZ, S, XL>(D, i, j0, k0, dx, dy, dz, sign, gnx, gny, gnz, R, live);
+    vel_zb_body<MODE, TX, TY, CY, CZ, S, XL>(D, i, j0, k0, dx, dy, dz, sign, live);
 }
 
 template <int MODE, int TX, int TY, int CY, int CZ, class S, bool XL = false>
 __global__ __launch_bounds__(TX *TY) DDX_BRICK_ATTR void k_stress_phy_zb(const PhyDesc *__restrict__ descs,
                                                           const int *__restrict__ starts, int n, float dx,
-                                                          float dy, float dz, float dt, int gnx, int gny, int gnz,
-                                                          int R) {
+                                                          float dy, float dz, float dt, int grp) {
   static_assert(!XL || TX == 64, "lane-exchange bricks need one wavefront per x row");
-  const int b = brick_block(blockIdx.x, gridDim.x);
+  const int b = brick_block(blockIdx.x, gridDim.x, grp);
   const PhyDesc &D = descs[find_desc(starts, n, b)];
-  gnx = D.gnx; gny = D.gny; gnz = D.gnz; R = D.R;  // per descriptor: fused batches mix grids
   int i, j0, k0;
   const bool live = zbrick<TX, TY, CY, CZ>(D, b - D.blk0, i, j0, k0);
   if (!XL && !live) return;
-  if (MODE == RTM_BACKWARD && brick_full_order<TX, TY, CY, CZ>(D, b - D.blk0, gnx, gny, gnz, R))
-    stress_zb_body<RTM_REVERSE, TX, TY, CY, CZ, S, XL>(D, i, j0, k0, dx, dy, dz, dt, gnx, gny, gnz, R, live);
+  if (MODE == RTM_BACKWARD && brick_full_order<TX, TY, CY, CZ>(D, b - D.blk0))
+    stress_zb_body<RTM_REVERSE, TX, TY, CY, CZ, S, XL>(D, i, j0, k0, dx, dy, dz, dt, live);
   else
-    stress_zb_body<MODE, TX, TY, CY, CZ, S, XL>(D, i, j0, k0, dx, dy, dz, dt, gnx, gny, gnz, R, live);
+    stress_zb_body<MODE, TX, TY, CY, CZ, S, XL>(D, i, j0, k0, dx, dy, dz, dt, live);
 }
 
 // ---------------------------------------------------------------------------
@@ -824,8 +746,7 @@ struct YlTile {
 
 template <int MODE, int TY, int CZ, class S>
 __device__ __forceinline__ void stress_yl_body(YlTile<3, TY, CZ> &ly, const PhyDesc &D, int i, int j0, int k0,
-                                               float dx, float dy, float dz, float dt, int gnx, int gny, int gnz,
-                                               int R, bool live) {
+                                               float dx, float dy, float dz, float dt, bool live) {
   typedef typename GPtr<S>::T gT;
   const long sy = D.sy, sz = D.sz;
   const int lane = (int)threadIdx.x & 63, w = (int)threadIdx.x >> 6;
@@ -892,15 +813,15 @@ __device__ __forceinline__ void stress_yl_body(YlTile<3, TY, CZ> &ly, const PhyD
   const gfloat *__restrict__ fmu = G(D.mu);
   const float a = dt / dx, bb = dt / dy, c = dt / dz;
   const Coef4 c4 = coef_row(4);
-  const Coef4 cx = MODE == RTM_BACKWARD ? coef_row(vowr_order(D.gx + i, gnx, R)) : c4;
-  const Coef4 cy = MODE == RTM_BACKWARD ? coef_row(vowr_order(D.gy + j, gny, R)) : c4;
+  const Coef4 cx = MODE == RTM_BACKWARD ? coef_row(vowr_order(i, D.nx, D.R)) : c4;
+  const Coef4 cy = MODE == RTM_BACKWARD ? coef_row(vowr_order(j, D.ny, D.R)) : c4;
   const long hbase = base + (xl.hx - ic);
   const int r0 = w + 4;  // the wave's row in the tile
 #pragma unroll
   for (int kk = 0; kk < CZ; kk++) {
     const int k = k0 + kk;
     if (k >= D.nz) break;
-    const Coef4 cz = MODE == RTM_BACKWARD ? coef_row(vowr_order(D.gz + k, gnz, R)) : c4;
+    const Coef4 cz = MODE == RTM_BACKWARD ? coef_row(vowr_order(k, D.nz, D.R)) : c4;
     const long id = base + (long)kk * sz;
     const float oxx = ld_stream(fsxx, id), oyy = ld_stream(fsyy, id), ozz = ld_stream(fszz, id);
     const float oxy = ld_stream(fsxy, id), oxz = ld_stream(fsxz, id), oyz = ld_stream(fsyz, id);
@@ -961,32 +882,22 @@ __device__ __forceinline__ void stress_yl_body(YlTile<3, TY, CZ> &ly, const PhyD
     st_stream(fsxz, id, nxz);
     st_stream(fsyz, id, nyz);
     if constexpr (rtm_mode(MODE)) st_stream(fsau, id, nau);
-    if (D.mir) {
-      const MirCell m = mir_cell(D.mir, D.ox + i, D.oy + j, D.oz + k);
-      if (m.any) {
-        mir_put<gT>(m, SXX, nxx); mir_put<gT>(m, SYY, nyy); mir_put<gT>(m, SZZ, nzz);
-        mir_put<gT>(m, SXY, nxy); mir_put<gT>(m, SXZ, nxz); mir_put<gT>(m, SYZ, nyz);
-        if constexpr (rtm_mode(MODE)) mir_put<gT>(m, SAU, nau);
-      }
-    }
   }
 }
 
 template <int MODE, int TY, int CZ, class S>
 __global__ __launch_bounds__(64 * TY) DDX_BRICK_ATTR void k_stress_phy_yl(const PhyDesc *__restrict__ descs,
                                                            const int *__restrict__ starts, int n, float dx,
-                                                           float dy, float dz, float dt, int gnx, int gny,
-                                                           int gnz, int R) {
+                                                           float dy, float dz, float dt, int grp) {
   __shared__ YlTile<3, TY, CZ> ly;
-  const int b = brick_block(blockIdx.x, gridDim.x);
+  const int b = brick_block(blockIdx.x, gridDim.x, grp);
   const PhyDesc &D = descs[find_desc(starts, n, b)];
-  gnx = D.gnx; gny = D.gny; gnz = D.gnz; R = D.R;  // per descriptor: fused batches mix grids
   int i, j0, k0;
   const bool live = zbrick<64, TY, 1, CZ>(D, b - D.blk0, i, j0, k0);
-  if (MODE == RTM_BACKWARD && brick_full_order<64, TY, 1, CZ>(D, b - D.blk0, gnx, gny, gnz, R))
-    stress_yl_body<RTM_REVERSE, TY, CZ, S>(ly, D, i, j0, k0, dx, dy, dz, dt, gnx, gny, gnz, R, live);
+  if (MODE == RTM_BACKWARD && brick_full_order<64, TY, 1, CZ>(D, b - D.blk0))
+    stress_yl_body<RTM_REVERSE, TY, CZ, S>(ly, D, i, j0, k0, dx, dy, dz, dt, live);
   else
-    stress_yl_body<MODE, TY, CZ, S>(ly, D, i, j0, k0, dx, dy, dz, dt, gnx, gny, gnz, R, live);
+    stress_yl_body<MODE, TY, CZ, S>(ly, D, i, j0, k0, dx, dy, dz, dt, live);
 }
 
 // Velocity update with the y arm from LDS: the tile holds syy, sxy, syz and,
@@ -995,7 +906,7 @@ __global__ __launch_bounds__(64 * TY) DDX_BRICK_ATTR void k_stress_phy_yl(const 
 template <int MODE, int TY, int CZ, class S>
 __device__ __forceinline__ void vel_yl_body(YlTile<(MODE == RTM_BACKWARD || MODE == RTM_REVERSE) ? 4 : 3, TY, CZ> &ly,
                                             const PhyDesc &D, int i, int j0, int k0, float dx, float dy, float dz,
-                                            float sign, int gnx, int gny, int gnz, int R, bool live) {
+                                            float sign, bool live) {
   typedef typename GPtr<S>::T gT;
   constexpr bool P = (MODE == RTM_BACKWARD || MODE == RTM_REVERSE);
   const long sy = D.sy, sz = D.sz;
@@ -1074,15 +985,15 @@ __device__ __forceinline__ void vel_yl_body(YlTile<(MODE == RTM_BACKWARD || MODE
   gT *__restrict__ fvzp = (gT *)D.f[VZP];
   const gfloat *__restrict__ fdtr = G(D.dtr);
   const Coef4 c4 = coef_row(4);
-  const Coef4 cx = MODE == RTM_BACKWARD ? coef_row(vowr_order(D.gx + i, gnx, R)) : c4;
-  const Coef4 cy = MODE == RTM_BACKWARD ? coef_row(vowr_order(D.gy + j, gny, R)) : c4;
+  const Coef4 cx = MODE == RTM_BACKWARD ? coef_row(vowr_order(i, D.nx, D.R)) : c4;
+  const Coef4 cy = MODE == RTM_BACKWARD ? coef_row(vowr_order(j, D.ny, D.R)) : c4;
   const long hbase = base + (xl.hx - ic);
   const int r0 = w + 4;
 #pragma unroll
   for (int kk = 0; kk < CZ; kk++) {
     const int k = k0 + kk;
     if (k >= D.nz) break;
-    const Coef4 cz = MODE == RTM_BACKWARD ? coef_row(vowr_order(D.gz + k, gnz, R)) : c4;
+    const Coef4 cz = MODE == RTM_BACKWARD ? coef_row(vowr_order(k, D.nz, D.R)) : c4;
     const long id = base + (long)kk * sz;
     const float ovx = ld_stream(fvx, id), ovy = ld_stream(fvy, id), ovz = ld_stream(fvz, id);
     const float ovxp = P ? ld_stream(fvxp, id) : 0.f, ovyp = P ? ld_stream(fvyp, id) : 0.f;
@@ -1148,10 +1059,6 @@ __device__ __forceinline__ void vel_yl_body(YlTile<(MODE == RTM_BACKWARD || MODE
     st_stream(fvx, id, nvx);
     st_stream(fvy, id, nvy);
     st_stream(fvz, id, nvz);
-    if (D.mir) {
-      const MirCell m = mir_cell(D.mir, D.ox + i, D.oy + j, D.oz + k);
-      if (m.any) { mir_put<gT>(m, VX, nvx); mir_put<gT>(m, VY, nvy); mir_put<gT>(m, VZ, nvz); }
-    }
     if constexpr (P) {
       st_stream(fvxp, id, ovxp + a * sx);
       st_stream(fvyp, id, ovyp + bb * sy_);
@@ -1163,21 +1070,20 @@ __device__ __forceinline__ void vel_yl_body(YlTile<(MODE == RTM_BACKWARD || MODE
 template <int MODE, int TY, int CZ, class S>
 __global__ __launch_bounds__(64 * TY) DDX_BRICK_ATTR void k_vel_phy_yl(const PhyDesc *__restrict__ descs,
                                                         const int *__restrict__ starts, int n, float dx, float dy,
-                                                        float dz, float sign, int gnx, int gny, int gnz, int R) {
+                                                        float dz, float sign, int grp) {
   __shared__ YlTile<(MODE == RTM_BACKWARD || MODE == RTM_REVERSE) ? 4 : 3, TY, CZ> ly;
-  const int b = brick_block(blockIdx.x, gridDim.x);
+  const int b = brick_block(blockIdx.x, gridDim.x, grp);
   const PhyDesc &D = descs[find_desc(starts, n, b)];
-  gnx = D.gnx; gny = D.gny; gnz = D.gnz; R = D.R;  // per descriptor: fused batches mix grids
   int i, j0, k0;
   const bool live = zbrick<64, TY, 1, CZ>(D, b - D.blk0, i, j0, k0);
   // backward mode and reverse mode differ only in the coefficient rows
   if constexpr (MODE == RTM_BACKWARD) {
-    if (brick_full_order<64, TY, 1, CZ>(D, b - D.blk0, gnx, gny, gnz, R))
-      vel_yl_body<RTM_REVERSE, TY, CZ, S>(ly, D, i, j0, k0, dx, dy, dz, sign, gnx, gny, gnz, R, live);
+    if (brick_full_order<64, TY, 1, CZ>(D, b - D.blk0))
+      vel_yl_body<RTM_REVERSE, TY, CZ, S>(ly, D, i, j0, k0, dx, dy, dz, sign, live);
     else
-      vel_yl_body<MODE, TY, CZ, S>(ly, D, i, j0, k0, dx, dy, dz, sign, gnx, gny, gnz, R, live);
+      vel_yl_body<MODE, TY, CZ, S>(ly, D, i, j0, k0, dx, dy, dz, sign, live);
   } else {
-    vel_yl_body<MODE, TY, CZ, S>(ly, D, i, j0, k0, dx, dy, dz, sign, gnx, gny, gnz, R, live);
+    vel_yl_body<MODE, TY, CZ, S>(ly, D, i, j0, k0, dx, dy, dz, sign, live);
   }
 }
 
@@ -1364,8 +1270,8 @@ __device__ __forceinline__ bool zbrick2(const PhyDesc &D, int t, int &i, int &j0
   return i < D.nx;
 }
 template <int TX, int TY, int CY, int CZ>
-__device__ __forceinline__ bool brick2_full_order(const PhyDesc &D, int t, int gnx, int gny, int gnz, int R) {
-  if (R >= 4) return true;
+__device__ __forceinline__ bool brick2_full_order(const PhyDesc &D, int t) {
+  if (D.R >= 4) return true;
   const int tiles_x = (D.nx + 2 * TX - 1) / (2 * TX);
   const int tiles_y = (D.ny + TY * CY - 1) / (TY * CY);
   const int per = tiles_x * tiles_y;
@@ -1373,15 +1279,15 @@ __device__ __forceinline__ bool brick2_full_order(const PhyDesc &D, int t, int g
   const int rem = t - zc * per;
   const int ty = rem / tiles_x;
   const int tx = rem - ty * tiles_x;
-  const int x0 = D.gx + tx * 2 * TX, x1 = D.gx + min(tx * 2 * TX + 2 * TX, D.nx) - 1;
-  const int y0 = D.gy + ty * TY * CY, y1 = D.gy + min((ty + 1) * TY * CY, D.ny) - 1;
-  const int z0 = D.gz + zc * CZ, z1 = D.gz + min(zc * CZ + CZ, D.nz) - 1;
-  return x0 >= 3 && x1 <= gnx - 4 && y0 >= 3 && y1 <= gny - 4 && z0 >= 3 && z1 <= gnz - 4;
+  const int x0 = tx * 2 * TX, x1 = min(tx * 2 * TX + 2 * TX, D.nx) - 1;
+  const int y0 = ty * TY * CY, y1 = min((ty + 1) * TY * CY, D.ny) - 1;
+  const int z0 = zc * CZ, z1 = min(zc * CZ + CZ, D.nz) - 1;
+  return x0 >= 3 && x1 <= D.nx - 4 && y0 >= 3 && y1 <= D.ny - 4 && z0 >= 3 && z1 <= D.nz - 4;
 }
 
 template <int MODE, int TX, int TY, int CY, int CZ, class S>
 __device__ __forceinline__ void vel_zb2_body(const PhyDesc &D, int i, int j0, int k0, float dx, float dy, float dz,
-                                             float sign, int gnx, int gny, int gnz, int R) {
+                                             float sign) {
   static_assert(MODE != FWI, "the FWI mode runs on the one-cell bricks");
   typedef typename GPtr<S>::T gT;
   const long sy = D.sy, sz = D.sz;
@@ -1402,13 +1308,13 @@ __device__ __forceinline__ void vel_zb2_body(const PhyDesc &D, int i, int j0, in
   constexpr bool P = (MODE == RTM_BACKWARD || MODE == RTM_REVERSE);
   const bool both = i + 1 < D.nx;
   const Coef4 c4 = coef_row(4);
-  const Coef4 cxa = MODE == RTM_BACKWARD ? coef_row(vowr_order(D.gx + i, gnx, R)) : c4;
-  const Coef4 cxb = MODE == RTM_BACKWARD ? coef_row(vowr_order(D.gx + i + 1, gnx, R)) : c4;
+  const Coef4 cxa = MODE == RTM_BACKWARD ? coef_row(vowr_order(i, D.nx, D.R)) : c4;
+  const Coef4 cxb = MODE == RTM_BACKWARD ? coef_row(vowr_order(i + 1, D.nx, D.R)) : c4;
 #pragma unroll
   for (int q = 0; q < CY; q++) {
     const int j = j0 + q * TY;
     if (j >= D.ny) continue;
-    const Coef4 cy = MODE == RTM_BACKWARD ? coef_row(vowr_order(D.gy + j, gny, R)) : c4;
+    const Coef4 cy = MODE == RTM_BACKWARD ? coef_row(vowr_order(j, D.ny, D.R)) : c4;
     const long base = (long)(D.ox + i) + sy * (D.oy + j) + sz * (D.oz + k0);
     float zzza[CZ + 7], zzzb[CZ + 7], zxza[CZ + 7], zxzb[CZ + 7], zyza[CZ + 7], zyzb[CZ + 7];
     float zsaa[P ? CZ + 7 : 1], zsab[P ? CZ + 7 : 1];
@@ -1420,7 +1326,7 @@ __device__ __forceinline__ void vel_zb2_body(const PhyDesc &D, int i, int j0, in
     for (int kk = 0; kk < CZ; kk++) {
       const int k = k0 + kk;
       if (k >= D.nz) break;
-      const Coef4 cz = MODE == RTM_BACKWARD ? coef_row(vowr_order(D.gz + k, gnz, R)) : c4;
+      const Coef4 cz = MODE == RTM_BACKWARD ? coef_row(vowr_order(k, D.nz, D.R)) : c4;
       const long id = base + (long)kk * sz;
       const F2 ovx = ld2_nt(fvx, id), ovy = ld2_nt(fvy, id), ovz = ld2_nt(fvz, id);
       F2 ovxp{0.f, 0.f}, ovyp{0.f, 0.f}, ovzp{0.f, 0.f};
@@ -1464,13 +1370,6 @@ __device__ __forceinline__ void vel_zb2_body(const PhyDesc &D, int i, int j0, in
       st2_nt(fvx, id, nxa, nxb, both);
       st2_nt(fvy, id, nya, nyb, both);
       st2_nt(fvz, id, nza, nzb, both);
-      if (D.mir) {
-        const MirCell ma = mir_cell(D.mir, D.ox + i, D.oy + j, D.oz + k);
-        const MirCell mb = mir_cell(D.mir, D.ox + i + 1, D.oy + j, D.oz + k);
-        mir_pair<gT>(ma, mb, both, VX, nxa, nxb);
-        mir_pair<gT>(ma, mb, both, VY, nya, nyb);
-        mir_pair<gT>(ma, mb, both, VZ, nza, nzb);
-      }
       if constexpr (P) {
         st2_nt(fvxp, id, ovxp.a + aa * sx.a, ovxp.b + ab * sx.b, both);
         st2_nt(fvyp, id, ovyp.a + ba * sy_.a, ovyp.b + bb * sy_.b, both);
@@ -1482,7 +1381,7 @@ __device__ __forceinline__ void vel_zb2_body(const PhyDesc &D, int i, int j0, in
 
 template <int MODE, int TX, int TY, int CY, int CZ, class S>
 __device__ __forceinline__ void stress_zb2_body(const PhyDesc &D, int i, int j0, int k0, float dx, float dy,
-                                                float dz, float dt, int gnx, int gny, int gnz, int R) {
+                                                float dz, float dt) {
   static_assert(MODE != FWI, "the FWI mode runs on the one-cell bricks");
   typedef typename GPtr<S>::T gT;
   const long sy = D.sy, sz = D.sz;
@@ -1501,13 +1400,13 @@ __device__ __forceinline__ void stress_zb2_body(const PhyDesc &D, int i, int j0,
   const float a = dt / dx, bb = dt / dy, c = dt / dz;
   const bool both = i + 1 < D.nx;
   const Coef4 c4 = coef_row(4);
-  const Coef4 cxa = MODE == RTM_BACKWARD ? coef_row(vowr_order(D.gx + i, gnx, R)) : c4;
-  const Coef4 cxb = MODE == RTM_BACKWARD ? coef_row(vowr_order(D.gx + i + 1, gnx, R)) : c4;
+  const Coef4 cxa = MODE == RTM_BACKWARD ? coef_row(vowr_order(i, D.nx, D.R)) : c4;
+  const Coef4 cxb = MODE == RTM_BACKWARD ? coef_row(vowr_order(i + 1, D.nx, D.R)) : c4;
 #pragma unroll
   for (int q = 0; q < CY; q++) {
     const int j = j0 + q * TY;
     if (j >= D.ny) continue;
-    const Coef4 cy = MODE == RTM_BACKWARD ? coef_row(vowr_order(D.gy + j, gny, R)) : c4;
+    const Coef4 cy = MODE == RTM_BACKWARD ? coef_row(vowr_order(j, D.ny, D.R)) : c4;
     const long base = (long)(D.ox + i) + sy * (D.oy + j) + sz * (D.oz + k0);
     float zxa[CZ + 7], zxb[CZ + 7], zya[CZ + 7], zyb[CZ + 7], zza[CZ + 7], zzb[CZ + 7];
     load_zcol2<CZ>(zxa, zxb, vx, base, sz, k0, -3, D.nz);  // vx, vy: forward-staggered in z
@@ -1517,7 +1416,7 @@ __device__ __forceinline__ void stress_zb2_body(const PhyDesc &D, int i, int j0,
     for (int kk = 0; kk < CZ; kk++) {
       const int k = k0 + kk;
       if (k >= D.nz) break;
-      const Coef4 cz = MODE == RTM_BACKWARD ? coef_row(vowr_order(D.gz + k, gnz, R)) : c4;
+      const Coef4 cz = MODE == RTM_BACKWARD ? coef_row(vowr_order(k, D.nz, D.R)) : c4;
       const long id = base + (long)kk * sz;
       const F2 oxx = ld2_nt(fsxx, id), oyy = ld2_nt(fsyy, id), ozz = ld2_nt(fszz, id);
       const F2 oxy = ld2_nt(fsxy, id), oxz = ld2_nt(fsxz, id), oyz = ld2_nt(fsyz, id);
@@ -1559,17 +1458,6 @@ __device__ __forceinline__ void stress_zb2_body(const PhyDesc &D, int i, int j0,
       st2_nt(fsxz, id, nxza, nxzb, both);
       st2_nt(fsyz, id, nyza, nyzb, both);
       if constexpr (rtm_mode(MODE)) st2_nt(fsau, id, naua, naub, both);
-      if (D.mir) {
-        const MirCell ma = mir_cell(D.mir, D.ox + i, D.oy + j, D.oz + k);
-        const MirCell mb = mir_cell(D.mir, D.ox + i + 1, D.oy + j, D.oz + k);
-        mir_pair<gT>(ma, mb, both, SXX, nxxa, nxxb);
-        mir_pair<gT>(ma, mb, both, SYY, nyya, nyyb);
-        mir_pair<gT>(ma, mb, both, SZZ, nzza, nzzb);
-        mir_pair<gT>(ma, mb, both, SXY, nxya, nxyb);
-        mir_pair<gT>(ma, mb, both, SXZ, nxza, nxzb);
-        mir_pair<gT>(ma, mb, both, SYZ, nyza, nyzb);
-        if constexpr (rtm_mode(MODE)) mir_pair<gT>(ma, mb, both, SAU, naua, naub);
-      }
     }
   }
 }
@@ -1577,32 +1465,29 @@ __device__ __forceinline__ void stress_zb2_body(const PhyDesc &D, int i, int j0,
 template <int MODE, int TX, int TY, int CY, int CZ, class S>
 __global__ __launch_bounds__(TX *TY) DDX_BRICK_ATTR void k_vel_phy_zb2(const PhyDesc *__restrict__ descs,
                                                         const int *__restrict__ starts, int n, float dx, float dy,
-                                                        float dz, float sign, int gnx, int gny, int gnz, int R) {
-  const int b = brick_block(blockIdx.x, gridDim.x);
+                                                        float dz, float sign, int grp) {
+  const int b = brick_block(blockIdx.x, gridDim.x, grp);
   const PhyDesc &D = descs[find_desc(starts, n, b)];
-  gnx = D.gnx; gny = D.gny; gnz = D.gnz; R = D.R;  // per descriptor: fused batches mix grids
   int i, j0, k0;
   if (!zbrick2<TX, TY, CY, CZ>(D, b - D.blk0, i, j0, k0)) return;
-  if (MODE == RTM_BACKWARD && brick2_full_order<TX, TY, CY, CZ>(D, b - D.blk0, gnx, gny, gnz, R))
-    vel_zb2_body<RTM_REVERSE, TX, TY, CY, CZ, S>(D, i, j0, k0, dx, dy, dz, sign, gnx, gny, gnz, R);
+  if (MODE == RTM_BACKWARD && brick2_full_order<TX, TY, CY, CZ>(D, b - D.blk0))
+    vel_zb2_body<RTM_REVERSE, TX, TY, CY, CZ, S>(D, i, j0, k0, dx, dy, dz, sign);
   else
-    vel_zb2_body<MODE, TX, TY, CY, CZ, S>(D, i, j0, k0, dx, dy, dz, sign, gnx, gny, gnz, R);
+    vel_zb2_body<MODE, TX, TY, CY, CZ, S>(D, i, j0, k0, dx, dy, dz, sign);
 }
 
 template <int MODE, int TX, int TY, int CY, int CZ, class S>
 __global__ __launch_bounds__(TX *TY) DDX_BRICK_ATTR void k_stress_phy_zb2(const PhyDesc *__restrict__ descs,
                                                            const int *__restrict__ starts, int n, float dx,
-                                                           float dy, float dz, float dt, int gnx, int gny, int gnz,
-                                                           int R) {
-  const int b = brick_block(blockIdx.x, gridDim.x);
+                                                           float dy, float dz, float dt, int grp) {
+  const int b = brick_block(blockIdx.x, gridDim.x, grp);
   const PhyDesc &D = descs[find_desc(starts, n, b)];
-  gnx = D.gnx; gny = D.gny; gnz = D.gnz; R = D.R;  // per descriptor: fused batches mix grids
   int i, j0, k0;
   if (!zbrick2<TX, TY, CY, CZ>(D, b - D.blk0, i, j0, k0)) return;
-  if (MODE == RTM_BACKWARD && brick2_full_order<TX, TY, CY, CZ>(D, b - D.blk0, gnx, gny, gnz, R))
-    stress_zb2_body<RTM_REVERSE, TX, TY, CY, CZ, S>(D, i, j0, k0, dx, dy, dz, dt, gnx, gny, gnz, R);
+  if (MODE == RTM_BACKWARD && brick2_full_order<TX, TY, CY, CZ>(D, b - D.blk0))
+    stress_zb2_body<RTM_REVERSE, TX, TY, CY, CZ, S>(D, i, j0, k0, dx, dy, dz, dt);
   else
-    stress_zb2_body<MODE, TX, TY, CY, CZ, S>(D, i, j0, k0, dx, dy, dz, dt, gnx, gny, gnz, R);
+    stress_zb2_body<MODE, TX, TY, CY, CZ, S>(D, i, j0, k0, dx, dy, dz, dt);
 }
 
 // ---------------------------------------------------------------------------
@@ -1649,7 +1534,7 @@ __device__ __forceinline__ LdsMap lds_map(const PhyDesc &D, int x0, int y0) {
 template <int MODE>
 __global__ __launch_bounds__(LX *LY) void k_vel_lds(const PhyDesc *__restrict__ descs,
                                                     const int *__restrict__ starts, int n, float dx, float dy,
-                                                    float dz, float sign, int gnx, int gny, int gnz, int R,
+                                                    float dz, float sign,
                                                     int kz) {
   constexpr bool P = (MODE == RTM_BACKWARD || MODE == RTM_REVERSE);
   __shared__ float Lxx[2][LY][HXW];
@@ -1660,7 +1545,6 @@ __global__ __launch_bounds__(LX *LY) void k_vel_lds(const PhyDesc *__restrict__ 
   __shared__ float Lsa[P ? 2 : 1][P ? HYW : 1][P ? HXW : 1];
   const int b = xcd_remap(blockIdx.x, gridDim.x);
   const PhyDesc &D = descs[find_desc(starts, n, b)];
-  gnx = D.gnx; gny = D.gny; gnz = D.gnz; R = D.R;  // per descriptor: fused batches mix grids
   const int t = b - D.blk0;
   const int tiles_x = (D.nx + LX - 1) / LX, tiles_y = (D.ny + LY - 1) / LY, per = tiles_x * tiles_y;
   const int zc = t / per, rem = t - zc * per, tyi = rem / tiles_x, txi = rem - tyi * tiles_x;
@@ -1674,8 +1558,8 @@ __global__ __launch_bounds__(LX *LY) void k_vel_lds(const PhyDesc *__restrict__ 
   const long hb = (long)(D.ox + m.i) + sy * (D.oy + m.hrow) + sz * D.oz;     // y-halo base
   const long xb = (long)(D.ox + m.xcol) + sy * (D.oy + y0 + m.xr) + sz * D.oz;  // x-halo base
   const Coef4 c4 = coef_row(4);
-  const Coef4 cx = MODE == RTM_BACKWARD ? coef_row(vowr_order(D.gx + min(m.i, D.nx - 1), gnx, R)) : c4;
-  const Coef4 cy = MODE == RTM_BACKWARD ? coef_row(vowr_order(D.gy + min(m.j, D.ny - 1), gny, R)) : c4;
+  const Coef4 cx = MODE == RTM_BACKWARD ? coef_row(vowr_order(min(m.i, D.nx - 1), D.nx, D.R)) : c4;
+  const Coef4 cy = MODE == RTM_BACKWARD ? coef_row(vowr_order(min(m.j, D.ny - 1), D.ny, D.R)) : c4;
   // z-arm queues: qzz, qsa planes k-3..k+4; qxz, qyz planes k-4..k+3
   float qzz[8], qxz[8], qyz[8], qsa[8];
 #pragma unroll
@@ -1738,7 +1622,7 @@ __global__ __launch_bounds__(LX *LY) void k_vel_lds(const PhyDesc *__restrict__ 
     }
     if (m.comp) {
       const long id = cb + (long)k * sz;
-      const Coef4 cz = MODE == RTM_BACKWARD ? coef_row(vowr_order(D.gz + k, gnz, R)) : c4;
+      const Coef4 cz = MODE == RTM_BACKWARD ? coef_row(vowr_order(k, D.nz, D.R)) : c4;
       const float dtr = sign * fdtr[id];
       const float a = dtr / dx, bb = dtr / dy, c = dtr / dz;
       const int X = tx + 4, Y = ty + 4;
@@ -1828,14 +1712,13 @@ __global__ __launch_bounds__(LX *LY) void k_vel_lds(const PhyDesc *__restrict__ 
 template <int MODE>
 __global__ __launch_bounds__(LX *LY) void k_stress_lds(const PhyDesc *__restrict__ descs,
                                                        const int *__restrict__ starts, int n, float dx, float dy,
-                                                       float dz, float dt, int gnx, int gny, int gnz, int R,
+                                                       float dz, float dt,
                                                        int kz) {
   __shared__ float Lx[2][HYW][HXW];
   __shared__ float Ly[2][HYW][HXW];
   __shared__ float Lz[2][HYW][HXW];
   const int b = xcd_remap(blockIdx.x, gridDim.x);
   const PhyDesc &D = descs[find_desc(starts, n, b)];
-  gnx = D.gnx; gny = D.gny; gnz = D.gnz; R = D.R;  // per descriptor: fused batches mix grids
   const int t = b - D.blk0;
   const int tiles_x = (D.nx + LX - 1) / LX, tiles_y = (D.ny + LY - 1) / LY, per = tiles_x * tiles_y;
   const int zc = t / per, rem = t - zc * per, tyi = rem / tiles_x, txi = rem - tyi * tiles_x;
@@ -1849,8 +1732,8 @@ __global__ __launch_bounds__(LX *LY) void k_stress_lds(const PhyDesc *__restrict
   const long xb = (long)(D.ox + m.xcol) + sy * (D.oy + y0 + m.xr) + sz * D.oz;
   const float a = dt / dx, bb = dt / dy, c = dt / dz;
   const Coef4 c4 = coef_row(4);
-  const Coef4 cx = MODE == RTM_BACKWARD ? coef_row(vowr_order(D.gx + min(m.i, D.nx - 1), gnx, R)) : c4;
-  const Coef4 cy = MODE == RTM_BACKWARD ? coef_row(vowr_order(D.gy + min(m.j, D.ny - 1), gny, R)) : c4;
+  const Coef4 cx = MODE == RTM_BACKWARD ? coef_row(vowr_order(min(m.i, D.nx - 1), D.nx, D.R)) : c4;
+  const Coef4 cy = MODE == RTM_BACKWARD ? coef_row(vowr_order(min(m.j, D.ny - 1), D.ny, D.R)) : c4;
   // queues: qx, qy planes k-3..k+4 (forward-staggered in z), qz planes k-4..k+3
   float qx[8], qy[8], qz[8];
 #pragma unroll
@@ -1894,7 +1777,7 @@ __global__ __launch_bounds__(LX *LY) void k_stress_lds(const PhyDesc *__restrict
     }
     if (m.comp) {
       const long id = cb + (long)k * sz;
-      const Coef4 cz = MODE == RTM_BACKWARD ? coef_row(vowr_order(D.gz + k, gnz, R)) : c4;
+      const Coef4 cz = MODE == RTM_BACKWARD ? coef_row(vowr_order(k, D.nz, D.R)) : c4;
       const float lm = flam[id], mu = fmu[id];
       const float l2m = lm + 2.0f * mu;
       const int X = tx + 4, Y = ty + 4;
@@ -2165,10 +2048,6 @@ __global__ __launch_bounds__(kBlock) DDX_PML_ATTR void k_vel_pml(const SlabDesc 
     stq(fvx, id, nv[kk][0]);
     stq(fvy, id, nv[kk][1]);
     stq(fvz, id, nv[kk][2]);
-    if (D.mir) {
-      const MirCell m = mir_cell(D.mir, ei, ej, ek);
-      if (m.any) { mir_put<gT>(m, VX, nv[kk][0]); mir_put<gT>(m, VY, nv[kk][1]); mir_put<gT>(m, VZ, nv[kk][2]); }
-    }
   }
 }
 
@@ -2289,14 +2168,6 @@ __global__ __launch_bounds__(kBlock) DDX_PML_ATTR void k_stress_pml(const SlabDe
     stq(fsxy, id, ns[kk][4]);
     stq(fsxz, id, ns[kk][5]);
     stq(fsyz, id, ns[kk][6]);
-    if (D.mir) {
-      const MirCell m = mir_cell(D.mir, ei, ej, ek);
-      if (m.any) {
-        mir_put<gT>(m, SXX, ns[kk][0]); mir_put<gT>(m, SYY, ns[kk][1]); mir_put<gT>(m, SZZ, ns[kk][2]);
-        if (WITH_SAU) mir_put<gT>(m, SAU, ns[kk][3]);
-        mir_put<gT>(m, SXY, ns[kk][4]); mir_put<gT>(m, SXZ, ns[kk][5]); mir_put<gT>(m, SYZ, ns[kk][6]);
-      }
-    }
   }
 }
 
@@ -2541,10 +2412,6 @@ __global__ __launch_bounds__(kBlock) DDX_PML_ATTR void k_vel_pml_t(const SlabDes
       stq(fvx, id, nv0);
       stq(fvy, id, nv1);
       stq(fvz, id, nv2);
-      if (D.mir) {
-        const MirCell m = mir_cell(D.mir, ei, ej, D.k0 + T.kc0 + kk);
-        if (m.any) { mir_put<gfloat>(m, VX, nv0); mir_put<gfloat>(m, VY, nv1); mir_put<gfloat>(m, VZ, nv2); }
-      }
     }
     if (more) {
       fill(b ^ 1, N);
@@ -2720,14 +2587,6 @@ __global__ __launch_bounds__(kBlock) DDX_PML_ATTR void k_stress_pml_t(const Slab
       stq(fsxy, id, ns[4]);
       stq(fsxz, id, ns[5]);
       stq(fsyz, id, ns[6]);
-      if (D.mir) {
-        const MirCell m = mir_cell(D.mir, ei, ej, D.k0 + T.kc0 + kk);
-        if (m.any) {
-          mir_put<gfloat>(m, SXX, ns[0]); mir_put<gfloat>(m, SYY, ns[1]); mir_put<gfloat>(m, SZZ, ns[2]);
-          if (WITH_SAU) mir_put<gfloat>(m, SAU, ns[3]);
-          mir_put<gfloat>(m, SXY, ns[4]); mir_put<gfloat>(m, SXZ, ns[5]); mir_put<gfloat>(m, SYZ, ns[6]);
-        }
-      }
     }
     if (more) {
       fill(b ^ 1, N);
@@ -2737,74 +2596,12 @@ __global__ __launch_bounds__(kBlock) DDX_PML_ATTR void k_stress_pml_t(const Slab
   }
 }
 
-// ---------------------------------------------------------------------------
-// CMM halo exchange between subdomains on one device
-// (OP/jarvis_2_mpicu_halo_comm_operator_meat.hpp:299-326 extract into the
-// send block, then the receiver's ghost layers): one copy per element from
-// the sender's boundary layers to the receiver's ghosts, all links of a
-// batch in one launch.  Boxes hold fewer than 2^31 elements (32-bit math).
-// ---------------------------------------------------------------------------
-// E: element type (float, or the 16-bit code of the 16-bit formats).  The
-// copy walks rows (j, k) of the box, row index j + nj k.  Narrow boxes (the
-// x-face links: 3-4 cells per row) take one cell per thread, a row's cells
-// on consecutive lanes (measured: one row per thread, 45 us per exchange
-// against 35, since each of its loads then touches 64 lines); wide boxes
-// take one row per wavefront, lanes 64 cells apart, up to four loads in
-// flight per lane before their stores, with no per-cell index division.
-template <typename E>
-__global__ __launch_bounds__(kBlock) void k_halo(const HaloDesc *__restrict__ descs,
-                                                 const int *__restrict__ starts, int n) {
-  typedef __attribute__((address_space(1))) E gE;
-  const int b = blockIdx.x;
-  const HaloDesc &D = descs[find_desc(starts, n, b)];
-  const int rows = D.nj * D.nk;
-  const gE *__restrict__ src = (const gE *)D.src;
-  gE *__restrict__ dst = (gE *)D.dst;
-  if (D.ni <= kHaloNarrow) {
-    // consecutive lanes take consecutive cells, so the lanes of one row
-    // share each load's cache line
-    const int e = (b - D.blk0) * kBlock + (int)threadIdx.x;
-    if (e >= rows * D.ni) return;
-    const int row = e / D.ni, i = e - row * D.ni;
-    const int k = row / D.nj, j = row - k * D.nj;
-    const long s = (long)(D.si + i) + D.ssy * (D.sj + j) + D.ssz * (D.sk + k);
-    const long d = (long)(D.di + i) + D.dsy * (D.dj + j) + D.dsz * (D.dk + k);
-    dst[d] = src[s];
-    return;
-  }
-  const int row = (b - D.blk0) * (kBlock / 64) + (int)(threadIdx.x >> 6);
-  if (row >= rows) return;
-  const int lane = (int)(threadIdx.x & 63);
-  const int k = row / D.nj, j = row - k * D.nj;
-  const long s = (long)D.si + D.ssy * (D.sj + j) + D.ssz * (D.sk + k);
-  const long d = (long)D.di + D.dsy * (D.dj + j) + D.dsz * (D.dk + k);
-  for (int i0 = 0; i0 < D.ni; i0 += 256) {
-    E v[4];
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int i = i0 + 64 * q + lane;
-      if (i < D.ni) v[q] = src[s + i];
-    }
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int i = i0 + 64 * q + lane;
-      if (i < D.ni) dst[d + i] = v[q];
-    }
-  }
-}
-
+#if DDX_PART == 0
 // ---------------------------------------------------------------------------
 // Box <-> contiguous buffer copies (FLD/jarvis_3_device_field_meat.hpp:23-60):
 // the VOWR boundary save / inject (BASE/fdtd3d_base_5_wave_recon_meat.hpp:89-133).  Boxes are walked
 // x-fastest, so both sides of every copy are coalesced along x.
 // ---------------------------------------------------------------------------
-// Buffer element of box element (i, j, k): the box may be a sub-box of the
-// buffer's box (CopyDesc::bi..bnj); for a whole box this is buf_off + the
-// element's x-fastest index.
-__device__ __forceinline__ long buf_index(const CopyDesc &D, int i, int j, int k) {
-  return D.buf_off + (long)(D.bi + i) + (long)D.bni * ((long)(D.bj + j) + (long)D.bnj * (D.bk + k));
-}
-
 template <int DIR, typename E>
 __global__ __launch_bounds__(kBlock) void k_copy(const CopyDesc *__restrict__ descs,
                                                  const int *__restrict__ starts, int n, void *__restrict__ buf) {
@@ -2820,7 +2617,7 @@ __global__ __launch_bounds__(kBlock) void k_copy(const CopyDesc *__restrict__ de
   const int i = e - r * D.ni;
   const int j = r - k * D.nj;
   const long id = (long)(D.i0 + i) + D.sy * (D.j0 + j) + D.sz * (D.k0 + k);
-  const long bo = buf_index(D, i, j, k);
+  const long bo = D.buf_off + e;
   if (DIR > 0) ((gE *)buf)[bo] = ((const gE *)D.field)[id];
   else ((gE *)D.field)[id] = ((const gE *)buf)[bo];
 }
@@ -2846,7 +2643,7 @@ __global__ __launch_bounds__(kBlock) void k_copy_conv(const CopyDesc *__restrict
   const long id = (long)(D.i0 + i) + D.sy * (D.j0 + j) + D.sz * (D.k0 + k);
   const float sc = D.cls == 0 ? sc_v : sc_s;
   gT *ring = (gT *)buf;
-  const long bo = buf_index(D, i, j, k);
+  const long bo = D.buf_off + e;
   if (DIR > 0) stq(ring, bo, G(D.field)[id] * sc);
   else G(D.field)[id] = ld(ring, bo) * (1.0f / sc);
 }
@@ -2912,7 +2709,7 @@ __global__ __launch_bounds__(kBlock) void k_copy_dyn(const CopyDesc *__restrict_
   const long id = (long)(D.i0 + i) + D.sy * (D.j0 + j) + D.sz * (D.k0 + k);
   const float sc = ldexpf(1.0f, exps[D.fid]);
   gT *ring = (gT *)buf;
-  const long bo = buf_index(D, i, j, k);
+  const long bo = D.buf_off + e;
   if (DIR > 0) stq(ring, bo, G(D.field)[id] * sc);
   else G(D.field)[id] = ld(ring, bo) * (1.0f / sc);
 }
@@ -3004,7 +2801,7 @@ __global__ __launch_bounds__(kBlock) void k_inject_bfp(const CopyDesc *__restric
   const int i = e - r * D.ni;
   const int j = r - k * D.nj;
   const long id = (long)(D.i0 + i) + D.sy * (D.j0 + j) + D.sz * (D.k0 + k);
-  const long bo = buf_index(D, i, j, k);
+  const long bo = D.buf_off + e;
   G(D.field)[id] = bfp_value(((const gshort *)buf)[bo], bexp[bo / kRingBlock]);
 }
 
@@ -3247,6 +3044,7 @@ __global__ __launch_bounds__(kBlock) void k_compensate(const ImgDesc *__restrict
     }
   }
 }
+#endif  // DDX_PART == 0
 
 // ---------------------------------------------------------------------------
 // Launchers
@@ -3264,6 +3062,7 @@ __global__ __launch_bounds__(kBlock) void k_compensate(const ImgDesc *__restrict
 // lane-exchange bricks (xl: x arm from neighbouring lanes, tx = 64), FP32
 #define DDX_TILINGSX(X) X(64, 4, 1, 2) X(64, 4, 1, 4) X(64, 4, 1, 8) X(64, 8, 1, 4) X(64, 2, 1, 8)
 
+#if DDX_PART == 0
 bool tiling_supported(const Tiling &t, int fmt) {
   if (t.xl == 2) {
     if (t.px != 1 || fmt != STORE_F32 || t.tx != 64 || t.cy != 1) return false;
@@ -3327,77 +3126,66 @@ int tiling_list(int fmt, Tiling *out, int max) {
   }
   return n;
 }
+#endif
+
+// Launch of one brick shape: the kernel of each mode (K: kernel template, PF:
+// the mode whose kernel the pure-forward and RTM-forward passes share or not).
+#define DDX_ARGS d, starts, n, dx, dy, dz, sc, grp
+#define DDX_SIG                                                                                              \
+  const Tiling &t, int mode, int fmt, dim3 g, hipStream_t st, const PhyDesc *d, const int *starts, int n,    \
+      float dx, float dy, float dz, float sc, int grp
+#define DDX_PASS t, mode, fmt, g, st, d, starts, n, dx, dy, dz, sc, grp
 
 template <int TX, int TY, int CY, int CZ, class S, bool XL = false>
-static void vel_zb(int mode, dim3 g, hipStream_t st, const PhyDesc *d, const int *starts, int n, float dx, float dy,
-                   float dz, float sign, int gnx, int gny, int gnz, int R) {
+static void vel_zb(DDX_SIG) {
   dim3 bl(TX * TY);
   switch (mode) {
     case PURE_FORWARD:
     case RTM_FORWARD:
-      hipLaunchKernelGGL((k_vel_phy_zb<PURE_FORWARD, TX, TY, CY, CZ, S, XL>), g, bl, 0, st, d, starts, n, dx, dy, dz, sign,
-                         gnx, gny, gnz, R);
+      hipLaunchKernelGGL((k_vel_phy_zb<PURE_FORWARD, TX, TY, CY, CZ, S, XL>), g, bl, 0, st, DDX_ARGS);
       break;
     case RTM_BACKWARD:
-      hipLaunchKernelGGL((k_vel_phy_zb<RTM_BACKWARD, TX, TY, CY, CZ, S, XL>), g, bl, 0, st, d, starts, n, dx, dy, dz, sign,
-                         gnx, gny, gnz, R);
+      hipLaunchKernelGGL((k_vel_phy_zb<RTM_BACKWARD, TX, TY, CY, CZ, S, XL>), g, bl, 0, st, DDX_ARGS);
       break;
     case FWI:
       if constexpr (std::is_same<S, F32>::value && !XL)
-        hipLaunchKernelGGL((k_vel_phy_zb<FWI, TX, TY, CY, CZ, F32>), g, bl, 0, st, d, starts, n, dx, dy, dz, sign, gnx,
-                           gny, gnz, R);
+        hipLaunchKernelGGL((k_vel_phy_zb<FWI, TX, TY, CY, CZ, F32>), g, bl, 0, st, DDX_ARGS);
       break;
     default:
-      hipLaunchKernelGGL((k_vel_phy_zb<RTM_REVERSE, TX, TY, CY, CZ, S, XL>), g, bl, 0, st, d, starts, n, dx, dy, dz, sign,
-                         gnx, gny, gnz, R);
+      hipLaunchKernelGGL((k_vel_phy_zb<RTM_REVERSE, TX, TY, CY, CZ, S, XL>), g, bl, 0, st, DDX_ARGS);
   }
 }
 
+// (FWI: the stress update is the pure-forward one)
 template <int TX, int TY, int CY, int CZ, class S, bool XL = false>
-static void stress_zb(int mode, dim3 g, hipStream_t st, const PhyDesc *d, const int *starts, int n, float dx,
-                      float dy, float dz, float dt, int gnx, int gny, int gnz, int R) {
+static void stress_zb(DDX_SIG) {
   dim3 bl(TX * TY);
   switch (mode) {
     case PURE_FORWARD:
-      hipLaunchKernelGGL((k_stress_phy_zb<PURE_FORWARD, TX, TY, CY, CZ, S, XL>), g, bl, 0, st, d, starts, n, dx, dy, dz,
-                         dt, gnx, gny, gnz, R);
-      break;
-    case RTM_FORWARD:
-      hipLaunchKernelGGL((k_stress_phy_zb<RTM_FORWARD, TX, TY, CY, CZ, S, XL>), g, bl, 0, st, d, starts, n, dx, dy, dz,
-                         dt, gnx, gny, gnz, R);
+    case FWI:
+      hipLaunchKernelGGL((k_stress_phy_zb<PURE_FORWARD, TX, TY, CY, CZ, S, XL>), g, bl, 0, st, DDX_ARGS);
       break;
     case RTM_BACKWARD:
-      hipLaunchKernelGGL((k_stress_phy_zb<RTM_BACKWARD, TX, TY, CY, CZ, S, XL>), g, bl, 0, st, d, starts, n, dx, dy, dz,
-                         dt, gnx, gny, gnz, R);
-      break;
-    case FWI:
-      if constexpr (std::is_same<S, F32>::value && !XL)
-        hipLaunchKernelGGL((k_stress_phy_zb<FWI, TX, TY, CY, CZ, F32>), g, bl, 0, st, d, starts, n, dx, dy, dz, dt,
-                           gnx, gny, gnz, R);
+      hipLaunchKernelGGL((k_stress_phy_zb<RTM_BACKWARD, TX, TY, CY, CZ, S, XL>), g, bl, 0, st, DDX_ARGS);
       break;
     default:
-      hipLaunchKernelGGL((k_stress_phy_zb<RTM_REVERSE, TX, TY, CY, CZ, S, XL>), g, bl, 0, st, d, starts, n, dx, dy, dz,
-                         dt, gnx, gny, gnz, R);
+      hipLaunchKernelGGL((k_stress_phy_zb<RTM_REVERSE, TX, TY, CY, CZ, S, XL>), g, bl, 0, st, DDX_ARGS);
   }
 }
 
 template <int TX, int TY, int CY, int CZ, class S>
-static void vel_zb2(int mode, dim3 g, hipStream_t st, const PhyDesc *d, const int *starts, int n, float dx,
-                    float dy, float dz, float sign, int gnx, int gny, int gnz, int R) {
+static void vel_zb2(DDX_SIG) {
   dim3 bl(TX * TY);
   switch (mode) {
     case PURE_FORWARD:
     case RTM_FORWARD:
-      hipLaunchKernelGGL((k_vel_phy_zb2<PURE_FORWARD, TX, TY, CY, CZ, S>), g, bl, 0, st, d, starts, n, dx, dy, dz,
-                         sign, gnx, gny, gnz, R);
+      hipLaunchKernelGGL((k_vel_phy_zb2<PURE_FORWARD, TX, TY, CY, CZ, S>), g, bl, 0, st, DDX_ARGS);
       break;
     case RTM_BACKWARD:
-      hipLaunchKernelGGL((k_vel_phy_zb2<RTM_BACKWARD, TX, TY, CY, CZ, S>), g, bl, 0, st, d, starts, n, dx, dy, dz,
-                         sign, gnx, gny, gnz, R);
+      hipLaunchKernelGGL((k_vel_phy_zb2<RTM_BACKWARD, TX, TY, CY, CZ, S>), g, bl, 0, st, DDX_ARGS);
       break;
     case RTM_REVERSE:
-      hipLaunchKernelGGL((k_vel_phy_zb2<RTM_REVERSE, TX, TY, CY, CZ, S>), g, bl, 0, st, d, starts, n, dx, dy, dz,
-                         sign, gnx, gny, gnz, R);
+      hipLaunchKernelGGL((k_vel_phy_zb2<RTM_REVERSE, TX, TY, CY, CZ, S>), g, bl, 0, st, DDX_ARGS);
       break;
     default:
       break;  // FWI: one-cell bricks only
@@ -3405,257 +3193,183 @@ static void vel_zb2(int mode, dim3 g, hipStream_t st, const PhyDesc *d, const in
 }
 
 template <int TX, int TY, int CY, int CZ, class S>
-static void stress_zb2(int mode, dim3 g, hipStream_t st, const PhyDesc *d, const int *starts, int n, float dx,
-                       float dy, float dz, float dt, int gnx, int gny, int gnz, int R) {
+static void stress_zb2(DDX_SIG) {
   dim3 bl(TX * TY);
   switch (mode) {
     case PURE_FORWARD:
-      hipLaunchKernelGGL((k_stress_phy_zb2<PURE_FORWARD, TX, TY, CY, CZ, S>), g, bl, 0, st, d, starts, n, dx, dy, dz,
-                         dt, gnx, gny, gnz, R);
-      break;
-    case RTM_FORWARD:
-      hipLaunchKernelGGL((k_stress_phy_zb2<RTM_FORWARD, TX, TY, CY, CZ, S>), g, bl, 0, st, d, starts, n, dx, dy, dz,
-                         dt, gnx, gny, gnz, R);
+      hipLaunchKernelGGL((k_stress_phy_zb2<PURE_FORWARD, TX, TY, CY, CZ, S>), g, bl, 0, st, DDX_ARGS);
       break;
     case RTM_BACKWARD:
-      hipLaunchKernelGGL((k_stress_phy_zb2<RTM_BACKWARD, TX, TY, CY, CZ, S>), g, bl, 0, st, d, starts, n, dx, dy,
-                         dz, dt, gnx, gny, gnz, R);
+      hipLaunchKernelGGL((k_stress_phy_zb2<RTM_BACKWARD, TX, TY, CY, CZ, S>), g, bl, 0, st, DDX_ARGS);
       break;
+    case RTM_FORWARD:
     case RTM_REVERSE:
-      hipLaunchKernelGGL((k_stress_phy_zb2<RTM_REVERSE, TX, TY, CY, CZ, S>), g, bl, 0, st, d, starts, n, dx, dy, dz,
-                         dt, gnx, gny, gnz, R);
+      hipLaunchKernelGGL((k_stress_phy_zb2<RTM_REVERSE, TX, TY, CY, CZ, S>), g, bl, 0, st, DDX_ARGS);
       break;
     default:
       break;  // FWI: one-cell bricks only
   }
 }
+
+template <int TY, int CZ>
+static void vel_yl(DDX_SIG) {
+  const dim3 bl(64 * TY);
+  switch (mode) {
+    case PURE_FORWARD:
+    case RTM_FORWARD:
+      hipLaunchKernelGGL((k_vel_phy_yl<PURE_FORWARD, TY, CZ, F32>), g, bl, 0, st, DDX_ARGS);
+      break;
+    case RTM_BACKWARD:
+      hipLaunchKernelGGL((k_vel_phy_yl<RTM_BACKWARD, TY, CZ, F32>), g, bl, 0, st, DDX_ARGS);
+      break;
+    default:
+      hipLaunchKernelGGL((k_vel_phy_yl<RTM_REVERSE, TY, CZ, F32>), g, bl, 0, st, DDX_ARGS);
+  }
+}
+
+template <int TY, int CZ>
+static void stress_yl(DDX_SIG) {
+  const dim3 bl(64 * TY);
+  switch (mode) {
+    case PURE_FORWARD:
+      hipLaunchKernelGGL((k_stress_phy_yl<PURE_FORWARD, TY, CZ, F32>), g, bl, 0, st, DDX_ARGS);
+      break;
+    case RTM_BACKWARD:
+      hipLaunchKernelGGL((k_stress_phy_yl<RTM_BACKWARD, TY, CZ, F32>), g, bl, 0, st, DDX_ARGS);
+      break;
+    default:
+      hipLaunchKernelGGL((k_stress_phy_yl<RTM_REVERSE, TY, CZ, F32>), g, bl, 0, st, DDX_ARGS);
+  }
+}
+
+// The families of brick shapes, each compiled in a part of its own: one
+// cell per thread in FP32 and in the 16-bit formats, paired, lane-exchange
+// and LDS y arm.  False when the shape is not one of the family's.
+#define DDX_FAMILY(X) X(one) X(half) X(pair) X(lane) X(ylds)
+#define DDX_T(F) bool vel_##F(DDX_SIG); bool stress_##F(DDX_SIG);
+DDX_FAMILY(DDX_T)
+#undef DDX_T
+#define DDX_IS(TX, TY, CY, CZ) (t.tx == TX && t.ty == TY && t.cy == CY && t.kz == CZ)
+#define DDX_T1(TX, TY, CY, CZ) if (DDX_IS(TX, TY, CY, CZ)) return DDX_F<TX, TY, CY, CZ, F32>(DDX_PASS), true;
+#define DDX_T16(TX, TY, CY, CZ)                                                        \
+  if (DDX_IS(TX, TY, CY, CZ))                                                          \
+    return (fmt == STORE_F16 ? DDX_F<TX, TY, CY, CZ, F16> : DDX_F<TX, TY, CY, CZ, BF16>)(DDX_PASS), true;
+#define DDX_T2(TX, TY, CY, CZ)                                                         \
+  if (DDX_IS(TX, TY, CY, CZ))                                                          \
+    return (fmt == STORE_F16 ? DDX_F<TX, TY, CY, CZ, F16> : fmt == STORE_BF16 ? DDX_F<TX, TY, CY, CZ, BF16> \
+                                                                    : DDX_F<TX, TY, CY, CZ, F32>)(DDX_PASS), true;
+#define DDX_TX(TX, TY, CY, CZ) if (DDX_IS(TX, TY, CY, CZ)) return DDX_F<TX, TY, CY, CZ, F32, true>(DDX_PASS), true;
+#define DDX_TY(TY, CZ) if (DDX_IS(64, TY, 1, CZ)) return DDX_F<TY, CZ>(DDX_PASS), true;
+#if DDX_PART == 1
+#define DDX_F vel_zb
+bool vel_one(DDX_SIG) { DDX_TILINGS(DDX_T1) return false; }
+#elif DDX_PART == 2
+#define DDX_F stress_zb
+bool stress_one(DDX_SIG) { DDX_TILINGS(DDX_T1) return false; }
+#elif DDX_PART == 3
+#define DDX_F vel_zb
+bool vel_half(DDX_SIG) { DDX_TILINGS16(DDX_T16) return false; }
+#elif DDX_PART == 4
+#define DDX_F stress_zb
+bool stress_half(DDX_SIG) { DDX_TILINGS16(DDX_T16) return false; }
+#elif DDX_PART == 5
+#define DDX_F vel_zb2
+bool vel_pair(DDX_SIG) { DDX_TILINGS2(DDX_T2) return false; }
+#elif DDX_PART == 6
+#define DDX_F stress_zb2
+bool stress_pair(DDX_SIG) { DDX_TILINGS2(DDX_T2) return false; }
+#elif DDX_PART == 7
+#define DDX_F vel_zb
+bool vel_lane(DDX_SIG) { DDX_TILINGSX(DDX_TX) return false; }
+#undef DDX_F
+#define DDX_F vel_yl
+bool vel_ylds(DDX_SIG) { DDX_TILINGSY(DDX_TY) return false; }
+#elif DDX_PART == 8
+#define DDX_F stress_zb
+bool stress_lane(DDX_SIG) { DDX_TILINGSX(DDX_TX) return false; }
+#undef DDX_F
+#define DDX_F stress_yl
+bool stress_ylds(DDX_SIG) { DDX_TILINGSY(DDX_TY) return false; }
+#else
 
 // kz == 0 selects the one-plane-per-block kernels (k_vel_phy / k_stress_phy),
 // cy == 0 the LDS-tiled ones (both FP32 storage only).  FWI mode and the
 // 16-bit formats run on the z-blocked bricks only (the engine never selects
 // another shape for them).
 bool launch_vel_phy(const Tiling &t, int mode, int fmt, const PhyDesc *d, const int *starts, int n, int nblk,
-                    float dx, float dy, float dz, float sign, int gnx, int gny, int gnz, int R, hipStream_t st) {
+                    float dx, float dy, float dz, float sc, int grp, hipStream_t st) {
   if (nblk <= 0) return true;
   if ((mode == FWI || fmt != STORE_F32) && !(t.kz > 0 && t.cy > 0)) return false;
   if (mode == FWI && (t.px != 1 || t.xl)) return false;
   dim3 g(nblk), bl(kBlock);
-  if (t.xl == 2) {
-    if (fmt != STORE_F32 || t.tx != 64 || t.cy != 1) return false;
-#define DDX_T(TY, CZ)                                                                                  \
-  if (t.ty == TY && t.kz == CZ) {                                                                      \
-    const dim3 b2(64 * TY);                                                                            \
-    switch (mode) {                                                                                    \
-      case PURE_FORWARD:                                                                               \
-      case RTM_FORWARD:                                                                                \
-        hipLaunchKernelGGL((k_vel_phy_yl<PURE_FORWARD, TY, CZ, F32>), g, b2, 0, st, d, starts, n, dx, dy, dz, sign, gnx, gny, gnz, R); \
-        break;                                                                                         \
-      case RTM_BACKWARD:                                                                               \
-        hipLaunchKernelGGL((k_vel_phy_yl<RTM_BACKWARD, TY, CZ, F32>), g, b2, 0, st, d, starts, n, dx, dy, dz, sign, gnx, gny, gnz, R); \
-        break;                                                                                         \
-      default:                                                                                         \
-        hipLaunchKernelGGL((k_vel_phy_yl<RTM_REVERSE, TY, CZ, F32>), g, b2, 0, st, d, starts, n, dx, dy, dz, sign, gnx, gny, gnz, R); \
-    }                                                                                                  \
-    return true;                                                                                      \
-  }
-    DDX_TILINGSY(DDX_T)
-#undef DDX_T
-    return false;
-  }
-  if (t.xl) {
-    if (fmt != STORE_F32) return false;
-#define DDX_T(TX, TY, CY, CZ)                                                                         \
-  if (t.tx == TX && t.ty == TY && t.cy == CY && t.kz == CZ) {                                         \
-    vel_zb<TX, TY, CY, CZ, F32, true>(mode, g, st, d, starts, n, dx, dy, dz, sign, gnx, gny, gnz, R);  \
-    return true;                                                                                     \
-  }
-    DDX_TILINGSX(DDX_T)
-#undef DDX_T
-    return false;
-  }
-  if (t.px == 2) {
-#define DDX_T(TX, TY, CY, CZ)                                                                          \
-  if (t.tx == TX && t.ty == TY && t.cy == CY && t.kz == CZ) {                                          \
-    if (fmt == STORE_F16)                                                                              \
-      vel_zb2<TX, TY, CY, CZ, F16>(mode, g, st, d, starts, n, dx, dy, dz, sign, gnx, gny, gnz, R);     \
-    else if (fmt == STORE_BF16)                                                                        \
-      vel_zb2<TX, TY, CY, CZ, BF16>(mode, g, st, d, starts, n, dx, dy, dz, sign, gnx, gny, gnz, R);    \
-    else                                                                                               \
-      vel_zb2<TX, TY, CY, CZ, F32>(mode, g, st, d, starts, n, dx, dy, dz, sign, gnx, gny, gnz, R);     \
-    return true;                                                                                      \
-  }
-    DDX_TILINGS2(DDX_T)
-#undef DDX_T
-    return false;
-  }
-  if (fmt == STORE_F16 || fmt == STORE_BF16) {
-#define DDX_T(TX, TY, CY, CZ)                                                                         \
-  if (t.tx == TX && t.ty == TY && t.cy == CY && t.kz == CZ) {                                         \
-    if (fmt == STORE_F16)                                                                             \
-      vel_zb<TX, TY, CY, CZ, F16>(mode, g, st, d, starts, n, dx, dy, dz, sign, gnx, gny, gnz, R);     \
-    else                                                                                              \
-      vel_zb<TX, TY, CY, CZ, BF16>(mode, g, st, d, starts, n, dx, dy, dz, sign, gnx, gny, gnz, R);    \
-    return true;                                                                                     \
-  }
-    DDX_TILINGS16(DDX_T)
-#undef DDX_T
-    return false;
-  }
+  if (t.xl) return fmt == STORE_F32 && (t.xl == 2 ? vel_ylds : vel_lane)(DDX_PASS);
+  if (t.px == 2) return vel_pair(DDX_PASS);
+  if (fmt != STORE_F32) return vel_half(DDX_PASS);
   if (t.cy == 0 && t.kz > 0) {
     dim3 bl2(LX * LY);
     switch (mode) {
       case PURE_FORWARD:
       case RTM_FORWARD:
-        hipLaunchKernelGGL(k_vel_lds<PURE_FORWARD>, g, bl2, 0, st, d, starts, n, dx, dy, dz, sign, gnx, gny, gnz, R, t.kz);
+        hipLaunchKernelGGL(k_vel_lds<PURE_FORWARD>, g, bl2, 0, st, d, starts, n, dx, dy, dz, sc, t.kz);
         break;
       case RTM_BACKWARD:
-        hipLaunchKernelGGL(k_vel_lds<RTM_BACKWARD>, g, bl2, 0, st, d, starts, n, dx, dy, dz, sign, gnx, gny, gnz, R, t.kz);
+        hipLaunchKernelGGL(k_vel_lds<RTM_BACKWARD>, g, bl2, 0, st, d, starts, n, dx, dy, dz, sc, t.kz);
         break;
       default:
-        hipLaunchKernelGGL(k_vel_lds<RTM_REVERSE>, g, bl2, 0, st, d, starts, n, dx, dy, dz, sign, gnx, gny, gnz, R, t.kz);
+        hipLaunchKernelGGL(k_vel_lds<RTM_REVERSE>, g, bl2, 0, st, d, starts, n, dx, dy, dz, sc, t.kz);
     }
     return true;
   }
-  if (t.kz > 0) {
-#define DDX_T(TX, TY, CY, CZ)                                                                      \
-  if (t.tx == TX && t.ty == TY && t.cy == CY && t.kz == CZ) {                                      \
-    vel_zb<TX, TY, CY, CZ, F32>(mode, g, st, d, starts, n, dx, dy, dz, sign, gnx, gny, gnz, R);     \
-    return true;                                                                                  \
-  }
-    DDX_TILINGS(DDX_T)
-#undef DDX_T
-    return false;
-  }
+  if (t.kz > 0) return vel_one(DDX_PASS);
   switch (mode) {
     case PURE_FORWARD:
     case RTM_FORWARD:
-      hipLaunchKernelGGL(k_vel_phy<PURE_FORWARD>, g, bl, 0, st, d, starts, n, dx, dy, dz, sign, gnx, gny, gnz, R);
+      hipLaunchKernelGGL(k_vel_phy<PURE_FORWARD>, g, bl, 0, st, d, starts, n, dx, dy, dz, sc);
       break;
     case RTM_BACKWARD:
-      hipLaunchKernelGGL(k_vel_phy<RTM_BACKWARD>, g, bl, 0, st, d, starts, n, dx, dy, dz, sign, gnx, gny, gnz, R);
+      hipLaunchKernelGGL(k_vel_phy<RTM_BACKWARD>, g, bl, 0, st, d, starts, n, dx, dy, dz, sc);
       break;
     default:
-      hipLaunchKernelGGL(k_vel_phy<RTM_REVERSE>, g, bl, 0, st, d, starts, n, dx, dy, dz, sign, gnx, gny, gnz, R);
+      hipLaunchKernelGGL(k_vel_phy<RTM_REVERSE>, g, bl, 0, st, d, starts, n, dx, dy, dz, sc);
   }
   return true;
 }
 
 bool launch_stress_phy(const Tiling &t, int mode, int fmt, const PhyDesc *d, const int *starts, int n, int nblk,
-                       float dx, float dy, float dz, float dt, int gnx, int gny, int gnz, int R, hipStream_t st) {
+                       float dx, float dy, float dz, float sc, int grp, hipStream_t st) {
   if (nblk <= 0) return true;
   if ((mode == FWI || fmt != STORE_F32) && !(t.kz > 0 && t.cy > 0)) return false;
   if (mode == FWI && (t.px != 1 || t.xl)) return false;
   dim3 g(nblk), bl(kBlock);
-  if (t.xl == 2) {
-    if (fmt != STORE_F32 || t.tx != 64 || t.cy != 1) return false;
-#define DDX_T(TY, CZ)                                                                                  \
-  if (t.ty == TY && t.kz == CZ) {                                                                      \
-    const dim3 b2(64 * TY);                                                                            \
-    switch (mode) {                                                                                    \
-      case PURE_FORWARD:                                                                               \
-        hipLaunchKernelGGL((k_stress_phy_yl<PURE_FORWARD, TY, CZ, F32>), g, b2, 0, st, d, starts, n, dx, dy, dz, dt, gnx, gny, gnz, R); \
-        break;                                                                                         \
-      case RTM_FORWARD:                                                                                \
-        hipLaunchKernelGGL((k_stress_phy_yl<RTM_FORWARD, TY, CZ, F32>), g, b2, 0, st, d, starts, n, dx, dy, dz, dt, gnx, gny, gnz, R); \
-        break;                                                                                         \
-      case RTM_BACKWARD:                                                                               \
-        hipLaunchKernelGGL((k_stress_phy_yl<RTM_BACKWARD, TY, CZ, F32>), g, b2, 0, st, d, starts, n, dx, dy, dz, dt, gnx, gny, gnz, R); \
-        break;                                                                                         \
-      default:                                                                                         \
-        hipLaunchKernelGGL((k_stress_phy_yl<RTM_REVERSE, TY, CZ, F32>), g, b2, 0, st, d, starts, n, dx, dy, dz, dt, gnx, gny, gnz, R); \
-    }                                                                                                  \
-    return true;                                                                                      \
-  }
-    DDX_TILINGSY(DDX_T)
-#undef DDX_T
-    return false;
-  }
-  if (t.xl) {
-    if (fmt != STORE_F32) return false;
-#define DDX_T(TX, TY, CY, CZ)                                                                          \
-  if (t.tx == TX && t.ty == TY && t.cy == CY && t.kz == CZ) {                                          \
-    stress_zb<TX, TY, CY, CZ, F32, true>(mode, g, st, d, starts, n, dx, dy, dz, dt, gnx, gny, gnz, R);  \
-    return true;                                                                                      \
-  }
-    DDX_TILINGSX(DDX_T)
-#undef DDX_T
-    return false;
-  }
-  if (t.px == 2) {
-#define DDX_T(TX, TY, CY, CZ)                                                                          \
-  if (t.tx == TX && t.ty == TY && t.cy == CY && t.kz == CZ) {                                          \
-    if (fmt == STORE_F16)                                                                              \
-      stress_zb2<TX, TY, CY, CZ, F16>(mode, g, st, d, starts, n, dx, dy, dz, dt, gnx, gny, gnz, R);    \
-    else if (fmt == STORE_BF16)                                                                        \
-      stress_zb2<TX, TY, CY, CZ, BF16>(mode, g, st, d, starts, n, dx, dy, dz, dt, gnx, gny, gnz, R);   \
-    else                                                                                               \
-      stress_zb2<TX, TY, CY, CZ, F32>(mode, g, st, d, starts, n, dx, dy, dz, dt, gnx, gny, gnz, R);    \
-    return true;                                                                                      \
-  }
-    DDX_TILINGS2(DDX_T)
-#undef DDX_T
-    return false;
-  }
-  if (fmt == STORE_F16 || fmt == STORE_BF16) {
-#define DDX_T(TX, TY, CY, CZ)                                                                          \
-  if (t.tx == TX && t.ty == TY && t.cy == CY && t.kz == CZ) {                                          \
-    if (fmt == STORE_F16)                                                                              \
-      stress_zb<TX, TY, CY, CZ, F16>(mode, g, st, d, starts, n, dx, dy, dz, dt, gnx, gny, gnz, R);     \
-    else                                                                                               \
-      stress_zb<TX, TY, CY, CZ, BF16>(mode, g, st, d, starts, n, dx, dy, dz, dt, gnx, gny, gnz, R);    \
-    return true;                                                                                      \
-  }
-    DDX_TILINGS16(DDX_T)
-#undef DDX_T
-    return false;
-  }
+  if (t.xl) return fmt == STORE_F32 && (t.xl == 2 ? stress_ylds : stress_lane)(DDX_PASS);
+  if (t.px == 2) return stress_pair(DDX_PASS);
+  if (fmt != STORE_F32) return stress_half(DDX_PASS);
   if (t.cy == 0 && t.kz > 0) {
     dim3 bl2(LX * LY);
     switch (mode) {
       case PURE_FORWARD:
-        hipLaunchKernelGGL(k_stress_lds<PURE_FORWARD>, g, bl2, 0, st, d, starts, n, dx, dy, dz, dt, gnx, gny, gnz, R, t.kz);
-        break;
-      case RTM_FORWARD:
-        hipLaunchKernelGGL(k_stress_lds<RTM_FORWARD>, g, bl2, 0, st, d, starts, n, dx, dy, dz, dt, gnx, gny, gnz, R, t.kz);
+        hipLaunchKernelGGL(k_stress_lds<PURE_FORWARD>, g, bl2, 0, st, d, starts, n, dx, dy, dz, sc, t.kz);
         break;
       case RTM_BACKWARD:
-        hipLaunchKernelGGL(k_stress_lds<RTM_BACKWARD>, g, bl2, 0, st, d, starts, n, dx, dy, dz, dt, gnx, gny, gnz, R, t.kz);
+        hipLaunchKernelGGL(k_stress_lds<RTM_BACKWARD>, g, bl2, 0, st, d, starts, n, dx, dy, dz, sc, t.kz);
         break;
       default:
-        hipLaunchKernelGGL(k_stress_lds<RTM_REVERSE>, g, bl2, 0, st, d, starts, n, dx, dy, dz, dt, gnx, gny, gnz, R, t.kz);
+        hipLaunchKernelGGL(k_stress_lds<RTM_REVERSE>, g, bl2, 0, st, d, starts, n, dx, dy, dz, sc, t.kz);
     }
     return true;
   }
-  if (t.kz > 0) {
-#define DDX_T(TX, TY, CY, CZ)                                                                      \
-  if (t.tx == TX && t.ty == TY && t.cy == CY && t.kz == CZ) {                                      \
-    stress_zb<TX, TY, CY, CZ, F32>(mode, g, st, d, starts, n, dx, dy, dz, dt, gnx, gny, gnz, R);    \
-    return true;                                                                                  \
-  }
-    DDX_TILINGS(DDX_T)
-#undef DDX_T
-    return false;
-  }
+  if (t.kz > 0) return stress_one(DDX_PASS);
   switch (mode) {
     case PURE_FORWARD:
-      hipLaunchKernelGGL(k_stress_phy<PURE_FORWARD>, g, bl, 0, st, d, starts, n, dx, dy, dz, dt, gnx, gny, gnz, R);
-      break;
-    case RTM_FORWARD:
-      hipLaunchKernelGGL(k_stress_phy<RTM_FORWARD>, g, bl, 0, st, d, starts, n, dx, dy, dz, dt, gnx, gny, gnz, R);
+      hipLaunchKernelGGL(k_stress_phy<PURE_FORWARD>, g, bl, 0, st, d, starts, n, dx, dy, dz, sc);
       break;
     case RTM_BACKWARD:
-      hipLaunchKernelGGL(k_stress_phy<RTM_BACKWARD>, g, bl, 0, st, d, starts, n, dx, dy, dz, dt, gnx, gny, gnz, R);
+      hipLaunchKernelGGL(k_stress_phy<RTM_BACKWARD>, g, bl, 0, st, d, starts, n, dx, dy, dz, sc);
       break;
     default:
-      hipLaunchKernelGGL(k_stress_phy<RTM_REVERSE>, g, bl, 0, st, d, starts, n, dx, dy, dz, dt, gnx, gny, gnz, R);
+      hipLaunchKernelGGL(k_stress_phy<RTM_REVERSE>, g, bl, 0, st, d, starts, n, dx, dy, dz, sc);
   }
   return true;
-}
-
-void launch_halo(int esz, const HaloDesc *d, const int *starts, int n, int nblk, hipStream_t st) {
-  if (nblk <= 0) return;
-  if (esz == 2) hipLaunchKernelGGL(k_halo<unsigned short>, dim3(nblk), dim3(kBlock), 0, st, d, starts, n);
-  else hipLaunchKernelGGL(k_halo<float>, dim3(nblk), dim3(kBlock), 0, st, d, starts, n);
 }
 
 template <int C, class S>
@@ -3936,4 +3650,5 @@ void launch_nonfinite(int fmt, const void *field, long n, int *flag, hipStream_t
   else hipLaunchKernelGGL(k_nonfinite<F32>, g, b, 0, st, field, n, flag);
 }
 
+#endif  // DDX_PART
 }  // namespace ddx

@@ -191,31 +191,25 @@ int ddx_step_stress(ddx_ctx *ctx, int set, int mode);
  * 163-268), and the CMM exchange of one batch on its own
  * (mpicu_halo_comm_Operator::extract_into_halo + the MPI exchange,
  * OP/jarvis_2_mpicu_halo_comm_operator_meat.hpp:299-326): batch 0 the
- * velocities, 1 the stresses, 2 the stresses and sau.  Every subdomain is
- * on the one device, so the exchange copies each sender's boundary layers
- * into the receiver's ghost layers. */
+ * velocities, 1 the stresses, 2 the stresses and sau.  Every field is one
+ * array over the global grid and a subdomain a window of it, so a
+ * subdomain's ghost layers are its neighbours' own cells: they are current
+ * after ddx_update_vel / ddx_update_stress, before the exchange is called. */
 int ddx_update_vel(ddx_ctx *ctx, int set, int mode);
 int ddx_update_stress(ddx_ctx *ctx, int set, int mode);
 int ddx_halo_exchange(ddx_ctx *ctx, int set, int batch);
 /* How the CMM exchange moves the halos (the reference exchanges them by
  * mpicu_halo_comm_Operator::extract_into_halo / inject_from_halo,
  * OP/jarvis_2_mpicu_halo_comm_operator_meat.hpp:299-326).  mode 0 (the
- * default): one copy per link from the sender's boundary layers straight
- * into the receiver's ghost layers.  mode 1: the reference's contiguous
- * message blocks -- every sender side packs the boundary layers of the
- * batch's fields into one contiguous block, each field at its offset in
- * push order (the blocks of the multiple-halo operator, :408-461), and the
- * receiver unpacks the block into its ghost layers; the block is what a
- * link between two GPUs would send.  mode 2: pack on store -- the kernels
- * that update a subdomain's boundary layers (z-blocked bricks, CPML
- * kernels, VOWR injection) also write each value into the receiver's ghost
- * layers, so no pass reads the layers again; after a half step run by the
- * one-plane or LDS-tiled kernels the mode-0 copy follows instead.  Mode 2
- * needs the context created with DDX_MIRROR=1 in the environment (it is
- * then the context's default), and is slower on this GPU than mode 0.
- * Results do not depend on the mode.  In mode 2, ddx_update_vel /
- * ddx_update_stress already leave the ghosts current, and ddx_halo_exchange
- * copies them again (same values). */
+ * default) and mode 2: nothing is moved, since the ghost layers are the
+ * neighbours' own cells.  mode 1: the reference's contiguous message blocks
+ * -- every sender side packs the boundary layers of the batch's fields into
+ * one contiguous block, each field at its offset in push order (the blocks
+ * of the multiple-halo operator, :408-461), and the receiver unpacks the
+ * block into its ghost layers; the block is what a link between two GPUs
+ * would send.  Mode 2 (ghosts written as their owner is updated) is offered
+ * to contexts created with DDX_MIRROR=1 in the environment and more than one
+ * subdomain, and is then the default.  Results do not depend on the mode. */
 int ddx_set_exchange(ddx_ctx *ctx, int mode);
 int ddx_get_exchange(const ddx_ctx *ctx, int *mode);
 /* VOWR boundary store of set 0: save time slice it (0..ntime-2) of every
