@@ -77,6 +77,7 @@ struct PhyDesc {
   int R;             // VOWR ring width
   int tiles_x, tiles_y;
   float dt;          // time step (FWI accumulators)
+  int io;            // member of a fused launch (StepIO)
   int blk0;
 };
 
@@ -92,7 +93,9 @@ struct SlabDesc {
   int axes;                          // damped axes: 1 x, 2 y, 4 z
   int xlo, xhi, ylo, yhi, zlo, zhi;  // a cell is in an axis' damping range iff c < lo || c >= hi
   void *psi;                         // [6 * naxes][ncell] memory variables (storage format)
-  const float *coef;                 // [4 * naxes][ncell]: a, b, a_half, b_half per axis
+  const float *coef;                 // [naxes][ncell][4]: a, b, a_half, b_half per axis and cell
+  float rdx, rdy, rdz;               // 1 / spacing
+  int io;                            // member of a fused launch (StepIO)
   int blk0;
 };
 
@@ -147,6 +150,7 @@ struct Tiling {
   int tx, ty, cy, kz;
   int px = 1;
   int xl = 0;
+  int whole = 1;  // the half step may run as one launch with the CPML cells (whole_half in engine.cpp)
 };
 // instantiated brick shapes (tx, ty, cy, kz) for a storage format
 bool tiling_supported(const Tiling &t, int fmt = STORE_F32);
@@ -168,6 +172,7 @@ inline int tiling_blocks(const Tiling &t, int nx, int ny, int nz) {
 struct MemberIO {
   void *sxx, *syy, *szz;  // source subdomain's fields; nullptr: the shot is outside gridext
   long src_off;
+  int src_x, src_y, src_z;  // the source cell in the whole grid's extended coordinates (-1: none)
   const float *wavelet;
   int src_mode;
   float ss;               // stress-class scale (16-bit formats)
@@ -183,6 +188,31 @@ struct MemberIO {
   int blk0;               // first block of this member's receivers
 };
 
+// Sources and receivers of a time step of the members of a launch (a shot on
+// its own is the one member); a descriptor's member is its `io`.  Time index:
+// gs, or *gsp when set (see launch_source_batch).  io null: no sources.
+// nblk: receiver blocks (0: the step samples none here).
+struct StepIO {
+  const MemberIO *io = nullptr;
+  const int *starts = nullptr;
+  int n = 0, nblk = 0;
+  int gs = 0;
+  const int *gsp = nullptr;
+};
+
+// A half step of the physical region and the CPML cells in one launch.
+struct HalfStep {
+  const PhyDesc *phy;
+  const int *pstarts;
+  int np, nphy;
+  const SlabDesc *slabs;
+  const int *sstarts;
+  int ns, npml;
+  float dx, dy, dz, sc;  // sc: as sign / dt of the separate kernels
+  float sx, sy, sz;      // sc over dx, dy, dz
+  int grp, pgrp;
+};
+
 // ---- launchers (kernels.hip) ----
 // fmt: storage format; the 16-bit formats fold their scale ratios into
 // `sign` (velocity: sv/ss), `dt` (stress: ss/sv) and `rv` (CPML velocity:
@@ -194,6 +224,13 @@ bool launch_vel_phy(const Tiling &t, int mode, int fmt, const PhyDesc *d, const 
                     float dx, float dy, float dz, float sign, int grp, hipStream_t st);
 bool launch_stress_phy(const Tiling &t, int mode, int fmt, const PhyDesc *d, const int *starts, int n, int nblk,
                        float dx, float dy, float dz, float dt, int grp, hipStream_t st);
+// One launch for a half step (CPML split 1, group-interleaved orders); false,
+// launching nothing, when no such kernel exists for the brick shape, format
+// and mode (the backward mode has no CPML cells).  The stress step also adds
+// the members' sources and samples their receivers (io).
+bool whole_shape(const Tiling &t, int fmt);  // the shapes they exist for
+bool launch_vel_all(const Tiling &t, int mode, int fmt, const HalfStep &a, hipStream_t st);
+bool launch_stress_all(const Tiling &t, int mode, int fmt, const HalfStep &a, const StepIO &io, hipStream_t st);
 // grp: blocks per XCD group of the group-interleaved block order (0: launch order)
 // ord (nullable): the XCD-partitioned block order of the table; without it
 // (or with ord->pieces null) the blocks follow the table's own order.
@@ -239,8 +276,7 @@ void launch_source_batch(int fmt, const MemberIO *io, int n, int gs, const int *
 // Observed data of every member of a fused RTM batch injected at its
 // receivers (io[q].vptr: the reverse set) at batch step gs.
 void launch_inject_batch(int fmt, const MemberIO *io, const int *starts, int n, int nblk, int gs, hipStream_t st);
-void launch_recv_batch(int fmt, const MemberIO *io, const int *starts, int n, int nblk, int gs, const int *gsp,
-                       hipStream_t st);
+void launch_recv_batch(int fmt, const StepIO &io, hipStream_t st);
 void launch_set_int(int *p, int v, hipStream_t st);
 void launch_recv_sample(int fmt, void *const *vptr, const int *rsub, const long *roff, int nrec, int it, int ntime,
                         float *seis, float inv_sv, const int *itp, hipStream_t st);

@@ -276,6 +276,15 @@ using namespace ddx;
 // of 0, 1, 2, 4, 8, 16 on the 256x256x200 RTM shot).
 static const int kBrickGroup = 8;
 
+// Half steps of at most so many cells (physical region and CPML) run as one
+// launch.  Measured, one launch against two, n^3 grids with 20 layers, 60
+// modelling steps: n = 64 3.06 against 3.85 ms, 96 6.29 / 7.10, 128 11.4 /
+// 12.1, 160 19.5 / 19.9, 192 (12.5 M cells) 28.2 / 28.4, 224 (18.4 M) 42.1 /
+// 41.7; the 256x256x200 RTM shot (20.1 M) is 1-2% slower in one launch: the
+// bricks then hold the CPML kernel's registers, and what one launch gains,
+// its last wave of blocks, is a small part of a large one.
+static const double kWholeCells = 14e6;
+
 struct ddx_ctx {
   ddx_desc d;
   std::string err;
@@ -295,13 +304,12 @@ struct ddx_ctx {
   std::vector<Geom> g;  // the subdomains (windows of the global arrays)
   Geom all;             // the whole grid
   int gext[3];
-  // Brick shape of the physical-region kernels per mode (index = mode),
-  // the fastest of a sweep on MI355X for the 2x2x1 256x256x200 RTM shot:
-  // deep z columns where the register budget allows, shallower ones for the
-  // backward/reverse velocity kernels, which carry the sau arms as well.
-  // (index 4: FWI mode, z-blocked bricks only)
-  Tiling tiling_vel[kModes] = {{64, 4, 1, 8}, {64, 4, 1, 8}, {64, 4, 1, 2}, {64, 4, 1, 4}, {64, 4, 1, 4}};
-  Tiling tiling_stress[kModes] = {{64, 4, 1, 2}, {64, 4, 1, 4}, {64, 4, 1, 4}, {64, 4, 1, 4}, {64, 4, 1, 2}};
+  // Brick shape of the physical-region kernels per mode (index = mode; 4: FWI
+  // mode, one-cell bricks only), default_bricks until tuned or set
+  Tiling tiling_vel[kModes], tiling_stress[kModes];
+  // and that of the physical region in a launch of its own, where it differs
+  // (batches too large for whole half steps): [velocity, stress]
+  Tiling apart[2][kModes];
   // device memory
   std::vector<void *> allocs;
   std::vector<size_t> alloc_bytes;  // size of each allocation in allocs
@@ -330,6 +338,8 @@ struct ddx_ctx {
   std::vector<Slab> slabs;
   std::vector<PhyTables> phy_cache;  // physical-region tables per brick shape
   int brick_group = kBrickGroup;     // XCD group size of the bricks' block order
+  int whole_group = -1;              // the same of the half steps that run as one launch (columns)
+  double whole_cells = kWholeCells;  // half steps of at most so many cells run as one launch
   int pml_cz = 1;                    // planes per thread of the CPML kernels (1, 2, 4, 8)
   int pml_group = 32;                // XCD group size of the CPML block order (0: launch order)
   int pml_order = 0;                 // 1: the XCD-partitioned CPML block order (PmlOrder); 0: pml_group
@@ -370,6 +380,7 @@ struct ddx_ctx {
   int nshot = 0;
   std::vector<int> shot_sub;    // per shot: owning subdomain or -1
   std::vector<long> shot_off;
+  std::vector<int> shot_ext;    // per shot: its cell in the whole grid's extended coordinates
   int nrec = 0;
   std::vector<int> rec_rank, rec_input;
   int *d_rsub = nullptr;
@@ -391,6 +402,8 @@ struct ddx_ctx {
   // its index and the next stage
   int chunk_kind = 0, chunk_shot = -1, chunk_next = 0;
   int *d_flag = nullptr;  // device flag of ddx_check_finite
+  MemberIO *d_io = nullptr;  // the shot in progress as the one member of its launches
+  int *d_zero = nullptr;     // its first block (0)
 };
 
 // ---------------------------------------------------------------------------
@@ -594,6 +607,36 @@ struct ProfScope {
 // ---------------------------------------------------------------------------
 static int build_tables(ddx_ctx *c);
 
+static void set_brick(ddx_ctx *c, int kernel, int mode, const Tiling &t) {
+  (kernel == 0 ? c->tiling_vel : c->tiling_stress)[mode] = c->apart[kernel][mode] = t;
+}
+// The shape of a launch over `cells` cells.
+static const Tiling &brick_for(const ddx_ctx *c, int kernel, int mode, double cells) {
+  if (cells > c->whole_cells) return c->apart[kernel][mode];
+  return (kernel == 0 ? c->tiling_vel : c->tiling_stress)[mode];
+}
+
+// Brick shapes of a context that is not tuned.  FP32: rows of 64 cells with
+// the y arm from LDS where they waste no more lanes than rows of 32 by over
+// 5%, else one-cell bricks of rows of 32 (n^3 grids, 15 layers, 60 modelling
+// steps, rows of 64 against 32: n = 48 1.77 / 1.84 ms, 72 3.38 / 3.20, 100
+// 5.59 / 5.65, 128 8.50 / 8.69, 160 16.1 / 15.8, 200 29.8 / 28.3).  16-bit:
+// paired bricks (161x150x131, BF16).
+static void default_bricks(ddx_ctx *c) {
+  const int nx = c->d.nx, w64 = (nx + 63) / 64 * 64, w32 = (nx + 31) / 32 * 32;
+  const bool narrow = w64 > 1.05 * w32;
+  Tiling t{64, 4, 1, 2}, f{64, 4, 1, 2};
+  if (c->fmt != STORE_F32) {
+    t = {64, 4, 1, 4};
+    t.px = 2;
+  } else if (narrow) {
+    t = f = {32, 8, 1, 4};
+  } else {
+    t.xl = 2;
+  }
+  for (int m = 0; m < kModes; m++) set_brick(c, 0, m, m == FWI ? f : t), set_brick(c, 1, m, m == FWI ? f : t);
+}
+
 extern "C" int ddx_create(const ddx_desc *desc, ddx_ctx **out) {
   if (!desc || !out) { g_create_error = "null argument"; return DDX_EINVAL; }
   *out = nullptr;
@@ -677,16 +720,19 @@ extern "C" int ddx_create(const ddx_desc *desc, ddx_ctx **out) {
   if (const char *e = getenv("DDX_PML_ORDER")) c->pml_order = atoi(e) != 0;
   if (const char *e = getenv("DDX_BRICK_GROUP")) {  // XCD group size of the brick blocks, for sweeps
     const int v = atoi(e);
-    if (v >= 0 && v <= 65536) c->brick_group = v;
+    if (v >= 0 && v <= 65536) c->brick_group = c->whole_group = v;
   }
+  if (const char *e = getenv("DDX_WHOLE_CELLS")) c->whole_cells = atof(e);  // for sweeps
+  default_bricks(c);
   if (const char *e = getenv("DDX_TILING")) {  // "TXxTYxCYxKZ[xFORM]", for tile sweeps
     Tiling t{0, 0, 0, 0};
     const int nf = sscanf(e, "%dx%dx%dx%dx%d", &t.tx, &t.ty, &t.cy, &t.kz, &t.px);
     if (t.px == 3) t.px = 1, t.xl = 1;
+    if (t.px == 4) t.px = 1, t.xl = 2;
     if (nf >= 4 && ((t.kz == 0 && t.px == 1 && !t.xl && c->fmt == STORE_F32) ||
                     (t.kz > 0 && tiling_supported(t, c->fmt))))
       for (int m = 0; m < kModes; m++)
-        if (m != FWI || (t.kz > 0 && t.cy > 0 && t.px == 1 && !t.xl)) c->tiling_vel[m] = c->tiling_stress[m] = t;
+        if (m != FWI || (t.kz > 0 && t.cy > 0 && t.px == 1 && !t.xl)) set_brick(c, 0, m, t), set_brick(c, 1, m, t);
   }
   int rc = build_tables(c);
   if (rc) {
@@ -736,6 +782,7 @@ static int build_phy_tables(ddx_ctx *c, const Tiling &t, int model, PhyTables &o
     p.ox = g.mlo[0]; p.oy = g.mlo[1]; p.oz = g.mlo[2];
     p.nx = g.pn[0]; p.ny = g.pn[1]; p.nz = g.pn[2];
     p.R = c->d.rec_width;
+    p.io = 0;
     p.tiles_x = (g.pn[0] + kTileX - 1) / kTileX;
     p.tiles_y = (g.pn[1] + kTileY - 1) / kTileY;
     p.blk0 = 0;
@@ -894,6 +941,10 @@ static int build_tables(ddx_ctx *c) {
   if (rc) return rc;
   rc = dalloc(c, (void **)&c->d_flag, sizeof(int));
   if (rc) return rc;
+  rc = dalloc(c, (void **)&c->d_io, sizeof(MemberIO));
+  if (rc) return rc;
+  rc = dalloc(c, (void **)&c->d_zero, sizeof(int));
+  if (rc) return rc;
   HIPCHECK(c, hipStreamSynchronize(c->st));
   return DDX_OK;
 }
@@ -1049,10 +1100,8 @@ static int load_model(ddx_ctx *c, int which, const float *vp, const float *vs, c
               float A, B, AH, BH;
               if (cpml_axis(en_[a], g.en[a], g.mlo[a], g.mhi[a], h_[a], v, d.fm, d.dt, A, B, AH, BH))
                 in_plane[(size_t)3 * k + a]++;
-              hc[(size_t)(slot * 4 + 0) * sl.ncell + cidx] = A;
-              hc[(size_t)(slot * 4 + 1) * sl.ncell + cidx] = B;
-              hc[(size_t)(slot * 4 + 2) * sl.ncell + cidx] = AH;
-              hc[(size_t)(slot * 4 + 3) * sl.ncell + cidx] = BH;
+              float *q = hc.data() + 4 * ((size_t)slot * sl.ncell + cidx);
+              q[0] = A; q[1] = B; q[2] = AH; q[3] = BH;
               slot++;
             }
           }
@@ -1084,6 +1133,10 @@ static int load_model(ddx_ctx *c, int which, const float *vp, const float *vs, c
         p.xlo = sl.xlo; p.xhi = sl.xhi; p.ylo = sl.ylo; p.yhi = sl.yhi; p.zlo = sl.zlo; p.zhi = sl.zhi;
         p.psi = sl.psi[set];
         p.coef = sl.coef[which];
+        // the short division is proven for spacings within 2^20 of 1 (DivGuard): NaN sends the rest the general way
+        auto recip = [](float h) { return h < 1048576.0f && h > 1.0f / 1048576.0f ? 1.0f / h : NAN; };
+        p.rdx = recip(d.dx); p.rdy = recip(d.dy); p.rdz = recip(d.dz);
+        p.io = 0;
         p.blk0 = blk;
         st.push_back(blk);
         blk += pml_blocks(sl.ni, sl.nj, sl.nk, c->pml_cz);
@@ -1236,6 +1289,7 @@ extern "C" int ddx_set_geometry(ddx_ctx *c, const float *shots, int nshot, const
   c->nshot = nshot;
   c->shot_sub.assign(nshot, -1);
   c->shot_off.assign(nshot, 0);
+  c->shot_ext.assign((size_t)3 * nshot, -1);
   for (int q = 0; q < nshot; q++) {
     const float *p = shots + 3 * q;
     for (int s = 0; s < c->nsub; s++) {
@@ -1247,6 +1301,7 @@ extern "C" int ddx_set_geometry(ddx_ctx *c, const float *shots, int nshot, const
       for (int a = 0; a < 3; a++) ii[a] = gap_num(g.lext[a], p[a], dd[a]);
       c->shot_sub[q] = s;
       c->shot_off[q] = ii[0] + g.sy * ii[1] + g.sz * ii[2];
+      for (int a = 0; a < 3; a++) c->shot_ext[(size_t)3 * q + a] = ii[a] + (int)g.ext_goff[a];
       break;
     }
   }
@@ -1431,10 +1486,30 @@ static int phy_launch(ddx_ctx *c, int kernel, int set, int mode, const Tiling &t
   return DDX_OK;
 }
 
+// The tables of a half step as one launch; false when the context's CPML work
+// split or block order, its stream overlap, a running profile (which times
+// the parts apart) or the launch's size rule it out.
+static bool whole_half(const ddx_ctx *c, const Tiling &t, const DevTable<PhyDesc> &p, const DevTable<SlabDesc> &q,
+                       float sc, HalfStep &a) {
+  if (!t.whole || c->prof.mask || c->pml_overlap || c->pml_cz != 1 || c->pml_order) return false;
+  if (p.cells + q.cells > c->whole_cells) return false;
+  a = {p.d, p.starts, p.n, p.nblk, q.d, q.starts, q.n, q.nblk, c->d.dx, c->d.dy, c->d.dz, sc,
+       sc / c->d.dx, sc / c->d.dy, sc / c->d.dz, c->whole_group, c->pml_group};
+  return true;
+}
+
 static int vel_update(ddx_ctx *c, int set, int mode) {
   if (!c || set < 0 || set > 1 || mode < 0 || mode >= kModes) return DDX_EINVAL;
   if (!c->have_model) { c->err = "no model"; return DDX_ESTATE; }
   if (int rc = check_mode(c, mode)) return rc;
+  if (mode != RTM_BACKWARD) {
+    const PhyTables *pt = phy_tables(c, c->tiling_vel[mode], model_for(c, mode));
+    if (!pt) return DDX_EHIP;
+    HalfStep a;
+    if (whole_half(c, c->tiling_vel[mode], pt->set[set], c->pml[model_for(c, mode)][set], ratio_vs(c), a) &&
+        launch_vel_all(c->tiling_vel[mode], mode, c->fmt, a, c->st))
+      return DDX_OK;
+  }
   const bool side = c->pml_overlap && mode != RTM_BACKWARD;
   hipStream_t pst = side ? c->st_pml : c->st;
   if (side) {
@@ -1458,10 +1533,21 @@ static int vel_update(ddx_ctx *c, int set, int mode) {
   return DDX_OK;
 }
 
+// The stress half step as one launch, with io's sources and receivers; false
+// (nothing launched) when it has to run as separate kernels.
+static bool stress_whole(ddx_ctx *c, int set, int mode, const StepIO &io) {
+  if (mode == RTM_BACKWARD) return false;
+  const PhyTables *pt = phy_tables(c, c->tiling_stress[mode], model_for(c, mode));
+  HalfStep a;
+  return pt && whole_half(c, c->tiling_stress[mode], pt->set[set], c->pml[model_for(c, mode)][set], c->d.dt * ratio_sv(c), a) &&
+         launch_stress_all(c->tiling_stress[mode], mode, c->fmt, a, io, c->st);
+}
+
 static int stress_update(ddx_ctx *c, int set, int mode) {
   if (!c || set < 0 || set > 1 || mode < 0 || mode >= kModes) return DDX_EINVAL;
   if (!c->have_model) { c->err = "no model"; return DDX_ESTATE; }
   if (int rc = check_mode(c, mode)) return rc;
+  if (stress_whole(c, set, mode, StepIO{})) return DDX_OK;
   const float dt = mode == RTM_BACKWARD ? -c->d.dt : c->d.dt;
   const bool side = c->pml_overlap && mode != RTM_BACKWARD;
   hipStream_t pst = side ? c->st_pml : c->st;
@@ -1586,20 +1672,87 @@ static int ensure_seis(ddx_ctx *c, int ishot) {
   return DDX_OK;
 }
 
-// One modelling time step (BLEND/fdtd3d_blend_elastic_model_mpi_meat.hpp:
-// 55-66): velocity, source, stress, receivers.  itp: read the time index
-// from this device int (graph capture) instead of it.
-static int model_step(ddx_ctx *c, int ishot, int it, const int *itp) {
-  int rc;
-  if ((rc = vel_half(c, 0, PURE_FORWARD))) return rc;
+// Shot ishot of c as a member of a launch: its source in set 0 and its
+// receivers in `set`.
+static MemberIO member_io(ddx_ctx *c, int ishot, int set) {
+  MemberIO x{};
+  const int s = c->shot_sub[ishot];
+  x.src_x = x.src_y = x.src_z = -1;
+  if (s >= 0) {
+    x.sxx = fptr(c, 0, s, SXX);
+    x.syy = fptr(c, 0, s, SYY);
+    x.szz = fptr(c, 0, s, SZZ);
+    x.src_off = c->shot_off[ishot];
+    x.src_x = c->shot_ext[(size_t)3 * ishot];
+    x.src_y = c->shot_ext[(size_t)3 * ishot + 1];
+    x.src_z = c->shot_ext[(size_t)3 * ishot + 2];
+  }
+  x.wavelet = c->wavelet;
+  x.src_mode = c->d.source_mode;
+  x.ss = scale_of(c, 1);
+  x.vptr = c->d_vptr[set];
+  x.rsub = c->d_rsub;
+  x.roff = c->d_roff;
+  x.nrec = c->nrec;
+  x.seis = c->seis[ishot];
+  x.inv_sv = 1.0f / scale_of(c, 0);
+  x.sv = scale_of(c, 0);
+  x.ntime = c->d.ntime;
+  return x;
+}
+static int recv_blocks(const ddx_ctx *c) { return (c->nrec + kBlock - 1) / kBlock; }
+
+// Whether the shot's cell is one that the stress update writes: the two
+// outermost layers of the extended grid are not, and a source there has to be
+// added by k_source.
+static bool source_owned(const ddx_ctx *c, int ishot) {
+  if (c->shot_sub[ishot] < 0) return true;  // src_x = -1: no cell has it
+  for (int a = 0; a < 3; a++) {
+    const int x = c->shot_ext[(size_t)3 * ishot + a];
+    if (x < 2 || x >= c->gext[a] - 2) return false;
+  }
+  return true;
+}
+
+// The second half of a forward step on set 0: source, stress, and (recv) the
+// receivers, which read velocities.  itp: read the time index from this
+// device int (graph capture) instead of it.
+static int source_stress(ddx_ctx *c, int mode, int ishot, int it, const int *itp, bool recv) {
+  StepIO io;
+  io.io = c->d_io;
+  io.starts = c->d_zero;
+  io.n = 1;
+  io.gs = it;
+  io.gsp = itp;
+  io.nblk = recv ? recv_blocks(c) : 0;
+  if (source_owned(c, ishot) && stress_whole(c, 0, mode, io)) {
+    exchange_on(c, 0, 1, c->st);
+    return DDX_OK;
+  }
   const int s = c->shot_sub[ishot];
   if (s >= 0)
     launch_source(c->fmt, fptr(c, 0, s, SXX), fptr(c, 0, s, SYY), fptr(c, 0, s, SZZ), c->shot_off[ishot], c->wavelet,
                   it, 1.f, c->d.source_mode, scale_of(c, 1), itp, c->st);
-  if ((rc = stress_half(c, 0, PURE_FORWARD))) return rc;
-  launch_recv_sample(c->fmt, c->d_vptr[0], c->d_rsub, c->d_roff, c->nrec, it, c->d.ntime, c->seis[ishot],
-                     1.0f / scale_of(c, 0), itp, c->st);
+  if (int rc = stress_half(c, 0, mode)) return rc;
+  if (recv)
+    launch_recv_sample(c->fmt, c->d_vptr[0], c->d_rsub, c->d_roff, c->nrec, it, c->d.ntime, c->seis[ishot],
+                       1.0f / scale_of(c, 0), itp, c->st);
   return DDX_OK;
+}
+
+// Shot ishot becomes the member of the context's launches (a small copy on
+// its stream; at the start of a shot, or of a piece of one).
+static int set_shot(ddx_ctx *c, int ishot) {
+  const MemberIO x = member_io(c, ishot, 0);
+  HIPCHECK(c, hipMemcpyAsync(c->d_io, &x, sizeof x, hipMemcpyHostToDevice, c->st));
+  return DDX_OK;
+}
+
+// One modelling time step (BLEND/fdtd3d_blend_elastic_model_mpi_meat.hpp:
+// 55-66): velocity, source, stress, receivers.
+static int model_step(ddx_ctx *c, int ishot, int it, const int *itp) {
+  if (int rc = vel_half(c, 0, PURE_FORWARD)) return rc;
+  return source_stress(c, PURE_FORWARD, ishot, it, itp, true);
 }
 
 // Capture one modelling step, with the step counter's advance, as a graph
@@ -1646,6 +1799,8 @@ extern "C" int ddx_model_shot(ddx_ctx *c, int ishot) {
   rc = ensure_seis(c, ishot);
   if (rc) return rc;
   rc = ddx_reset_wave(c, 0);
+  if (rc) return rc;
+  rc = set_shot(c, ishot);
   if (rc) return rc;
   const int nt = c->d.ntime;
   if (c->use_graph && c->prof.mask == 0 && !c->pml_overlap) {
@@ -1774,17 +1929,22 @@ struct BatchMember {
 
 // What members of one fused launch must share.
 struct BatchKey {
-  int device = 0, fmt = 0, lg0 = 0, lg1 = 0, pml_cz = 1, pml_group = 0, pml_order = 1, brick_group = 0;
+  int device = 0, fmt = 0, lg0 = 0, lg1 = 0, pml_cz = 1, pml_group = 0, pml_order = 1, brick_group = 0, whole_group = 0;
   float dt = 0.f, dx = 0.f, dy = 0.f, dz = 0.f;
   Tiling tv{0, 0, 0, 0}, ts{0, 0, 0, 0};
 };
-static BatchKey batch_key(const ddx_ctx *c) {
+static double batch_cells(ddx_ctx *const *cs, int n) {
+  double cells = 0;
+  for (int q = 0; q < n; q++) cells += ext_cells(cs[q]);
+  return cells;
+}
+static BatchKey batch_key(const ddx_ctx *c, double cells) {
   BatchKey k;
   k.device = c->d.device; k.fmt = c->fmt; k.lg0 = c->lg[0]; k.lg1 = c->lg[1];
-  k.pml_cz = c->pml_cz; k.pml_group = c->pml_group; k.pml_order = c->pml_order; k.brick_group = c->brick_group;
+  k.pml_cz = c->pml_cz; k.pml_group = c->pml_group; k.pml_order = c->pml_order; k.brick_group = c->brick_group; k.whole_group = c->whole_group;
   k.dt = c->d.dt; k.dx = c->d.dx; k.dy = c->d.dy; k.dz = c->d.dz;
-  k.tv = c->tiling_vel[PURE_FORWARD];
-  k.ts = c->tiling_stress[PURE_FORWARD];
+  k.tv = brick_for(c, 0, PURE_FORWARD, cells);
+  k.ts = brick_for(c, 1, PURE_FORWARD, cells);
   return k;
 }
 static bool batch_compatible(const BatchKey &k, const ddx_ctx *c) {
@@ -1831,10 +1991,17 @@ static int batch_prepare(ddx_ctx *c, int ishot, const BatchKey &k, BatchMember &
   return DDX_OK;
 }
 
+// The descriptors of a member carry its place in the launch's MemberIO table.
+template <class T>
+static void set_member(HostTable<T> &t, int q) {
+  for (T &x : t.d) x.io = q;
+}
+
 struct FusedSet {
   FusedTable<PhyDesc> v, s;
   FusedTable<SlabDesc> p;
   FusedTable<MemberIO> io;  // sources and receivers of the members
+  bool whole = false;       // the half steps may run as one launch each
 };
 // The fused tables of a batch on the host.
 struct FusedHost {
@@ -1842,7 +2009,7 @@ struct FusedHost {
   HostTable<SlabDesc> p;
   HostTable<MemberIO> io;
 };
-static void fuse_host(const std::vector<BatchMember> &ms, FusedHost &f) {
+static void fuse_host(std::vector<BatchMember> &ms, FusedHost &f) {
   std::vector<const HostTable<PhyDesc> *> pv, ps;
   std::vector<const HostTable<SlabDesc> *> pp;
   // one MemberIO part per member (its receiver blocks), so upload_fused
@@ -1850,35 +2017,17 @@ static void fuse_host(const std::vector<BatchMember> &ms, FusedHost &f) {
   std::vector<HostTable<MemberIO>> parts(ms.size());
   std::vector<const HostTable<MemberIO> *> pio;
   for (size_t q = 0; q < ms.size(); q++) {
-    const BatchMember &m = ms[q];
+    BatchMember &m = ms[q];
+    set_member(m.hs, (int)q);
+    set_member(m.hp, (int)q);
     pv.push_back(&m.hv);
     ps.push_back(&m.hs);
     pp.push_back(&m.hp);
-    ddx_ctx *c = m.c;
-    MemberIO x{};
-    const int s = c->shot_sub[m.ishot];
-    if (s >= 0) {
-      x.sxx = fptr(c, 0, s, SXX);
-      x.syy = fptr(c, 0, s, SYY);
-      x.szz = fptr(c, 0, s, SZZ);
-      x.src_off = c->shot_off[m.ishot];
-    }
-    x.wavelet = c->wavelet;
-    x.src_mode = c->d.source_mode;
-    x.ss = scale_of(c, 1);
-    x.vptr = c->d_vptr[0];
-    x.rsub = c->d_rsub;
-    x.roff = c->d_roff;
-    x.nrec = c->nrec;
-    x.seis = c->seis[m.ishot];
-    x.inv_sv = 1.0f / scale_of(c, 0);
-    x.sv = scale_of(c, 0);
+    MemberIO x = member_io(m.c, m.ishot, 0);
     x.join = m.join;
-    x.ntime = c->d.ntime;
-    x.blk0 = 0;
     parts[q].d.push_back(x);
     parts[q].s.push_back(0);
-    parts[q].nblk = (x.nrec + kBlock - 1) / kBlock;
+    parts[q].nblk = recv_blocks(m.c);
     pio.push_back(&parts[q]);
   }
   concat_tables(pv, f.v);
@@ -1886,9 +2035,23 @@ static void fuse_host(const std::vector<BatchMember> &ms, FusedHost &f) {
   concat_tables(pp, f.p);
   concat_tables(pio, f.io);
 }
-static hipError_t fuse_members(const std::vector<BatchMember> &ms, FusedSet &f) {
+// The half steps of ms as one launch each: the split and order of their CPML
+// kernels, the blocks' number and the sources' cells allow it.
+static bool batch_whole(const std::vector<BatchMember> &ms) {
+  if (ms.empty()) return false;
+  const ddx_ctx *c0 = ms[0].c;
+  double cells = 0;
+  bool ok = c0->pml_cz == 1 && !c0->pml_order;
+  for (const BatchMember &m : ms) {
+    ok = ok && source_owned(m.c, m.ishot);
+    cells += ext_cells(m.c);
+  }
+  return ok && cells <= c0->whole_cells;
+}
+static hipError_t fuse_members(std::vector<BatchMember> &ms, FusedSet &f) {
   FusedHost h;
   fuse_host(ms, h);
+  f.whole = batch_whole(ms);
   hipError_t e = upload_owned(h.v, f.v);
   if (e == hipSuccess) e = upload_owned(h.s, f.s);
   if (e == hipSuccess) e = upload_owned_pml(h.p, ms.empty() ? 1 : ms[0].c->pml_cz, f.p);
@@ -1896,23 +2059,41 @@ static hipError_t fuse_members(const std::vector<BatchMember> &ms, FusedSet &f) 
   return e;
 }
 
+static HalfStep half_of(const BatchKey &k, const FusedTable<PhyDesc> &p, const FusedTable<SlabDesc> &q, float sc) {
+  return {p.d, p.starts, p.n, p.nblk, q.d, q.starts, q.n, q.nblk, k.dx, k.dy, k.dz, sc,
+          sc / k.dx, sc / k.dy, sc / k.dz, k.whole_group, k.pml_group};
+}
+
 // One modelling time step of every member (each at its own time index, the
 // batch step gs minus its join step), in the order of model_step.
 static bool fused_step(const BatchKey &k, const FusedSet &f, const std::vector<BatchMember> &ms, int gs,
                        hipStream_t st, const int *gsp = nullptr) {
   const float rvs = std::ldexp(1.0f, k.lg0 - k.lg1), rsv = std::ldexp(1.0f, k.lg1 - k.lg0);
-  if (!launch_vel_phy(k.tv, PURE_FORWARD, k.fmt, f.v.d, f.v.starts, f.v.n, f.v.nblk, k.dx, k.dy, k.dz, rvs, k.brick_group, st))
-    return false;
-  launch_vel_pml(k.pml_cz, k.fmt, f.p.d, f.p.starts, f.p.n, f.p.nblk, k.dx, k.dy, k.dz, rvs, k.pml_group,
-                 k.pml_order ? &f.p.ord : nullptr, st);
+  if (!f.whole || !k.tv.whole || !launch_vel_all(k.tv, PURE_FORWARD, k.fmt, half_of(k, f.v, f.p, rvs), st)) {
+    if (!launch_vel_phy(k.tv, PURE_FORWARD, k.fmt, f.v.d, f.v.starts, f.v.n, f.v.nblk, k.dx, k.dy, k.dz, rvs,
+                        k.brick_group, st))
+      return false;
+    launch_vel_pml(k.pml_cz, k.fmt, f.p.d, f.p.starts, f.p.n, f.p.nblk, k.dx, k.dy, k.dz, rvs, k.pml_group,
+                   k.pml_order ? &f.p.ord : nullptr, st);
+  }
   for (const BatchMember &m : ms) exchange_on(m.c, 0, 0, st);
-  launch_source_batch(k.fmt, f.io.d, f.io.n, gs, gsp, st);
-  if (!launch_stress_phy(k.ts, PURE_FORWARD, k.fmt, f.s.d, f.s.starts, f.s.n, f.s.nblk, k.dx, k.dy, k.dz, k.dt * rsv, k.brick_group, st))
-    return false;
-  launch_stress_pml(k.pml_cz, 0, k.fmt, f.p.d, f.p.starts, f.p.n, f.p.nblk, k.dx, k.dy, k.dz, k.dt * rsv,
-                    k.pml_group, k.pml_order ? &f.p.ord : nullptr, st);
+  StepIO io;
+  io.io = f.io.d;
+  io.starts = f.io.starts;
+  io.n = f.io.n;
+  io.nblk = f.io.nblk;
+  io.gs = gs;
+  io.gsp = gsp;
+  if (!f.whole || !k.ts.whole || !launch_stress_all(k.ts, PURE_FORWARD, k.fmt, half_of(k, f.s, f.p, k.dt * rsv), io, st)) {
+    launch_source_batch(k.fmt, f.io.d, f.io.n, gs, gsp, st);
+    if (!launch_stress_phy(k.ts, PURE_FORWARD, k.fmt, f.s.d, f.s.starts, f.s.n, f.s.nblk, k.dx, k.dy, k.dz,
+                           k.dt * rsv, k.brick_group, st))
+      return false;
+    launch_stress_pml(k.pml_cz, 0, k.fmt, f.p.d, f.p.starts, f.p.n, f.p.nblk, k.dx, k.dy, k.dz, k.dt * rsv,
+                      k.pml_group, k.pml_order ? &f.p.ord : nullptr, st);
+    launch_recv_batch(k.fmt, io, st);
+  }
   for (const BatchMember &m : ms) exchange_on(m.c, 0, 1, st);
-  launch_recv_batch(k.fmt, f.io.d, f.io.starts, f.io.n, f.io.nblk, gs, gsp, st);
   return true;
 }
 static const char *kNoKernel = "no physical-region kernel for the batch's brick shape and storage format";
@@ -1978,7 +2159,7 @@ extern "C" int ddx_model_batch(ddx_ctx *const *ctxs, const int *ishots, int n) {
   for (int q = 0; q < n; q++)
     if (!ctxs[q]) return DDX_EINVAL;
   ddx_ctx *c0 = ctxs[0];
-  const BatchKey k = batch_key(c0);
+  const BatchKey k = batch_key(c0, batch_cells(ctxs, n));
   HIPCHECK(c0, hipSetDevice(k.device));
   std::vector<BatchMember> ms(n);
   for (int q = 0; q < n; q++) {
@@ -2054,10 +2235,11 @@ static void view(FusedTable<T> &t, const HostTable<T> &h, unsigned char *dev, si
 }
 
 // The fused tables of ms copied into scratch (dev) on stream st; f gets views.
-static int fuse_into_scratch(const std::vector<BatchMember> &ms, FusedSet &f, unsigned char *dev, hipStream_t st,
+static int fuse_into_scratch(std::vector<BatchMember> &ms, FusedSet &f, unsigned char *dev, hipStream_t st,
                              std::string &err) {
   FusedHost h;
   fuse_host(ms, h);
+  f.whole = batch_whole(ms);
   std::vector<PmlPiece> pieces;
   PmlOrder ord;
   pml_order_host(h.p.d, ms[0].c->pml_cz, pieces, ord);
@@ -2088,7 +2270,7 @@ extern "C" int ddx_model_batch_noalloc(ddx_ctx *const *ctxs, const int *ishots, 
   for (int q = 0; q < n; q++)
     if (!ctxs[q]) return DDX_EINVAL;
   ddx_ctx *c0 = ctxs[0];
-  const BatchKey k = batch_key(c0);
+  const BatchKey k = batch_key(c0, batch_cells(ctxs, n));
   HIPCHECK(c0, hipSetDevice(k.device));
   unsigned char *dev = nullptr;
   if (int rc = scratch_of(k.device, &dev, c0->err)) return rc;
@@ -2135,6 +2317,8 @@ struct RtmTables {  // the fused tables of one RTM batch
   FusedTable<SlabDesc> fp, rp;                 // CPML of the forward and reverse sets
   FusedTable<MemberIO> src, inj;               // sources (set 0) and receiver injection (set 1)
   FusedTable<ImgDesc> img;
+  bool whole = false;  // the forward and reverse half steps may run as one launch each
+  Tiling sh[6];        // brick shapes of fv, fs, bv, bs, rv, rs
 };
 
 // joins (nullable): each member's MemberIO::join, with rev its direction
@@ -2143,8 +2327,10 @@ static int rtm_batch_tables(const std::vector<ddx_ctx *> &cs, const std::vector<
                             std::string &err, const std::vector<int> *joins = nullptr, int rev = 0) {
   ddx_ctx *c0 = cs[0];
   const int F = RTM_FORWARD, B = RTM_BACKWARD, R = RTM_REVERSE;
-  const Tiling sh[6] = {c0->tiling_vel[F], c0->tiling_stress[F], c0->tiling_vel[B],
-                        c0->tiling_stress[B], c0->tiling_vel[R], c0->tiling_stress[R]};
+  const double cells = batch_cells(cs.data(), (int)cs.size());
+  const Tiling sh[6] = {brick_for(c0, 0, F, cells), brick_for(c0, 1, F, cells), brick_for(c0, 0, B, cells),
+                        brick_for(c0, 1, B, cells), brick_for(c0, 0, R, cells), brick_for(c0, 1, R, cells)};
+  std::copy(sh, sh + 6, T.sh);
   const int mode_of[6] = {F, F, B, B, R, R}, set_of[6] = {0, 0, 0, 0, 1, 1};
   std::vector<HostTable<PhyDesc>> hp[6];
   std::vector<HostTable<SlabDesc>> hf(cs.size()), hr(cs.size());
@@ -2162,35 +2348,20 @@ static int rtm_batch_tables(const std::vector<ddx_ctx *> &cs, const std::vector<
     if (e == hipSuccess) e = download_table(c->pml[model_for(c, F)][0], hf[q]);
     if (e == hipSuccess) e = download_table(c->pml[model_for(c, R)][1], hr[q]);
     if (e == hipSuccess) e = download_table(c->img, him[q]);
-    const int ishot = shots[q];
-    MemberIO x{};
-    const int s = c->shot_sub[ishot];
-    if (s >= 0) {
-      x.sxx = fptr(c, 0, s, SXX);
-      x.syy = fptr(c, 0, s, SYY);
-      x.szz = fptr(c, 0, s, SZZ);
-      x.src_off = c->shot_off[ishot];
-    }
-    x.wavelet = c->wavelet;
-    x.src_mode = c->d.source_mode;
-    x.ss = scale_of(c, 1);
-    x.rsub = c->d_rsub;
-    x.roff = c->d_roff;
-    x.nrec = c->nrec;
-    x.seis = c->seis[ishot];
-    x.inv_sv = 1.0f / scale_of(c, 0);
-    x.sv = scale_of(c, 0);
+    MemberIO x = member_io(c, shots[q], 0);
     x.join = joins ? (*joins)[q] : 0;
     x.rev = rev;
-    x.ntime = c->d.ntime;
-    x.vptr = c->d_vptr[0];
+    for (int k = 0; k < 6; k++) set_member(hp[k][q], (int)q);
+    set_member(hf[q], (int)q);
+    set_member(hr[q], (int)q);
     hs[q].d.push_back(x);
     hs[q].s.push_back(0);
     hs[q].nblk = 0;
     x.vptr = c->d_vptr[1];  // the observed data go into the reverse set
     hi[q].d.push_back(x);
     hi[q].s.push_back(0);
-    hi[q].nblk = (x.nrec + kBlock - 1) / kBlock;
+    hi[q].nblk = recv_blocks(c);
+    T.whole = (q ? T.whole : c0->pml_cz == 1 && !c0->pml_order) && source_owned(c, shots[q]);
   }
   if (e == hipSuccess) e = hipStreamSynchronize(c0->st);
   auto ptrs = [](auto &v) {
@@ -2217,6 +2388,7 @@ static int rtm_batch_tables(const std::vector<ddx_ctx *> &cs, const std::vector<
   if (e == hipSuccess) e = upload_owned(m1, T.src);
   if (e == hipSuccess) e = upload_owned(m2, T.inj);
   if (e == hipSuccess) e = upload_owned(im, T.img);
+  T.whole = T.whole && cells <= c0->whole_cells;
   if (e != hipSuccess) { err = std::string("HIP: ") + hipGetErrorString(e); return DDX_EHIP; }
   return DDX_OK;
 }
@@ -2228,17 +2400,25 @@ static bool rtm_fused_forward(const BatchKey &k, const ddx_ctx *c0, const RtmTab
                               const std::vector<ddx_ctx *> &cs, const std::vector<int> &its, int gs, hipStream_t st) {
   const int F = RTM_FORWARD;
   const float rvs = std::ldexp(1.0f, k.lg0 - k.lg1), rsv = std::ldexp(1.0f, k.lg1 - k.lg0);
-  if (!launch_vel_phy(c0->tiling_vel[F], F, k.fmt, T.fv.d, T.fv.starts, T.fv.n, T.fv.nblk, k.dx, k.dy, k.dz, rvs, k.brick_group, st))
-    return false;
-  launch_vel_pml(k.pml_cz, k.fmt, T.fp.d, T.fp.starts, T.fp.n, T.fp.nblk, k.dx, k.dy, k.dz, rvs, k.pml_group,
-                 k.pml_order ? &T.fp.ord : nullptr, st);
+  if (!T.whole || !T.sh[0].whole || !launch_vel_all(T.sh[0], F, k.fmt, half_of(k, T.fv, T.fp, rvs), st)) {
+    if (!launch_vel_phy(T.sh[0], F, k.fmt, T.fv.d, T.fv.starts, T.fv.n, T.fv.nblk, k.dx, k.dy, k.dz, rvs,
+                        k.brick_group, st))
+      return false;
+    launch_vel_pml(k.pml_cz, k.fmt, T.fp.d, T.fp.starts, T.fp.n, T.fp.nblk, k.dx, k.dy, k.dz, rvs, k.pml_group,
+                   k.pml_order ? &T.fp.ord : nullptr, st);
+  }
   for (ddx_ctx *c : cs) exchange_on(c, 0, 0, st);
-  launch_source_batch(k.fmt, T.src.d, T.src.n, gs, nullptr, st, 1.f);
-  if (!launch_stress_phy(c0->tiling_stress[F], F, k.fmt, T.fs.d, T.fs.starts, T.fs.n, T.fs.nblk, k.dx, k.dy, k.dz,
-                         k.dt * rsv, k.brick_group, st))
-    return false;
-  launch_stress_pml(k.pml_cz, 1, k.fmt, T.fp.d, T.fp.starts, T.fp.n, T.fp.nblk, k.dx, k.dy, k.dz, k.dt * rsv,
-                    k.pml_group, k.pml_order ? &T.fp.ord : nullptr, st);
+  StepIO io;
+  io.io = T.src.d;
+  io.gs = gs;
+  if (!T.whole || !T.sh[1].whole || !launch_stress_all(T.sh[1], F, k.fmt, half_of(k, T.fs, T.fp, k.dt * rsv), io, st)) {
+    launch_source_batch(k.fmt, T.src.d, T.src.n, gs, nullptr, st, 1.f);
+    if (!launch_stress_phy(T.sh[1], F, k.fmt, T.fs.d, T.fs.starts, T.fs.n, T.fs.nblk, k.dx, k.dy, k.dz,
+                           k.dt * rsv, k.brick_group, st))
+      return false;
+    launch_stress_pml(k.pml_cz, 1, k.fmt, T.fp.d, T.fp.starts, T.fp.n, T.fp.nblk, k.dx, k.dy, k.dz, k.dt * rsv,
+                      k.pml_group, k.pml_order ? &T.fp.ord : nullptr, st);
+  }
   for (ddx_ctx *c : cs) exchange_on(c, 0, 1, st);
   // each member saves slices 0 .. its own ntime - 2 (members of a
   // continuous batch may differ in ntime)
@@ -2255,10 +2435,10 @@ static bool rtm_fused_reverse(const BatchKey &k, const ddx_ctx *c0, const RtmTab
   const float rvs = std::ldexp(1.0f, k.lg0 - k.lg1), rsv = std::ldexp(1.0f, k.lg1 - k.lg0);
   const float dx = k.dx, dy = k.dy, dz = k.dz, dt = k.dt;
   auto vel = [&](const FusedTable<PhyDesc> &t, int mode, float sign) {
-    return launch_vel_phy(c0->tiling_vel[mode], mode, k.fmt, t.d, t.starts, t.n, t.nblk, dx, dy, dz, sign * rvs, k.brick_group, st);
+    return launch_vel_phy(T.sh[mode == B ? 2 : 4], mode, k.fmt, t.d, t.starts, t.n, t.nblk, dx, dy, dz, sign * rvs, k.brick_group, st);
   };
   auto stress = [&](const FusedTable<PhyDesc> &t, int mode, float d) {
-    return launch_stress_phy(c0->tiling_stress[mode], mode, k.fmt, t.d, t.starts, t.n, t.nblk, dx, dy, dz, d * rsv, k.brick_group, st);
+    return launch_stress_phy(T.sh[mode == B ? 3 : 5], mode, k.fmt, t.d, t.starts, t.n, t.nblk, dx, dy, dz, d * rsv, k.brick_group, st);
   };
   launch_source_batch(k.fmt, T.src.d, T.src.n, gs, nullptr, st, -1.f);
   launch_inject_batch(k.fmt, T.inj.d, T.inj.starts, T.inj.n, T.inj.nblk, gs, st);
@@ -2266,17 +2446,21 @@ static bool rtm_fused_reverse(const BatchKey &k, const ddx_ctx *c0, const RtmTab
   for (size_t q = 0; q < cs.size(); q++)
     if (its[q] >= 1) ring(cs[q], -1, 2, its[q] - 1, st);
   for (ddx_ctx *c : cs) exchange_on(c, 0, 2, st);
-  if (!vel(T.rv, R, 1.f)) return false;
-  launch_vel_pml(k.pml_cz, k.fmt, T.rp.d, T.rp.starts, T.rp.n, T.rp.nblk, dx, dy, dz, rvs, k.pml_group,
-                 k.pml_order ? &T.rp.ord : nullptr, st);
+  if (!T.whole || !T.sh[4].whole || !launch_vel_all(T.sh[4], R, k.fmt, half_of(k, T.rv, T.rp, rvs), st)) {
+    if (!vel(T.rv, R, 1.f)) return false;
+    launch_vel_pml(k.pml_cz, k.fmt, T.rp.d, T.rp.starts, T.rp.n, T.rp.nblk, dx, dy, dz, rvs, k.pml_group,
+                   k.pml_order ? &T.rp.ord : nullptr, st);
+  }
   for (ddx_ctx *c : cs) exchange_on(c, 1, 0, st);
   if (!vel(T.bv, B, -1.f)) return false;
   for (size_t q = 0; q < cs.size(); q++)
     if (its[q] >= 1) ring(cs[q], -1, 1, its[q] - 1, st);
   for (ddx_ctx *c : cs) exchange_on(c, 0, 0, st);
-  if (!stress(T.rs, R, dt)) return false;
-  launch_stress_pml(k.pml_cz, 1, k.fmt, T.rp.d, T.rp.starts, T.rp.n, T.rp.nblk, dx, dy, dz, dt * rsv, k.pml_group,
-                    k.pml_order ? &T.rp.ord : nullptr, st);
+  if (!T.whole || !T.sh[5].whole || !launch_stress_all(T.sh[5], R, k.fmt, half_of(k, T.rs, T.rp, dt * rsv), StepIO{}, st)) {
+    if (!stress(T.rs, R, dt)) return false;
+    launch_stress_pml(k.pml_cz, 1, k.fmt, T.rp.d, T.rp.starts, T.rp.n, T.rp.nblk, dx, dy, dz, dt * rsv, k.pml_group,
+                      k.pml_order ? &T.rp.ord : nullptr, st);
+  }
   for (ddx_ctx *c : cs) exchange_on(c, 1, 2, st);
   launch_image(c0->d.image_fp64, k.fmt, T.img.d, T.img.starts, T.img.n, T.img.nblk, 1.0f / std::ldexp(1.0f, k.lg0),
                st);
@@ -2288,7 +2472,7 @@ extern "C" int ddx_rtm_batch(ddx_ctx *const *ctxs, const int *ishots, int n) {
   for (int q = 0; q < n; q++)
     if (!ctxs[q]) return DDX_EINVAL;
   ddx_ctx *c0 = ctxs[0];
-  const BatchKey k = batch_key(c0);
+  const BatchKey k = batch_key(c0, batch_cells(ctxs, n));
   HIPCHECK(c0, hipSetDevice(k.device));
   std::vector<ddx_ctx *> cs(ctxs, ctxs + n);
   std::vector<int> shots(ishots, ishots + n);
@@ -2393,7 +2577,7 @@ extern "C" int ddx_batch_add(ddx_batch *b, ddx_ctx *c, int ishot) {
     if (d == c) { b->err = "the context's finished shot has not been collected"; return DDX_EINVAL; }
   // the first member to join sets what the others must share
   const bool first = !b->keyed;
-  const BatchKey key = first ? batch_key(c) : b->key;
+  const BatchKey key = first ? batch_key(c, ext_cells(c)) : b->key;
   if (!batch_compatible(key, c)) {
     b->err = kBatchMismatch;
     return DDX_EINVAL;
@@ -2428,7 +2612,7 @@ extern "C" int ddx_batch_add_rtm(ddx_batch *b, ddx_ctx *c, int ishot) {
   for (ddx_ctx *d : b->done)
     if (d == c) { b->err = "the context's finished shot has not been collected"; return DDX_EINVAL; }
   const bool first = !b->keyed;
-  const BatchKey key = first ? batch_key(c) : b->key;
+  const BatchKey key = first ? batch_key(c, ext_cells(c)) : b->key;
   if (!batch_compatible(key, c) || c->set_overlap || (b->image_fp64 >= 0 && c->d.image_fp64 != b->image_fp64)) {
     b->err = std::string(kBatchMismatch) + ", one image precision for the RTM members, and no reverse-set overlap";
     return DDX_EINVAL;
@@ -2858,8 +3042,7 @@ static int rtm_forward_step(ddx_ctx *c, int ishot, int it) {
   const int nt = c->d.ntime;
   int rc;
   if ((rc = vel_half(c, 0, RTM_FORWARD))) return rc;
-  if ((rc = ddx_source(c, 0, ishot, it, +1))) return rc;
-  if ((rc = stress_half(c, 0, RTM_FORWARD))) return rc;
+  if ((rc = source_stress(c, RTM_FORWARD, ishot, it, nullptr, false))) return rc;
   if (it <= nt - 2) ring(c, +1, 0, it);
   // forward state after step it == backward state after reverse iteration it + 1
   if (c->snap_every > 0 && (nt - 1 - it) % c->snap_every == 0) snapshot(c, 0, (nt - 1 - it) / c->snap_every);
@@ -2928,6 +3111,7 @@ extern "C" int ddx_rtm_shot(ddx_ctx *c, int ishot) {
   if (!c) return DDX_EINVAL;
   int rc = rtm_begin(c, ishot);
   if (rc) return rc;
+  if ((rc = set_shot(c, ishot))) return rc;
   const int nt = c->d.ntime;
   for (int it = 0; it < nt; it++)
     if ((rc = rtm_forward_step(c, ishot, it))) return rc;
@@ -2965,6 +3149,7 @@ extern "C" int ddx_model_steps(ddx_ctx *c, int ishot, int s0, int n) {
     if ((rc = ensure_seis(c, ishot))) return rc;
     if ((rc = ddx_reset_wave(c, 0))) return rc;
   }
+  if ((rc = set_shot(c, ishot))) return rc;
   c->chunk_kind = 1;
   c->chunk_shot = ishot;
   for (int it = s0; it < s0 + n; it++) {
@@ -2982,6 +3167,7 @@ extern "C" int ddx_rtm_steps(ddx_ctx *c, int ishot, int s0, int n) {
   int rc;
   if ((rc = chunk_order(c, 2, ishot, s0, n, 2 * nt))) return rc;
   if (s0 == 0 && (rc = rtm_begin(c, ishot))) return rc;
+  if ((rc = set_shot(c, ishot))) return rc;
   c->chunk_kind = 2;
   c->chunk_shot = ishot;
   for (int st = s0; st < s0 + n; st++) {
@@ -3122,7 +3308,7 @@ extern "C" int ddx_set_tiling_mode(ddx_ctx *c, int kernel, int mode, int tx, int
     return DDX_EINVAL;
   }
   HIPCHECK(c, hipStreamSynchronize(c->st));
-  (kernel == 0 ? c->tiling_vel : c->tiling_stress)[mode] = t;
+  set_brick(c, kernel, mode, t);
   for (int m = 0; m < 2; m++)
     if (c->model[m] && !phy_tables(c, t, m)) return DDX_EHIP;
   return DDX_OK;
@@ -3138,7 +3324,7 @@ extern "C" int ddx_set_tiling_mode(ddx_ctx *c, int kernel, int mode, int tx, int
 // timing launches run on the current wavefields; both sets are reset
 // afterwards.
 static std::mutex g_tune_mu;
-static std::map<std::string, Tiling> g_tune_cache;
+static std::map<std::string, std::pair<Tiling, Tiling>> g_tune_cache;  // a launch of its own, and as used
 
 static std::string tune_key(const ddx_ctx *c, int kernel, int mode) {
   char b[160];
@@ -3147,6 +3333,19 @@ static std::string tune_key(const ddx_ctx *c, int kernel, int mode) {
   snprintf(b, sizeof b, "f%d k%d m%d R%d b%dx%dx%d mig%d", c->fmt, kernel, mode,
            mode == RTM_BACKWARD ? c->d.rec_width : 0, big[0], big[1], big[2], (int)model_for(c, mode));
   return b;
+}
+
+// Milliseconds of `reps` calls of f on the context's stream, after one that
+// warms up and builds tables.
+template <class F>
+static int time_launches(ddx_ctx *c, hipEvent_t e0, hipEvent_t e1, int reps, float &ms, F &&f) {
+  if (int rc = f()) return rc;
+  if (hipEventRecord(e0, c->st) != hipSuccess) return DDX_EHIP;
+  for (int r = 0; r < reps; r++)
+    if (int rc = f()) return rc;
+  if (hipEventRecord(e1, c->st) != hipSuccess || hipEventSynchronize(e1) != hipSuccess) return DDX_EHIP;
+  (void)hipEventElapsedTime(&ms, e0, e1);
+  return DDX_OK;
 }
 
 extern "C" int ddx_autotune(ddx_ctx *c, int reps, int *timed) {
@@ -3171,29 +3370,40 @@ extern "C" int ddx_autotune(ddx_ctx *c, int reps, int *timed) {
         std::lock_guard<std::mutex> lk(g_tune_mu);
         auto it = g_tune_cache.find(key);
         if (it != g_tune_cache.end()) {
-          slot = it->second;
+          c->apart[kernel][mode] = it->second.first;
+          slot = it->second.second;
           continue;
         }
       }
       float best = 1e30f;
       Tiling bt = slot;
       for (int q = 0; q < nc && !rc; q++) {
-        if ((rc = phy_launch(c, kernel, 0, mode, cand[q]))) break;  // warm-up (and table build)
-        if (hipEventRecord(e0, c->st) != hipSuccess) { rc = DDX_EHIP; break; }
-        for (int r = 0; r < reps && !rc; r++) rc = phy_launch(c, kernel, 0, mode, cand[q]);
-        if (rc || hipEventRecord(e1, c->st) != hipSuccess || hipEventSynchronize(e1) != hipSuccess) {
-          rc = rc ? rc : DDX_EHIP;
-          break;
-        }
         float ms = 0.f;
-        (void)hipEventElapsedTime(&ms, e0, e1);
+        if ((rc = time_launches(c, e0, e1, reps, ms, [&] { return phy_launch(c, kernel, 0, mode, cand[q]); }))) break;
         count++;
         if (ms < best) { best = ms; bt = cand[q]; }
       }
+      const Tiling apart = bt;
+      // the whole half step (CPML cells too): that brick and the CPML kernel
+      // apart, against every shape that runs them as one launch
+      if (!rc && mode != RTM_BACKWARD && c->pml[model_for(c, mode)][0].cells + phy_cells(c) <= c->whole_cells) {
+        float whole_best = 1e30f;
+        for (int q = -1; q < nc && !rc; q++) {
+          Tiling t = q < 0 ? apart : cand[q];
+          t.whole = q >= 0;
+          if (q >= 0 && !whole_shape(t, c->fmt)) continue;
+          slot = t;
+          float ms = 0.f;
+          rc = time_launches(c, e0, e1, reps, ms, [&] { return kernel == 0 ? vel_update(c, 0, mode) : stress_update(c, 0, mode); });
+          count++;
+          if (!rc && ms < whole_best) { whole_best = ms; bt = t; }
+        }
+      }
       if (rc) break;
       slot = bt;
+      c->apart[kernel][mode] = apart;
       std::lock_guard<std::mutex> lk(g_tune_mu);
-      g_tune_cache[key] = bt;
+      g_tune_cache[key] = {apart, bt};
     }
   c->prof.mask = prof_mask;
   (void)hipEventDestroy(e0);
@@ -3225,7 +3435,7 @@ extern "C" int ddx_set_brick(ddx_ctx *c, int kernel, int mode, int tx, int ty, i
     return DDX_EINVAL;
   }
   HIPCHECK(c, hipStreamSynchronize(c->st));
-  (kernel == 0 ? c->tiling_vel : c->tiling_stress)[mode] = t;
+  set_brick(c, kernel, mode, t);
   for (int m = 0; m < 2; m++)
     if (c->model[m] && !phy_tables(c, t, m)) return DDX_EHIP;
   return DDX_OK;

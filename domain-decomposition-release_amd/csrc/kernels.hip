@@ -63,12 +63,50 @@ __device__ __forceinline__ int xcd_group_remap(int b, int nblk, int g) {
   return ((i / g) * 8 + x) * g + (i % g);
 }
 
-// Block order of the z-blocked bricks: grp = 0 one contiguous chunk per XCD
-// (xcd_remap), grp > 0 groups of grp blocks dealt round-robin (the engine
-// passes 8: measured 1-3.5% faster than contiguous chunks on the 256x256x200
-// RTM shot, every group size from 1 to 16 within 1% of each other).
+// Block order of the z-blocked bricks (grp): > 0 the bricks in x, y, z order,
+// groups of grp blocks dealt to the XCDs round-robin; 0 that order, one
+// contiguous chunk per XCD; < 0 columns of 256 cells x 16 rows that run
+// through z, one contiguous chunk per XCD.  Launches of the physical region
+// alone take groups of 8 (1-3.5% faster than contiguous chunks on the
+// 256x256x200 grid, sizes 1 to 16 within 1% of each other; 676x676x210:
+// 81.0 ms per 20 steps against 82.4 for columns).  Whole half steps take the
+// columns: how far apart a brick and its z neighbour then run does not
+// depend on how many bricks a plane has (100^3 grid, 15 layers, 60 steps:
+// groups 6.09 ms, contiguous 5.67, columns 5.70; 128^3 8.60, 8.77, 8.58).
 __device__ __forceinline__ int brick_block(int b, int nblk, int grp) {
   return grp > 0 ? xcd_group_remap(b, nblk, grp) : xcd_remap(b, nblk);
+}
+
+// Place of brick t in a region of nx x ny x nz cells, W x H x kz cells per brick.
+struct TileAt {
+  int x, y, z;
+};
+template <int W, int H>
+__device__ __forceinline__ TileAt tile_at(int nx, int ny, int nz, int kz, int t, int grp) {
+  const int tiles_x = (nx + W - 1) / W, tiles_y = (ny + H - 1) / H;
+  TileAt r;
+  if (grp >= 0) {
+    const int per = tiles_x * tiles_y;
+    r.z = t / per;
+    const int rem = t - r.z * per;
+    r.y = rem / tiles_x;
+    r.x = rem - r.y * tiles_x;
+    return r;
+  }
+  constexpr int X = W < 256 ? 256 / W : 1, Y = H < 16 ? 16 / H : 1;
+  const int chunks = (nz + kz - 1) / kz;
+  const int strip = t / (tiles_x * Y * chunks);
+  t -= strip * (tiles_x * Y * chunks);
+  const int h = min(Y, tiles_y - strip * Y);
+  const int col = t / (X * h * chunks);
+  t -= col * (X * h * chunks);
+  const int w = min(X, tiles_x - col * X);
+  r.z = t / (w * h);
+  t -= r.z * (w * h);
+  const int y = t / w;
+  r.x = col * X + (t - y * w);
+  r.y = strip * Y + y;
+  return r;
 }
 
 // Field pointers reach the kernels through descriptor tables in global
@@ -133,6 +171,44 @@ template <typename GT>
 __device__ __forceinline__ void add_to(GT *p, long i, float v) {
   p[i] = narrow(widen(p[i]) + v, p);
 }
+
+// Accesses at a block-uniform pointer plus a per-lane byte offset: one scalar
+// register pair per array and one vector register per offset, shared by all
+// arrays, instead of a 64-bit vector address per access.
+typedef __attribute__((address_space(1))) char gchar;
+typedef float f4v __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(1))) f4v gf4v;
+template <typename GT>
+__device__ __forceinline__ float ldo(const GT *p, unsigned off, int elem = 0) {
+  return widen(*((const GT *)((const gchar *)p + off) + elem));
+}
+template <typename GT>
+__device__ __forceinline__ float sto(GT *p, unsigned off, float v) {
+  const auto r = narrow(v, p);
+  *(GT *)((gchar *)p + off) = r;
+  return widen(r);
+}
+
+// x / d for a block-uniform d with r = RN(1 / d): RN(q + r (x - q d)) with
+// q = RN(x r) is the correctly rounded quotient (Markstein) as long as the
+// remainder is exact, which div_ok tells for a group of results: 0, or
+// magnitudes that neither x nor the remainder can under- or overflow at.
+// (Three operations against eleven of the general division.)
+__device__ __forceinline__ float div_u(float x, float d, float r) {
+  const float q = x * r;
+  return __builtin_fmaf(__builtin_fmaf(-q, d, x), r, q);
+}
+struct DivGuard {
+  unsigned lo = 0xffffffffu, hi = 0;
+  // magnitudes shifted up, less one for the minimum: a zero never is it
+  __device__ __forceinline__ void add(float y) {
+    const unsigned u = __float_as_uint(y) << 1;
+    lo = min(lo, u - 1u);
+    hi = max(hi, u);
+  }
+  // every result 0, or between 2^-90 and 2^100 (d and 1 / d are within 2^20)
+  __device__ __forceinline__ bool ok() const { return lo >= (37u << 24) && hi < (227u << 24); }
+};
 
 // Cells that one thread alone reads and writes in a launch (the updated
 // fields and the per-cell model arrays of the physical-region bricks, the
@@ -201,6 +277,36 @@ __device__ __forceinline__ float dm2(PT f, long i, long s, float c0, float c1) {
 __device__ __forceinline__ int vowr_order(int p, int n, int R) {
   int d = min(p, n - 1 - p);
   return d >= 4 ? 4 : max(R, d + 1);
+}
+
+// The source of a shot inside a stress update: the thread that owns the cell
+// adds the sample to the values it has read (what k_source would have stored
+// before the update).  x = -1: none.
+struct SrcCell {
+  int x = -1, y = 0, z = 0, all = 0;
+  float w = 0.f;
+};
+// Member q's source at batch step gs (or *gsp), as k_source_batch has it.
+template <class S>
+__device__ __forceinline__ SrcCell src_cell(const StepIO &io, int q) {
+  SrcCell c;
+  if (!io.io) return c;
+  const MemberIO *m = io.io + q;
+  const int g = io.gsp ? *io.gsp : io.gs;
+  const int it = m->rev ? m->join - g : g - m->join;
+  if (it >= 0 && it < m->ntime) {
+    c.x = m->src_x; c.y = m->src_y; c.z = m->src_z;
+    c.all = m->src_mode == 0;
+    c.w = std::is_same<S, F32>::value ? m->wavelet[it] : m->wavelet[it] * m->ss;
+  }
+  return c;
+}
+template <typename GT>
+__device__ __forceinline__ void add_source(const SrcCell &c, int x, int y, int z, float &xx, float &yy, float &zz) {
+  const bool hit = x == c.x && y == c.y && z == c.z;
+  const GT *t = nullptr;
+  if (hit && c.all) { xx = quant(t, xx + c.w); yy = quant(t, yy + c.w); }
+  if (hit) zz = quant(t, zz + c.w);
 }
 
 struct Coef4 {
@@ -284,8 +390,7 @@ __global__ __launch_bounds__(kBlock) void k_vel_phy(const PhyDesc *__restrict__ 
 // ---------------------------------------------------------------------------
 template <int MODE>
 __global__ __launch_bounds__(kBlock) void k_stress_phy(const PhyDesc *__restrict__ descs,
-                                                       const int *__restrict__ starts, int n, float dx,
-                                                       float dy, float dz, float dt) {
+                                                       const int *__restrict__ starts, int n, float a, float bb, float c) {
   const int b = xcd_remap(blockIdx.x, gridDim.x);
   const PhyDesc &D = descs[find_desc(starts, n, b)];
   const int t = b - D.blk0;
@@ -311,7 +416,6 @@ __global__ __launch_bounds__(kBlock) void k_stress_phy(const PhyDesc *__restrict
     cz = cx;
   }
   const gfloat *vx = G(D.f[VX]), *vy = G(D.f[VY]), *vz = G(D.f[VZ]);
-  const float a = dt / dx, bb = dt / dy, c = dt / dz;
   const float lm = G(D.lam)[id], mu = G(D.mu)[id];
   const float l2m = lm + 2.0f * mu;
   const float vx_x = dm4(vx, id, 1, cx.c0, cx.c1, cx.c2, cx.c3);
@@ -343,17 +447,10 @@ __global__ __launch_bounds__(kBlock) void k_stress_phy(const PhyDesc *__restrict
 // k_vel_phy / k_stress_phy, so results are bit-identical.
 // ---------------------------------------------------------------------------
 template <int TX, int TY, int CY, int CZ>
-__device__ __forceinline__ bool zbrick(const PhyDesc &D, int t, int &i, int &j0, int &k0) {
-  const int tiles_x = (D.nx + TX - 1) / TX;
-  const int tiles_y = (D.ny + TY * CY - 1) / (TY * CY);
-  const int per = tiles_x * tiles_y;
-  const int zc = t / per;
-  const int rem = t - zc * per;
-  const int ty = rem / tiles_x;
-  const int tx = rem - ty * tiles_x;
-  i = tx * TX + (int)(threadIdx.x % TX);
-  j0 = ty * TY * CY + (int)(threadIdx.x / TX);
-  k0 = zc * CZ;
+__device__ __forceinline__ bool zbrick(const PhyDesc &D, const TileAt &t, int &i, int &j0, int &k0) {
+  i = t.x * TX + (int)(threadIdx.x % TX);
+  j0 = t.y * TY * CY + (int)(threadIdx.x / TX);
+  k0 = t.z * CZ;
   return i < D.nx;
 }
 
@@ -572,10 +669,8 @@ __device__ __forceinline__ void vel_zb_body(const PhyDesc &D, int i, int j0, int
 }
 
 // `dt` carries the stress-over-velocity scale ratio of the 16-bit formats.
-template <int MODE, int TX, int TY, int CY, int CZ, class S, bool XL = false>
-__device__ __forceinline__ void stress_zb_body(const PhyDesc &D, int i, int j0, int k0, float dx, float dy,
-                                               float dz, float dt,
-                                               bool live = true) {
+template <int MODE, int TX, int TY, int CY, int CZ, class S, bool XL = false, bool SRC = false>
+__device__ __forceinline__ void stress_zb_body(const PhyDesc &D, int i, int j0, int k0, float a, float bb, float c, bool live = true, const SrcCell &src = SrcCell{}) {
   typedef typename GPtr<S>::T gT;
   const long sy = D.sy, sz = D.sz;
   const XLane xl = xlane(i, D.nx);
@@ -592,7 +687,6 @@ __device__ __forceinline__ void stress_zb_body(const PhyDesc &D, int i, int j0, 
   gT *__restrict__ fsau = (gT *)D.f[SAU];
   const gfloat *__restrict__ flam = G(D.lam);
   const gfloat *__restrict__ fmu = G(D.mu);
-  const float a = dt / dx, bb = dt / dy, c = dt / dz;
   const Coef4 c4 = coef_row(4);
   const Coef4 cx = MODE == RTM_BACKWARD ? coef_row(vowr_order(i, D.nx, D.R)) : c4;
 #pragma unroll
@@ -615,7 +709,8 @@ __device__ __forceinline__ void stress_zb_body(const PhyDesc &D, int i, int j0, 
       // the updated cells are read before the stencil taps: on this target
       // the memory counter also tracks stores, so a read issued after a
       // store waits for that store, which would serialise the updates
-      const float oxx = ld_stream(fsxx, id), oyy = ld_stream(fsyy, id), ozz = ld_stream(fszz, id);
+      float oxx = ld_stream(fsxx, id), oyy = ld_stream(fsyy, id), ozz = ld_stream(fszz, id);
+      if constexpr (SRC) add_source<gT>(src, D.ox + i, D.oy + j, D.oz + k, oxx, oyy, ozz);
       const float oxy = ld_stream(fsxy, id), oxz = ld_stream(fsxz, id), oyz = ld_stream(fsyz, id);
       const float oau = rtm_mode(MODE) ? ld_stream(fsau, id) : 0.f;
       const float lm = ld_stream(flam, id), mu = ld_stream(fmu, id);
@@ -673,18 +768,11 @@ __device__ __forceinline__ void stress_zb_body(const PhyDesc &D, int i, int j0, 
 // gridphy boundary (vowr_order gives 4 for d >= 3, and always for R = 4).
 // Block-uniform, so interior bricks run the constant-coefficient code.
 template <int TX, int TY, int CY, int CZ>
-__device__ __forceinline__ bool brick_full_order(const PhyDesc &D, int t) {
+__device__ __forceinline__ bool brick_full_order(const PhyDesc &D, const TileAt &t) {
   if (D.R >= 4) return true;
-  const int tiles_x = (D.nx + TX - 1) / TX;
-  const int tiles_y = (D.ny + TY * CY - 1) / (TY * CY);
-  const int per = tiles_x * tiles_y;
-  const int zc = t / per;
-  const int rem = t - zc * per;
-  const int ty = rem / tiles_x;
-  const int tx = rem - ty * tiles_x;
-  const int x0 = tx * TX, x1 = min(tx * TX + TX, D.nx) - 1;
-  const int y0 = ty * TY * CY, y1 = min((ty + 1) * TY * CY, D.ny) - 1;
-  const int z0 = zc * CZ, z1 = min(zc * CZ + CZ, D.nz) - 1;
+  const int x0 = t.x * TX, x1 = min(x0 + TX, D.nx) - 1;
+  const int y0 = t.y * TY * CY, y1 = min(y0 + TY * CY, D.ny) - 1;
+  const int z0 = t.z * CZ, z1 = min(z0 + CZ, D.nz) - 1;
   return x0 >= 3 && x1 <= D.nx - 4 && y0 >= 3 && y1 <= D.ny - 4 && z0 >= 3 && z1 <= D.nz - 4;
 }
 
@@ -704,10 +792,11 @@ __global__ __launch_bounds__(TX *TY) DDX_BRICK_ATTR void k_vel_phy_zb(const PhyD
   const int b = brick_block(blockIdx.x, gridDim.x, grp);
   const PhyDesc &D = descs[find_desc(starts, n, b)];
   int i, j0, k0;
-  const bool live = zbrick<TX, TY, CY, CZ>(D, b - D.blk0, i, j0, k0);
+  const TileAt at = tile_at<TX, TY * CY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp);
+  const bool live = zbrick<TX, TY, CY, CZ>(D, at, i, j0, k0);
   if (!XL && !live) return;
   // backward mode and reverse mode differ only in the coefficient rows
-  if (MODE == RTM_BACKWARD && brick_full_order<TX, TY, CY, CZ>(D, b - D.blk0))
+  if (MODE == RTM_BACKWARD && brick_full_order<TX, TY, CY, CZ>(D, at))
     vel_zb_body<RTM_REVERSE, TX, TY, CY, CZ, S, XL>(D, i, j0, k0, dx, dy, dz, sign, live);
   else
     vel_zb_body<MODE, TX, TY, CY, CZ, S, XL>(D, i, j0, k0, dx, dy, dz, sign, live);
@@ -715,18 +804,18 @@ __global__ __launch_bounds__(TX *TY) DDX_BRICK_ATTR void k_vel_phy_zb(const PhyD
 
 template <int MODE, int TX, int TY, int CY, int CZ, class S, bool XL = false>
 __global__ __launch_bounds__(TX *TY) DDX_BRICK_ATTR void k_stress_phy_zb(const PhyDesc *__restrict__ descs,
-                                                          const int *__restrict__ starts, int n, float dx,
-                                                          float dy, float dz, float dt, int grp) {
+                                                          const int *__restrict__ starts, int n, float a, float bb, float c, int grp) {
   static_assert(!XL || TX == 64, "lane-exchange bricks need one wavefront per x row");
   const int b = brick_block(blockIdx.x, gridDim.x, grp);
   const PhyDesc &D = descs[find_desc(starts, n, b)];
   int i, j0, k0;
-  const bool live = zbrick<TX, TY, CY, CZ>(D, b - D.blk0, i, j0, k0);
+  const TileAt at = tile_at<TX, TY * CY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp);
+  const bool live = zbrick<TX, TY, CY, CZ>(D, at, i, j0, k0);
   if (!XL && !live) return;
-  if (MODE == RTM_BACKWARD && brick_full_order<TX, TY, CY, CZ>(D, b - D.blk0))
-    stress_zb_body<RTM_REVERSE, TX, TY, CY, CZ, S, XL>(D, i, j0, k0, dx, dy, dz, dt, live);
+  if (MODE == RTM_BACKWARD && brick_full_order<TX, TY, CY, CZ>(D, at))
+    stress_zb_body<RTM_REVERSE, TX, TY, CY, CZ, S, XL>(D, i, j0, k0, a, bb, c, live);
   else
-    stress_zb_body<MODE, TX, TY, CY, CZ, S, XL>(D, i, j0, k0, dx, dy, dz, dt, live);
+    stress_zb_body<MODE, TX, TY, CY, CZ, S, XL>(D, i, j0, k0, a, bb, c, live);
 }
 
 // ---------------------------------------------------------------------------
@@ -744,9 +833,9 @@ struct YlTile {
   float v[NF][CZ][TY + 8][64];  // field, plane, row (j0-4 ..), x
 };
 
-template <int MODE, int TY, int CZ, class S>
+template <int MODE, int TY, int CZ, class S, bool SRC = false>
 __device__ __forceinline__ void stress_yl_body(YlTile<3, TY, CZ> &ly, const PhyDesc &D, int i, int j0, int k0,
-                                               float dx, float dy, float dz, float dt, bool live) {
+                                               float a, float bb, float c, bool live, const SrcCell &src = SrcCell{}) {
   typedef typename GPtr<S>::T gT;
   const long sy = D.sy, sz = D.sz;
   const int lane = (int)threadIdx.x & 63, w = (int)threadIdx.x >> 6;
@@ -811,7 +900,6 @@ __device__ __forceinline__ void stress_yl_body(YlTile<3, TY, CZ> &ly, const PhyD
   gT *__restrict__ fsau = (gT *)D.f[SAU];
   const gfloat *__restrict__ flam = G(D.lam);
   const gfloat *__restrict__ fmu = G(D.mu);
-  const float a = dt / dx, bb = dt / dy, c = dt / dz;
   const Coef4 c4 = coef_row(4);
   const Coef4 cx = MODE == RTM_BACKWARD ? coef_row(vowr_order(i, D.nx, D.R)) : c4;
   const Coef4 cy = MODE == RTM_BACKWARD ? coef_row(vowr_order(j, D.ny, D.R)) : c4;
@@ -823,7 +911,8 @@ __device__ __forceinline__ void stress_yl_body(YlTile<3, TY, CZ> &ly, const PhyD
     if (k >= D.nz) break;
     const Coef4 cz = MODE == RTM_BACKWARD ? coef_row(vowr_order(k, D.nz, D.R)) : c4;
     const long id = base + (long)kk * sz;
-    const float oxx = ld_stream(fsxx, id), oyy = ld_stream(fsyy, id), ozz = ld_stream(fszz, id);
+    float oxx = ld_stream(fsxx, id), oyy = ld_stream(fsyy, id), ozz = ld_stream(fszz, id);
+    if constexpr (SRC) add_source<gT>(src, D.ox + i, D.oy + j, D.oz + k, oxx, oyy, ozz);
     const float oxy = ld_stream(fsxy, id), oxz = ld_stream(fsxz, id), oyz = ld_stream(fsyz, id);
     const float oau = rtm_mode(MODE) ? ld_stream(fsau, id) : 0.f;
     const float lm = ld_stream(flam, id), mu = ld_stream(fmu, id);
@@ -887,17 +976,17 @@ __device__ __forceinline__ void stress_yl_body(YlTile<3, TY, CZ> &ly, const PhyD
 
 template <int MODE, int TY, int CZ, class S>
 __global__ __launch_bounds__(64 * TY) DDX_BRICK_ATTR void k_stress_phy_yl(const PhyDesc *__restrict__ descs,
-                                                           const int *__restrict__ starts, int n, float dx,
-                                                           float dy, float dz, float dt, int grp) {
+                                                           const int *__restrict__ starts, int n, float a, float bb, float c, int grp) {
   __shared__ YlTile<3, TY, CZ> ly;
   const int b = brick_block(blockIdx.x, gridDim.x, grp);
   const PhyDesc &D = descs[find_desc(starts, n, b)];
   int i, j0, k0;
-  const bool live = zbrick<64, TY, 1, CZ>(D, b - D.blk0, i, j0, k0);
-  if (MODE == RTM_BACKWARD && brick_full_order<64, TY, 1, CZ>(D, b - D.blk0))
-    stress_yl_body<RTM_REVERSE, TY, CZ, S>(ly, D, i, j0, k0, dx, dy, dz, dt, live);
+  const TileAt at = tile_at<64, TY * 1>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp);
+  const bool live = zbrick<64, TY, 1, CZ>(D, at, i, j0, k0);
+  if (MODE == RTM_BACKWARD && brick_full_order<64, TY, 1, CZ>(D, at))
+    stress_yl_body<RTM_REVERSE, TY, CZ, S>(ly, D, i, j0, k0, a, bb, c, live);
   else
-    stress_yl_body<MODE, TY, CZ, S>(ly, D, i, j0, k0, dx, dy, dz, dt, live);
+    stress_yl_body<MODE, TY, CZ, S>(ly, D, i, j0, k0, a, bb, c, live);
 }
 
 // Velocity update with the y arm from LDS: the tile holds syy, sxy, syz and,
@@ -1075,10 +1164,11 @@ __global__ __launch_bounds__(64 * TY) DDX_BRICK_ATTR void k_vel_phy_yl(const Phy
   const int b = brick_block(blockIdx.x, gridDim.x, grp);
   const PhyDesc &D = descs[find_desc(starts, n, b)];
   int i, j0, k0;
-  const bool live = zbrick<64, TY, 1, CZ>(D, b - D.blk0, i, j0, k0);
+  const TileAt at = tile_at<64, TY * 1>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp);
+  const bool live = zbrick<64, TY, 1, CZ>(D, at, i, j0, k0);
   // backward mode and reverse mode differ only in the coefficient rows
   if constexpr (MODE == RTM_BACKWARD) {
-    if (brick_full_order<64, TY, 1, CZ>(D, b - D.blk0))
+    if (brick_full_order<64, TY, 1, CZ>(D, at))
       vel_yl_body<RTM_REVERSE, TY, CZ, S>(ly, D, i, j0, k0, dx, dy, dz, sign, live);
     else
       vel_yl_body<MODE, TY, CZ, S>(ly, D, i, j0, k0, dx, dy, dz, sign, live);
@@ -1256,32 +1346,18 @@ __device__ __forceinline__ float dzq(const float (&zc)[N], int kk, const Coef4 &
 
 // brick of pairs: TX threads cover 2*TX cells in x
 template <int TX, int TY, int CY, int CZ>
-__device__ __forceinline__ bool zbrick2(const PhyDesc &D, int t, int &i, int &j0, int &k0) {
-  const int tiles_x = (D.nx + 2 * TX - 1) / (2 * TX);
-  const int tiles_y = (D.ny + TY * CY - 1) / (TY * CY);
-  const int per = tiles_x * tiles_y;
-  const int zc = t / per;
-  const int rem = t - zc * per;
-  const int ty = rem / tiles_x;
-  const int tx = rem - ty * tiles_x;
-  i = tx * 2 * TX + 2 * (int)(threadIdx.x % TX);
-  j0 = ty * TY * CY + (int)(threadIdx.x / TX);
-  k0 = zc * CZ;
+__device__ __forceinline__ bool zbrick2(const PhyDesc &D, const TileAt &t, int &i, int &j0, int &k0) {
+  i = t.x * 2 * TX + 2 * (int)(threadIdx.x % TX);
+  j0 = t.y * TY * CY + (int)(threadIdx.x / TX);
+  k0 = t.z * CZ;
   return i < D.nx;
 }
 template <int TX, int TY, int CY, int CZ>
-__device__ __forceinline__ bool brick2_full_order(const PhyDesc &D, int t) {
+__device__ __forceinline__ bool brick2_full_order(const PhyDesc &D, const TileAt &t) {
   if (D.R >= 4) return true;
-  const int tiles_x = (D.nx + 2 * TX - 1) / (2 * TX);
-  const int tiles_y = (D.ny + TY * CY - 1) / (TY * CY);
-  const int per = tiles_x * tiles_y;
-  const int zc = t / per;
-  const int rem = t - zc * per;
-  const int ty = rem / tiles_x;
-  const int tx = rem - ty * tiles_x;
-  const int x0 = tx * 2 * TX, x1 = min(tx * 2 * TX + 2 * TX, D.nx) - 1;
-  const int y0 = ty * TY * CY, y1 = min((ty + 1) * TY * CY, D.ny) - 1;
-  const int z0 = zc * CZ, z1 = min(zc * CZ + CZ, D.nz) - 1;
+  const int x0 = t.x * 2 * TX, x1 = min(x0 + 2 * TX, D.nx) - 1;
+  const int y0 = t.y * TY * CY, y1 = min(y0 + TY * CY, D.ny) - 1;
+  const int z0 = t.z * CZ, z1 = min(z0 + CZ, D.nz) - 1;
   return x0 >= 3 && x1 <= D.nx - 4 && y0 >= 3 && y1 <= D.ny - 4 && z0 >= 3 && z1 <= D.nz - 4;
 }
 
@@ -1379,9 +1455,8 @@ __device__ __forceinline__ void vel_zb2_body(const PhyDesc &D, int i, int j0, in
   }
 }
 
-template <int MODE, int TX, int TY, int CY, int CZ, class S>
-__device__ __forceinline__ void stress_zb2_body(const PhyDesc &D, int i, int j0, int k0, float dx, float dy,
-                                                float dz, float dt) {
+template <int MODE, int TX, int TY, int CY, int CZ, class S, bool SRC = false>
+__device__ __forceinline__ void stress_zb2_body(const PhyDesc &D, int i, int j0, int k0, float a, float bb, float c, const SrcCell &src = SrcCell{}) {
   static_assert(MODE != FWI, "the FWI mode runs on the one-cell bricks");
   typedef typename GPtr<S>::T gT;
   const long sy = D.sy, sz = D.sz;
@@ -1397,7 +1472,6 @@ __device__ __forceinline__ void stress_zb2_body(const PhyDesc &D, int i, int j0,
   gT *__restrict__ fsau = (gT *)D.f[SAU];
   const gfloat *__restrict__ flam = G(D.lam);
   const gfloat *__restrict__ fmu = G(D.mu);
-  const float a = dt / dx, bb = dt / dy, c = dt / dz;
   const bool both = i + 1 < D.nx;
   const Coef4 c4 = coef_row(4);
   const Coef4 cxa = MODE == RTM_BACKWARD ? coef_row(vowr_order(i, D.nx, D.R)) : c4;
@@ -1418,7 +1492,11 @@ __device__ __forceinline__ void stress_zb2_body(const PhyDesc &D, int i, int j0,
       if (k >= D.nz) break;
       const Coef4 cz = MODE == RTM_BACKWARD ? coef_row(vowr_order(k, D.nz, D.R)) : c4;
       const long id = base + (long)kk * sz;
-      const F2 oxx = ld2_nt(fsxx, id), oyy = ld2_nt(fsyy, id), ozz = ld2_nt(fszz, id);
+      F2 oxx = ld2_nt(fsxx, id), oyy = ld2_nt(fsyy, id), ozz = ld2_nt(fszz, id);
+      if constexpr (SRC) {
+        add_source<gT>(src, D.ox + i, D.oy + j, D.oz + k, oxx.a, oyy.a, ozz.a);
+        add_source<gT>(src, D.ox + i + 1, D.oy + j, D.oz + k, oxx.b, oyy.b, ozz.b);
+      }
       const F2 oxy = ld2_nt(fsxy, id), oxz = ld2_nt(fsxz, id), oyz = ld2_nt(fsyz, id);
       F2 oau{0.f, 0.f};
       if constexpr (rtm_mode(MODE)) oau = ld2_nt(fsau, id);
@@ -1469,8 +1547,9 @@ __global__ __launch_bounds__(TX *TY) DDX_BRICK_ATTR void k_vel_phy_zb2(const Phy
   const int b = brick_block(blockIdx.x, gridDim.x, grp);
   const PhyDesc &D = descs[find_desc(starts, n, b)];
   int i, j0, k0;
-  if (!zbrick2<TX, TY, CY, CZ>(D, b - D.blk0, i, j0, k0)) return;
-  if (MODE == RTM_BACKWARD && brick2_full_order<TX, TY, CY, CZ>(D, b - D.blk0))
+  const TileAt at = tile_at<2 * TX, TY * CY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp);
+  if (!zbrick2<TX, TY, CY, CZ>(D, at, i, j0, k0)) return;
+  if (MODE == RTM_BACKWARD && brick2_full_order<TX, TY, CY, CZ>(D, at))
     vel_zb2_body<RTM_REVERSE, TX, TY, CY, CZ, S>(D, i, j0, k0, dx, dy, dz, sign);
   else
     vel_zb2_body<MODE, TX, TY, CY, CZ, S>(D, i, j0, k0, dx, dy, dz, sign);
@@ -1478,16 +1557,16 @@ __global__ __launch_bounds__(TX *TY) DDX_BRICK_ATTR void k_vel_phy_zb2(const Phy
 
 template <int MODE, int TX, int TY, int CY, int CZ, class S>
 __global__ __launch_bounds__(TX *TY) DDX_BRICK_ATTR void k_stress_phy_zb2(const PhyDesc *__restrict__ descs,
-                                                           const int *__restrict__ starts, int n, float dx,
-                                                           float dy, float dz, float dt, int grp) {
+                                                           const int *__restrict__ starts, int n, float a, float bb, float c, int grp) {
   const int b = brick_block(blockIdx.x, gridDim.x, grp);
   const PhyDesc &D = descs[find_desc(starts, n, b)];
   int i, j0, k0;
-  if (!zbrick2<TX, TY, CY, CZ>(D, b - D.blk0, i, j0, k0)) return;
-  if (MODE == RTM_BACKWARD && brick2_full_order<TX, TY, CY, CZ>(D, b - D.blk0))
-    stress_zb2_body<RTM_REVERSE, TX, TY, CY, CZ, S>(D, i, j0, k0, dx, dy, dz, dt);
+  const TileAt at = tile_at<2 * TX, TY * CY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp);
+  if (!zbrick2<TX, TY, CY, CZ>(D, at, i, j0, k0)) return;
+  if (MODE == RTM_BACKWARD && brick2_full_order<TX, TY, CY, CZ>(D, at))
+    stress_zb2_body<RTM_REVERSE, TX, TY, CY, CZ, S>(D, i, j0, k0, a, bb, c);
   else
-    stress_zb2_body<MODE, TX, TY, CY, CZ, S>(D, i, j0, k0, dx, dy, dz, dt);
+    stress_zb2_body<MODE, TX, TY, CY, CZ, S>(D, i, j0, k0, a, bb, c);
 }
 
 // ---------------------------------------------------------------------------
@@ -1711,8 +1790,7 @@ __global__ __launch_bounds__(LX *LY) void k_vel_lds(const PhyDesc *__restrict__ 
 
 template <int MODE>
 __global__ __launch_bounds__(LX *LY) void k_stress_lds(const PhyDesc *__restrict__ descs,
-                                                       const int *__restrict__ starts, int n, float dx, float dy,
-                                                       float dz, float dt,
+                                                       const int *__restrict__ starts, int n, float a, float bb, float c,
                                                        int kz) {
   __shared__ float Lx[2][HYW][HXW];
   __shared__ float Ly[2][HYW][HXW];
@@ -1730,7 +1808,6 @@ __global__ __launch_bounds__(LX *LY) void k_stress_lds(const PhyDesc *__restrict
   const long cb = (long)(D.ox + m.i) + sy * (D.oy + m.j) + sz * D.oz;
   const long hb = (long)(D.ox + m.i) + sy * (D.oy + m.hrow) + sz * D.oz;
   const long xb = (long)(D.ox + m.xcol) + sy * (D.oy + y0 + m.xr) + sz * D.oz;
-  const float a = dt / dx, bb = dt / dy, c = dt / dz;
   const Coef4 c4 = coef_row(4);
   const Coef4 cx = MODE == RTM_BACKWARD ? coef_row(vowr_order(min(m.i, D.nx - 1), D.nx, D.R)) : c4;
   const Coef4 cy = MODE == RTM_BACKWARD ? coef_row(vowr_order(min(m.j, D.ny - 1), D.ny, D.R)) : c4;
@@ -1871,10 +1948,10 @@ __global__ __launch_bounds__(LX *LY) void k_stress_lds(const PhyDesc *__restrict
 // order after the group-interleaved remap grp.  Returns false for the
 // surplus workgroups of an XCD with fewer blocks than the largest.
 __device__ __forceinline__ bool pml_block(const SlabDesc *__restrict__ descs, const int *__restrict__ starts,
-                                          int n, int grp, const PmlOrder &ord, int cz, int &di, int &zc,
-                                          int &tile) {
+                                          int n, int block, int nblk, int grp, const PmlOrder &ord, int cz, int &di,
+                                          int &zc, int &tile) {
   if (ord.pieces) {
-    const int x = (int)blockIdx.x & 7, local = (int)blockIdx.x >> 3;
+    const int x = block & 7, local = block >> 3;
     if (local >= ord.xn[x]) return false;
     int lo = ord.xoff[x], hi = ord.xoff[x + 1] - 1;
     while (lo < hi) {
@@ -1889,7 +1966,7 @@ __device__ __forceinline__ bool pml_block(const SlabDesc *__restrict__ descs, co
     tile = P.t0 + (off - q * P.tcnt);
     return true;
   }
-  const int b = xcd_group_remap(blockIdx.x, gridDim.x, grp);
+  const int b = xcd_group_remap(block, nblk, grp);
   di = find_desc(starts, n, b);
   const SlabDesc &D = descs[di];
   const int tiles = pml_plane_tiles(D.ni, D.nj, cz);
@@ -1912,13 +1989,35 @@ __device__ __forceinline__ bool slab_column(const SlabDesc &D, int zc, int tile,
   return ci < plane;
 }
 
-// zq[r] = f(slab plane kc0 + lo + r) for the planes the outputs need
-// (up to kend + 1); the rest read as 0 and are never used.
-template <int CZ, typename GT>
-__device__ __forceinline__ void load_pml_zq(float (&zq)[CZ + 3], const GT *__restrict__ f, long base,
-                                            long sz, int kc0, int lo, int kend) {
-#pragma unroll
-  for (int r = 0; r < CZ + 3; r++) zq[r] = (kc0 + lo + r <= kend + 1) ? ld(f, base + (long)(lo + r) * sz) : 0.f;
+// 4th-order staggered difference of the taps (a - b) and (p - q)
+__device__ __forceinline__ float d2(float a, float b, float p, float q, float c0, float c1) {
+  float r = 0.f;
+  r += c0 * (a - b);
+  r += c1 * (p - q);
+  return r;
+}
+
+// The nine differences of a cell over their spacings, x, y, z three each: the
+// short division where it is exact for every cell of the wavefront.
+__device__ __forceinline__ void div9(float &x0, float &x1, float &x2, float &y0, float &y1, float &y2, float &z0,
+                                     float &z1, float &z2, float dx, float dy, float dz, float rdx, float rdy,
+                                     float rdz) {
+  const float a0 = div_u(x0, dx, rdx), a1 = div_u(x1, dx, rdx), a2 = div_u(x2, dx, rdx);
+  const float b0 = div_u(y0, dy, rdy), b1 = div_u(y1, dy, rdy), b2 = div_u(y2, dy, rdy);
+  const float e0 = div_u(z0, dz, rdz), e1 = div_u(z1, dz, rdz), e2 = div_u(z2, dz, rdz);
+  DivGuard g;
+  g.add(a0); g.add(a1); g.add(a2);
+  g.add(b0); g.add(b1); g.add(b2);
+  g.add(e0); g.add(e1); g.add(e2);
+  if (__builtin_expect(__all(g.ok()), 1)) {
+    x0 = a0; x1 = a1; x2 = a2;
+    y0 = b0; y1 = b1; y2 = b2;
+    z0 = e0; z1 = e1; z2 = e2;
+  } else {
+    x0 = x0 / dx; x1 = x1 / dx; x2 = x2 / dx;
+    y0 = y0 / dy; y1 = y1 / dy; y2 = y2 / dy;
+    z0 = z0 / dz; z1 = z1 / dz; z2 = z2 / dz;
+  }
 }
 
 // Extra attributes of the CPML kernels (occupancy experiments), empty by default.
@@ -1935,40 +2034,76 @@ struct PsiCell {
   GT *p;
   float a, b, ah, bh, m0, m1, m2;
 };
+// psi: the axis' first variable at the block's plane; o: the cell in it
+template <typename GT>
+__device__ __forceinline__ PsiCell<GT> psi_cell(GT *psi, const gfloat *coef, long ncell, unsigned c) {
+  const f4v q = *(const gf4v *)((const gchar *)coef + (size_t)(c * 16u));
+  const unsigned o = c * (unsigned)sizeof(typename std::remove_reference<decltype(*psi)>::type);
+  return {psi, q.x, q.y, q.z, q.w, ldo(psi, o), ldo(psi + ncell, o), ldo(psi + 2 * ncell, o)};
+}
+// the same from the cell's own addresses (planar memory variables, q: its four coefficients)
 template <typename GT>
 __device__ __forceinline__ PsiCell<GT> psi_cell(GT *p, const gfloat *q, long ncell) {
-  return {p, q[0], q[ncell], q[2 * ncell], q[3 * ncell], ld(p, 0), ld(p, ncell), ld(p, 2 * ncell)};
+  const f4v v = *(const gf4v *)q;
+  return {p, v.x, v.y, v.z, v.w, ld(p, 0), ld(p, ncell), ld(p, 2 * ncell)};
+}
+template <typename GT>
+__device__ __forceinline__ void psi_store(GT *psi, long ncell, unsigned c, float p0, float p1, float p2) {
+  const unsigned o = c * (unsigned)sizeof(typename std::remove_reference<decltype(*psi)>::type);
+  sto(psi, o, p0);
+  sto(psi + ncell, o, p1);
+  sto(psi + 2 * ncell, o, p2);
 }
 
 // S: storage format of fields and memory variables; rv: velocity-over-stress
-// scale ratio (1 for F32), folded into dt/rho.
+// scale ratio (1 for F32), folded into dt/rho.  The cells of block (zc, tile)
+// of slab D.
+//
+// What bounds it: the slab's own bytes (42-48 loads and 12-16 stores per
+// cell), moved at 4.6 TB/s on large grids, the rate of a plain copy; on small
+// ones, how many blocks fit the GPU and their vector instructions.  Hence one
+// scalar base per array and nine 32-bit offsets (the cell, two rows either
+// way, two planes either way) shared by all arrays, the coefficients of an
+// axis as one 16-byte load, and div_u: the stress kernel needs 89 vector
+// registers instead of 102 (5 wavefronts per SIMD, 4 before).  256x256x200,
+// 20 layers (7.0 M cells): velocity 180 -> 177 us, stress 224 -> 214 us; BF16
+// 161x150x131 82.7 -> 70.5 and 101.8 -> 79.4 us.
 template <int CZ, class S>
-__global__ __launch_bounds__(kBlock) DDX_PML_ATTR void k_vel_pml(const SlabDesc *__restrict__ descs,
-                                                    const int *__restrict__ starts, int n, float dx, float dy,
-                                                    float dz, float rv, int grp, PmlOrder ord) {
+__device__ __forceinline__ void vel_pml_body(const SlabDesc &D, int zc, int tile, float dx, float dy, float dz, float rv) {
   typedef typename GPtr<S>::T gT;
-  int di, zc, tile;
-  if (!pml_block(descs, starts, n, grp, ord, CZ, di, zc, tile)) return;
-  const SlabDesc &D = descs[di];
   int ci, ei, ej, kc0, kend;
   if (!slab_column<CZ>(D, zc, tile, ci, ei, ej, kc0, kend)) return;
   const long ncell = (long)D.ni * D.nj * D.nk;
   const int plane = D.ni * D.nj;
-  const long sy = D.sy, sz = D.sz;
-  const long base = (long)ei + sy * ej + sz * (D.k0 + kc0);
+  constexpr unsigned E = sizeof(typename GPtr<S>::raw);
+  const unsigned syb = (unsigned)D.sy * E, szb = (unsigned)D.sz * E;
+  const long pb = D.sz * (D.k0 + kc0 - 2);  // two planes below the block's first
   const float c0 = c_fd[2][0], c1 = c_fd[2][1];
-  const gT *sxx = (const gT *)D.f[SXX], *syy = (const gT *)D.f[SYY], *szz = (const gT *)D.f[SZZ];
-  const gT *sxy = (const gT *)D.f[SXY], *sxz = (const gT *)D.f[SXZ], *syz = (const gT *)D.f[SYZ];
-  gT *fvx = (gT *)D.f[VX], *fvy = (gT *)D.f[VY], *fvz = (gT *)D.f[VZ];
-  gT *psi = (gT *)D.psi;
-  const gfloat *fdtr = G(D.dtr);
-  float qzz[CZ + 3], qxz[CZ + 3], qyz[CZ + 3];
-  load_pml_zq<CZ>(qzz, szz, base, sz, kc0, -1, kend);  // szz: forward-staggered, planes k-1 .. k+2
-  load_pml_zq<CZ>(qxz, sxz, base, sz, kc0, -2, kend);  // sxz, syz: backward-staggered, planes k-2 .. k+1
-  load_pml_zq<CZ>(qyz, syz, base, sz, kc0, -2, kend);
+  const float rdx = D.rdx, rdy = D.rdy, rdz = D.rdz;
+  const gT *sxx = (const gT *)D.f[SXX] + pb, *syy = (const gT *)D.f[SYY] + pb, *szz = (const gT *)D.f[SZZ] + pb;
+  const gT *sxy = (const gT *)D.f[SXY] + pb, *sxz = (const gT *)D.f[SXZ] + pb, *syz = (const gT *)D.f[SYZ] + pb;
+  gT *fvx = (gT *)D.f[VX] + pb, *fvy = (gT *)D.f[VY] + pb, *fvz = (gT *)D.f[VZ] + pb;
+  const gfloat *fdtr = G(D.dtr) + pb;
   const bool inx = (D.axes & 1) && (ei < D.xlo || ei >= D.xhi);
   const bool iny = (D.axes & 2) && (ej < D.ylo || ej >= D.yhi);
   const int sx_slot = 0, sy_slot = (D.axes & 1) ? 1 : 0, sz_slot = sy_slot + ((D.axes & 2) ? 1 : 0);
+  const long cb = (long)plane * kc0;
+  gT *px = (gT *)D.psi + (long)(sx_slot * 6) * ncell + cb;
+  gT *py = (gT *)D.psi + (long)(sy_slot * 6) * ncell + cb;
+  gT *pz = (gT *)D.psi + (long)(sz_slot * 6) * ncell + cb;
+  const gfloat *qx = G(D.coef) + 4 * ((long)sx_slot * ncell + cb);
+  const gfloat *qy = G(D.coef) + 4 * ((long)sy_slot * ncell + cb);
+  const gfloat *qz = G(D.coef) + 4 * ((long)sz_slot * ncell + cb);
+  const unsigned o0 = (unsigned)ei * E + syb * (unsigned)ej;  // the cell in plane pb
+  // z arms: szz forward-staggered, planes k-1 .. k+2; sxz, syz backward-staggered, planes k-2 .. k+1
+  float qzz[CZ + 3], qxz[CZ + 3], qyz[CZ + 3];
+#pragma unroll
+  for (int r = 0; r < CZ + 3; r++) {
+    const bool in = kc0 + r - 2 <= kend;
+    qzz[r] = in ? ldo(szz, o0 + (unsigned)(r + 1) * szb) : 0.f;
+    qxz[r] = in ? ldo(sxz, o0 + (unsigned)r * szb) : 0.f;
+    qyz[r] = in ? ldo(syz, o0 + (unsigned)r * szb) : 0.f;
+  }
   // Two phases: every plane's loads and results first, then every store,
   // so that no load of a later plane waits behind an earlier plane's
   // stores (the memory counter tracks both).  A memory variable's new value
@@ -1980,28 +2115,31 @@ __global__ __launch_bounds__(kBlock) DDX_PML_ATTR void k_vel_pml(const SlabDesc 
     inz[kk] = false;
     if (kc0 + kk >= kend) break;
     const int ek = D.k0 + kc0 + kk;
-    const long id = base + (long)kk * sz;
-    const long c = (long)ci + (long)plane * (kc0 + kk);
-    const float ovx = ld(fvx, id), ovy = ld(fvy, id), ovz = ld(fvz, id);
-    const float dtr = std::is_same<S, F32>::value ? fdtr[id] : rv * fdtr[id];
-    float sxx_x = dp2(sxx, id, 1, c0, c1), syx_x = dm2(sxy, id, 1, c0, c1), szx_x = dm2(sxz, id, 1, c0, c1);
-    float syy_y = dp2(syy, id, sy, c0, c1), sxy_y = dm2(sxy, id, sy, c0, c1), szy_y = dm2(syz, id, sy, c0, c1);
-    float szz_z = 0.f, sxz_z = 0.f, syz_z = 0.f;
-    szz_z += c0 * (qzz[kk + 2] - qzz[kk + 1]);
-    szz_z += c1 * (qzz[kk + 3] - qzz[kk]);
-    sxz_z += c0 * (qxz[kk + 2] - qxz[kk + 1]);
-    sxz_z += c1 * (qxz[kk + 3] - qxz[kk]);
-    syz_z += c0 * (qyz[kk + 2] - qyz[kk + 1]);
-    syz_z += c1 * (qyz[kk + 3] - qyz[kk]);
+    const unsigned o = o0 + (unsigned)(kk + 2) * szb, c = (unsigned)ci + (unsigned)(plane * kk);
+    const unsigned ym2 = o - 2 * syb, ym1 = o - syb, yp1 = o + syb, yp2 = o + 2 * syb;
+    const unsigned of = E == 4 ? o : (o / E) * 4u;  // dt/rho is FP32
+    const float ovx = ldo(fvx, o), ovy = ldo(fvy, o), ovz = ldo(fvz, o);
+    const float dtr = std::is_same<S, F32>::value ? ldo(fdtr, of) : rv * ldo(fdtr, of);
+    const float xx0 = ldo(sxx, o), xxm = ldo(sxx, o, -1), xx1 = ldo(sxx, o, 1), xx2 = ldo(sxx, o, 2);
+    const float xy0 = ldo(sxy, o), xym1 = ldo(sxy, o, -1), xym2 = ldo(sxy, o, -2), xy1 = ldo(sxy, o, 1);
+    const float xzm1 = ldo(sxz, o, -1), xzm2 = ldo(sxz, o, -2), xz1 = ldo(sxz, o, 1);
+    const float yy0 = ldo(syy, o), yym = ldo(syy, ym1), yy1 = ldo(syy, yp1), yy2 = ldo(syy, yp2);
+    const float xyYm1 = ldo(sxy, ym1), xyYm2 = ldo(sxy, ym2), xyY1 = ldo(sxy, yp1);
+    const float yzm1 = ldo(syz, ym1), yzm2 = ldo(syz, ym2), yz1 = ldo(syz, yp1);
+    const float xz0 = qxz[kk + 2], yz0 = qyz[kk + 2];
     inz[kk] = (D.axes & 4) && (ek < D.zlo || ek >= D.zhi);
-    PsiCell<gT> mx{}, my{}, mz{};
-    if (inx) mx = psi_cell(psi + (long)(sx_slot * 6) * ncell + c, G(D.coef) + (long)(sx_slot * 4) * ncell + c, ncell);
-    if (iny) my = psi_cell(psi + (long)(sy_slot * 6) * ncell + c, G(D.coef) + (long)(sy_slot * 4) * ncell + c, ncell);
-    if (inz[kk])
-      mz = psi_cell(psi + (long)(sz_slot * 6) * ncell + c, G(D.coef) + (long)(sz_slot * 4) * ncell + c, ncell);
-    sxx_x = sxx_x / dx; syy_y = syy_y / dy; szz_z = szz_z / dz;
-    sxy_y = sxy_y / dy; sxz_z = sxz_z / dz; syx_x = syx_x / dx;
-    syz_z = syz_z / dz; szx_x = szx_x / dx; szy_y = szy_y / dy;
+    PsiCell<gT> mx, my, mz;
+    if (inx) mx = psi_cell(px, qx, ncell, c);
+    if (iny) my = psi_cell(py, qy, ncell, c);
+    if (inz[kk]) mz = psi_cell(pz, qz, ncell, c);
+    float sxx_x = d2(xx1, xx0, xx2, xxm, c0, c1), syx_x = d2(xy0, xym1, xy1, xym2, c0, c1);
+    float szx_x = d2(xz0, xzm1, xz1, xzm2, c0, c1);
+    float syy_y = d2(yy1, yy0, yy2, yym, c0, c1), sxy_y = d2(xy0, xyYm1, xyY1, xyYm2, c0, c1);
+    float szy_y = d2(yz0, yzm1, yz1, yzm2, c0, c1);
+    float szz_z = d2(qzz[kk + 2], qzz[kk + 1], qzz[kk + 3], qzz[kk], c0, c1);
+    float sxz_z = d2(qxz[kk + 2], qxz[kk + 1], qxz[kk + 3], qxz[kk], c0, c1);
+    float syz_z = d2(qyz[kk + 2], qyz[kk + 1], qyz[kk + 3], qyz[kk], c0, c1);
+    div9(sxx_x, syx_x, szx_x, sxy_y, syy_y, szy_y, sxz_z, syz_z, szz_z, dx, dy, dz, rdx, rdy, rdz);
     if (inx) {
       const float p0 = quant(fvx, mx.bh * mx.m0 + mx.ah * sxx_x);
       const float p1 = quant(fvx, mx.b * mx.m1 + mx.a * syx_x);
@@ -2030,56 +2168,67 @@ __global__ __launch_bounds__(kBlock) DDX_PML_ATTR void k_vel_pml(const SlabDesc 
 #pragma unroll
   for (int kk = 0; kk < CZ; kk++) {
     if (kc0 + kk >= kend) break;
-    const int ek = D.k0 + kc0 + kk;
-    const long id = base + (long)kk * sz;
-    const long c = (long)ci + (long)plane * (kc0 + kk);
-    if (inx) {
-      gT *q = psi + (long)(sx_slot * 6) * ncell + c;
-      stq(q, 0, np[kk][0]); stq(q, ncell, np[kk][1]); stq(q, 2 * ncell, np[kk][2]);
-    }
-    if (iny) {
-      gT *q = psi + (long)(sy_slot * 6) * ncell + c;
-      stq(q, 0, np[kk][3]); stq(q, ncell, np[kk][4]); stq(q, 2 * ncell, np[kk][5]);
-    }
-    if (inz[kk]) {
-      gT *q = psi + (long)(sz_slot * 6) * ncell + c;
-      stq(q, 0, np[kk][6]); stq(q, ncell, np[kk][7]); stq(q, 2 * ncell, np[kk][8]);
-    }
-    stq(fvx, id, nv[kk][0]);
-    stq(fvy, id, nv[kk][1]);
-    stq(fvz, id, nv[kk][2]);
+    const unsigned o = o0 + (unsigned)(kk + 2) * szb, c = (unsigned)ci + (unsigned)(plane * kk);
+    if (inx) psi_store(px, ncell, c, np[kk][0], np[kk][1], np[kk][2]);
+    if (iny) psi_store(py, ncell, c, np[kk][3], np[kk][4], np[kk][5]);
+    if (inz[kk]) psi_store(pz, ncell, c, np[kk][6], np[kk][7], np[kk][8]);
+    sto(fvx, o, nv[kk][0]);
+    sto(fvy, o, nv[kk][1]);
+    sto(fvz, o, nv[kk][2]);
   }
 }
 
-// `dt` carries the stress-over-velocity scale ratio of the 16-bit formats.
-template <int WITH_SAU, int CZ, class S>
-__global__ __launch_bounds__(kBlock) DDX_PML_ATTR void k_stress_pml(const SlabDesc *__restrict__ descs,
-                                                       const int *__restrict__ starts, int n, float dx,
-                                                       float dy, float dz, float dt, int grp, PmlOrder ord) {
-  typedef typename GPtr<S>::T gT;
+template <int CZ, class S>
+__global__ __launch_bounds__(kBlock) DDX_PML_ATTR void k_vel_pml(const SlabDesc *__restrict__ descs,
+                                                    const int *__restrict__ starts, int n, float dx, float dy,
+                                                    float dz, float rv, int grp, PmlOrder ord) {
   int di, zc, tile;
-  if (!pml_block(descs, starts, n, grp, ord, CZ, di, zc, tile)) return;
-  const SlabDesc &D = descs[di];
+  if (!pml_block(descs, starts, n, blockIdx.x, gridDim.x, grp, ord, CZ, di, zc, tile)) return;
+  vel_pml_body<CZ, S>(descs[di], zc, tile, dx, dy, dz, rv);
+}
+
+
+// `dt` carries the stress-over-velocity scale ratio of the 16-bit formats.
+// (Bounds and layout as vel_pml_body.)
+template <int WITH_SAU, int CZ, class S, bool SRC = false>
+__device__ __forceinline__ void stress_pml_body(const SlabDesc &D, int zc, int tile, float dx, float dy, float dz,
+                                                float dt, const SrcCell &src = SrcCell{}) {
+  typedef typename GPtr<S>::T gT;
   int ci, ei, ej, kc0, kend;
   if (!slab_column<CZ>(D, zc, tile, ci, ei, ej, kc0, kend)) return;
   const long ncell = (long)D.ni * D.nj * D.nk;
   const int plane = D.ni * D.nj;
-  const long sy = D.sy, sz = D.sz;
-  const long base = (long)ei + sy * ej + sz * (D.k0 + kc0);
+  constexpr unsigned E = sizeof(typename GPtr<S>::raw);
+  const unsigned syb = (unsigned)D.sy * E, szb = (unsigned)D.sz * E;
+  const long pb = D.sz * (D.k0 + kc0 - 2);  // two planes below the block's first
   const float c0 = c_fd[2][0], c1 = c_fd[2][1];
-  const gT *vx = (const gT *)D.f[VX], *vy = (const gT *)D.f[VY], *vz = (const gT *)D.f[VZ];
-  gT *fsxx = (gT *)D.f[SXX], *fsyy = (gT *)D.f[SYY], *fszz = (gT *)D.f[SZZ];
-  gT *fsxy = (gT *)D.f[SXY], *fsxz = (gT *)D.f[SXZ], *fsyz = (gT *)D.f[SYZ], *fsau = (gT *)D.f[SAU];
-  gT *psi = (gT *)D.psi;
-  const gfloat *flam = G(D.lam), *fmu = G(D.mu);
-  float qx[CZ + 3], qy[CZ + 3], qz[CZ + 3];
-  load_pml_zq<CZ>(qx, vx, base, sz, kc0, -1, kend);  // vx, vy: forward-staggered in z
-  load_pml_zq<CZ>(qy, vy, base, sz, kc0, -1, kend);
-  load_pml_zq<CZ>(qz, vz, base, sz, kc0, -2, kend);  // vz: backward-staggered in z
+  const float rdx = D.rdx, rdy = D.rdy, rdz = D.rdz;
+  const gT *vx = (const gT *)D.f[VX] + pb, *vy = (const gT *)D.f[VY] + pb, *vz = (const gT *)D.f[VZ] + pb;
+  gT *fsxx = (gT *)D.f[SXX] + pb, *fsyy = (gT *)D.f[SYY] + pb, *fszz = (gT *)D.f[SZZ] + pb;
+  gT *fsxy = (gT *)D.f[SXY] + pb, *fsxz = (gT *)D.f[SXZ] + pb, *fsyz = (gT *)D.f[SYZ] + pb;
+  gT *fsau = (gT *)D.f[SAU] + pb;
+  const gfloat *flam = G(D.lam) + pb, *fmu = G(D.mu) + pb;
   const bool inx = (D.axes & 1) && (ei < D.xlo || ei >= D.xhi);
   const bool iny = (D.axes & 2) && (ej < D.ylo || ej >= D.yhi);
   const int sx_slot = 0, sy_slot = (D.axes & 1) ? 1 : 0, sz_slot = sy_slot + ((D.axes & 2) ? 1 : 0);
-  // loads and results of every plane first, then the stores (as k_vel_pml)
+  const long cb = (long)plane * kc0;
+  gT *px = (gT *)D.psi + (long)(sx_slot * 6 + 3) * ncell + cb;
+  gT *py = (gT *)D.psi + (long)(sy_slot * 6 + 3) * ncell + cb;
+  gT *pz = (gT *)D.psi + (long)(sz_slot * 6 + 3) * ncell + cb;
+  const gfloat *qx = G(D.coef) + 4 * ((long)sx_slot * ncell + cb);
+  const gfloat *qy = G(D.coef) + 4 * ((long)sy_slot * ncell + cb);
+  const gfloat *qz = G(D.coef) + 4 * ((long)sz_slot * ncell + cb);
+  const unsigned o0 = (unsigned)ei * E + syb * (unsigned)ej;
+  // z arms: vx, vy forward-staggered, planes k-1 .. k+2; vz backward-staggered, planes k-2 .. k+1
+  float zx[CZ + 3], zy[CZ + 3], zz[CZ + 3];
+#pragma unroll
+  for (int r = 0; r < CZ + 3; r++) {
+    const bool in = kc0 + r - 2 <= kend;
+    zx[r] = in ? ldo(vx, o0 + (unsigned)(r + 1) * szb) : 0.f;
+    zy[r] = in ? ldo(vy, o0 + (unsigned)(r + 1) * szb) : 0.f;
+    zz[r] = in ? ldo(vz, o0 + (unsigned)r * szb) : 0.f;
+  }
+  // loads and results of every plane first, then the stores (as vel_pml_body)
   float ns[CZ][7], np[CZ][9];
   bool inz[CZ];
 #pragma unroll
@@ -2087,33 +2236,35 @@ __global__ __launch_bounds__(kBlock) DDX_PML_ATTR void k_stress_pml(const SlabDe
     inz[kk] = false;
     if (kc0 + kk >= kend) break;
     const int ek = D.k0 + kc0 + kk;
-    const long id = base + (long)kk * sz;
-    const long c = (long)ci + (long)plane * (kc0 + kk);
-    float vx_x = dm2(vx, id, 1, c0, c1), vy_x = dp2(vy, id, 1, c0, c1), vz_x = dp2(vz, id, 1, c0, c1);
-    float vy_y = dm2(vy, id, sy, c0, c1), vx_y = dp2(vx, id, sy, c0, c1), vz_y = dp2(vz, id, sy, c0, c1);
-    float vz_z = 0.f, vx_z = 0.f, vy_z = 0.f;
-    vz_z += c0 * (qz[kk + 2] - qz[kk + 1]);
-    vz_z += c1 * (qz[kk + 3] - qz[kk]);
-    vx_z += c0 * (qx[kk + 2] - qx[kk + 1]);
-    vx_z += c1 * (qx[kk + 3] - qx[kk]);
-    vy_z += c0 * (qy[kk + 2] - qy[kk + 1]);
-    vy_z += c1 * (qy[kk + 3] - qy[kk]);
-    const float lm = flam[id], mu = fmu[id];
+    const unsigned o = o0 + (unsigned)(kk + 2) * szb, c = (unsigned)ci + (unsigned)(plane * kk);
+    const unsigned ym2 = o - 2 * syb, ym1 = o - syb, yp1 = o + syb, yp2 = o + 2 * syb;
+    const unsigned of = E == 4 ? o : (o / E) * 4u;  // the model is FP32
+    const float x0 = zx[kk + 1], y0 = zy[kk + 1], z0 = zz[kk + 2];
+    const float xm1 = ldo(vx, o, -1), xm2 = ldo(vx, o, -2), x1 = ldo(vx, o, 1);
+    const float yxm = ldo(vy, o, -1), yx1 = ldo(vy, o, 1), yx2 = ldo(vy, o, 2);
+    const float zxm = ldo(vz, o, -1), zx1 = ldo(vz, o, 1), zx2 = ldo(vz, o, 2);
+    const float xym = ldo(vx, ym1), xy1 = ldo(vx, yp1), xy2 = ldo(vx, yp2);
+    const float yym1 = ldo(vy, ym1), yym2 = ldo(vy, ym2), yy1 = ldo(vy, yp1);
+    const float zym = ldo(vz, ym1), zy1 = ldo(vz, yp1), zy2 = ldo(vz, yp2);
+    const float lm = ldo(flam, of), mu = ldo(fmu, of);
     const float l2m = lm + 2.0f * mu;
-    const float oxx = ld(fsxx, id), oyy = ld(fsyy, id), ozz = ld(fszz, id);
-    const float oxy = ld(fsxy, id), oxz = ld(fsxz, id), oyz = ld(fsyz, id);
-    const float oau = WITH_SAU ? ld(fsau, id) : 0.f;
+    float oxx = ldo(fsxx, o), oyy = ldo(fsyy, o), ozz = ldo(fszz, o);
+    if constexpr (SRC) add_source<gT>(src, ei, ej, ek, oxx, oyy, ozz);
+    const float oxy = ldo(fsxy, o), oxz = ldo(fsxz, o), oyz = ldo(fsyz, o);
+    const float oau = WITH_SAU ? ldo(fsau, o) : 0.f;
     inz[kk] = (D.axes & 4) && (ek < D.zlo || ek >= D.zhi);
-    PsiCell<gT> mx{}, my{}, mz{};
-    if (inx)
-      mx = psi_cell(psi + (long)(sx_slot * 6 + 3) * ncell + c, G(D.coef) + (long)(sx_slot * 4) * ncell + c, ncell);
-    if (iny)
-      my = psi_cell(psi + (long)(sy_slot * 6 + 3) * ncell + c, G(D.coef) + (long)(sy_slot * 4) * ncell + c, ncell);
-    if (inz[kk])
-      mz = psi_cell(psi + (long)(sz_slot * 6 + 3) * ncell + c, G(D.coef) + (long)(sz_slot * 4) * ncell + c, ncell);
-    vx_x = vx_x / dx; vy_y = vy_y / dy; vz_z = vz_z / dz;
-    vy_x = vy_x / dx; vz_x = vz_x / dx; vx_y = vx_y / dy;
-    vz_y = vz_y / dy; vx_z = vx_z / dz; vy_z = vy_z / dz;
+    PsiCell<gT> mx, my, mz;
+    if (inx) mx = psi_cell(px, qx, ncell, c);
+    if (iny) my = psi_cell(py, qy, ncell, c);
+    if (inz[kk]) mz = psi_cell(pz, qz, ncell, c);
+    float vx_x = d2(x0, xm1, x1, xm2, c0, c1), vy_x = d2(yx1, y0, yx2, yxm, c0, c1);
+    float vz_x = d2(zx1, z0, zx2, zxm, c0, c1);
+    float vy_y = d2(y0, yym1, yy1, yym2, c0, c1), vx_y = d2(xy1, x0, xy2, xym, c0, c1);
+    float vz_y = d2(zy1, z0, zy2, zym, c0, c1);
+    float vz_z = d2(zz[kk + 2], zz[kk + 1], zz[kk + 3], zz[kk], c0, c1);
+    float vx_z = d2(zx[kk + 2], zx[kk + 1], zx[kk + 3], zx[kk], c0, c1);
+    float vy_z = d2(zy[kk + 2], zy[kk + 1], zy[kk + 3], zy[kk], c0, c1);
+    div9(vx_x, vy_x, vz_x, vy_y, vx_y, vz_y, vz_z, vx_z, vy_z, dx, dy, dz, rdx, rdy, rdz);
     if (inx) {
       const float p0 = quant(fsxx, mx.b * mx.m0 + mx.a * vx_x);
       const float p1 = quant(fsxx, mx.bh * mx.m1 + mx.ah * vy_x);
@@ -2146,30 +2297,29 @@ __global__ __launch_bounds__(kBlock) DDX_PML_ATTR void k_stress_pml(const SlabDe
 #pragma unroll
   for (int kk = 0; kk < CZ; kk++) {
     if (kc0 + kk >= kend) break;
-    const int ek = D.k0 + kc0 + kk;
-    const long id = base + (long)kk * sz;
-    const long c = (long)ci + (long)plane * (kc0 + kk);
-    if (inx) {
-      gT *q = psi + (long)(sx_slot * 6 + 3) * ncell + c;
-      stq(q, 0, np[kk][0]); stq(q, ncell, np[kk][1]); stq(q, 2 * ncell, np[kk][2]);
-    }
-    if (iny) {
-      gT *q = psi + (long)(sy_slot * 6 + 3) * ncell + c;
-      stq(q, 0, np[kk][3]); stq(q, ncell, np[kk][4]); stq(q, 2 * ncell, np[kk][5]);
-    }
-    if (inz[kk]) {
-      gT *q = psi + (long)(sz_slot * 6 + 3) * ncell + c;
-      stq(q, 0, np[kk][6]); stq(q, ncell, np[kk][7]); stq(q, 2 * ncell, np[kk][8]);
-    }
-    stq(fsxx, id, ns[kk][0]);
-    stq(fsyy, id, ns[kk][1]);
-    stq(fszz, id, ns[kk][2]);
-    if (WITH_SAU) stq(fsau, id, ns[kk][3]);
-    stq(fsxy, id, ns[kk][4]);
-    stq(fsxz, id, ns[kk][5]);
-    stq(fsyz, id, ns[kk][6]);
+    const unsigned o = o0 + (unsigned)(kk + 2) * szb, c = (unsigned)ci + (unsigned)(plane * kk);
+    if (inx) psi_store(px, ncell, c, np[kk][0], np[kk][1], np[kk][2]);
+    if (iny) psi_store(py, ncell, c, np[kk][3], np[kk][4], np[kk][5]);
+    if (inz[kk]) psi_store(pz, ncell, c, np[kk][6], np[kk][7], np[kk][8]);
+    sto(fsxx, o, ns[kk][0]);
+    sto(fsyy, o, ns[kk][1]);
+    sto(fszz, o, ns[kk][2]);
+    if (WITH_SAU) sto(fsau, o, ns[kk][3]);
+    sto(fsxy, o, ns[kk][4]);
+    sto(fsxz, o, ns[kk][5]);
+    sto(fsyz, o, ns[kk][6]);
   }
 }
+
+template <int WITH_SAU, int CZ, class S>
+__global__ __launch_bounds__(kBlock) DDX_PML_ATTR void k_stress_pml(const SlabDesc *__restrict__ descs,
+                                                       const int *__restrict__ starts, int n, float dx,
+                                                       float dy, float dz, float dt, int grp, PmlOrder ord) {
+  int di, zc, tile;
+  if (!pml_block(descs, starts, n, blockIdx.x, gridDim.x, grp, ord, CZ, di, zc, tile)) return;
+  stress_pml_body<WITH_SAU, CZ, S>(descs[di], zc, tile, dx, dy, dz, dt);
+}
+
 
 // ---------------------------------------------------------------------------
 // CPML halves on LDS-staged plane tiles (FP32 storage; work split
@@ -2271,7 +2421,7 @@ __global__ __launch_bounds__(kBlock) DDX_PML_ATTR void k_vel_pml_t(const SlabDes
                                                       float dz, int grp, PmlOrder ord) {
   __shared__ float lt[2][5][kPmlLds];  // sxx, sxy, sxz, syy, syz
   int di, zc, tile;
-  if (!pml_block(descs, starts, n, grp, ord, kPmlTiled + P, di, zc, tile)) return;
+  if (!pml_block(descs, starts, n, blockIdx.x, gridDim.x, grp, ord, kPmlTiled + P, di, zc, tile)) return;
   const SlabDesc &D = descs[di];
   const PmlTile T = pml_tile(D, zc, tile, P);
   const long ncell = (long)D.ni * D.nj * D.nk;
@@ -2312,10 +2462,10 @@ __global__ __launch_bounds__(kBlock) DDX_PML_ATTR void k_vel_pml_t(const SlabDes
       const long c = c00 + (long)plane * kk;
       const int ek = D.k0 + T.kc0 + kk;
       L.inz = (D.axes & 4) && (ek < D.zlo || ek >= D.zhi);
-      if (inx) L.mx = psi_cell(psi + (long)(sx_slot * 6) * ncell + c, coef + (long)(sx_slot * 4) * ncell + c, ncell);
-      if (iny) L.my = psi_cell(psi + (long)(sy_slot * 6) * ncell + c, coef + (long)(sy_slot * 4) * ncell + c, ncell);
+      if (inx) L.mx = psi_cell(psi + (long)(sx_slot * 6) * ncell + c, coef + 4 * ((long)sx_slot * ncell + c), ncell);
+      if (iny) L.my = psi_cell(psi + (long)(sy_slot * 6) * ncell + c, coef + 4 * ((long)sy_slot * ncell + c), ncell);
       if (L.inz)
-        L.mz = psi_cell(psi + (long)(sz_slot * 6) * ncell + c, coef + (long)(sz_slot * 4) * ncell + c, ncell);
+        L.mz = psi_cell(psi + (long)(sz_slot * 6) * ncell + c, coef + 4 * ((long)sz_slot * ncell + c), ncell);
     }
     return L;
   };
@@ -2436,7 +2586,7 @@ __global__ __launch_bounds__(kBlock) DDX_PML_ATTR void k_stress_pml_t(const Slab
                                                          float dy, float dz, float dt, int grp, PmlOrder ord) {
   __shared__ float lt[2][3][kPmlLds];  // vx, vy, vz
   int di, zc, tile;
-  if (!pml_block(descs, starts, n, grp, ord, kPmlTiled + P, di, zc, tile)) return;
+  if (!pml_block(descs, starts, n, blockIdx.x, gridDim.x, grp, ord, kPmlTiled + P, di, zc, tile)) return;
   const SlabDesc &D = descs[di];
   const PmlTile T = pml_tile(D, zc, tile, P);
   const long ncell = (long)D.ni * D.nj * D.nk;
@@ -2479,11 +2629,11 @@ __global__ __launch_bounds__(kBlock) DDX_PML_ATTR void k_stress_pml_t(const Slab
       const int ek = D.k0 + T.kc0 + kk;
       L.inz = (D.axes & 4) && (ek < D.zlo || ek >= D.zhi);
       if (inx)
-        L.mx = psi_cell(psi + (long)(sx_slot * 6 + 3) * ncell + c, coef + (long)(sx_slot * 4) * ncell + c, ncell);
+        L.mx = psi_cell(psi + (long)(sx_slot * 6 + 3) * ncell + c, coef + 4 * ((long)sx_slot * ncell + c), ncell);
       if (iny)
-        L.my = psi_cell(psi + (long)(sy_slot * 6 + 3) * ncell + c, coef + (long)(sy_slot * 4) * ncell + c, ncell);
+        L.my = psi_cell(psi + (long)(sy_slot * 6 + 3) * ncell + c, coef + 4 * ((long)sy_slot * ncell + c), ncell);
       if (L.inz)
-        L.mz = psi_cell(psi + (long)(sz_slot * 6 + 3) * ncell + c, coef + (long)(sz_slot * 4) * ncell + c, ncell);
+        L.mz = psi_cell(psi + (long)(sz_slot * 6 + 3) * ncell + c, coef + 4 * ((long)sz_slot * ncell + c), ncell);
     }
     return L;
   };
@@ -2593,6 +2743,99 @@ __global__ __launch_bounds__(kBlock) DDX_PML_ATTR void k_stress_pml_t(const Slab
       __syncthreads();
       C = N;
     }
+  }
+}
+
+// Receiver samples of the members of a batch (or of one shot): blocks of
+// kBlock receivers, each block within one member; the same operations as
+// k_recv_sample.
+template <class S>
+__device__ __forceinline__ void recv_block(const StepIO &io, int b) {
+  typedef typename GPtr<S>::T gT;
+  const MemberIO &m = io.io[find_desc(io.starts, io.n, b)];
+  const int r = (b - m.blk0) * kBlock + (int)threadIdx.x;
+  const int it = (io.gsp ? *io.gsp : io.gs) - m.join;
+  if (r >= m.nrec || it < 0 || it >= m.ntime) return;
+  const int s = m.rsub[r];
+  const long o = m.roff[r];
+#pragma unroll
+  for (int q = 0; q < 3; q++) {
+    const float v = ld((const gT *)m.vptr[s * 3 + q], o);
+    m.seis[((long)q * m.nrec + r) * m.ntime + it] = std::is_same<S, F32>::value ? v : v * m.inv_sv;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Whole half steps in one launch: blocks [0, nphy) are the physical region's
+// bricks, the next npml the CPML cells, and after them (stress only) the
+// receivers of the step; the thread that owns the source cell adds the
+// sample.  The parts of a half step are independent of each other: the
+// bricks and the CPML cells update different cells from fields that the half
+// step does not write, and the receivers read velocities.  One launch fills
+// the GPU's last wave of bricks with CPML blocks and drops the launches'
+// gaps; what each block does is what the separate kernels do.  Where it pays
+// and where not: kWholeCells in engine.cpp.  A modelling step is two launches
+// instead of six: 32x28x24 cells 31.8 -> 15.2 us per step, 64^3 with 20
+// layers 66 -> 52 us, 100^3 with 10 layers 96 -> 76 us.
+// ---------------------------------------------------------------------------
+enum { FORM_ONE = 0, FORM_PAIR = 2, FORM_YL = 4 };
+template <int FORM, int MODE, int TX, int TY, int CZ, class S>
+__global__ __launch_bounds__(kBlock) void k_vel_all(HalfStep a) {
+  static_assert(TX * TY == kBlock, "the bricks and the CPML cells share a block size");
+  if ((int)blockIdx.x >= a.nphy) {
+    int di, zc, tile;
+    const PmlOrder ord{};
+    if (pml_block(a.slabs, a.sstarts, a.ns, blockIdx.x - a.nphy, a.npml, a.pgrp, ord, 1, di, zc, tile))
+      vel_pml_body<1, S>(a.slabs[di], zc, tile, a.dx, a.dy, a.dz, a.sc);
+    return;
+  }
+  const int grp = a.grp, b = brick_block(blockIdx.x, a.nphy, grp);
+  const PhyDesc &D = a.phy[find_desc(a.pstarts, a.np, b)];
+  int i, j0, k0;
+  if constexpr (FORM == FORM_YL) {
+    __shared__ YlTile<(MODE == RTM_BACKWARD || MODE == RTM_REVERSE) ? 4 : 3, TY, CZ> ly;
+    const TileAt at = tile_at<64, TY * 1>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp);
+  const bool live = zbrick<64, TY, 1, CZ>(D, at, i, j0, k0);
+    vel_yl_body<MODE, TY, CZ, S>(ly, D, i, j0, k0, a.dx, a.dy, a.dz, a.sc, live);
+  } else if constexpr (FORM == FORM_PAIR) {
+    if (zbrick2<TX, TY, 1, CZ>(D, tile_at<2 * TX, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp), i, j0, k0))
+      vel_zb2_body<MODE, TX, TY, 1, CZ, S>(D, i, j0, k0, a.dx, a.dy, a.dz, a.sc);
+  } else {
+    if (zbrick<TX, TY, 1, CZ>(D, tile_at<TX, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp), i, j0, k0))
+      vel_zb_body<MODE, TX, TY, 1, CZ, S>(D, i, j0, k0, a.dx, a.dy, a.dz, a.sc);
+  }
+}
+
+template <int FORM, int MODE, int TX, int TY, int CZ, class S>
+__global__ __launch_bounds__(kBlock) void k_stress_all(HalfStep a, StepIO io) {
+  static_assert(TX * TY == kBlock, "the bricks and the CPML cells share a block size");
+  if ((int)blockIdx.x >= a.nphy) {
+    if ((int)blockIdx.x >= a.nphy + a.npml) {
+      recv_block<S>(io, blockIdx.x - a.nphy - a.npml);
+      return;
+    }
+    int di, zc, tile;
+    const PmlOrder ord{};
+    if (pml_block(a.slabs, a.sstarts, a.ns, blockIdx.x - a.nphy, a.npml, a.pgrp, ord, 1, di, zc, tile))
+      stress_pml_body<rtm_mode(MODE), 1, S, true>(a.slabs[di], zc, tile, a.dx, a.dy, a.dz, a.sc,
+                                                  src_cell<S>(io, a.slabs[di].io));
+    return;
+  }
+  const int grp = a.grp, b = brick_block(blockIdx.x, a.nphy, grp);
+  const PhyDesc &D = a.phy[find_desc(a.pstarts, a.np, b)];
+  const SrcCell src = src_cell<S>(io, D.io);
+  int i, j0, k0;
+  if constexpr (FORM == FORM_YL) {
+    __shared__ YlTile<3, TY, CZ> ly;
+    const TileAt at = tile_at<64, TY * 1>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp);
+  const bool live = zbrick<64, TY, 1, CZ>(D, at, i, j0, k0);
+    stress_yl_body<MODE, TY, CZ, S, true>(ly, D, i, j0, k0, a.sx, a.sy, a.sz, live, src);
+  } else if constexpr (FORM == FORM_PAIR) {
+    if (zbrick2<TX, TY, 1, CZ>(D, tile_at<2 * TX, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp), i, j0, k0))
+      stress_zb2_body<MODE, TX, TY, 1, CZ, S, true>(D, i, j0, k0, a.sx, a.sy, a.sz, src);
+  } else {
+    if (zbrick<TX, TY, 1, CZ>(D, tile_at<TX, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp), i, j0, k0))
+      stress_zb_body<MODE, TX, TY, 1, CZ, S, false, true>(D, i, j0, k0, a.sx, a.sy, a.sz, true, src);
   }
 }
 
@@ -2847,25 +3090,9 @@ __global__ void k_source_batch(const MemberIO *__restrict__ io, int n, int gs, c
   add_to((gT *)M.szz, M.src_off, v);
 }
 
-// Receiver samples of every member of a fused batch: blocks of kBlock
-// receivers, each block within one member; the same operations as
-// k_recv_sample.
 template <class S>
-__global__ __launch_bounds__(kBlock) void k_recv_batch(const MemberIO *__restrict__ io, const int *__restrict__ starts,
-                                                       int n, int gs, const int *__restrict__ gsp) {
-  typedef typename GPtr<S>::T gT;
-  const int b = blockIdx.x;
-  const MemberIO &M = io[find_desc(starts, n, b)];
-  const int r = (b - M.blk0) * kBlock + (int)threadIdx.x;
-  const int it = (gsp ? *gsp : gs) - M.join;
-  if (r >= M.nrec || it < 0 || it >= M.ntime) return;
-  const int s = M.rsub[r];
-  const long o = M.roff[r];
-#pragma unroll
-  for (int q = 0; q < 3; q++) {
-    const float v = ld((const gT *)M.vptr[s * 3 + q], o);
-    M.seis[((long)q * M.nrec + r) * M.ntime + it] = std::is_same<S, F32>::value ? v : v * M.inv_sv;
-  }
+__global__ __launch_bounds__(kBlock) void k_recv_batch(StepIO io) {
+  recv_block<S>(io, blockIdx.x);
 }
 
 // Reverse-time receiver injection of every member of a fused RTM batch
@@ -3131,6 +3358,7 @@ int tiling_list(int fmt, Tiling *out, int max) {
 // Launch of one brick shape: the kernel of each mode (K: kernel template, PF:
 // the mode whose kernel the pure-forward and RTM-forward passes share or not).
 #define DDX_ARGS d, starts, n, dx, dy, dz, sc, grp
+#define DDX_ARGS_S d, starts, n, sc / dx, sc / dy, sc / dz, grp
 #define DDX_SIG                                                                                              \
   const Tiling &t, int mode, int fmt, dim3 g, hipStream_t st, const PhyDesc *d, const int *starts, int n,    \
       float dx, float dy, float dz, float sc, int grp
@@ -3163,13 +3391,13 @@ static void stress_zb(DDX_SIG) {
   switch (mode) {
     case PURE_FORWARD:
     case FWI:
-      hipLaunchKernelGGL((k_stress_phy_zb<PURE_FORWARD, TX, TY, CY, CZ, S, XL>), g, bl, 0, st, DDX_ARGS);
+      hipLaunchKernelGGL((k_stress_phy_zb<PURE_FORWARD, TX, TY, CY, CZ, S, XL>), g, bl, 0, st, DDX_ARGS_S);
       break;
     case RTM_BACKWARD:
-      hipLaunchKernelGGL((k_stress_phy_zb<RTM_BACKWARD, TX, TY, CY, CZ, S, XL>), g, bl, 0, st, DDX_ARGS);
+      hipLaunchKernelGGL((k_stress_phy_zb<RTM_BACKWARD, TX, TY, CY, CZ, S, XL>), g, bl, 0, st, DDX_ARGS_S);
       break;
     default:
-      hipLaunchKernelGGL((k_stress_phy_zb<RTM_REVERSE, TX, TY, CY, CZ, S, XL>), g, bl, 0, st, DDX_ARGS);
+      hipLaunchKernelGGL((k_stress_phy_zb<RTM_REVERSE, TX, TY, CY, CZ, S, XL>), g, bl, 0, st, DDX_ARGS_S);
   }
 }
 
@@ -3197,14 +3425,14 @@ static void stress_zb2(DDX_SIG) {
   dim3 bl(TX * TY);
   switch (mode) {
     case PURE_FORWARD:
-      hipLaunchKernelGGL((k_stress_phy_zb2<PURE_FORWARD, TX, TY, CY, CZ, S>), g, bl, 0, st, DDX_ARGS);
+      hipLaunchKernelGGL((k_stress_phy_zb2<PURE_FORWARD, TX, TY, CY, CZ, S>), g, bl, 0, st, DDX_ARGS_S);
       break;
     case RTM_BACKWARD:
-      hipLaunchKernelGGL((k_stress_phy_zb2<RTM_BACKWARD, TX, TY, CY, CZ, S>), g, bl, 0, st, DDX_ARGS);
+      hipLaunchKernelGGL((k_stress_phy_zb2<RTM_BACKWARD, TX, TY, CY, CZ, S>), g, bl, 0, st, DDX_ARGS_S);
       break;
     case RTM_FORWARD:
     case RTM_REVERSE:
-      hipLaunchKernelGGL((k_stress_phy_zb2<RTM_REVERSE, TX, TY, CY, CZ, S>), g, bl, 0, st, DDX_ARGS);
+      hipLaunchKernelGGL((k_stress_phy_zb2<RTM_REVERSE, TX, TY, CY, CZ, S>), g, bl, 0, st, DDX_ARGS_S);
       break;
     default:
       break;  // FWI: one-cell bricks only
@@ -3232,13 +3460,13 @@ static void stress_yl(DDX_SIG) {
   const dim3 bl(64 * TY);
   switch (mode) {
     case PURE_FORWARD:
-      hipLaunchKernelGGL((k_stress_phy_yl<PURE_FORWARD, TY, CZ, F32>), g, bl, 0, st, DDX_ARGS);
+      hipLaunchKernelGGL((k_stress_phy_yl<PURE_FORWARD, TY, CZ, F32>), g, bl, 0, st, DDX_ARGS_S);
       break;
     case RTM_BACKWARD:
-      hipLaunchKernelGGL((k_stress_phy_yl<RTM_BACKWARD, TY, CZ, F32>), g, bl, 0, st, DDX_ARGS);
+      hipLaunchKernelGGL((k_stress_phy_yl<RTM_BACKWARD, TY, CZ, F32>), g, bl, 0, st, DDX_ARGS_S);
       break;
     default:
-      hipLaunchKernelGGL((k_stress_phy_yl<RTM_REVERSE, TY, CZ, F32>), g, bl, 0, st, DDX_ARGS);
+      hipLaunchKernelGGL((k_stress_phy_yl<RTM_REVERSE, TY, CZ, F32>), g, bl, 0, st, DDX_ARGS_S);
   }
 }
 
@@ -3260,6 +3488,82 @@ DDX_FAMILY(DDX_T)
                                                                     : DDX_F<TX, TY, CY, CZ, F32>)(DDX_PASS), true;
 #define DDX_TX(TX, TY, CY, CZ) if (DDX_IS(TX, TY, CY, CZ)) return DDX_F<TX, TY, CY, CZ, F32, true>(DDX_PASS), true;
 #define DDX_TY(TY, CZ) if (DDX_IS(64, TY, 1, CZ)) return DDX_F<TY, CZ>(DDX_PASS), true;
+// Fused half steps: the shapes they exist for, (form, tx, ty, kz), FP32 and
+// 16-bit; each part compiles one kind.
+#define DDX_FUSED32(X) X(FORM_ONE, 32, 8, 4) X(FORM_ONE, 64, 4, 2) X(FORM_YL, 64, 4, 2) X(FORM_YL, 64, 4, 4)
+#define DDX_FUSED16(X) X(FORM_PAIR, 64, 4, 2) X(FORM_PAIR, 64, 4, 4)
+bool vel_all_32(const Tiling &t, int form, int mode, const HalfStep &a, hipStream_t st);
+bool vel_all_16(const Tiling &t, int form, int mode, int fmt, const HalfStep &a, hipStream_t st);
+bool stress_all_32(const Tiling &t, int form, int mode, const HalfStep &a, const StepIO &io, int grid, hipStream_t st);
+bool stress_all_16(const Tiling &t, int form, int mode, int fmt, const HalfStep &a, const StepIO &io, int grid,
+                   hipStream_t st);
+#define DDX_V(FORM, MODE, TX, TY, CZ, S) \
+  hipLaunchKernelGGL((k_vel_all<FORM, MODE, TX, TY, CZ, S>), dim3(a.nphy + a.npml), dim3(kBlock), 0, st, a)
+#define DDX_S(FORM, MODE, TX, TY, CZ, S) \
+  hipLaunchKernelGGL((k_stress_all<FORM, MODE, TX, TY, CZ, S>), dim3(grid), dim3(kBlock), 0, st, a, io)
+#if DDX_PART == 9
+bool vel_all_32(const Tiling &t, int form, int mode, const HalfStep &a, hipStream_t st) {
+#define DDX_T(FORM, TX, TY, CZ)                                               \
+  if (form == FORM && DDX_IS(TX, TY, 1, CZ)) {                                \
+    if (mode == RTM_REVERSE) DDX_V(FORM, RTM_REVERSE, TX, TY, CZ, F32);       \
+    else if (mode != FWI) DDX_V(FORM, PURE_FORWARD, TX, TY, CZ, F32);         \
+    else if (FORM != FORM_ONE) return false;                                  \
+    else DDX_V(FORM_ONE, FWI, TX, TY, CZ, F32);                               \
+    return true;                                                              \
+  }
+  DDX_FUSED32(DDX_T)
+#undef DDX_T
+  return false;
+}
+#elif DDX_PART == 10
+bool stress_all_32(const Tiling &t, int form, int mode, const HalfStep &a, const StepIO &io, int grid,
+                   hipStream_t st) {
+#define DDX_T(FORM, TX, TY, CZ)                                               \
+  if (form == FORM && DDX_IS(TX, TY, 1, CZ)) {                                \
+    if (rtm_mode(mode)) DDX_S(FORM, RTM_REVERSE, TX, TY, CZ, F32);            \
+    else DDX_S(FORM, PURE_FORWARD, TX, TY, CZ, F32);                          \
+    return true;                                                              \
+  }
+  DDX_FUSED32(DDX_T)
+#undef DDX_T
+  return false;
+}
+#elif DDX_PART == 11
+bool vel_all_16(const Tiling &t, int form, int mode, int fmt, const HalfStep &a, hipStream_t st) {
+#define DDX_T(FORM, TX, TY, CZ)                                               \
+  if (form == FORM && DDX_IS(TX, TY, 1, CZ)) {                                \
+    if (fmt == STORE_F16) {                                                   \
+      if (mode == RTM_REVERSE) DDX_V(FORM, RTM_REVERSE, TX, TY, CZ, F16);     \
+      else DDX_V(FORM, PURE_FORWARD, TX, TY, CZ, F16);                        \
+    } else {                                                                  \
+      if (mode == RTM_REVERSE) DDX_V(FORM, RTM_REVERSE, TX, TY, CZ, BF16);    \
+      else DDX_V(FORM, PURE_FORWARD, TX, TY, CZ, BF16);                       \
+    }                                                                         \
+    return true;                                                              \
+  }
+  DDX_FUSED16(DDX_T)
+#undef DDX_T
+  return false;
+}
+bool stress_all_16(const Tiling &t, int form, int mode, int fmt, const HalfStep &a, const StepIO &io, int grid,
+                   hipStream_t st) {
+#define DDX_T(FORM, TX, TY, CZ)                                               \
+  if (form == FORM && DDX_IS(TX, TY, 1, CZ)) {                                \
+    if (fmt == STORE_F16) {                                                   \
+      if (rtm_mode(mode)) DDX_S(FORM, RTM_REVERSE, TX, TY, CZ, F16);          \
+      else DDX_S(FORM, PURE_FORWARD, TX, TY, CZ, F16);                        \
+    } else {                                                                  \
+      if (rtm_mode(mode)) DDX_S(FORM, RTM_REVERSE, TX, TY, CZ, BF16);         \
+      else DDX_S(FORM, PURE_FORWARD, TX, TY, CZ, BF16);                       \
+    }                                                                         \
+    return true;                                                              \
+  }
+  DDX_FUSED16(DDX_T)
+#undef DDX_T
+  return false;
+}
+#endif
+
 #if DDX_PART == 1
 #define DDX_F vel_zb
 bool vel_one(DDX_SIG) { DDX_TILINGS(DDX_T1) return false; }
@@ -3290,7 +3594,31 @@ bool stress_lane(DDX_SIG) { DDX_TILINGSX(DDX_TX) return false; }
 #undef DDX_F
 #define DDX_F stress_yl
 bool stress_ylds(DDX_SIG) { DDX_TILINGSY(DDX_TY) return false; }
-#else
+#elif DDX_PART == 0
+
+bool whole_shape(const Tiling &t, int fmt) {
+  const int form = t.xl == 2 ? FORM_YL : t.xl ? 3 : t.px == 2 ? FORM_PAIR : FORM_ONE;
+#define DDX_T(FORM, TX, TY, CZ) if (form == FORM && DDX_IS(TX, TY, 1, CZ)) return true;
+  if (fmt == STORE_F32) { DDX_FUSED32(DDX_T) } else { DDX_FUSED16(DDX_T) }
+#undef DDX_T
+  return false;
+}
+
+static int form_of(const Tiling &t) { return t.xl == 2 ? FORM_YL : t.xl ? 3 : t.px == 2 ? FORM_PAIR : FORM_ONE; }
+
+bool launch_vel_all(const Tiling &t, int mode, int fmt, const HalfStep &a, hipStream_t st) {
+  if (mode == RTM_BACKWARD || t.cy != 1 || (mode == FWI && fmt != STORE_F32)) return false;
+  if (a.nphy + a.npml <= 0) return true;
+  return fmt == STORE_F32 ? vel_all_32(t, form_of(t), mode, a, st) : vel_all_16(t, form_of(t), mode, fmt, a, st);
+}
+
+bool launch_stress_all(const Tiling &t, int mode, int fmt, const HalfStep &a, const StepIO &io, hipStream_t st) {
+  if (mode == RTM_BACKWARD || t.cy != 1) return false;
+  const int grid = a.nphy + a.npml + io.nblk;
+  if (grid <= 0) return true;
+  return fmt == STORE_F32 ? stress_all_32(t, form_of(t), mode, a, io, grid, st)
+                          : stress_all_16(t, form_of(t), mode, fmt, a, io, grid, st);
+}
 
 // kz == 0 selects the one-plane-per-block kernels (k_vel_phy / k_stress_phy),
 // cy == 0 the LDS-tiled ones (both FP32 storage only).  FWI mode and the
@@ -3348,26 +3676,26 @@ bool launch_stress_phy(const Tiling &t, int mode, int fmt, const PhyDesc *d, con
     dim3 bl2(LX * LY);
     switch (mode) {
       case PURE_FORWARD:
-        hipLaunchKernelGGL(k_stress_lds<PURE_FORWARD>, g, bl2, 0, st, d, starts, n, dx, dy, dz, sc, t.kz);
+        hipLaunchKernelGGL(k_stress_lds<PURE_FORWARD>, g, bl2, 0, st, d, starts, n, sc / dx, sc / dy, sc / dz, t.kz);
         break;
       case RTM_BACKWARD:
-        hipLaunchKernelGGL(k_stress_lds<RTM_BACKWARD>, g, bl2, 0, st, d, starts, n, dx, dy, dz, sc, t.kz);
+        hipLaunchKernelGGL(k_stress_lds<RTM_BACKWARD>, g, bl2, 0, st, d, starts, n, sc / dx, sc / dy, sc / dz, t.kz);
         break;
       default:
-        hipLaunchKernelGGL(k_stress_lds<RTM_REVERSE>, g, bl2, 0, st, d, starts, n, dx, dy, dz, sc, t.kz);
+        hipLaunchKernelGGL(k_stress_lds<RTM_REVERSE>, g, bl2, 0, st, d, starts, n, sc / dx, sc / dy, sc / dz, t.kz);
     }
     return true;
   }
   if (t.kz > 0) return stress_one(DDX_PASS);
   switch (mode) {
     case PURE_FORWARD:
-      hipLaunchKernelGGL(k_stress_phy<PURE_FORWARD>, g, bl, 0, st, d, starts, n, dx, dy, dz, sc);
+      hipLaunchKernelGGL(k_stress_phy<PURE_FORWARD>, g, bl, 0, st, d, starts, n, sc / dx, sc / dy, sc / dz);
       break;
     case RTM_BACKWARD:
-      hipLaunchKernelGGL(k_stress_phy<RTM_BACKWARD>, g, bl, 0, st, d, starts, n, dx, dy, dz, sc);
+      hipLaunchKernelGGL(k_stress_phy<RTM_BACKWARD>, g, bl, 0, st, d, starts, n, sc / dx, sc / dy, sc / dz);
       break;
     default:
-      hipLaunchKernelGGL(k_stress_phy<RTM_REVERSE>, g, bl, 0, st, d, starts, n, dx, dy, dz, sc);
+      hipLaunchKernelGGL(k_stress_phy<RTM_REVERSE>, g, bl, 0, st, d, starts, n, sc / dx, sc / dy, sc / dz);
   }
   return true;
 }
@@ -3555,13 +3883,12 @@ void launch_inject_batch(int fmt, const MemberIO *io, const int *starts, int n, 
   else hipLaunchKernelGGL(k_inject_batch<F32>, g, b, 0, st, io, starts, n, gs);
 }
 
-void launch_recv_batch(int fmt, const MemberIO *io, const int *starts, int n, int nblk, int gs, const int *gsp,
-                       hipStream_t st) {
-  if (n <= 0 || nblk <= 0) return;
-  const dim3 g(nblk), b(kBlock);
-  if (fmt == STORE_F16) hipLaunchKernelGGL(k_recv_batch<F16>, g, b, 0, st, io, starts, n, gs, gsp);
-  else if (fmt == STORE_BF16) hipLaunchKernelGGL(k_recv_batch<BF16>, g, b, 0, st, io, starts, n, gs, gsp);
-  else hipLaunchKernelGGL(k_recv_batch<F32>, g, b, 0, st, io, starts, n, gs, gsp);
+void launch_recv_batch(int fmt, const StepIO &io, hipStream_t st) {
+  if (io.nblk <= 0) return;
+  const dim3 g(io.nblk), b(kBlock);
+  if (fmt == STORE_F16) hipLaunchKernelGGL(k_recv_batch<F16>, g, b, 0, st, io);
+  else if (fmt == STORE_BF16) hipLaunchKernelGGL(k_recv_batch<BF16>, g, b, 0, st, io);
+  else hipLaunchKernelGGL(k_recv_batch<F32>, g, b, 0, st, io);
 }
 
 void launch_recv_sample(int fmt, void *const *vptr, const int *rsub, const long *roff, int nrec, int it, int ntime,

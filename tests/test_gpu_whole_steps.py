@@ -1,0 +1,125 @@
+"""Half steps run as one launch (bricks, CPML cells, source and receivers)
+against the separate kernels, and the CPML kernels' short division against
+the general one: equal bit for bit."""
+import numpy as np
+import pytest
+
+import ddx
+import pyoracle as po
+from cases import case, random_fields
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = {
+    "fp32": [(32, 8, 1, 4, 1), (64, 4, 1, 2, 1), (64, 4, 1, 2, 4), (64, 4, 1, 4, 4)],
+    "bf16": [(64, 4, 1, 2, 2), (64, 4, 1, 4, 2)],
+    "fp16": [(64, 4, 1, 2, 2), (64, 4, 1, 4, 2)],
+}
+
+
+def engine(c, storage="fp32", shots=None, **kw):
+    e = ddx.Engine(ddx.make_desc(c["nx"], c["ny"], c["nz"], c["dx"], c["pml"], c["dt"], c["fm"], c["ntime"],
+                                 rec_width=c["rec_width"], cfl_policy=1, storage=storage, **kw))
+    e.set_model(c["vp"], c["vs"], c["rho"])
+    e.set_wavelet(po.ricker(c["fm"], c["dt"], c["ntime"]))
+    e.set_geometry(c["shots"] if shots is None else shots, c["recv"])
+    return e
+
+
+# partial tiles on every axis; a row of exactly 64; several columns of bricks (256 cells x 16 rows)
+GRIDS = [(75, 21, 19, 6), (64, 9, 8, 4), (300, 37, 9, 5)]
+
+
+@pytest.mark.parametrize("grid", GRIDS)
+@pytest.mark.parametrize("storage", list(SHAPES))
+def test_whole_half_steps_equal_separate_kernels(storage, grid, monkeypatch):
+    nx, ny, nz, pml = grid
+    c = case(nx=nx, ny=ny, nz=nz, pml=pml, ntime=20, rec_width=2)
+    dx = c["dx"]
+    # in the physical region, in a CPML corner, in the layers that no kernel updates
+    shots = np.array([c["shots"][0], [-(pml - 3) * dx, -(pml - 2) * dx, 2 * dx],
+                      [-pml * dx, 3 * dx, 3 * dx]], np.float32)
+    ref = None
+    for shape in [None] + SHAPES[storage]:
+        monkeypatch.setenv("DDX_WHOLE_CELLS", "0" if shape is None else "1e9")
+        e = engine(c, storage, shots)
+        modes = [po.PURE_FORWARD, po.RTM_FORWARD, po.RTM_REVERSE]
+        if shape is not None:
+            for k in (0, 1):
+                for m in modes:
+                    e.set_brick(k, m, *shape)
+        out = []
+        fwi = [po.FWI] if storage == "fp32" else []
+        for m in modes + fwi:
+            if m == po.FWI and shape is not None and shape[4] == 1:
+                for k in (0, 1):
+                    e.set_brick(k, m, *shape)
+            for s in (0, 1):
+                for f, arr in enumerate(random_fields(e.ext_shape, seed=5 + m, scale=1e-3)):
+                    e.set(s, f, arr)
+            s = 1 if m == po.RTM_REVERSE else 0
+            for _ in range(2):
+                e.step_vel(s, m)
+                e.step_stress(s, m)
+            out += [e.get(s, f) for f in range(19 if m == po.FWI else 13)]
+        for q in range(len(shots)):
+            e.model_shot(q)
+            out += [e.seismograms(q), e.get(0, ddx.SZZ)]
+        e.rtm_shot(0)
+        out += [e.image(q, 0) for q in range(5)]
+        e.close()
+        if ref is None:
+            ref = out
+            continue
+        for i, (a, b) in enumerate(zip(ref, out)):
+            assert np.array_equal(a, b, equal_nan=True), (shape, i)
+
+
+def test_whole_batches_equal_separate_kernels(monkeypatch):
+    """Fused batches of modelling and RTM shots of uneven grids, one member's
+    shot in the CPML, in whole half steps and apart."""
+    cs = [case(nx=41, ny=22, nz=20, ntime=24), case(nx=70, ny=18, nz=26, pml=5, ntime=24, seed=3)]
+    outs = []
+    for cells in ("0", "1e9"):
+        monkeypatch.setenv("DDX_WHOLE_CELLS", cells)
+        es = [engine(c, shots=s) for c, s in zip(cs, (None, np.array([[-20.0, 50.0, 40.0]], np.float32)))]
+        ddx.model_batch(es)
+        ddx.rtm_batch(es)
+        outs.append([e.seismograms(0) for e in es] + [e.image(q, 0) for e in es for q in range(5)])
+        for e in es:
+            e.close()
+    for a, b in zip(*outs):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("spacing", [(10.0, 10.0, 10.0), (7.3, 12.9, 0.3), (8.0, 1000.0, 3.0)])
+def test_cpml_division_is_exact_at_every_magnitude(spacing, monkeypatch):
+    """The one-cell CPML kernels divide by the spacing in three operations
+    where that is exact, else in general; the LDS-tile kernels always in
+    general.  Fields from subnormals to the largest floats, with zeros and
+    infinities in some of them."""
+    c = case(nx=20, ny=18, nz=16, pml=6)
+    for scale in (1e-44, 1e-38, 3e-28, 1e-3, 1e30, 1e37, None):
+        outs = []
+        for cz in ("1", "18"):
+            monkeypatch.setenv("DDX_PML_CZ", cz)
+            e = ddx.Engine(ddx.make_desc(c["nx"], c["ny"], c["nz"], spacing[0], c["pml"], 1e-6, c["fm"], 10,
+                                         dy=spacing[1], dz=spacing[2], cfl_policy=1))
+            e.set_model(c["vp"], c["vs"], c["rho"])
+            rng = np.random.default_rng(3)
+            for f in range(13):
+                a = rng.standard_normal(e.ext_shape)
+                if scale is None:  # every magnitude side by side, zeros and a few infinities
+                    a = np.sign(a) * 10.0 ** rng.uniform(-46, 37, e.ext_shape)
+                    a[rng.random(e.ext_shape) < 0.3] = 0.0
+                    a[rng.random(e.ext_shape) < 1e-3] = np.inf
+                else:
+                    a = a * scale
+                e.set(0, f, a.astype(np.float32))
+            for m in (po.PURE_FORWARD, po.RTM_REVERSE):
+                e.step_vel(0, m)
+                e.step_stress(0, m)
+            outs.append([e.get(0, f) for f in range(10)])
+            e.close()
+        for f, (a, b) in enumerate(zip(*outs)):
+            assert np.array_equal(a, b, equal_nan=True), (scale, ddx.FIELD_NAMES[f])
