@@ -39,27 +39,41 @@ constexpr int kBlock = 256;
 constexpr int kTileX = 64;
 constexpr int kTileY = 4;
 // Work split of the CPML kernels (a context's pml_cz):
+//   kPmlPairs (the default): kBlock consecutive pairs of x cells of a slab
+//     plane per block;
 //   1, 2, 4, 8: kBlock consecutive cells of a slab plane per block, cz
 //     planes per thread, the x and y stencil taps read through the caches;
 //   kPmlTiled + p (p = 2, 4, 8): a tile of pml_tile_x(ni) x (kBlock /
 //     pml_tile_x(ni)) plane cells per block, staged in LDS with its halo,
 //     p planes marched per block (FP32 storage only).
+constexpr int kPmlPairs = 0;
 constexpr int kPmlTiled = 16;
+// The split inside half steps that run as one launch.  FP32 has one cell per
+// thread there: pairs take 120 registers where the bricks and one-cell CPML
+// blocks take 85 to 110, and such grids live in the last-level cache, so the
+// wavefronts in flight count for more than the loads saved (100^3 with 10
+// layers: 75 us per step with one cell, 99 with pairs; 64^3 with 20: 51 and
+// 53).  The 16-bit bricks take 136 registers or more anyway, and their pairs
+// are ahead everywhere.
+__host__ __device__ constexpr int pml_whole(int fmt) { return fmt == STORE_F32 ? 1 : kPmlPairs; }
 __host__ __device__ constexpr bool pml_tiled(int cz) { return cz > kPmlTiled; }
-__host__ __device__ constexpr int pml_planes(int cz) { return cz > kPmlTiled ? cz - kPmlTiled : cz; }
+__host__ __device__ constexpr int pml_planes(int cz) {
+  return cz > kPmlTiled ? cz - kPmlTiled : cz == kPmlPairs ? 1 : cz;
+}
 // Tile width: the whole slab row when it is at most 64 cells (the 18-cell
 // x slabs), else 64 (one wavefront per row).
 __host__ __device__ constexpr int pml_tile_x(int ni) { return ni < 4 ? 4 : ni > 64 ? 64 : ni; }
-// Plane tiles of one slab plane.
-__host__ __device__ inline int pml_plane_tiles(int ni, int nj, int cz) {
+// Plane tiles of one slab plane (ip: elements of a row of memory variables).
+__host__ __device__ inline int pml_plane_tiles(int ni, int nj, int ip, int cz) {
+  if (cz == kPmlPairs) return ((ip >> 1) * nj + kBlock - 1) / kBlock;
   if (!pml_tiled(cz)) return (ni * nj + kBlock - 1) / kBlock;
   const int tx = pml_tile_x(ni), ty = kBlock / tx;
   return ((ni + tx - 1) / tx) * ((nj + ty - 1) / ty);
 }
 // blocks of one CPML slab: plane tiles times chunks of pml_planes(cz) planes
-inline int pml_blocks(int ni, int nj, int nk, int cz) {
+inline int pml_blocks(int ni, int nj, int nk, int ip, int cz) {
   const int p = pml_planes(cz);
-  return pml_plane_tiles(ni, nj, cz) * ((nk + p - 1) / p);
+  return pml_plane_tiles(ni, nj, ip, cz) * ((nk + p - 1) / p);
 }
 
 // One physical region (gridphy) of the whole grid, all subdomains of the
@@ -92,8 +106,13 @@ struct SlabDesc {
   int i0, j0, k0, ni, nj, nk;        // box in extended coordinates
   int axes;                          // damped axes: 1 x, 2 y, 4 z
   int xlo, xhi, ylo, yhi, zlo, zhi;  // a cell is in an axis' damping range iff c < lo || c >= hi
-  void *psi;                         // [6 * naxes][ncell] memory variables (storage format)
-  const float *coef;                 // [naxes][ncell][4]: a, b, a_half, b_half per axis and cell
+  // rows of memory variables and coefficients hold ip elements, an even
+  // number, cell i0 at element sh (0 or 1): pairs of elements 2q, 2q + 1 are
+  // pairs of cells whose first lies on an even element of the fields' storage
+  int ip, sh;
+  unsigned mni, mnp;                 // (2^32 - 1) / ni, / (ip / 2), rounded down
+  void *psi;                         // [6 * naxes][nk][nj][ip] memory variables (storage format)
+  const float *coef;                 // [naxes][nk][nj][ip][4]: a, b, a_half, b_half per axis and cell
   float rdx, rdy, rdz;               // 1 / spacing
   int io;                            // member of a fused launch (StepIO)
   int blk0;

@@ -249,7 +249,9 @@ struct PhyTables {  // physical-region tables of one brick shape and model, per 
 struct Slab {
   int i0, j0, k0, ni, nj, nk, axes;
   int xlo, xhi, ylo, yhi, zlo, zhi;
-  long ncell;
+  long ncell;   // cells
+  int ip, sh;   // elements of a row of memory variables, and of them before the first cell (SlabDesc)
+  long nstore;  // elements of one memory variable
   void *psi[2] = {nullptr, nullptr};  // memory variables of each set (storage format)
   float *coef[2] = {nullptr, nullptr};  // CPML coefficients of the modelling / migration model
   long in_range[3] = {0, 0, 0};
@@ -340,10 +342,11 @@ struct ddx_ctx {
   int brick_group = kBrickGroup;     // XCD group size of the bricks' block order
   int whole_group = -1;              // the same of the half steps that run as one launch (columns)
   double whole_cells = kWholeCells;  // half steps of at most so many cells run as one launch
-  int pml_cz = 1;                    // planes per thread of the CPML kernels (1, 2, 4, 8)
+  int pml_cz = kPmlPairs;            // work split of the CPML kernels
   int pml_group = 32;                // XCD group size of the CPML block order (0: launch order)
   int pml_order = 0;                 // 1: the XCD-partitioned CPML block order (PmlOrder); 0: pml_group
-  DevTable<SlabDesc> pml[2][2];  // [model][set]
+  DevTable<SlabDesc> pml[2][2];        // [model][set]
+  DevTable<SlabDesc> pml_whole[2][2];  // the same, split for half steps that run as one launch
   // exchange mode (ddx_set_exchange): 0 and 2 need no copy, since a
   // subdomain's ghosts are its neighbours' cells; 1 runs the CMM message
   // blocks: every sender side packs the boundary layers of the batch's
@@ -469,6 +472,18 @@ static int upload_table(ddx_ctx *c, DevTable<T> &t, std::vector<T> &h, const std
   return DDX_OK;
 }
 
+// First blocks of the slabs d for the work split cz; returns the number of blocks.
+static int split_pml(std::vector<SlabDesc> &d, std::vector<int> &starts, int cz) {
+  int blk = 0;
+  starts.clear();
+  for (SlabDesc &p : d) {
+    p.blk0 = blk;
+    starts.push_back(blk);
+    blk += pml_blocks(p.ni, p.nj, p.nk, p.ip, cz);
+  }
+  return blk;
+}
+
 // XCD-partitioned block order of a CPML table (PmlOrder): every slab is
 // split into one part per XCD, by z chunks of cz planes when the slab is
 // deeper than its y extent (the y slabs and the x slabs), else by plane
@@ -479,7 +494,7 @@ static void pml_order_host(const std::vector<SlabDesc> &d, int cz, std::vector<P
   std::vector<PmlPiece> per[8];
   o = PmlOrder{};
   for (int s = 0; s < (int)d.size(); s++) {
-    const int T = pml_plane_tiles(d[s].ni, d[s].nj, cz);
+    const int T = pml_plane_tiles(d[s].ni, d[s].nj, d[s].ip, cz);
     const int Z = (d[s].nk + pml_planes(cz) - 1) / pml_planes(cz);
     const bool by_chunk = Z >= 8 && d[s].nk > d[s].nj;
     for (int x = 0; x < 8; x++) {
@@ -705,12 +720,13 @@ extern "C" int ddx_create(const ddx_desc *desc, ddx_ctx **out) {
     delete c;
     return DDX_EHIP;
   }
-  // CPML work split, for sweeps (FP32 storage): 1, 2, 4, 8 planes per thread
+  // CPML work split, for sweeps (FP32 storage; half steps then run as separate
+  // launches unless it is 0): 0 pairs, 1, 2, 4, 8 planes per thread
   // with cached taps, or kPmlTiled + 2, 4, 8 (18, 20, 24) for LDS plane tiles
   if (const char *e = getenv("DDX_PML_CZ")) {
     const int v = atoi(e);
     const int p = pml_planes(v);
-    if (c->fmt == STORE_F32 && (p == 1 || p == 2 || p == 4 || p == 8) && (v < kPmlTiled || p > 1)) c->pml_cz = v;
+    if (c->fmt == STORE_F32 && v >= 0 && (p == 1 || p == 2 || p == 4 || p == 8) && (v < kPmlTiled || p > 1)) c->pml_cz = v;
   }
   if (const char *e = getenv("DDX_PML_GROUP")) {  // XCD group size of the CPML blocks, for sweeps
     const int v = atoi(e);
@@ -1049,7 +1065,8 @@ static int load_model(ddx_ctx *c, int which, const float *vp, const float *vs, c
     if (first) {
       auto add = [&](int i0, int i1, int j0, int j1, int k0, int k1, int axes) {
         // the CPML kernels index a slab in 32 bits: larger ones are cut along z
-        const long plane = (long)(i1 - i0) * (j1 - j0), most = INT_MAX - kBlock;
+        const int sh = (int)((g.origin + i0) & 1), ip = (i1 - i0 + sh + 1) / 2 * 2;
+        const long plane = (long)ip * (j1 - j0), most = INT_MAX - kBlock;
         if (plane > most) { too_big = true; return; }
         const int step = (int)std::min<long>(k1 - k0, most / plane);
         for (int kb = k0; kb < k1; kb += step) {
@@ -1060,7 +1077,9 @@ static int load_model(ddx_ctx *c, int which, const float *vp, const float *vs, c
         sl.xlo = g.mlo[0]; sl.xhi = g.en[0] - g.mhi[0];
         sl.ylo = g.mlo[1]; sl.yhi = g.en[1] - g.mhi[1];
         sl.zlo = g.mlo[2]; sl.zhi = g.en[2] - g.mhi[2];
-        sl.ncell = plane * sl.nk;
+        sl.ncell = (long)sl.ni * sl.nj * sl.nk;
+        sl.ip = ip; sl.sh = sh;
+        sl.nstore = plane * sl.nk;
         c->slabs.push_back(sl);
         }
       };
@@ -1075,20 +1094,20 @@ static int load_model(ddx_ctx *c, int which, const float *vp, const float *vs, c
     for (auto &sl : c->slabs) {
       const int naxes = __builtin_popcount(sl.axes);
       if (!sl.coef[which]) {
-        int rc = dalloc(c, (void **)&sl.coef[which], sizeof(float) * 4 * naxes * sl.ncell);
+        int rc = dalloc(c, (void **)&sl.coef[which], sizeof(float) * 4 * naxes * sl.nstore);
         if (rc) return rc;
       }
       if (!sl.psi[0]) {
         for (int set = 0; set < 2; set++) {
-          int rc = dalloc(c, (void **)&sl.psi[set], (size_t)c->esz * 6 * naxes * sl.ncell);
+          int rc = dalloc(c, (void **)&sl.psi[set], (size_t)c->esz * 6 * naxes * sl.nstore);
           if (rc) return rc;
         }
       }
-      std::vector<float> hc((size_t)4 * naxes * sl.ncell, 0.f);
+      std::vector<float> hc((size_t)4 * naxes * sl.nstore, 0.f);
       std::vector<long> in_plane((size_t)3 * sl.nk, 0);  // cells in each axis' damping range, per plane
       parallel_for(sl.nk, [&](int k) {
-        long cidx = (long)sl.ni * sl.nj * k;
-        for (int j = 0; j < sl.nj; j++)
+        for (int j = 0; j < sl.nj; j++) {
+          long cidx = (long)sl.ip * ((long)sl.nj * k + j) + sl.sh;
           for (int i = 0; i < sl.ni; i++, cidx++) {
             const int ei = sl.i0 + i, ej = sl.j0 + j, ek = sl.k0 + k;
             const float v = evp[(size_t)ei + (size_t)g.en[0] * ((size_t)ej + (size_t)g.en[1] * ek)];
@@ -1100,11 +1119,12 @@ static int load_model(ddx_ctx *c, int which, const float *vp, const float *vs, c
               float A, B, AH, BH;
               if (cpml_axis(en_[a], g.en[a], g.mlo[a], g.mhi[a], h_[a], v, d.fm, d.dt, A, B, AH, BH))
                 in_plane[(size_t)3 * k + a]++;
-              float *q = hc.data() + 4 * ((size_t)slot * sl.ncell + cidx);
+              float *q = hc.data() + 4 * ((size_t)slot * sl.nstore + cidx);
               q[0] = A; q[1] = B; q[2] = AH; q[3] = BH;
               slot++;
             }
           }
+        }
       });
       sl.in_range[0] = sl.in_range[1] = sl.in_range[2] = 0;
       for (int k = 0; k < sl.nk; k++)
@@ -1118,7 +1138,6 @@ static int load_model(ddx_ctx *c, int which, const float *vp, const float *vs, c
     for (int set = 0; set < 2; set++) {
       std::vector<SlabDesc> h;
       std::vector<int> st;
-      int blk = 0;
       double cells = 0, psi_cells = 0;
       for (auto &sl : c->slabs) {
         const Geom &g = c->all;
@@ -1131,22 +1150,25 @@ static int load_model(ddx_ctx *c, int which, const float *vp, const float *vs, c
         p.i0 = sl.i0; p.j0 = sl.j0; p.k0 = sl.k0; p.ni = sl.ni; p.nj = sl.nj; p.nk = sl.nk;
         p.axes = sl.axes;
         p.xlo = sl.xlo; p.xhi = sl.xhi; p.ylo = sl.ylo; p.yhi = sl.yhi; p.zlo = sl.zlo; p.zhi = sl.zhi;
+        p.ip = sl.ip; p.sh = sl.sh;
+        p.mni = 0xffffffffu / (unsigned)sl.ni; p.mnp = 0xffffffffu / (unsigned)(sl.ip / 2);
         p.psi = sl.psi[set];
         p.coef = sl.coef[which];
         // the short division is proven for spacings within 2^20 of 1 (DivGuard): NaN sends the rest the general way
         auto recip = [](float h) { return h < 1048576.0f && h > 1.0f / 1048576.0f ? 1.0f / h : NAN; };
         p.rdx = recip(d.dx); p.rdy = recip(d.dy); p.rdz = recip(d.dz);
         p.io = 0;
-        p.blk0 = blk;
-        st.push_back(blk);
-        blk += pml_blocks(sl.ni, sl.nj, sl.nk, c->pml_cz);
         h.push_back(p);
         cells += (double)sl.ncell;
         psi_cells += (double)(sl.in_range[0] + sl.in_range[1] + sl.in_range[2]);
       }
+      int blk = split_pml(h, st, c->pml_cz);
       int rc = upload_table(c, c->pml[which][set], h, st, blk);
       if (rc) return rc;
       if ((rc = upload_pml_order(c, c->pml[which][set], h))) return rc;
+      blk = split_pml(h, st, pml_whole(c->fmt));
+      if ((rc = upload_table(c, c->pml_whole[which][set], h, st, blk))) return rc;
+      c->pml_whole[which][set].cells = cells;
       c->pml[which][set].cells = cells;
       c->pml[which][set].psi_cells = psi_cells;
     }
@@ -1491,7 +1513,7 @@ static int phy_launch(ddx_ctx *c, int kernel, int set, int mode, const Tiling &t
 // the parts apart) or the launch's size rule it out.
 static bool whole_half(const ddx_ctx *c, const Tiling &t, const DevTable<PhyDesc> &p, const DevTable<SlabDesc> &q,
                        float sc, HalfStep &a) {
-  if (!t.whole || c->prof.mask || c->pml_overlap || c->pml_cz != 1 || c->pml_order) return false;
+  if (!t.whole || c->prof.mask || c->pml_overlap || c->pml_cz != kPmlPairs || c->pml_order) return false;
   if (p.cells + q.cells > c->whole_cells) return false;
   a = {p.d, p.starts, p.n, p.nblk, q.d, q.starts, q.n, q.nblk, c->d.dx, c->d.dy, c->d.dz, sc,
        sc / c->d.dx, sc / c->d.dy, sc / c->d.dz, c->whole_group, c->pml_group};
@@ -1506,7 +1528,7 @@ static int vel_update(ddx_ctx *c, int set, int mode) {
     const PhyTables *pt = phy_tables(c, c->tiling_vel[mode], model_for(c, mode));
     if (!pt) return DDX_EHIP;
     HalfStep a;
-    if (whole_half(c, c->tiling_vel[mode], pt->set[set], c->pml[model_for(c, mode)][set], ratio_vs(c), a) &&
+    if (whole_half(c, c->tiling_vel[mode], pt->set[set], c->pml_whole[model_for(c, mode)][set], ratio_vs(c), a) &&
         launch_vel_all(c->tiling_vel[mode], mode, c->fmt, a, c->st))
       return DDX_OK;
   }
@@ -1539,7 +1561,8 @@ static bool stress_whole(ddx_ctx *c, int set, int mode, const StepIO &io) {
   if (mode == RTM_BACKWARD) return false;
   const PhyTables *pt = phy_tables(c, c->tiling_stress[mode], model_for(c, mode));
   HalfStep a;
-  return pt && whole_half(c, c->tiling_stress[mode], pt->set[set], c->pml[model_for(c, mode)][set], c->d.dt * ratio_sv(c), a) &&
+  return pt && whole_half(c, c->tiling_stress[mode], pt->set[set], c->pml_whole[model_for(c, mode)][set],
+                          c->d.dt * ratio_sv(c), a) &&
          launch_stress_all(c->tiling_stress[mode], mode, c->fmt, a, io, c->st);
 }
 
@@ -1649,7 +1672,7 @@ extern "C" int ddx_reset_wave(ddx_ctx *c, int set) {
   HIPCHECK(c, hipMemsetAsync(c->wave[set], 0, (size_t)c->esz * NF * c->all.fpitch, c->st));
   for (auto &sl : c->slabs)
     if (sl.psi[set])
-      HIPCHECK(c, hipMemsetAsync(sl.psi[set], 0, (size_t)c->esz * 6 * __builtin_popcount(sl.axes) * sl.ncell, c->st));
+      HIPCHECK(c, hipMemsetAsync(sl.psi[set], 0, (size_t)c->esz * 6 * __builtin_popcount(sl.axes) * sl.nstore, c->st));
   return DDX_OK;
 }
 
@@ -1929,7 +1952,7 @@ struct BatchMember {
 
 // What members of one fused launch must share.
 struct BatchKey {
-  int device = 0, fmt = 0, lg0 = 0, lg1 = 0, pml_cz = 1, pml_group = 0, pml_order = 1, brick_group = 0, whole_group = 0;
+  int device = 0, fmt = 0, lg0 = 0, lg1 = 0, pml_cz = kPmlPairs, pml_group = 0, pml_order = 1, brick_group = 0, whole_group = 0;
   float dt = 0.f, dx = 0.f, dy = 0.f, dz = 0.f;
   Tiling tv{0, 0, 0, 0}, ts{0, 0, 0, 0};
 };
@@ -1999,7 +2022,7 @@ static void set_member(HostTable<T> &t, int q) {
 
 struct FusedSet {
   FusedTable<PhyDesc> v, s;
-  FusedTable<SlabDesc> p;
+  FusedTable<SlabDesc> p, pw;  // CPML: split for launches of their own, for whole half steps
   FusedTable<MemberIO> io;  // sources and receivers of the members
   bool whole = false;       // the half steps may run as one launch each
 };
@@ -2041,7 +2064,7 @@ static bool batch_whole(const std::vector<BatchMember> &ms) {
   if (ms.empty()) return false;
   const ddx_ctx *c0 = ms[0].c;
   double cells = 0;
-  bool ok = c0->pml_cz == 1 && !c0->pml_order;
+  bool ok = c0->pml_cz == kPmlPairs && !c0->pml_order;
   for (const BatchMember &m : ms) {
     ok = ok && source_owned(m.c, m.ishot);
     cells += ext_cells(m.c);
@@ -2052,9 +2075,12 @@ static hipError_t fuse_members(std::vector<BatchMember> &ms, FusedSet &f) {
   FusedHost h;
   fuse_host(ms, h);
   f.whole = batch_whole(ms);
+  HostTable<SlabDesc> pw = h.p;
+  if (f.whole) pw.nblk = split_pml(pw.d, pw.s, pml_whole(ms[0].c->fmt));
   hipError_t e = upload_owned(h.v, f.v);
   if (e == hipSuccess) e = upload_owned(h.s, f.s);
-  if (e == hipSuccess) e = upload_owned_pml(h.p, ms.empty() ? 1 : ms[0].c->pml_cz, f.p);
+  if (e == hipSuccess) e = upload_owned_pml(h.p, ms.empty() ? kPmlPairs : ms[0].c->pml_cz, f.p);
+  if (e == hipSuccess && f.whole) e = upload_owned(pw, f.pw);
   if (e == hipSuccess) e = upload_owned(h.io, f.io);
   return e;
 }
@@ -2069,7 +2095,7 @@ static HalfStep half_of(const BatchKey &k, const FusedTable<PhyDesc> &p, const F
 static bool fused_step(const BatchKey &k, const FusedSet &f, const std::vector<BatchMember> &ms, int gs,
                        hipStream_t st, const int *gsp = nullptr) {
   const float rvs = std::ldexp(1.0f, k.lg0 - k.lg1), rsv = std::ldexp(1.0f, k.lg1 - k.lg0);
-  if (!f.whole || !k.tv.whole || !launch_vel_all(k.tv, PURE_FORWARD, k.fmt, half_of(k, f.v, f.p, rvs), st)) {
+  if (!f.whole || !k.tv.whole || !launch_vel_all(k.tv, PURE_FORWARD, k.fmt, half_of(k, f.v, f.pw, rvs), st)) {
     if (!launch_vel_phy(k.tv, PURE_FORWARD, k.fmt, f.v.d, f.v.starts, f.v.n, f.v.nblk, k.dx, k.dy, k.dz, rvs,
                         k.brick_group, st))
       return false;
@@ -2084,7 +2110,7 @@ static bool fused_step(const BatchKey &k, const FusedSet &f, const std::vector<B
   io.nblk = f.io.nblk;
   io.gs = gs;
   io.gsp = gsp;
-  if (!f.whole || !k.ts.whole || !launch_stress_all(k.ts, PURE_FORWARD, k.fmt, half_of(k, f.s, f.p, k.dt * rsv), io, st)) {
+  if (!f.whole || !k.ts.whole || !launch_stress_all(k.ts, PURE_FORWARD, k.fmt, half_of(k, f.s, f.pw, k.dt * rsv), io, st)) {
     launch_source_batch(k.fmt, f.io.d, f.io.n, gs, gsp, st);
     if (!launch_stress_phy(k.ts, PURE_FORWARD, k.fmt, f.s.d, f.s.starts, f.s.n, f.s.nblk, k.dx, k.dy, k.dz,
                            k.dt * rsv, k.brick_group, st))
@@ -2247,6 +2273,12 @@ static int fuse_into_scratch(std::vector<BatchMember> &ms, FusedSet &f, unsigned
   const size_t vd = stage(buf, h.v.d), vs = stage(buf, h.v.s);
   const size_t sd = stage(buf, h.s.d), ss = stage(buf, h.s.s);
   const size_t pd = stage(buf, h.p.d), ps = stage(buf, h.p.s), pp = stage(buf, pieces);
+  HostTable<SlabDesc> pw;
+  if (f.whole) {
+    pw.d = h.p.d;
+    pw.nblk = split_pml(pw.d, pw.s, pml_whole(ms[0].c->fmt));
+  }
+  const size_t wd = stage(buf, pw.d), ws = stage(buf, pw.s);
   const size_t id = stage(buf, h.io.d), is = stage(buf, h.io.s);
   if (buf.size() > kScratchBytes) {
     err = "the batch's descriptor tables need " + std::to_string(buf.size()) + " bytes, more than the " +
@@ -2259,6 +2291,7 @@ static int fuse_into_scratch(std::vector<BatchMember> &ms, FusedSet &f, unsigned
   view(f.v, h.v, dev, vd, vs);
   view(f.s, h.s, dev, sd, ss);
   view(f.p, h.p, dev, pd, ps);
+  view(f.pw, pw, dev, wd, ws);
   view(f.io, h.io, dev, id, is);
   f.p.ord = ord;
   f.p.ord.pieces = pieces.empty() ? nullptr : (const PmlPiece *)(dev + pp);
@@ -2315,6 +2348,7 @@ static int ring_status(ddx_ctx *c, std::string &err);
 struct RtmTables {  // the fused tables of one RTM batch
   FusedTable<PhyDesc> fv, fs, bv, bs, rv, rs;  // forward (set 0), backward (set 0), reverse (set 1)
   FusedTable<SlabDesc> fp, rp;                 // CPML of the forward and reverse sets
+  FusedTable<SlabDesc> fpw, rpw;               // the same, split for whole half steps
   FusedTable<MemberIO> src, inj;               // sources (set 0) and receiver injection (set 1)
   FusedTable<ImgDesc> img;
   bool whole = false;  // the forward and reverse half steps may run as one launch each
@@ -2361,7 +2395,7 @@ static int rtm_batch_tables(const std::vector<ddx_ctx *> &cs, const std::vector<
     hi[q].d.push_back(x);
     hi[q].s.push_back(0);
     hi[q].nblk = recv_blocks(c);
-    T.whole = (q ? T.whole : c0->pml_cz == 1 && !c0->pml_order) && source_owned(c, shots[q]);
+    T.whole = (q ? T.whole : c0->pml_cz == kPmlPairs && !c0->pml_order) && source_owned(c, shots[q]);
   }
   if (e == hipSuccess) e = hipStreamSynchronize(c0->st);
   auto ptrs = [](auto &v) {
@@ -2389,6 +2423,12 @@ static int rtm_batch_tables(const std::vector<ddx_ctx *> &cs, const std::vector<
   if (e == hipSuccess) e = upload_owned(m2, T.inj);
   if (e == hipSuccess) e = upload_owned(im, T.img);
   T.whole = T.whole && cells <= c0->whole_cells;
+  if (T.whole) {
+    a.nblk = split_pml(a.d, a.s, pml_whole(c0->fmt));
+    b.nblk = split_pml(b.d, b.s, pml_whole(c0->fmt));
+    if (e == hipSuccess) e = upload_owned(a, T.fpw);
+    if (e == hipSuccess) e = upload_owned(b, T.rpw);
+  }
   if (e != hipSuccess) { err = std::string("HIP: ") + hipGetErrorString(e); return DDX_EHIP; }
   return DDX_OK;
 }
@@ -2400,7 +2440,7 @@ static bool rtm_fused_forward(const BatchKey &k, const ddx_ctx *c0, const RtmTab
                               const std::vector<ddx_ctx *> &cs, const std::vector<int> &its, int gs, hipStream_t st) {
   const int F = RTM_FORWARD;
   const float rvs = std::ldexp(1.0f, k.lg0 - k.lg1), rsv = std::ldexp(1.0f, k.lg1 - k.lg0);
-  if (!T.whole || !T.sh[0].whole || !launch_vel_all(T.sh[0], F, k.fmt, half_of(k, T.fv, T.fp, rvs), st)) {
+  if (!T.whole || !T.sh[0].whole || !launch_vel_all(T.sh[0], F, k.fmt, half_of(k, T.fv, T.fpw, rvs), st)) {
     if (!launch_vel_phy(T.sh[0], F, k.fmt, T.fv.d, T.fv.starts, T.fv.n, T.fv.nblk, k.dx, k.dy, k.dz, rvs,
                         k.brick_group, st))
       return false;
@@ -2411,7 +2451,7 @@ static bool rtm_fused_forward(const BatchKey &k, const ddx_ctx *c0, const RtmTab
   StepIO io;
   io.io = T.src.d;
   io.gs = gs;
-  if (!T.whole || !T.sh[1].whole || !launch_stress_all(T.sh[1], F, k.fmt, half_of(k, T.fs, T.fp, k.dt * rsv), io, st)) {
+  if (!T.whole || !T.sh[1].whole || !launch_stress_all(T.sh[1], F, k.fmt, half_of(k, T.fs, T.fpw, k.dt * rsv), io, st)) {
     launch_source_batch(k.fmt, T.src.d, T.src.n, gs, nullptr, st, 1.f);
     if (!launch_stress_phy(T.sh[1], F, k.fmt, T.fs.d, T.fs.starts, T.fs.n, T.fs.nblk, k.dx, k.dy, k.dz,
                            k.dt * rsv, k.brick_group, st))
@@ -2446,7 +2486,7 @@ static bool rtm_fused_reverse(const BatchKey &k, const ddx_ctx *c0, const RtmTab
   for (size_t q = 0; q < cs.size(); q++)
     if (its[q] >= 1) ring(cs[q], -1, 2, its[q] - 1, st);
   for (ddx_ctx *c : cs) exchange_on(c, 0, 2, st);
-  if (!T.whole || !T.sh[4].whole || !launch_vel_all(T.sh[4], R, k.fmt, half_of(k, T.rv, T.rp, rvs), st)) {
+  if (!T.whole || !T.sh[4].whole || !launch_vel_all(T.sh[4], R, k.fmt, half_of(k, T.rv, T.rpw, rvs), st)) {
     if (!vel(T.rv, R, 1.f)) return false;
     launch_vel_pml(k.pml_cz, k.fmt, T.rp.d, T.rp.starts, T.rp.n, T.rp.nblk, dx, dy, dz, rvs, k.pml_group,
                    k.pml_order ? &T.rp.ord : nullptr, st);
@@ -2456,7 +2496,7 @@ static bool rtm_fused_reverse(const BatchKey &k, const ddx_ctx *c0, const RtmTab
   for (size_t q = 0; q < cs.size(); q++)
     if (its[q] >= 1) ring(cs[q], -1, 1, its[q] - 1, st);
   for (ddx_ctx *c : cs) exchange_on(c, 0, 0, st);
-  if (!T.whole || !T.sh[5].whole || !launch_stress_all(T.sh[5], R, k.fmt, half_of(k, T.rs, T.rp, dt * rsv), StepIO{}, st)) {
+  if (!T.whole || !T.sh[5].whole || !launch_stress_all(T.sh[5], R, k.fmt, half_of(k, T.rs, T.rpw, dt * rsv), StepIO{}, st)) {
     if (!stress(T.rs, R, dt)) return false;
     launch_stress_pml(k.pml_cz, 1, k.fmt, T.rp.d, T.rp.starts, T.rp.n, T.rp.nblk, dx, dy, dz, dt * rsv, k.pml_group,
                       k.pml_order ? &T.rp.ord : nullptr, st);
@@ -3353,6 +3393,9 @@ extern "C" int ddx_autotune(ddx_ctx *c, int reps, int *timed) {
   if (!c || reps < 1 || reps > 100) return DDX_EINVAL;
   if (!c->have_model) { c->err = "set the model before ddx_autotune"; return DDX_ESTATE; }
   HIPCHECK(c, hipStreamSynchronize(c->st));
+  // The velocity bricks' LDS y arm is ahead on large grids only (676x676x210:
+  // 80.2 ms of 20 steps with it, 82.0 without; RTM of 88^3: 21.6 and 21.7).
+  const bool small = ext_cells(c) <= kWholeCells;
   Tiling cand[64];
   const int nc = std::min(tiling_list(c->fmt, cand, 64), 64);
   hipEvent_t e0, e1;
@@ -3378,6 +3421,7 @@ extern "C" int ddx_autotune(ddx_ctx *c, int reps, int *timed) {
       float best = 1e30f;
       Tiling bt = slot;
       for (int q = 0; q < nc && !rc; q++) {
+        if (kernel == 0 && cand[q].xl == 2 && small) continue;
         float ms = 0.f;
         if ((rc = time_launches(c, e0, e1, reps, ms, [&] { return phy_launch(c, kernel, 0, mode, cand[q]); }))) break;
         count++;
@@ -3391,7 +3435,7 @@ extern "C" int ddx_autotune(ddx_ctx *c, int reps, int *timed) {
         for (int q = -1; q < nc && !rc; q++) {
           Tiling t = q < 0 ? apart : cand[q];
           t.whole = q >= 0;
-          if (q >= 0 && !whole_shape(t, c->fmt)) continue;
+          if (q >= 0 && (!whole_shape(t, c->fmt) || (kernel == 0 && t.xl == 2))) continue;
           slot = t;
           float ms = 0.f;
           rc = time_launches(c, e0, e1, reps, ms, [&] { return kernel == 0 ? vel_update(c, 0, mode) : stress_update(c, 0, mode); });
@@ -3558,7 +3602,8 @@ extern "C" int ddx_estimate_bytes(const ddx_desc *d, int nrec, int nshot, int rt
       b += (2.0 * NF * fsz + 4.0 * 3.0 * models) * (double)w.fpitch;
       for_each_slab(w, [&](int i0, int i1, int j0, int j1, int k0, int k1, int axes) {
         if (i1 <= i0 || j1 <= j0 || k1 <= k0) return;
-        const double ncell = (double)(i1 - i0) * (j1 - j0) * (k1 - k0);
+        const int sh = (int)((w.origin + i0) & 1);
+        const double ncell = (double)((i1 - i0 + sh + 1) / 2 * 2) * (j1 - j0) * (k1 - k0);
         b += ncell * __builtin_popcount(axes) * (4.0 * 4.0 * models + 12.0 * fsz);  // coefficients + 2 sets of psi
       });
     }

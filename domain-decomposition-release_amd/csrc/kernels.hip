@@ -132,6 +132,7 @@ __device__ __forceinline__ const gfloat *G(const void *p) { return (const gfloat
 struct F32 {};
 struct F16 {};
 struct BF16 {};
+template <class S> constexpr bool kF32 = std::is_same<S, F32>::value;
 typedef __attribute__((address_space(1))) _Float16 ghalf;
 typedef __attribute__((address_space(1))) unsigned short gbf16;
 template <class S> struct GPtr;
@@ -1969,11 +1970,19 @@ __device__ __forceinline__ bool pml_block(const SlabDesc *__restrict__ descs, co
   const int b = xcd_group_remap(block, nblk, grp);
   di = find_desc(starts, n, b);
   const SlabDesc &D = descs[di];
-  const int tiles = pml_plane_tiles(D.ni, D.nj, cz);
+  const int tiles = pml_plane_tiles(D.ni, D.nj, D.ip, cz);
   const int t = b - D.blk0;
   zc = t / tiles;
   tile = t - zc * tiles;
   return true;
+}
+
+// Row r and column col of element e of rows of n; m: (2^32 - 1) / n rounded
+// down, so the product's high word is the quotient or one less.
+__device__ __forceinline__ void split_row(int e, int n, unsigned m, int &r, int &col) {
+  r = (int)__umulhi((unsigned)e, m);
+  col = e - r * n;
+  if (col >= n) { col -= n; r++; }
 }
 
 template <int CZ>
@@ -1981,12 +1990,15 @@ __device__ __forceinline__ bool slab_column(const SlabDesc &D, int zc, int tile,
                                             int &kc0, int &kend) {
   const int plane = D.ni * D.nj;
   ci = tile * kBlock + (int)threadIdx.x;
-  const int r = ci / D.ni;
-  ei = D.i0 + (ci - r * D.ni);
+  const bool in = ci < plane;
+  int r, col;
+  split_row(ci, D.ni, D.mni, r, col);
+  ei = D.i0 + col;
   ej = D.j0 + r;
   kc0 = zc * CZ;
   kend = min(kc0 + CZ, D.nk);
-  return ci < plane;
+  ci = r * D.ip + D.sh + col;  // the cell's place in its plane of memory variables
+  return in;
 }
 
 // 4th-order staggered difference of the taps (a - b) and (p - q)
@@ -2036,8 +2048,8 @@ struct PsiCell {
 };
 // psi: the axis' first variable at the block's plane; o: the cell in it
 template <typename GT>
-__device__ __forceinline__ PsiCell<GT> psi_cell(GT *psi, const gfloat *coef, long ncell, unsigned c) {
-  const f4v q = *(const gf4v *)((const gchar *)coef + (size_t)(c * 16u));
+__device__ __forceinline__ PsiCell<GT> psi_cell(GT *psi, const gfloat *coef, long ncell, unsigned c, unsigned cq) {
+  const f4v q = *(const gf4v *)((const gchar *)coef + ((size_t)cq << 4));
   const unsigned o = c * (unsigned)sizeof(typename std::remove_reference<decltype(*psi)>::type);
   return {psi, q.x, q.y, q.z, q.w, ldo(psi, o), ldo(psi + ncell, o), ldo(psi + 2 * ncell, o)};
 }
@@ -2055,9 +2067,8 @@ __device__ __forceinline__ void psi_store(GT *psi, long ncell, unsigned c, float
   sto(psi + 2 * ncell, o, p2);
 }
 
-// S: storage format of fields and memory variables; rv: velocity-over-stress
-// scale ratio (1 for F32), folded into dt/rho.  The cells of block (zc, tile)
-// of slab D.
+// One x cell per thread (FP32 storage).  The cells of block (zc, tile) of slab
+// D; rv: 1, as the pairs' ratio of scales.
 //
 // What bounds it: the slab's own bytes (42-48 loads and 12-16 stores per
 // cell), moved at 4.6 TB/s on large grids, the rate of a plain copy; on small
@@ -2066,16 +2077,19 @@ __device__ __forceinline__ void psi_store(GT *psi, long ncell, unsigned c, float
 // way, two planes either way) shared by all arrays, the coefficients of an
 // axis as one 16-byte load, and div_u: the stress kernel needs 89 vector
 // registers instead of 102 (5 wavefronts per SIMD, 4 before).  256x256x200,
-// 20 layers (7.0 M cells): velocity 180 -> 177 us, stress 224 -> 214 us; BF16
-// 161x150x131 82.7 -> 70.5 and 101.8 -> 79.4 us.
+// 20 layers (7.0 M cells): velocity 180 -> 177 us, stress 224 -> 214 us.  The
+// z slabs' shared model and coefficients and the row found by a product
+// instead of a division: 64^3 with 20 layers 52 -> 51 us per step (clamping
+// the model's row and column too costs vector instructions: 53.6).
 template <int CZ, class S>
 __device__ __forceinline__ void vel_pml_body(const SlabDesc &D, int zc, int tile, float dx, float dy, float dz, float rv) {
   typedef typename GPtr<S>::T gT;
   int ci, ei, ej, kc0, kend;
   if (!slab_column<CZ>(D, zc, tile, ci, ei, ej, kc0, kend)) return;
-  const long ncell = (long)D.ni * D.nj * D.nk;
-  const int plane = D.ni * D.nj;
-  constexpr unsigned E = sizeof(typename GPtr<S>::raw);
+  const long ncell = (long)D.ip * D.nj * D.nk;
+  const int plane = D.ip * D.nj;
+  static_assert(kF32<S>, "the 16-bit formats run pairs");
+  constexpr unsigned E = 4;
   const unsigned syb = (unsigned)D.sy * E, szb = (unsigned)D.sz * E;
   const long pb = D.sz * (D.k0 + kc0 - 2);  // two planes below the block's first
   const float c0 = c_fd[2][0], c1 = c_fd[2][1];
@@ -2083,7 +2097,6 @@ __device__ __forceinline__ void vel_pml_body(const SlabDesc &D, int zc, int tile
   const gT *sxx = (const gT *)D.f[SXX] + pb, *syy = (const gT *)D.f[SYY] + pb, *szz = (const gT *)D.f[SZZ] + pb;
   const gT *sxy = (const gT *)D.f[SXY] + pb, *sxz = (const gT *)D.f[SXZ] + pb, *syz = (const gT *)D.f[SYZ] + pb;
   gT *fvx = (gT *)D.f[VX] + pb, *fvy = (gT *)D.f[VY] + pb, *fvz = (gT *)D.f[VZ] + pb;
-  const gfloat *fdtr = G(D.dtr) + pb;
   const bool inx = (D.axes & 1) && (ei < D.xlo || ei >= D.xhi);
   const bool iny = (D.axes & 2) && (ej < D.ylo || ej >= D.yhi);
   const int sx_slot = 0, sy_slot = (D.axes & 1) ? 1 : 0, sz_slot = sy_slot + ((D.axes & 2) ? 1 : 0);
@@ -2091,8 +2104,11 @@ __device__ __forceinline__ void vel_pml_body(const SlabDesc &D, int zc, int tile
   gT *px = (gT *)D.psi + (long)(sx_slot * 6) * ncell + cb;
   gT *py = (gT *)D.psi + (long)(sy_slot * 6) * ncell + cb;
   gT *pz = (gT *)D.psi + (long)(sz_slot * 6) * ncell + cb;
-  const gfloat *qx = G(D.coef) + 4 * ((long)sx_slot * ncell + cb);
-  const gfloat *qy = G(D.coef) + 4 * ((long)sy_slot * ncell + cb);
+  // the model and the x and y coefficients do not change along a z slab's
+  // normal: those of its first plane, which the caches hold
+  const bool zs = D.axes & 4;
+  const gfloat *qx = G(D.coef) + 4 * ((long)sx_slot * ncell + (zs ? 0 : cb));
+  const gfloat *qy = G(D.coef) + 4 * ((long)sy_slot * ncell + (zs ? 0 : cb));
   const gfloat *qz = G(D.coef) + 4 * ((long)sz_slot * ncell + cb);
   const unsigned o0 = (unsigned)ei * E + syb * (unsigned)ej;  // the cell in plane pb
   // z arms: szz forward-staggered, planes k-1 .. k+2; sxz, syz backward-staggered, planes k-2 .. k+1
@@ -2117,9 +2133,9 @@ __device__ __forceinline__ void vel_pml_body(const SlabDesc &D, int zc, int tile
     const int ek = D.k0 + kc0 + kk;
     const unsigned o = o0 + (unsigned)(kk + 2) * szb, c = (unsigned)ci + (unsigned)(plane * kk);
     const unsigned ym2 = o - 2 * syb, ym1 = o - syb, yp1 = o + syb, yp2 = o + 2 * syb;
-    const unsigned of = E == 4 ? o : (o / E) * 4u;  // dt/rho is FP32
+    const gfloat *fdtr = G(D.dtr) + D.sz * min(max(ek, D.zlo), D.zhi - 1);
     const float ovx = ldo(fvx, o), ovy = ldo(fvy, o), ovz = ldo(fvz, o);
-    const float dtr = std::is_same<S, F32>::value ? ldo(fdtr, of) : rv * ldo(fdtr, of);
+    const float dtr = ldo(fdtr, o0);
     const float xx0 = ldo(sxx, o), xxm = ldo(sxx, o, -1), xx1 = ldo(sxx, o, 1), xx2 = ldo(sxx, o, 2);
     const float xy0 = ldo(sxy, o), xym1 = ldo(sxy, o, -1), xym2 = ldo(sxy, o, -2), xy1 = ldo(sxy, o, 1);
     const float xzm1 = ldo(sxz, o, -1), xzm2 = ldo(sxz, o, -2), xz1 = ldo(sxz, o, 1);
@@ -2129,9 +2145,9 @@ __device__ __forceinline__ void vel_pml_body(const SlabDesc &D, int zc, int tile
     const float xz0 = qxz[kk + 2], yz0 = qyz[kk + 2];
     inz[kk] = (D.axes & 4) && (ek < D.zlo || ek >= D.zhi);
     PsiCell<gT> mx, my, mz;
-    if (inx) mx = psi_cell(px, qx, ncell, c);
-    if (iny) my = psi_cell(py, qy, ncell, c);
-    if (inz[kk]) mz = psi_cell(pz, qz, ncell, c);
+    if (inx) mx = psi_cell(px, qx, ncell, c, zs ? (unsigned)ci : c);
+    if (iny) my = psi_cell(py, qy, ncell, c, zs ? (unsigned)ci : c);
+    if (inz[kk]) mz = psi_cell(pz, qz, ncell, c, c);
     float sxx_x = d2(xx1, xx0, xx2, xxm, c0, c1), syx_x = d2(xy0, xym1, xy1, xym2, c0, c1);
     float szx_x = d2(xz0, xzm1, xz1, xzm2, c0, c1);
     float syy_y = d2(yy1, yy0, yy2, yym, c0, c1), sxy_y = d2(xy0, xyYm1, xyY1, xyYm2, c0, c1);
@@ -2196,9 +2212,10 @@ __device__ __forceinline__ void stress_pml_body(const SlabDesc &D, int zc, int t
   typedef typename GPtr<S>::T gT;
   int ci, ei, ej, kc0, kend;
   if (!slab_column<CZ>(D, zc, tile, ci, ei, ej, kc0, kend)) return;
-  const long ncell = (long)D.ni * D.nj * D.nk;
-  const int plane = D.ni * D.nj;
-  constexpr unsigned E = sizeof(typename GPtr<S>::raw);
+  const long ncell = (long)D.ip * D.nj * D.nk;
+  const int plane = D.ip * D.nj;
+  static_assert(kF32<S>, "the 16-bit formats run pairs");
+  constexpr unsigned E = 4;
   const unsigned syb = (unsigned)D.sy * E, szb = (unsigned)D.sz * E;
   const long pb = D.sz * (D.k0 + kc0 - 2);  // two planes below the block's first
   const float c0 = c_fd[2][0], c1 = c_fd[2][1];
@@ -2207,7 +2224,6 @@ __device__ __forceinline__ void stress_pml_body(const SlabDesc &D, int zc, int t
   gT *fsxx = (gT *)D.f[SXX] + pb, *fsyy = (gT *)D.f[SYY] + pb, *fszz = (gT *)D.f[SZZ] + pb;
   gT *fsxy = (gT *)D.f[SXY] + pb, *fsxz = (gT *)D.f[SXZ] + pb, *fsyz = (gT *)D.f[SYZ] + pb;
   gT *fsau = (gT *)D.f[SAU] + pb;
-  const gfloat *flam = G(D.lam) + pb, *fmu = G(D.mu) + pb;
   const bool inx = (D.axes & 1) && (ei < D.xlo || ei >= D.xhi);
   const bool iny = (D.axes & 2) && (ej < D.ylo || ej >= D.yhi);
   const int sx_slot = 0, sy_slot = (D.axes & 1) ? 1 : 0, sz_slot = sy_slot + ((D.axes & 2) ? 1 : 0);
@@ -2215,8 +2231,11 @@ __device__ __forceinline__ void stress_pml_body(const SlabDesc &D, int zc, int t
   gT *px = (gT *)D.psi + (long)(sx_slot * 6 + 3) * ncell + cb;
   gT *py = (gT *)D.psi + (long)(sy_slot * 6 + 3) * ncell + cb;
   gT *pz = (gT *)D.psi + (long)(sz_slot * 6 + 3) * ncell + cb;
-  const gfloat *qx = G(D.coef) + 4 * ((long)sx_slot * ncell + cb);
-  const gfloat *qy = G(D.coef) + 4 * ((long)sy_slot * ncell + cb);
+  // the model and the x and y coefficients do not change along a z slab's
+  // normal: those of its first plane, which the caches hold
+  const bool zs = D.axes & 4;
+  const gfloat *qx = G(D.coef) + 4 * ((long)sx_slot * ncell + (zs ? 0 : cb));
+  const gfloat *qy = G(D.coef) + 4 * ((long)sy_slot * ncell + (zs ? 0 : cb));
   const gfloat *qz = G(D.coef) + 4 * ((long)sz_slot * ncell + cb);
   const unsigned o0 = (unsigned)ei * E + syb * (unsigned)ej;
   // z arms: vx, vy forward-staggered, planes k-1 .. k+2; vz backward-staggered, planes k-2 .. k+1
@@ -2238,7 +2257,8 @@ __device__ __forceinline__ void stress_pml_body(const SlabDesc &D, int zc, int t
     const int ek = D.k0 + kc0 + kk;
     const unsigned o = o0 + (unsigned)(kk + 2) * szb, c = (unsigned)ci + (unsigned)(plane * kk);
     const unsigned ym2 = o - 2 * syb, ym1 = o - syb, yp1 = o + syb, yp2 = o + 2 * syb;
-    const unsigned of = E == 4 ? o : (o / E) * 4u;  // the model is FP32
+    const long mb = D.sz * min(max(ek, D.zlo), D.zhi - 1);
+    const gfloat *flam = G(D.lam) + mb, *fmu = G(D.mu) + mb;
     const float x0 = zx[kk + 1], y0 = zy[kk + 1], z0 = zz[kk + 2];
     const float xm1 = ldo(vx, o, -1), xm2 = ldo(vx, o, -2), x1 = ldo(vx, o, 1);
     const float yxm = ldo(vy, o, -1), yx1 = ldo(vy, o, 1), yx2 = ldo(vy, o, 2);
@@ -2246,7 +2266,7 @@ __device__ __forceinline__ void stress_pml_body(const SlabDesc &D, int zc, int t
     const float xym = ldo(vx, ym1), xy1 = ldo(vx, yp1), xy2 = ldo(vx, yp2);
     const float yym1 = ldo(vy, ym1), yym2 = ldo(vy, ym2), yy1 = ldo(vy, yp1);
     const float zym = ldo(vz, ym1), zy1 = ldo(vz, yp1), zy2 = ldo(vz, yp2);
-    const float lm = ldo(flam, of), mu = ldo(fmu, of);
+    const float lm = ldo(flam, o0), mu = ldo(fmu, o0);
     const float l2m = lm + 2.0f * mu;
     float oxx = ldo(fsxx, o), oyy = ldo(fsyy, o), ozz = ldo(fszz, o);
     if constexpr (SRC) add_source<gT>(src, ei, ej, ek, oxx, oyy, ozz);
@@ -2254,9 +2274,9 @@ __device__ __forceinline__ void stress_pml_body(const SlabDesc &D, int zc, int t
     const float oau = WITH_SAU ? ldo(fsau, o) : 0.f;
     inz[kk] = (D.axes & 4) && (ek < D.zlo || ek >= D.zhi);
     PsiCell<gT> mx, my, mz;
-    if (inx) mx = psi_cell(px, qx, ncell, c);
-    if (iny) my = psi_cell(py, qy, ncell, c);
-    if (inz[kk]) mz = psi_cell(pz, qz, ncell, c);
+    if (inx) mx = psi_cell(px, qx, ncell, c, zs ? (unsigned)ci : c);
+    if (iny) my = psi_cell(py, qy, ncell, c, zs ? (unsigned)ci : c);
+    if (inz[kk]) mz = psi_cell(pz, qz, ncell, c, c);
     float vx_x = d2(x0, xm1, x1, xm2, c0, c1), vy_x = d2(yx1, y0, yx2, yxm, c0, c1);
     float vz_x = d2(zx1, z0, zx2, zxm, c0, c1);
     float vy_y = d2(y0, yym1, yy1, yym2, c0, c1), vx_y = d2(xy1, x0, xy2, xym, c0, c1);
@@ -2320,6 +2340,323 @@ __global__ __launch_bounds__(kBlock) DDX_PML_ATTR void k_stress_pml(const SlabDe
   stress_pml_body<WITH_SAU, CZ, S>(descs[di], zc, tile, dx, dy, dz, dt);
 }
 
+
+// ---------------------------------------------------------------------------
+// CPML halves, two neighbouring x cells per thread (work split kPmlPairs, the
+// default).  A plane's rows are cut into pairs whose first cell lies on an
+// even element of the storage (D.sh shifts a slab's rows; the memory variables
+// and coefficients have rows of D.ip elements in the same pairs), so every
+// access of a pair is one aligned 2-element load or store in every format.  A
+// pair's cell outside the slab (a row's first, last) is read, never written.
+//
+// What bounds it: the bytes on large FP32 grids (its kernels run at the copy
+// rate), instruction issue for the 16-bit formats, whose one-cell loads move
+// 2 bytes per lane and whose conversions come on top.  Pairs halve the loads
+// and the addressing.  The model is constant along the normal of the layers
+// (extended by its edge values), and so are the coefficients of the axes
+// other than the slab's own, so both are read from the layer's first plane,
+// row or column, which the caches hold.  161x150x131 cells with 20 layers in
+// BF16: 320 -> 282 us per step; 676x676x210 in FP32: 4055 -> 4026 us.
+// Operands and order of operations per cell are those of vel_pml_body and
+// stress_pml_body.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ F2 ldp(const gfloat *p, unsigned off, int elem = 0) {
+  const f2v v = *(const gf2v *)((const gchar *)p + off + elem * 4);
+  return {v.x, v.y};
+}
+__device__ __forceinline__ F2 ldp(const ghalf *p, unsigned off, int elem = 0) {
+  const h2v v = *(const gh2v *)((const gchar *)p + off + elem * 2);
+  return {(float)v.x, (float)v.y};
+}
+__device__ __forceinline__ F2 ldp(const gbf16 *p, unsigned off, int elem = 0) {
+  const unsigned u = *(const gu32 *)((const gchar *)p + off + elem * 2);
+  return {__uint_as_float(u << 16), __uint_as_float(u & 0xffff0000u)};
+}
+__device__ __forceinline__ void stp2(gfloat *p, unsigned off, float a, float b) {
+  f2v v;
+  v.x = a;
+  v.y = b;
+  *(gf2v *)((gchar *)p + off) = v;
+}
+__device__ __forceinline__ void stp2(ghalf *p, unsigned off, float a, float b) {
+  h2v v;
+  v.x = (_Float16)a;
+  v.y = (_Float16)b;
+  *(gh2v *)((gchar *)p + off) = v;
+}
+__device__ __forceinline__ void stp2(gbf16 *p, unsigned off, float a, float b) {
+  *(gu32 *)((gchar *)p + off) = (unsigned)bf16_rne(a) | ((unsigned)bf16_rne(b) << 16);
+}
+// the pair, or the one of its cells that is in the slab (m: bit 0 first, 1 second)
+template <typename GT>
+__device__ __forceinline__ void stp(GT *p, unsigned off, float a, float b, int m) {
+  if (m == 3) stp2(p, off, a, b);
+  else if (m == 1) sto(p, off, a);
+  else sto(p + 1, off, b);
+}
+
+// A thread's pair: first cell's extended coordinates, place in the plane's
+// memory variables (c) and in its row (cx), which of its cells are in the slab.
+struct PairAt {
+  int ei, ej, c, cx, m;
+};
+__device__ __forceinline__ bool pml_pair(const SlabDesc &D, int tile, PairAt &a) {
+  const int np = D.ip >> 1;
+  const int e = tile * kBlock + (int)threadIdx.x;
+  if (e >= np * D.nj) return false;
+  int r, q;
+  split_row(e, np, D.mnp, r, q);
+  a.cx = 2 * q;
+  a.c = r * D.ip + a.cx;
+  a.ei = D.i0 - D.sh + a.cx;
+  a.ej = D.j0 + r;
+  a.m = (a.ei >= D.i0 ? 1 : 0) | (a.ei + 1 < D.i0 + D.ni ? 2 : 0);
+  return true;
+}
+
+// The pair whose model the pair at ei has: the outermost one of the edge's value in the layers.
+__device__ __forceinline__ int pair_edge(const SlabDesc &D, int ei) {
+  const int first = D.i0 - D.sh, lo = D.xlo - 1, hi = D.xhi - 1;
+  return min(max(ei, lo - ((lo - first) & 1)), hi + ((hi - first) & 1));
+}
+
+// Memory variables and coefficients of one damped axis of a pair.
+struct PsiPair {
+  f4v qa, qb;  // a, b, a_half, b_half of the two cells
+  F2 m0, m1, m2;
+};
+template <typename GT>
+__device__ __forceinline__ PsiPair psi_pair(const GT *psi, const gfloat *coef, long ncell, unsigned c, unsigned cq) {
+  constexpr unsigned E = sizeof(typename std::remove_reference<decltype(*psi)>::type);
+  const gf4v *q = (const gf4v *)((const gchar *)coef + ((size_t)cq << 4));
+  return {q[0], q[1], ldp(psi, c * E), ldp(psi + ncell, c * E), ldp(psi + 2 * ncell, c * E)};
+}
+template <typename GT>
+__device__ __forceinline__ void psi_pair_store(GT *psi, long ncell, unsigned c, const float (&a)[3],
+                                               const float (&b)[3], int m) {
+  constexpr unsigned E = sizeof(typename std::remove_reference<decltype(*psi)>::type);
+  stp(psi, c * E, a[0], b[0], m);
+  stp(psi + ncell, c * E, a[1], b[1], m);
+  stp(psi + 2 * ncell, c * E, a[2], b[2], m);
+}
+// new memory variables p of the derivatives d (h: bit q set where d[q] takes
+// the half-grid coefficients), which enter the derivatives as stored
+template <typename GT, int H>
+__device__ __forceinline__ void psi_step(const f4v &q, float m0, float m1, float m2, float &d0, float &d1, float &d2,
+                                         float (&p)[3]) {
+  const GT *t = nullptr;
+  p[0] = quant(t, (H & 1 ? q.w : q.y) * m0 + (H & 1 ? q.z : q.x) * d0);
+  p[1] = quant(t, (H & 2 ? q.w : q.y) * m1 + (H & 2 ? q.z : q.x) * d1);
+  p[2] = quant(t, (H & 4 ? q.w : q.y) * m2 + (H & 4 ? q.z : q.x) * d2);
+  d0 += p[0];
+  d1 += p[1];
+  d2 += p[2];
+}
+
+// A slab's scalar bases for a plane: memory variables (first: 0 velocity, 3
+// stress) and coefficients per axis, and the plane of the model it shares.
+template <typename GT>
+struct PmlBase {
+  GT *px, *py, *pz;
+  const gfloat *qx, *qy, *qz;
+  long ncell;
+  bool cx_row;  // the x coefficients are those of the plane's first row
+};
+template <typename GT>
+__device__ __forceinline__ PmlBase<GT> pml_base(const SlabDesc &D, int zc, int first) {
+  PmlBase<GT> b;
+  b.ncell = (long)D.ip * D.nj * D.nk;
+  const long at = (long)D.ip * D.nj * zc;
+  GT *p = (GT *)D.psi + (long)first * b.ncell + at;
+  const bool zs = D.axes & 4, ys = !zs && (D.axes & 2);
+  b.px = p;
+  b.py = p + 6 * b.ncell;
+  b.pz = p + 12 * b.ncell;
+  const gfloat *q = G(D.coef);
+  b.qx = q + (zs ? 0 : 4 * at);
+  b.qy = q + 4 * b.ncell + (zs ? 0 : 4 * at);
+  b.qz = q + 8 * b.ncell + 4 * at;
+  b.cx_row = ys;
+  return b;
+}
+
+template <class S>
+__device__ __forceinline__ void vel_pml_pair(const SlabDesc &D, int zc, int tile, float dx, float dy, float dz,
+                                             float rv) {
+  typedef typename GPtr<S>::T gT;
+  PairAt at;
+  if (!pml_pair(D, tile, at)) return;
+  constexpr unsigned E = sizeof(typename GPtr<S>::raw);
+  const unsigned syb = (unsigned)D.sy * E, szb = (unsigned)D.sz * E;
+  const int ek = D.k0 + zc;
+  const long pb = D.sz * (ek - 2);  // two planes below
+  const float c0 = c_fd[2][0], c1 = c_fd[2][1];
+  const gT *sxx = (const gT *)D.f[SXX] + pb, *syy = (const gT *)D.f[SYY] + pb, *szz = (const gT *)D.f[SZZ] + pb;
+  const gT *sxy = (const gT *)D.f[SXY] + pb, *sxz = (const gT *)D.f[SXZ] + pb, *syz = (const gT *)D.f[SYZ] + pb;
+  gT *fvx = (gT *)D.f[VX] + pb, *fvy = (gT *)D.f[VY] + pb, *fvz = (gT *)D.f[VZ] + pb;
+  const gfloat *fdtr = G(D.dtr) + D.sz * min(max(ek, D.zlo), D.zhi - 1);
+  const PmlBase<gT> B = pml_base<gT>(D, zc, 0);
+  const unsigned ob = (unsigned)at.ei * E + syb * (unsigned)at.ej, o = ob + 2 * szb;
+  const unsigned om = (unsigned)pair_edge(D, at.ei) * 4u + (unsigned)D.sy * 4u * (unsigned)min(max(at.ej, D.ylo), D.yhi - 1);
+  const unsigned ym2 = o - 2 * syb, ym1 = o - syb, yp1 = o + syb, yp2 = o + 2 * syb;
+  const unsigned zm1 = ob + szb, zp1 = o + szb, zp2 = o + 2 * szb;
+  const bool ixa = (D.axes & 1) && (at.ei < D.xlo || at.ei >= D.xhi);
+  const bool ixb = (D.axes & 1) && (at.ei + 1 < D.xlo || at.ei + 1 >= D.xhi);
+  const bool iy = (D.axes & 2) && (at.ej < D.ylo || at.ej >= D.yhi);
+  const bool iz = D.axes & 4;  // every cell of a z slab, no other slab's
+  const F2 ovx = ldp(fvx, o), ovy = ldp(fvy, o), ovz = ldp(fvz, o);
+  const F2 dr = ldp(fdtr, om);
+  const F2 xx0 = ldp(sxx, o), xxm = ldp(sxx, o, -2), xxp = ldp(sxx, o, 2);
+  const F2 xy0 = ldp(sxy, o), xym = ldp(sxy, o, -2), xyp = ldp(sxy, o, 2);
+  const F2 xz0 = ldp(sxz, o), xzm = ldp(sxz, o, -2), xzp = ldp(sxz, o, 2);
+  const F2 yy0 = ldp(syy, o), yym = ldp(syy, ym1), yy1 = ldp(syy, yp1), yy2 = ldp(syy, yp2);
+  const F2 xym2 = ldp(sxy, ym2), xym1 = ldp(sxy, ym1), xy1 = ldp(sxy, yp1);
+  const F2 yz0 = ldp(syz, o), yzm2 = ldp(syz, ym2), yzm1 = ldp(syz, ym1), yz1 = ldp(syz, yp1);
+  const F2 zz0 = ldp(szz, o), zzm = ldp(szz, zm1), zz1 = ldp(szz, zp1), zz2 = ldp(szz, zp2);
+  const F2 xzm2 = ldp(sxz, ob), xzm1 = ldp(sxz, zm1), xz1 = ldp(sxz, zp1);
+  const F2 yzZm2 = ldp(syz, ob), yzZm1 = ldp(syz, zm1), yzZ1 = ldp(syz, zp1);
+  PsiPair mx, my, mz;
+  if (ixa || ixb) mx = psi_pair(B.px, B.qx, B.ncell, at.c, B.cx_row ? at.cx : at.c);
+  if (iy) my = psi_pair(B.py, B.qy, B.ncell, at.c, at.c);
+  if (iz) mz = psi_pair(B.pz, B.qz, B.ncell, at.c, at.c);
+  float xa0 = d2(xx0.b, xx0.a, xxp.a, xxm.b, c0, c1), xb0 = d2(xxp.a, xx0.b, xxp.b, xx0.a, c0, c1);  // sxx_x
+  float xa1 = d2(xy0.a, xym.b, xy0.b, xym.a, c0, c1), xb1 = d2(xy0.b, xy0.a, xyp.a, xym.b, c0, c1);  // syx_x
+  float xa2 = d2(xz0.a, xzm.b, xz0.b, xzm.a, c0, c1), xb2 = d2(xz0.b, xz0.a, xzp.a, xzm.b, c0, c1);  // szx_x
+  float ya0 = d2(xy0.a, xym1.a, xy1.a, xym2.a, c0, c1), yb0 = d2(xy0.b, xym1.b, xy1.b, xym2.b, c0, c1);  // sxy_y
+  float ya1 = d2(yy1.a, yy0.a, yy2.a, yym.a, c0, c1), yb1 = d2(yy1.b, yy0.b, yy2.b, yym.b, c0, c1);      // syy_y
+  float ya2 = d2(yz0.a, yzm1.a, yz1.a, yzm2.a, c0, c1), yb2 = d2(yz0.b, yzm1.b, yz1.b, yzm2.b, c0, c1);  // szy_y
+  float za0 = d2(xz0.a, xzm1.a, xz1.a, xzm2.a, c0, c1), zb0 = d2(xz0.b, xzm1.b, xz1.b, xzm2.b, c0, c1);  // sxz_z
+  float za1 = d2(yz0.a, yzZm1.a, yzZ1.a, yzZm2.a, c0, c1);
+  float zb1 = d2(yz0.b, yzZm1.b, yzZ1.b, yzZm2.b, c0, c1);                                               // syz_z
+  float za2 = d2(zz1.a, zz0.a, zz2.a, zzm.a, c0, c1), zb2 = d2(zz1.b, zz0.b, zz2.b, zzm.b, c0, c1);      // szz_z
+  div9(xa0, xa1, xa2, ya0, ya1, ya2, za0, za1, za2, dx, dy, dz, D.rdx, D.rdy, D.rdz);
+  div9(xb0, xb1, xb2, yb0, yb1, yb2, zb0, zb1, zb2, dx, dy, dz, D.rdx, D.rdy, D.rdz);
+  float pa[3][3], pc[3][3];
+  if (ixa) psi_step<gT, 1>(mx.qa, mx.m0.a, mx.m1.a, mx.m2.a, xa0, xa1, xa2, pa[0]);
+  if (ixb) psi_step<gT, 1>(mx.qb, mx.m0.b, mx.m1.b, mx.m2.b, xb0, xb1, xb2, pc[0]);
+  if (iy) {
+    psi_step<gT, 2>(my.qa, my.m0.a, my.m1.a, my.m2.a, ya0, ya1, ya2, pa[1]);
+    psi_step<gT, 2>(my.qb, my.m0.b, my.m1.b, my.m2.b, yb0, yb1, yb2, pc[1]);
+  }
+  if (iz) {
+    psi_step<gT, 4>(mz.qa, mz.m0.a, mz.m1.a, mz.m2.a, za0, za1, za2, pa[2]);
+    psi_step<gT, 4>(mz.qb, mz.m0.b, mz.m1.b, mz.m2.b, zb0, zb1, zb2, pc[2]);
+  }
+  const float da = std::is_same<S, F32>::value ? dr.a : rv * dr.a, db = std::is_same<S, F32>::value ? dr.b : rv * dr.b;
+  const int mxm = at.m & ((ixa ? 1 : 0) | (ixb ? 2 : 0));
+  if (mxm) psi_pair_store(B.px, B.ncell, at.c, pa[0], pc[0], mxm);
+  if (iy) psi_pair_store(B.py, B.ncell, at.c, pa[1], pc[1], at.m);
+  if (iz) psi_pair_store(B.pz, B.ncell, at.c, pa[2], pc[2], at.m);
+  stp(fvx, o, ovx.a + da * (xa0 + ya0 + za0), ovx.b + db * (xb0 + yb0 + zb0), at.m);
+  stp(fvy, o, ovy.a + da * (xa1 + ya1 + za1), ovy.b + db * (xb1 + yb1 + zb1), at.m);
+  stp(fvz, o, ovz.a + da * (xa2 + ya2 + za2), ovz.b + db * (xb2 + yb2 + zb2), at.m);
+}
+
+template <int WITH_SAU, class S, bool SRC = false>
+__device__ __forceinline__ void stress_pml_pair(const SlabDesc &D, int zc, int tile, float dx, float dy, float dz,
+                                                float dt, const SrcCell &src = SrcCell{}) {
+  typedef typename GPtr<S>::T gT;
+  PairAt at;
+  if (!pml_pair(D, tile, at)) return;
+  constexpr unsigned E = sizeof(typename GPtr<S>::raw);
+  const unsigned syb = (unsigned)D.sy * E, szb = (unsigned)D.sz * E;
+  const int ek = D.k0 + zc;
+  const long pb = D.sz * (ek - 2);
+  const float c0 = c_fd[2][0], c1 = c_fd[2][1];
+  const gT *vx = (const gT *)D.f[VX] + pb, *vy = (const gT *)D.f[VY] + pb, *vz = (const gT *)D.f[VZ] + pb;
+  gT *fsxx = (gT *)D.f[SXX] + pb, *fsyy = (gT *)D.f[SYY] + pb, *fszz = (gT *)D.f[SZZ] + pb;
+  gT *fsxy = (gT *)D.f[SXY] + pb, *fsxz = (gT *)D.f[SXZ] + pb, *fsyz = (gT *)D.f[SYZ] + pb;
+  gT *fsau = (gT *)D.f[SAU] + pb;
+  const long mb = D.sz * min(max(ek, D.zlo), D.zhi - 1);
+  const gfloat *flam = G(D.lam) + mb, *fmu = G(D.mu) + mb;
+  const PmlBase<gT> B = pml_base<gT>(D, zc, 3);
+  const unsigned ob = (unsigned)at.ei * E + syb * (unsigned)at.ej, o = ob + 2 * szb;
+  const unsigned om = (unsigned)pair_edge(D, at.ei) * 4u + (unsigned)D.sy * 4u * (unsigned)min(max(at.ej, D.ylo), D.yhi - 1);
+  const unsigned ym2 = o - 2 * syb, ym1 = o - syb, yp1 = o + syb, yp2 = o + 2 * syb;
+  const unsigned zm1 = ob + szb, zp1 = o + szb, zp2 = o + 2 * szb;
+  const bool ixa = (D.axes & 1) && (at.ei < D.xlo || at.ei >= D.xhi);
+  const bool ixb = (D.axes & 1) && (at.ei + 1 < D.xlo || at.ei + 1 >= D.xhi);
+  const bool iy = (D.axes & 2) && (at.ej < D.ylo || at.ej >= D.yhi);
+  const bool iz = D.axes & 4;
+  const F2 x0 = ldp(vx, o), xm = ldp(vx, o, -2), xp = ldp(vx, o, 2);
+  const F2 y0 = ldp(vy, o), yxm = ldp(vy, o, -2), yxp = ldp(vy, o, 2);
+  const F2 z0 = ldp(vz, o), zxm = ldp(vz, o, -2), zxp = ldp(vz, o, 2);
+  const F2 xym = ldp(vx, ym1), xy1 = ldp(vx, yp1), xy2 = ldp(vx, yp2);
+  const F2 yym2 = ldp(vy, ym2), yym1 = ldp(vy, ym1), yy1 = ldp(vy, yp1);
+  const F2 zym = ldp(vz, ym1), zy1 = ldp(vz, yp1), zy2 = ldp(vz, yp2);
+  const F2 xzm = ldp(vx, zm1), xz1 = ldp(vx, zp1), xz2 = ldp(vx, zp2);
+  const F2 yzm = ldp(vy, zm1), yz1 = ldp(vy, zp1), yz2 = ldp(vy, zp2);
+  const F2 zzm2 = ldp(vz, ob), zzm1 = ldp(vz, zm1), zz1 = ldp(vz, zp1);
+  const F2 lm = ldp(flam, om), mu = ldp(fmu, om);
+  F2 oxx = ldp(fsxx, o), oyy = ldp(fsyy, o), ozz = ldp(fszz, o);
+  const F2 oxy = ldp(fsxy, o), oxz = ldp(fsxz, o), oyz = ldp(fsyz, o);
+  F2 oau{0.f, 0.f};
+  if constexpr (WITH_SAU) oau = ldp(fsau, o);
+  PsiPair mx, my, mz;
+  if (ixa || ixb) mx = psi_pair(B.px, B.qx, B.ncell, at.c, B.cx_row ? at.cx : at.c);
+  if (iy) my = psi_pair(B.py, B.qy, B.ncell, at.c, at.c);
+  if (iz) mz = psi_pair(B.pz, B.qz, B.ncell, at.c, at.c);
+  if constexpr (SRC) {
+    add_source<gT>(src, at.ei, at.ej, ek, oxx.a, oyy.a, ozz.a);
+    add_source<gT>(src, at.ei + 1, at.ej, ek, oxx.b, oyy.b, ozz.b);
+  }
+  float xa0 = d2(x0.a, xm.b, x0.b, xm.a, c0, c1), xb0 = d2(x0.b, x0.a, xp.a, xm.b, c0, c1);       // vx_x
+  float xa1 = d2(y0.b, y0.a, yxp.a, yxm.b, c0, c1), xb1 = d2(yxp.a, y0.b, yxp.b, y0.a, c0, c1);   // vy_x
+  float xa2 = d2(z0.b, z0.a, zxp.a, zxm.b, c0, c1), xb2 = d2(zxp.a, z0.b, zxp.b, z0.a, c0, c1);   // vz_x
+  float ya0 = d2(xy1.a, x0.a, xy2.a, xym.a, c0, c1), yb0 = d2(xy1.b, x0.b, xy2.b, xym.b, c0, c1);      // vx_y
+  float ya1 = d2(y0.a, yym1.a, yy1.a, yym2.a, c0, c1), yb1 = d2(y0.b, yym1.b, yy1.b, yym2.b, c0, c1);  // vy_y
+  float ya2 = d2(zy1.a, z0.a, zy2.a, zym.a, c0, c1), yb2 = d2(zy1.b, z0.b, zy2.b, zym.b, c0, c1);      // vz_y
+  float za0 = d2(xz1.a, x0.a, xz2.a, xzm.a, c0, c1), zb0 = d2(xz1.b, x0.b, xz2.b, xzm.b, c0, c1);      // vx_z
+  float za1 = d2(yz1.a, y0.a, yz2.a, yzm.a, c0, c1), zb1 = d2(yz1.b, y0.b, yz2.b, yzm.b, c0, c1);      // vy_z
+  float za2 = d2(z0.a, zzm1.a, zz1.a, zzm2.a, c0, c1), zb2 = d2(z0.b, zzm1.b, zz1.b, zzm2.b, c0, c1);  // vz_z
+  div9(xa0, xa1, xa2, ya0, ya1, ya2, za0, za1, za2, dx, dy, dz, D.rdx, D.rdy, D.rdz);
+  div9(xb0, xb1, xb2, yb0, yb1, yb2, zb0, zb1, zb2, dx, dy, dz, D.rdx, D.rdy, D.rdz);
+  float pa[3][3], pc[3][3];
+  if (ixa) psi_step<gT, 6>(mx.qa, mx.m0.a, mx.m1.a, mx.m2.a, xa0, xa1, xa2, pa[0]);
+  if (ixb) psi_step<gT, 6>(mx.qb, mx.m0.b, mx.m1.b, mx.m2.b, xb0, xb1, xb2, pc[0]);
+  if (iy) {
+    psi_step<gT, 5>(my.qa, my.m0.a, my.m1.a, my.m2.a, ya0, ya1, ya2, pa[1]);
+    psi_step<gT, 5>(my.qb, my.m0.b, my.m1.b, my.m2.b, yb0, yb1, yb2, pc[1]);
+  }
+  if (iz) {
+    psi_step<gT, 3>(mz.qa, mz.m0.a, mz.m1.a, mz.m2.a, za0, za1, za2, pa[2]);
+    psi_step<gT, 3>(mz.qb, mz.m0.b, mz.m1.b, mz.m2.b, zb0, zb1, zb2, pc[2]);
+  }
+  const float la = lm.a + 2.0f * mu.a, lb = lm.b + 2.0f * mu.b;
+  const int mxm = at.m & ((ixa ? 1 : 0) | (ixb ? 2 : 0));
+  if (mxm) psi_pair_store(B.px, B.ncell, at.c, pa[0], pc[0], mxm);
+  if (iy) psi_pair_store(B.py, B.ncell, at.c, pa[1], pc[1], at.m);
+  if (iz) psi_pair_store(B.pz, B.ncell, at.c, pa[2], pc[2], at.m);
+  stp(fsxx, o, oxx.a + dt * (la * xa0 + lm.a * ya1 + lm.a * za2), oxx.b + dt * (lb * xb0 + lm.b * yb1 + lm.b * zb2),
+      at.m);
+  stp(fsyy, o, oyy.a + dt * (lm.a * xa0 + la * ya1 + lm.a * za2), oyy.b + dt * (lm.b * xb0 + lb * yb1 + lm.b * zb2),
+      at.m);
+  stp(fszz, o, ozz.a + dt * (lm.a * xa0 + lm.a * ya1 + la * za2), ozz.b + dt * (lm.b * xb0 + lm.b * yb1 + lb * zb2),
+      at.m);
+  if constexpr (WITH_SAU)
+    stp(fsau, o, oau.a + dt * (la * xa0 + la * ya1 + la * za2), oau.b + dt * (lb * xb0 + lb * yb1 + lb * zb2), at.m);
+  stp(fsxy, o, oxy.a + dt * mu.a * (xa1 + ya0), oxy.b + dt * mu.b * (xb1 + yb0), at.m);
+  stp(fsxz, o, oxz.a + dt * mu.a * (xa2 + za0), oxz.b + dt * mu.b * (xb2 + zb0), at.m);
+  stp(fsyz, o, oyz.a + dt * mu.a * (ya2 + za1), oyz.b + dt * mu.b * (yb2 + zb1), at.m);
+}
+
+template <class S>
+__global__ __launch_bounds__(kBlock) DDX_PML_ATTR void k_vel_pml_p(const SlabDesc *__restrict__ descs,
+                                                      const int *__restrict__ starts, int n, float dx, float dy,
+                                                      float dz, float rv, int grp, PmlOrder ord) {
+  int di, zc, tile;
+  if (!pml_block(descs, starts, n, blockIdx.x, gridDim.x, grp, ord, kPmlPairs, di, zc, tile)) return;
+  vel_pml_pair<S>(descs[di], zc, tile, dx, dy, dz, rv);
+}
+
+template <int WITH_SAU, class S>
+__global__ __launch_bounds__(kBlock) DDX_PML_ATTR void k_stress_pml_p(const SlabDesc *__restrict__ descs,
+                                                         const int *__restrict__ starts, int n, float dx, float dy,
+                                                         float dz, float dt, int grp, PmlOrder ord) {
+  int di, zc, tile;
+  if (!pml_block(descs, starts, n, blockIdx.x, gridDim.x, grp, ord, kPmlPairs, di, zc, tile)) return;
+  stress_pml_pair<WITH_SAU, S>(descs[di], zc, tile, dx, dy, dz, dt);
+}
 
 // ---------------------------------------------------------------------------
 // CPML halves on LDS-staged plane tiles (FP32 storage; work split
@@ -2424,13 +2761,13 @@ __global__ __launch_bounds__(kBlock) DDX_PML_ATTR void k_vel_pml_t(const SlabDes
   if (!pml_block(descs, starts, n, blockIdx.x, gridDim.x, grp, ord, kPmlTiled + P, di, zc, tile)) return;
   const SlabDesc &D = descs[di];
   const PmlTile T = pml_tile(D, zc, tile, P);
-  const long ncell = (long)D.ni * D.nj * D.nk;
-  const int plane = D.ni * D.nj;
+  const long ncell = (long)D.ip * D.nj * D.nk;
+  const int plane = D.ip * D.nj;
   const int sy = (int)D.sy;
   const long sz = D.sz;
   const long tb0 = (long)(D.i0 + T.x0) + D.sy * (D.j0 + T.y0) + sz * (D.k0 + T.kc0);  // tile origin
   const long id0 = tb0 + T.tx + (long)T.ty * sy;                                       // this cell
-  const long c00 = (long)(T.x0 + T.tx) + (long)D.ni * (T.y0 + T.ty) + (long)plane * T.kc0;
+  const long c00 = (long)(D.sh + T.x0 + T.tx) + (long)D.ip * (T.y0 + T.ty) + (long)plane * T.kc0;
   const int ei = D.i0 + T.x0 + T.tx, ej = D.j0 + T.y0 + T.ty;
   const int t = (int)threadIdx.x;
   const TileSlot x12 = tile_slot(t, true, 1, 2, T.w, T.h, T.px, sy);
@@ -2589,13 +2926,13 @@ __global__ __launch_bounds__(kBlock) DDX_PML_ATTR void k_stress_pml_t(const Slab
   if (!pml_block(descs, starts, n, blockIdx.x, gridDim.x, grp, ord, kPmlTiled + P, di, zc, tile)) return;
   const SlabDesc &D = descs[di];
   const PmlTile T = pml_tile(D, zc, tile, P);
-  const long ncell = (long)D.ni * D.nj * D.nk;
-  const int plane = D.ni * D.nj;
+  const long ncell = (long)D.ip * D.nj * D.nk;
+  const int plane = D.ip * D.nj;
   const int sy = (int)D.sy;
   const long sz = D.sz;
   const long tb0 = (long)(D.i0 + T.x0) + D.sy * (D.j0 + T.y0) + sz * (D.k0 + T.kc0);
   const long id0 = tb0 + T.tx + (long)T.ty * sy;
-  const long c00 = (long)(T.x0 + T.tx) + (long)D.ni * (T.y0 + T.ty) + (long)plane * T.kc0;
+  const long c00 = (long)(D.sh + T.x0 + T.tx) + (long)D.ip * (T.y0 + T.ty) + (long)plane * T.kc0;
   const int ei = D.i0 + T.x0 + T.tx, ej = D.j0 + T.y0 + T.ty;
   const int t = (int)threadIdx.x;
   const TileSlot x12 = tile_slot(t, true, 1, 2, T.w, T.h, T.px, sy);
@@ -2776,7 +3113,7 @@ __device__ __forceinline__ void recv_block(const StepIO &io, int b) {
 // gaps; what each block does is what the separate kernels do.  Where it pays
 // and where not: kWholeCells in engine.cpp.  A modelling step is two launches
 // instead of six: 32x28x24 cells 31.8 -> 15.2 us per step, 64^3 with 20
-// layers 66 -> 52 us, 100^3 with 10 layers 96 -> 76 us.
+// layers 66 -> 51 us, 100^3 with 10 layers 96 -> 75 us.
 // ---------------------------------------------------------------------------
 enum { FORM_ONE = 0, FORM_PAIR = 2, FORM_YL = 4 };
 template <int FORM, int MODE, int TX, int TY, int CZ, class S>
@@ -2785,8 +3122,11 @@ __global__ __launch_bounds__(kBlock) void k_vel_all(HalfStep a) {
   if ((int)blockIdx.x >= a.nphy) {
     int di, zc, tile;
     const PmlOrder ord{};
-    if (pml_block(a.slabs, a.sstarts, a.ns, blockIdx.x - a.nphy, a.npml, a.pgrp, ord, 1, di, zc, tile))
-      vel_pml_body<1, S>(a.slabs[di], zc, tile, a.dx, a.dy, a.dz, a.sc);
+    if (pml_block(a.slabs, a.sstarts, a.ns, blockIdx.x - a.nphy, a.npml, a.pgrp, ord,
+                  pml_whole(kF32<S> ? STORE_F32 : STORE_F16), di, zc, tile)) {
+      if constexpr (kF32<S>) vel_pml_body<1, S>(a.slabs[di], zc, tile, a.dx, a.dy, a.dz, a.sc);
+      else vel_pml_pair<S>(a.slabs[di], zc, tile, a.dx, a.dy, a.dz, a.sc);
+    }
     return;
   }
   const int grp = a.grp, b = brick_block(blockIdx.x, a.nphy, grp);
@@ -2816,9 +3156,14 @@ __global__ __launch_bounds__(kBlock) void k_stress_all(HalfStep a, StepIO io) {
     }
     int di, zc, tile;
     const PmlOrder ord{};
-    if (pml_block(a.slabs, a.sstarts, a.ns, blockIdx.x - a.nphy, a.npml, a.pgrp, ord, 1, di, zc, tile))
-      stress_pml_body<rtm_mode(MODE), 1, S, true>(a.slabs[di], zc, tile, a.dx, a.dy, a.dz, a.sc,
-                                                  src_cell<S>(io, a.slabs[di].io));
+    if (pml_block(a.slabs, a.sstarts, a.ns, blockIdx.x - a.nphy, a.npml, a.pgrp, ord,
+                  pml_whole(kF32<S> ? STORE_F32 : STORE_F16), di, zc, tile)) {
+      const SrcCell src = src_cell<S>(io, a.slabs[di].io);
+      if constexpr (kF32<S>)
+        stress_pml_body<rtm_mode(MODE), 1, S, true>(a.slabs[di], zc, tile, a.dx, a.dy, a.dz, a.sc, src);
+      else
+        stress_pml_pair<rtm_mode(MODE), S, true>(a.slabs[di], zc, tile, a.dx, a.dy, a.dz, a.sc, src);
+    }
     return;
   }
   const int grp = a.grp, b = brick_block(blockIdx.x, a.nphy, grp);
@@ -3706,6 +4051,17 @@ static void vel_pml_launch(const SlabDesc *d, const int *starts, int n, int grid
   hipLaunchKernelGGL((k_vel_pml<C, S>), dim3(grid), dim3(kBlock), 0, st, d, starts, n, dx, dy, dz, rv, grp, o);
 }
 
+template <class S>
+static void vel_pml_p_launch(const SlabDesc *d, const int *starts, int n, int grid, float dx, float dy, float dz,
+                             float rv, int grp, const PmlOrder &o, hipStream_t st) {
+  hipLaunchKernelGGL(k_vel_pml_p<S>, dim3(grid), dim3(kBlock), 0, st, d, starts, n, dx, dy, dz, rv, grp, o);
+}
+template <int W, class S>
+static void stress_pml_p_launch(const SlabDesc *d, const int *starts, int n, int grid, float dx, float dy, float dz,
+                                float dt, int grp, const PmlOrder &o, hipStream_t st) {
+  hipLaunchKernelGGL((k_stress_pml_p<W, S>), dim3(grid), dim3(kBlock), 0, st, d, starts, n, dx, dy, dz, dt, grp, o);
+}
+
 // The grid of a CPML launch: the table's blocks, or 8 x the largest XCD
 // share of the XCD-partitioned order.
 static int pml_grid(int nblk, const PmlOrder *ord, PmlOrder &o) {
@@ -3723,8 +4079,7 @@ static void vel_pml_t_launch(const SlabDesc *d, const int *starts, int n, int gr
   hipLaunchKernelGGL((k_vel_pml_t<P>), dim3(grid), dim3(kBlock), 0, st, d, starts, n, dx, dy, dz, grp, o);
 }
 
-// The 16-bit formats run one cell per thread (cz is ignored for them; the
-// tables of a 16-bit context are built for cz = 1).
+// The 16-bit formats run pairs (their tables are built for that split).
 void launch_vel_pml(int cz, int fmt, const SlabDesc *d, const int *starts, int n, int nblk, float dx, float dy,
                     float dz, float rv, int grp, const PmlOrder *ord, hipStream_t st) {
   if (nblk <= 0) return;
@@ -3733,10 +4088,11 @@ void launch_vel_pml(int cz, int fmt, const SlabDesc *d, const int *starts, int n
   if (grid <= 0) return;
   void (*f)(const SlabDesc *, const int *, int, int, float, float, float, float, int, const PmlOrder &,
             hipStream_t);
-  if (fmt == STORE_F32 && pml_tiled(cz))
+  if (fmt == STORE_F16) f = vel_pml_p_launch<F16>;
+  else if (fmt == STORE_BF16) f = vel_pml_p_launch<BF16>;
+  else if (cz == kPmlPairs) f = vel_pml_p_launch<F32>;
+  else if (pml_tiled(cz))
     f = cz == kPmlTiled + 2 ? vel_pml_t_launch<2> : cz == kPmlTiled + 4 ? vel_pml_t_launch<4> : vel_pml_t_launch<8>;
-  else if (fmt == STORE_F16) f = vel_pml_launch<1, F16>;
-  else if (fmt == STORE_BF16) f = vel_pml_launch<1, BF16>;
   else f = cz == 1 ? vel_pml_launch<1, F32> : cz == 2 ? vel_pml_launch<2, F32>
            : cz == 4 ? vel_pml_launch<4, F32> : vel_pml_launch<8, F32>;
   f(d, starts, n, grid, dx, dy, dz, rv, grp, o, st);
@@ -3756,7 +4112,6 @@ static void stress_pml_t_launch(const SlabDesc *d, const int *starts, int n, int
   hipLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), 0, st, d, starts, n, dx, dy, dz, dt, grp, o);
 }
 
-// The 16-bit formats run one cell per thread (cz is ignored for them).
 void launch_stress_pml(int cz, int with_sau, int fmt, const SlabDesc *d, const int *starts, int n, int nblk,
                        float dx, float dy, float dz, float dt, int grp, const PmlOrder *ord, hipStream_t st) {
   if (nblk <= 0) return;
@@ -3765,18 +4120,17 @@ void launch_stress_pml(int cz, int with_sau, int fmt, const SlabDesc *d, const i
   if (grid <= 0) return;
   void (*f)(const SlabDesc *, const int *, int, int, float, float, float, float, int, const PmlOrder &,
             hipStream_t);
-  if (fmt == STORE_F32 && pml_tiled(cz)) {
+  if (fmt == STORE_F16) f = with_sau ? stress_pml_p_launch<1, F16> : stress_pml_p_launch<0, F16>;
+  else if (fmt == STORE_BF16) f = with_sau ? stress_pml_p_launch<1, BF16> : stress_pml_p_launch<0, BF16>;
+  else if (cz == kPmlPairs) f = with_sau ? stress_pml_p_launch<1, F32> : stress_pml_p_launch<0, F32>;
+  else if (pml_tiled(cz)) {
     if (with_sau)
       f = cz == kPmlTiled + 2 ? stress_pml_t_launch<1, 2> : cz == kPmlTiled + 4 ? stress_pml_t_launch<1, 4>
           : stress_pml_t_launch<1, 8>;
     else
       f = cz == kPmlTiled + 2 ? stress_pml_t_launch<0, 2> : cz == kPmlTiled + 4 ? stress_pml_t_launch<0, 4>
           : stress_pml_t_launch<0, 8>;
-  } else if (fmt == STORE_F16)
-    f = with_sau ? stress_pml_launch<1, 1, F16> : stress_pml_launch<0, 1, F16>;
-  else if (fmt == STORE_BF16)
-    f = with_sau ? stress_pml_launch<1, 1, BF16> : stress_pml_launch<0, 1, BF16>;
-  else if (with_sau)
+  } else if (with_sau)
     f = cz == 1 ? stress_pml_launch<1, 1, F32> : cz == 2 ? stress_pml_launch<1, 2, F32>
         : cz == 4 ? stress_pml_launch<1, 4, F32> : stress_pml_launch<1, 8, F32>;
   else

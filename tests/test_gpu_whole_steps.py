@@ -92,6 +92,32 @@ def test_whole_batches_equal_separate_kernels(monkeypatch):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("grid", [(75, 21, 19, 6), (20, 9, 8, 4), (33, 10, 9, 5), (512, 9, 8, 5)])
+def test_cpml_pairs_equal_one_cell_kernels(grid, monkeypatch):
+    """Two x cells per thread against one: rows that begin or end inside a
+    pair, slabs two cells thick, damping edges inside a pair, rows of more
+    pairs than a block."""
+    nx, ny, nz, pml = grid
+    c = case(nx=nx, ny=ny, nz=nz, pml=pml, rec_width=2)
+    monkeypatch.setenv("DDX_WHOLE_CELLS", "0")
+    outs = []
+    for cz in ("1", "0"):
+        monkeypatch.setenv("DDX_PML_CZ", cz)
+        e = engine(c)
+        e.set_migration_model(c["vp"][::-1, ::-1, ::-1].copy(), c["vs"][::-1, ::-1, ::-1].copy(),
+                              c["rho"][::-1, ::-1, ::-1].copy())
+        for f, arr in enumerate(random_fields(e.ext_shape, seed=23, scale=1e-3)):
+            e.set(0, f, arr)
+        for m in (po.PURE_FORWARD, po.RTM_FORWARD, po.RTM_REVERSE):
+            for _ in range(2):
+                e.step_vel(0, m)
+                e.step_stress(0, m)
+        outs.append([e.get(0, f) for f in range(13)])
+        e.close()
+    for f, (a, b) in enumerate(zip(*outs)):
+        assert np.array_equal(a, b), ddx.FIELD_NAMES[f]
+
+
 @pytest.mark.parametrize("spacing", [(10.0, 10.0, 10.0), (7.3, 12.9, 0.3), (8.0, 1000.0, 3.0)])
 def test_cpml_division_is_exact_at_every_magnitude(spacing, monkeypatch):
     """The one-cell CPML kernels divide by the spacing in three operations
