@@ -34,7 +34,7 @@ COMMON = [
     "-Wall", "-Wno-unused-function", "-Wno-unused-variable", "-Wno-unused-command-line-argument",
 ]
 # kernels.hip once per family of kernels (DDX_PART), so that they compile in parallel
-PARTS = 12
+PARTS = 14
 SOURCES = [("kernels.hip", p) for p in range(PARTS)] + [("engine.cpp", None)]
 
 

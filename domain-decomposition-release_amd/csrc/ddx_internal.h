@@ -146,8 +146,11 @@ struct CopyDesc {
   long buf_off;
   int cls;   // field class (0 velocity, 1 stress): the scale of a converting copy
   int fid;   // ring field index (0..9): the per-slice scale of a converting copy
+  int io;    // member of a fused launch (StepIO)
   int blk0;
 };
+// How a boundary store holds its values (RING_F16, RING_BF16: converted, scaled).
+enum : int { RING_COPY4, RING_COPY2, RING_F16, RING_BF16, RING_BFP };
 
 // Imaging over one subdomain's gridphy.
 struct ImgDesc {
@@ -204,6 +207,13 @@ struct MemberIO {
   float sv;               // velocity-class scale (receiver injection of the 16-bit formats)
   int join, ntime;
   int rev;                // 0: time index = batch step - join; 1: join - batch step (a reverse loop)
+  // the member's boundary store (k_rev_vel, k_rev_stress)
+  const float *store;     // [ring_slices][ring_slice], by ring_kind
+  long ring_slice, ring_runs;
+  int ring_slices, ring_kind;
+  float ring_sv, ring_ss;         // class scales of a converted store
+  const int *store_exp;           // per-slice scales instead (nullptr: the class scales)
+  const signed char *store_bexp;  // run exponents of a block-scaled store
   int blk0;               // first block of this member's receivers
 };
 
@@ -217,6 +227,7 @@ struct StepIO {
   int n = 0, nblk = 0;
   int gs = 0;
   const int *gsp = nullptr;
+  float sign = 1.f;  // of the sources
 };
 
 // A half step of the physical region and the CPML cells in one launch.
@@ -230,6 +241,19 @@ struct HalfStep {
   float dx, dy, dz, sc;  // sc: as sign / dt of the separate kernels
   float sx, sy, sz;      // sc over dx, dy, dz
   int grp, pgrp;
+};
+// The backward bricks of half a reverse iteration (sc, sx, sy, sz as HalfStep).
+struct BackBricks {
+  const PhyDesc *phy;
+  const int *starts;
+  int n, nblk;
+  float sc, sx, sy, sz;
+};
+// Boundary-store boxes to inject, of the members of a StepIO.
+struct RingBoxes {
+  const CopyDesc *d;
+  const int *starts;
+  int n, nblk;
 };
 
 // ---- launchers (kernels.hip) ----
@@ -250,6 +274,15 @@ bool launch_stress_phy(const Tiling &t, int mode, int fmt, const PhyDesc *d, con
 bool whole_shape(const Tiling &t, int fmt);  // the shapes they exist for
 bool launch_vel_all(const Tiling &t, int mode, int fmt, const HalfStep &a, hipStream_t st);
 bool launch_stress_all(const Tiling &t, int mode, int fmt, const HalfStep &a, const StepIO &io, hipStream_t st);
+// The halves of a reverse iteration, one launch each, in the shapes of
+// whole_shape: the reverse set's half step a, the backward set's bricks q (of
+// the same shape; stress next to the velocity half step and the other way
+// round) and boxes rb; io: the members, their sources subtracted by the
+// backward stress.  False, launching nothing, as launch_vel_all.
+bool launch_rev_vel(const Tiling &t, int fmt, const HalfStep &a, const BackBricks &q, const StepIO &io,
+                    const RingBoxes &rb, hipStream_t st);
+bool launch_rev_stress(const Tiling &t, int fmt, const HalfStep &a, const BackBricks &q, const StepIO &io,
+                       const RingBoxes &rb, hipStream_t st);
 // grp: blocks per XCD group of the group-interleaved block order (0: launch order)
 // ord (nullable): the XCD-partitioned block order of the table; without it
 // (or with ord->pieces null) the blocks follow the table's own order.

@@ -298,7 +298,7 @@ __device__ __forceinline__ SrcCell src_cell(const StepIO &io, int q) {
   if (it >= 0 && it < m->ntime) {
     c.x = m->src_x; c.y = m->src_y; c.z = m->src_z;
     c.all = m->src_mode == 0;
-    c.w = std::is_same<S, F32>::value ? m->wavelet[it] : m->wavelet[it] * m->ss;
+    c.w = (std::is_same<S, F32>::value ? m->wavelet[it] : m->wavelet[it] * m->ss) * io.sign;
   }
   return c;
 }
@@ -3116,26 +3116,29 @@ __device__ __forceinline__ void recv_block(const StepIO &io, int b) {
 // layers 66 -> 51 us, 100^3 with 10 layers 96 -> 75 us.
 // ---------------------------------------------------------------------------
 enum { FORM_ONE = 0, FORM_PAIR = 2, FORM_YL = 4 };
+struct NoLds {};
+template <int FORM, int NF, int TY, int CZ>
+using YlLds = typename std::conditional<FORM == FORM_YL, YlTile<NF, TY, CZ>, NoLds>::type;
 template <int FORM, int MODE, int TX, int TY, int CZ, class S>
-__global__ __launch_bounds__(kBlock) void k_vel_all(HalfStep a) {
+__device__ __forceinline__ void vel_all_block(const HalfStep &a, int blk, void *lds) {
   static_assert(TX * TY == kBlock, "the bricks and the CPML cells share a block size");
-  if ((int)blockIdx.x >= a.nphy) {
+  if (blk >= a.nphy) {
     int di, zc, tile;
     const PmlOrder ord{};
-    if (pml_block(a.slabs, a.sstarts, a.ns, blockIdx.x - a.nphy, a.npml, a.pgrp, ord,
+    if (pml_block(a.slabs, a.sstarts, a.ns, blk - a.nphy, a.npml, a.pgrp, ord,
                   pml_whole(kF32<S> ? STORE_F32 : STORE_F16), di, zc, tile)) {
       if constexpr (kF32<S>) vel_pml_body<1, S>(a.slabs[di], zc, tile, a.dx, a.dy, a.dz, a.sc);
       else vel_pml_pair<S>(a.slabs[di], zc, tile, a.dx, a.dy, a.dz, a.sc);
     }
     return;
   }
-  const int grp = a.grp, b = brick_block(blockIdx.x, a.nphy, grp);
+  const int grp = a.grp, b = brick_block(blk, a.nphy, grp);
   const PhyDesc &D = a.phy[find_desc(a.pstarts, a.np, b)];
   int i, j0, k0;
   if constexpr (FORM == FORM_YL) {
-    __shared__ YlTile<(MODE == RTM_BACKWARD || MODE == RTM_REVERSE) ? 4 : 3, TY, CZ> ly;
-    const TileAt at = tile_at<64, TY * 1>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp);
-  const bool live = zbrick<64, TY, 1, CZ>(D, at, i, j0, k0);
+    auto &ly = *(YlTile<MODE == RTM_REVERSE ? 4 : 3, TY, CZ> *)lds;
+    const TileAt at = tile_at<64, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp);
+    const bool live = zbrick<64, TY, 1, CZ>(D, at, i, j0, k0);
     vel_yl_body<MODE, TY, CZ, S>(ly, D, i, j0, k0, a.dx, a.dy, a.dz, a.sc, live);
   } else if constexpr (FORM == FORM_PAIR) {
     if (zbrick2<TX, TY, 1, CZ>(D, tile_at<2 * TX, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp), i, j0, k0))
@@ -3147,16 +3150,22 @@ __global__ __launch_bounds__(kBlock) void k_vel_all(HalfStep a) {
 }
 
 template <int FORM, int MODE, int TX, int TY, int CZ, class S>
-__global__ __launch_bounds__(kBlock) void k_stress_all(HalfStep a, StepIO io) {
+__global__ __launch_bounds__(kBlock) void k_vel_all(HalfStep a) {
+  __shared__ YlLds<FORM, MODE == RTM_REVERSE ? 4 : 3, TY, CZ> lds;
+  vel_all_block<FORM, MODE, TX, TY, CZ, S>(a, blockIdx.x, &lds);
+}
+
+template <int FORM, int MODE, int TX, int TY, int CZ, class S>
+__device__ __forceinline__ void stress_all_block(const HalfStep &a, const StepIO &io, int blk, void *lds) {
   static_assert(TX * TY == kBlock, "the bricks and the CPML cells share a block size");
-  if ((int)blockIdx.x >= a.nphy) {
-    if ((int)blockIdx.x >= a.nphy + a.npml) {
-      recv_block<S>(io, blockIdx.x - a.nphy - a.npml);
+  if (blk >= a.nphy) {
+    if (blk >= a.nphy + a.npml) {
+      recv_block<S>(io, blk - a.nphy - a.npml);
       return;
     }
     int di, zc, tile;
     const PmlOrder ord{};
-    if (pml_block(a.slabs, a.sstarts, a.ns, blockIdx.x - a.nphy, a.npml, a.pgrp, ord,
+    if (pml_block(a.slabs, a.sstarts, a.ns, blk - a.nphy, a.npml, a.pgrp, ord,
                   pml_whole(kF32<S> ? STORE_F32 : STORE_F16), di, zc, tile)) {
       const SrcCell src = src_cell<S>(io, a.slabs[di].io);
       if constexpr (kF32<S>)
@@ -3166,14 +3175,14 @@ __global__ __launch_bounds__(kBlock) void k_stress_all(HalfStep a, StepIO io) {
     }
     return;
   }
-  const int grp = a.grp, b = brick_block(blockIdx.x, a.nphy, grp);
+  const int grp = a.grp, b = brick_block(blk, a.nphy, grp);
   const PhyDesc &D = a.phy[find_desc(a.pstarts, a.np, b)];
   const SrcCell src = src_cell<S>(io, D.io);
   int i, j0, k0;
   if constexpr (FORM == FORM_YL) {
-    __shared__ YlTile<3, TY, CZ> ly;
-    const TileAt at = tile_at<64, TY * 1>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp);
-  const bool live = zbrick<64, TY, 1, CZ>(D, at, i, j0, k0);
+    auto &ly = *(YlTile<3, TY, CZ> *)lds;
+    const TileAt at = tile_at<64, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp);
+    const bool live = zbrick<64, TY, 1, CZ>(D, at, i, j0, k0);
     stress_yl_body<MODE, TY, CZ, S, true>(ly, D, i, j0, k0, a.sx, a.sy, a.sz, live, src);
   } else if constexpr (FORM == FORM_PAIR) {
     if (zbrick2<TX, TY, 1, CZ>(D, tile_at<2 * TX, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp), i, j0, k0))
@@ -3182,6 +3191,122 @@ __global__ __launch_bounds__(kBlock) void k_stress_all(HalfStep a, StepIO io) {
     if (zbrick<TX, TY, 1, CZ>(D, tile_at<TX, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp), i, j0, k0))
       stress_zb_body<MODE, TX, TY, 1, CZ, S, false, true>(D, i, j0, k0, a.sx, a.sy, a.sz, true, src);
   }
+}
+
+template <int FORM, int MODE, int TX, int TY, int CZ, class S>
+__global__ __launch_bounds__(kBlock) void k_stress_all(HalfStep a, StepIO io) {
+  __shared__ YlLds<FORM, 3, TY, CZ> lds;
+  stress_all_block<FORM, MODE, TX, TY, CZ, S>(a, io, blockIdx.x, &lds);
+}
+
+typedef __attribute__((address_space(1))) short gshort;
+// The value of a code of the block-scaled boundary store (format: k_save_bfp), run exponent s.
+__device__ __forceinline__ float bfp_value(short q, int s) {
+  const int c = q < 0 ? -(int)q : (int)q;
+  const float u = c < 4096 ? ldexpf((float)c, -19) : ldexpf((float)(4096 + (c & 4095)), (c >> 12) - 20);
+  return ldexpf(q < 0 ? -u : u, s);
+}
+
+// ---------------------------------------------------------------------------
+// The two halves of a reverse iteration, each one launch: the backward
+// (source) set's bricks and boundary-store boxes next to the reverse
+// (receiver) set's bricks and CPML cells.
+//   k_rev_vel: backward stress and its boxes, reverse velocity;
+//   k_rev_stress: backward velocity and its boxes, reverse stress.
+// The sets do not meet, and the boxes lie outside the region that the
+// backward bricks update and hold fields that they do not read.  The brick
+// that owns the source cell subtracts the sample.  Blocks: the backward
+// bricks [0, nb), then as k_vel_all / k_stress_all, then the boxes'.
+// What bounds a reverse iteration of a small grid beyond its bytes is the
+// launches' tails and the 4.7 us of each small one (source, two injections).
+// 88^3 with 20 layers: 75 + 81 us as nine launches, 63 + 71 as two; 141x97x75
+// with 12: 84 + 90 and 77 + 80.  Four wavefronts per SIMD are asked for, as
+// the reverse half steps alone have; it costs the (32, 8, 4) and (64, 4, 2)
+// shapes 12 and 8 bytes of scratch.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ void ring_cell(const CopyDesc &D, int e, int cnt, const MemberIO &m, int slice) {
+  if (e >= cnt) return;
+  const int r = e / D.ni;
+  const int k = r / D.nj;
+  const int i = e - r * D.ni;
+  const int j = r - k * D.nj;
+  const long id = (long)(D.i0 + i) + D.sy * (D.j0 + j) + D.sz * (D.k0 + k);
+  const long at = (long)slice * m.ring_slice + D.buf_off + e;  // the box's element in the store
+  switch (m.ring_kind) {
+    case RING_COPY4: G(D.field)[id] = G(m.store)[at]; break;
+    case RING_COPY2: ((gshort *)D.field)[id] = ((const gshort *)m.store)[at]; break;
+    case RING_BFP: {
+      const long run = (long)slice * m.ring_runs + (D.buf_off + e) / kRingBlock;
+      G(D.field)[id] = bfp_value(((const gshort *)m.store)[at], m.store_bexp[run]);
+      break;
+    }
+    default: {
+      const float sc = m.store_exp ? ldexpf(1.0f, m.store_exp[(long)slice * 10 + D.fid]) : D.cls == 0 ? m.ring_sv : m.ring_ss;
+      const float v = m.ring_kind == RING_F16 ? ld((const ghalf *)m.store, at) : ld((const gbf16 *)m.store, at);
+      G(D.field)[id] = v * (1.0f / sc);
+    }
+  }
+}
+// Block b of the boxes of an iteration: the slice of the step before the member's own.
+__device__ __forceinline__ void ring_block(const StepIO &io, const RingBoxes &r, int b) {
+  const CopyDesc &D = r.d[find_desc(r.starts, r.n, b)];
+  const MemberIO &m = io.io[D.io];
+  const int slice = (m.rev ? m.join - io.gs : io.gs - m.join) - 1;
+  if (slice < 0 || slice >= m.ring_slices) return;
+  ring_cell(D, (b - D.blk0) * kBlock + (int)threadIdx.x, D.ni * D.nj * D.nk, m, slice);
+}
+
+template <int FORM, int TX, int TY, int CZ, class S>
+__global__ __launch_bounds__(kBlock, kF32<S> ? 4 : 2) void k_rev_vel(HalfStep a, BackBricks q, StepIO io, RingBoxes rb) {
+  __shared__ YlLds<FORM, 4, TY, CZ> lds;
+  int i, j0, k0;
+  const int grp = a.grp, blk = (int)blockIdx.x - q.nblk;
+  if (blk < 0) {
+    const int b = brick_block(blockIdx.x, q.nblk, grp);
+    const PhyDesc &D = q.phy[find_desc(q.starts, q.n, b)];
+    const SrcCell src = src_cell<S>(io, D.io);
+    if constexpr (FORM == FORM_YL) {
+      auto &ly = *(YlTile<3, TY, CZ> *)&lds;
+      const TileAt at = tile_at<64, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp);
+      const bool live = zbrick<64, TY, 1, CZ>(D, at, i, j0, k0);
+      stress_yl_body<RTM_BACKWARD, TY, CZ, S, true>(ly, D, i, j0, k0, q.sx, q.sy, q.sz, live, src);
+    } else if constexpr (FORM == FORM_PAIR) {
+      if (zbrick2<TX, TY, 1, CZ>(D, tile_at<2 * TX, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp), i, j0, k0))
+        stress_zb2_body<RTM_BACKWARD, TX, TY, 1, CZ, S, true>(D, i, j0, k0, q.sx, q.sy, q.sz, src);
+    } else {
+      if (zbrick<TX, TY, 1, CZ>(D, tile_at<TX, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp), i, j0, k0))
+        stress_zb_body<RTM_BACKWARD, TX, TY, 1, CZ, S, false, true>(D, i, j0, k0, q.sx, q.sy, q.sz, true, src);
+    }
+    return;
+  }
+  if (blk >= a.nphy + a.npml) return ring_block(io, rb, blk - a.nphy - a.npml);
+  vel_all_block<FORM, RTM_REVERSE, TX, TY, CZ, S>(a, blk, &lds);
+}
+
+template <int FORM, int TX, int TY, int CZ, class S>
+__global__ __launch_bounds__(kBlock, kF32<S> ? 4 : 2) void k_rev_stress(HalfStep a, BackBricks q, StepIO io, RingBoxes rb) {
+  __shared__ YlLds<FORM, 4, TY, CZ> lds;
+  int i, j0, k0;
+  const int grp = a.grp, blk = (int)blockIdx.x - q.nblk;
+  if (blk < 0) {
+    const int b = brick_block(blockIdx.x, q.nblk, grp);
+    const PhyDesc &D = q.phy[find_desc(q.starts, q.n, b)];
+    if constexpr (FORM == FORM_YL) {
+      auto &ly = *(YlTile<4, TY, CZ> *)&lds;
+      const TileAt at = tile_at<64, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp);
+      const bool live = zbrick<64, TY, 1, CZ>(D, at, i, j0, k0);
+      vel_yl_body<RTM_BACKWARD, TY, CZ, S>(ly, D, i, j0, k0, a.dx, a.dy, a.dz, q.sc, live);
+    } else if constexpr (FORM == FORM_PAIR) {
+      if (zbrick2<TX, TY, 1, CZ>(D, tile_at<2 * TX, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp), i, j0, k0))
+        vel_zb2_body<RTM_BACKWARD, TX, TY, 1, CZ, S>(D, i, j0, k0, a.dx, a.dy, a.dz, q.sc);
+    } else {
+      if (zbrick<TX, TY, 1, CZ>(D, tile_at<TX, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp), i, j0, k0))
+        vel_zb_body<RTM_BACKWARD, TX, TY, 1, CZ, S>(D, i, j0, k0, a.dx, a.dy, a.dz, q.sc);
+    }
+    return;
+  }
+  if (blk >= a.nphy + a.npml) return ring_block(io, rb, blk - a.nphy - a.npml);
+  stress_all_block<FORM, RTM_REVERSE, TX, TY, CZ, S>(a, StepIO{}, blk, &lds);
 }
 
 #if DDX_PART == 0
@@ -3312,7 +3437,6 @@ __global__ __launch_bounds__(kBlock) void k_copy_dyn(const CopyDesc *__restrict_
 // is 2^-11); below, c = u 2^19.  The codes are monotonic in u, so a mantissa
 // that rounds up carries into the exponent.  Every scaling is by a power of
 // two and exact.
-typedef __attribute__((address_space(1))) short gshort;
 
 __device__ __forceinline__ short bfp_code(float v, int s) {
   const float u = ldexpf(fabsf(v), -s);
@@ -3328,11 +3452,6 @@ __device__ __forceinline__ short bfp_code(float v, int s) {
   return (short)(v < 0.f ? -c : c);
 }
 
-__device__ __forceinline__ float bfp_value(short q, int s) {
-  const int c = q < 0 ? -(int)q : (int)q;
-  const float u = c < 4096 ? ldexpf((float)c, -19) : ldexpf((float)(4096 + (c & 4095)), (c >> 12) - 20);
-  return ldexpf(q < 0 ? -u : u, s);
-}
 
 // Save: the save table holds whole boxes (buffer index = buf_off + the
 // cell's x-fastest index e, buf_off a multiple of kRingBlock) and a block
@@ -3846,6 +3965,16 @@ bool stress_all_16(const Tiling &t, int form, int mode, int fmt, const HalfStep 
   hipLaunchKernelGGL((k_vel_all<FORM, MODE, TX, TY, CZ, S>), dim3(a.nphy + a.npml), dim3(kBlock), 0, st, a)
 #define DDX_S(FORM, MODE, TX, TY, CZ, S) \
   hipLaunchKernelGGL((k_stress_all<FORM, MODE, TX, TY, CZ, S>), dim3(grid), dim3(kBlock), 0, st, a, io)
+bool rev_vel_32(const Tiling &t, int form, const HalfStep &a, const BackBricks &q, const StepIO &io,
+                const RingBoxes &rb, int grid, hipStream_t st);
+bool rev_vel_16(const Tiling &t, int form, int fmt, const HalfStep &a, const BackBricks &q, const StepIO &io,
+                const RingBoxes &rb, int grid, hipStream_t st);
+bool rev_stress_32(const Tiling &t, int form, const HalfStep &a, const BackBricks &q, const StepIO &io,
+                   const RingBoxes &rb, int grid, hipStream_t st);
+bool rev_stress_16(const Tiling &t, int form, int fmt, const HalfStep &a, const BackBricks &q, const StepIO &io,
+                   const RingBoxes &rb, int grid, hipStream_t st);
+#define DDX_R(K, FORM, TX, TY, CZ, S) \
+  hipLaunchKernelGGL((K<FORM, TX, TY, CZ, S>), dim3(grid), dim3(kBlock), 0, st, a, q, io, rb)
 #if DDX_PART == 9
 bool vel_all_32(const Tiling &t, int form, int mode, const HalfStep &a, hipStream_t st) {
 #define DDX_T(FORM, TX, TY, CZ)                                               \
@@ -3909,6 +4038,44 @@ bool stress_all_16(const Tiling &t, int form, int mode, int fmt, const HalfStep 
 }
 #endif
 
+#if DDX_PART == 12 || DDX_PART == 13
+#if DDX_PART == 12
+#define DDX_K k_rev_vel
+bool rev_vel_32(const Tiling &t, int form, const HalfStep &a, const BackBricks &q, const StepIO &io,
+                const RingBoxes &rb, int grid, hipStream_t st) {
+#else
+#define DDX_K k_rev_stress
+bool rev_stress_32(const Tiling &t, int form, const HalfStep &a, const BackBricks &q, const StepIO &io,
+                   const RingBoxes &rb, int grid, hipStream_t st) {
+#endif
+#define DDX_T(FORM, TX, TY, CZ)                  \
+  if (form == FORM && DDX_IS(TX, TY, 1, CZ)) {   \
+    DDX_R(DDX_K, FORM, TX, TY, CZ, F32);         \
+    return true;                                 \
+  }
+  DDX_FUSED32(DDX_T)
+#undef DDX_T
+  return false;
+}
+#if DDX_PART == 12
+bool rev_vel_16(const Tiling &t, int form, int fmt, const HalfStep &a, const BackBricks &q, const StepIO &io,
+                const RingBoxes &rb, int grid, hipStream_t st) {
+#else
+bool rev_stress_16(const Tiling &t, int form, int fmt, const HalfStep &a, const BackBricks &q, const StepIO &io,
+                   const RingBoxes &rb, int grid, hipStream_t st) {
+#endif
+#define DDX_T(FORM, TX, TY, CZ)                                     \
+  if (form == FORM && DDX_IS(TX, TY, 1, CZ)) {                      \
+    if (fmt == STORE_F16) DDX_R(DDX_K, FORM, TX, TY, CZ, F16);      \
+    else DDX_R(DDX_K, FORM, TX, TY, CZ, BF16);                      \
+    return true;                                                    \
+  }
+  DDX_FUSED16(DDX_T)
+#undef DDX_T
+  return false;
+}
+#endif
+
 #if DDX_PART == 1
 #define DDX_F vel_zb
 bool vel_one(DDX_SIG) { DDX_TILINGS(DDX_T1) return false; }
@@ -3963,6 +4130,22 @@ bool launch_stress_all(const Tiling &t, int mode, int fmt, const HalfStep &a, co
   if (grid <= 0) return true;
   return fmt == STORE_F32 ? stress_all_32(t, form_of(t), mode, a, io, grid, st)
                           : stress_all_16(t, form_of(t), mode, fmt, a, io, grid, st);
+}
+
+bool launch_rev_vel(const Tiling &t, int fmt, const HalfStep &a, const BackBricks &q, const StepIO &io,
+                    const RingBoxes &rb, hipStream_t st) {
+  const int grid = q.nblk + a.nphy + a.npml + rb.nblk;
+  if (grid <= 0) return true;
+  return fmt == STORE_F32 ? rev_vel_32(t, form_of(t), a, q, io, rb, grid, st)
+                          : rev_vel_16(t, form_of(t), fmt, a, q, io, rb, grid, st);
+}
+
+bool launch_rev_stress(const Tiling &t, int fmt, const HalfStep &a, const BackBricks &q, const StepIO &io,
+                       const RingBoxes &rb, hipStream_t st) {
+  const int grid = q.nblk + a.nphy + a.npml + rb.nblk;
+  if (grid <= 0) return true;
+  return fmt == STORE_F32 ? rev_stress_32(t, form_of(t), a, q, io, rb, grid, st)
+                          : rev_stress_16(t, form_of(t), fmt, a, q, io, rb, grid, st);
 }
 
 // kz == 0 selects the one-plane-per-block kernels (k_vel_phy / k_stress_phy),

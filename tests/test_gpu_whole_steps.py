@@ -92,6 +92,33 @@ def test_whole_batches_equal_separate_kernels(monkeypatch):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("ring,scaling", [("fp32", 0), ("fp16", 0), ("fp16", 1), ("bf16", 1), ("bfp16", 0)])
+def test_reverse_halves_equal_separate_kernels(ring, scaling, monkeypatch):
+    """A reverse iteration in two launches against separate ones, for every
+    boundary store, with subdomains, with the shot in and outside the region
+    that the backward bricks update, alone and as a batch."""
+    c = case(nx=70, ny=21, nz=19, pml=6, ntime=30, rec_width=2)
+    shots = np.array([c["shots"][0], [-2 * c["dx"], 3 * c["dx"], 2 * c["dx"]]], np.float32)
+    outs = []
+    for cells in ("0", "1e9"):
+        monkeypatch.setenv("DDX_WHOLE_CELLS", cells)
+        out = []
+        es = [engine(c, shots=shots, divide=d, ring_storage=ring) for d in ((1, 1, 1), (2, 1, 2))]
+        for e in es:
+            e.set_ring_scaling(scaling)
+            for q in range(2):
+                e.model_shot(q)
+                e.rtm_shot(q)
+                out += [e.image(i, 0) for i in range(5)] + [e.get(0, f) for f in range(10)]
+        ddx.rtm_batch(es)
+        out += [e.image(i, 0) for e in es for i in range(5)]
+        for e in es:
+            e.close()
+        outs.append(out)
+    for a, b in zip(*outs):
+        assert np.array_equal(a, b)
+
+
 @pytest.mark.parametrize("grid", [(75, 21, 19, 6), (20, 9, 8, 4), (33, 10, 9, 5), (512, 9, 8, 5)])
 def test_cpml_pairs_equal_one_cell_kernels(grid, monkeypatch):
     """Two x cells per thread against one: rows that begin or end inside a
