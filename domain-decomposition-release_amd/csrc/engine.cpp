@@ -636,13 +636,17 @@ static const Tiling &brick_for(const ddx_ctx *c, int kernel, int mode, double ce
 // 5%, else one-cell bricks of rows of 32 (n^3 grids, 15 layers, 60 modelling
 // steps, rows of 64 against 32: n = 48 1.77 / 1.84 ms, 72 3.38 / 3.20, 100
 // 5.59 / 5.65, 128 8.50 / 8.69, 160 16.1 / 15.8, 200 29.8 / 28.3).  16-bit:
-// paired bricks (161x150x131, BF16).
+// paired bricks, rows of 64 pairs where they waste no more lanes than rows of
+// 32 by over 5% (161x150x131 in BF16, 60 steps, rows of 64 pairs against 32:
+// 17.1 / 14.9 ms).
 static void default_bricks(ddx_ctx *c) {
   const int nx = c->d.nx, w64 = (nx + 63) / 64 * 64, w32 = (nx + 31) / 32 * 32;
   const bool narrow = w64 > 1.05 * w32;
   Tiling t{64, 4, 1, 2}, f{64, 4, 1, 2};
   if (c->fmt != STORE_F32) {
-    t = {64, 4, 1, 4};
+    // pairs: a row of 128 cells or of 64, by the lanes they leave idle
+    const bool half_row = (nx + 127) / 128 * 128 > 1.05 * w64;
+    t = half_row ? Tiling{32, 8, 1, 4} : Tiling{64, 4, 1, 4};
     t.px = 2;
   } else if (narrow) {
     t = f = {32, 8, 1, 4};

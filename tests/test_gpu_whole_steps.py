@@ -12,8 +12,8 @@ pytestmark = pytest.mark.gpu
 
 SHAPES = {
     "fp32": [(32, 8, 1, 4, 1), (64, 4, 1, 2, 1), (64, 4, 1, 2, 4), (64, 4, 1, 4, 4)],
-    "bf16": [(64, 4, 1, 2, 2), (64, 4, 1, 4, 2)],
-    "fp16": [(64, 4, 1, 2, 2), (64, 4, 1, 4, 2)],
+    "bf16": [(32, 8, 1, 2, 2), (32, 8, 1, 4, 2), (64, 4, 1, 2, 2), (64, 4, 1, 4, 2)],
+    "fp16": [(32, 8, 1, 4, 2), (64, 4, 1, 2, 2), (64, 4, 1, 4, 2)],
 }
 
 
