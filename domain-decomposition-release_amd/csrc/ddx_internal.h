@@ -241,6 +241,7 @@ struct HalfStep {
   float dx, dy, dz, sc;  // sc: as sign / dt of the separate kernels
   float sx, sy, sz;      // sc over dx, dy, dz
   int grp, pgrp;
+  int cached;            // the bricks' own cells go through ordinary accesses (cached_limit in engine.cpp)
 };
 // The backward bricks of half a reverse iteration (sc, sx, sy, sz as HalfStep).
 struct BackBricks {
@@ -337,7 +338,7 @@ void launch_recv_inject(int fmt, void *const *vptr, const int *rsub, const long 
 // v += obs - syn at the receivers (FWI adjoint source; FP32 storage)
 void launch_recv_residual(void *const *vptr, const int *rsub, const long *roff, int nrec, int it, int ntime,
                           const float *obs, const float *syn, hipStream_t st);
-void launch_image(int fp64, int fmt, const ImgDesc *d, const int *starts, int n, int nblk, float inv_sv,
+void launch_image(int fp64, int fmt, const ImgDesc *d, const int *starts, int n, int nblk, float inv_sv, bool cached,
                   hipStream_t st);
 void launch_image_post(int fp64, const ImgDesc *d, const int *starts, int n, int nblk, hipStream_t st);
 

@@ -287,6 +287,16 @@ static const int kBrickGroup = 8;
 // its last wave of blocks, is a small part of a large one.
 static const double kWholeCells = 14e6;
 
+// A wavefield set of at most so many cells stays in the 256 MB last-level cache
+// from one launch to the next; then the bricks read and write their own cells,
+// and the imaging its inputs, with ordinary accesses instead of streaming ones,
+// which keep nothing there.  n^3 grids with 15 layers, 40 steps, streaming
+// against ordinary: FP32 n = 64 1.71 / 1.65 ms, 100 (2.2 M cells) 3.83 / 3.53,
+// 128 (3.9 M) 5.72 / 6.01, 200 19.1 / 19.6; BF16 100 3.89 / 3.33, 160 (6.9 M)
+// 11.0 / 10.1, 180 (9.3 M) 15.1 / 14.7, 200 (12.2 M) 21.46 / 21.45.  RTM of
+// 141x97x75 with 12 layers (2.0 M), 140 steps: 52.9 / 46.8 ms.
+static double cached_limit(int fmt) { return fmt == STORE_F32 ? 3e6 : 10e6; }
+
 struct ddx_ctx {
   ddx_desc d;
   std::string err;
@@ -342,6 +352,7 @@ struct ddx_ctx {
   int brick_group = kBrickGroup;     // XCD group size of the bricks' block order
   int whole_group = -1;              // the same of the half steps that run as one launch (columns)
   double whole_cells = kWholeCells;  // half steps of at most so many cells run as one launch
+  double cached_cells = 0;           // and of at most so many through ordinary accesses (cached_limit)
   int pml_cz = kPmlPairs;            // work split of the CPML kernels
   int pml_group = 32;                // XCD group size of the CPML block order (0: launch order)
   int pml_order = 0;                 // 1: the XCD-partitioned CPML block order (PmlOrder); 0: pml_group
@@ -743,6 +754,8 @@ extern "C" int ddx_create(const ddx_desc *desc, ddx_ctx **out) {
     if (v >= 0 && v <= 65536) c->brick_group = c->whole_group = v;
   }
   if (const char *e = getenv("DDX_WHOLE_CELLS")) c->whole_cells = atof(e);  // for sweeps
+  c->cached_cells = cached_limit(c->fmt);
+  if (const char *e = getenv("DDX_CACHED_CELLS")) c->cached_cells = atof(e);  // for sweeps
   default_bricks(c);
   if (const char *e = getenv("DDX_TILING")) {  // "TXxTYxCYxKZ[xFORM]", for tile sweeps
     Tiling t{0, 0, 0, 0};
@@ -1521,7 +1534,8 @@ static bool whole_half(const ddx_ctx *c, const Tiling &t, const DevTable<PhyDesc
   if (!t.whole || c->prof.mask || c->pml_overlap || c->pml_cz != kPmlPairs || c->pml_order) return false;
   if (p.cells + q.cells > c->whole_cells) return false;
   a = {p.d, p.starts, p.n, p.nblk, q.d, q.starts, q.n, q.nblk, c->d.dx, c->d.dy, c->d.dz, sc,
-       sc / c->d.dx, sc / c->d.dy, sc / c->d.dz, c->whole_group, c->pml_group};
+       sc / c->d.dx, sc / c->d.dy, sc / c->d.dz, c->whole_group, c->pml_group,
+       p.cells + q.cells <= c->cached_cells};
   return true;
 }
 
@@ -1980,6 +1994,7 @@ struct BatchKey {
   int device = 0, fmt = 0, lg0 = 0, lg1 = 0, pml_cz = kPmlPairs, pml_group = 0, pml_order = 1, brick_group = 0, whole_group = 0;
   float dt = 0.f, dx = 0.f, dy = 0.f, dz = 0.f;
   Tiling tv{0, 0, 0, 0}, ts{0, 0, 0, 0};
+  double cached_cells = 0;
 };
 static double batch_cells(ddx_ctx *const *cs, int n) {
   double cells = 0;
@@ -1988,6 +2003,7 @@ static double batch_cells(ddx_ctx *const *cs, int n) {
 }
 static BatchKey batch_key(const ddx_ctx *c, double cells) {
   BatchKey k;
+  k.cached_cells = c->cached_cells;
   k.device = c->d.device; k.fmt = c->fmt; k.lg0 = c->lg[0]; k.lg1 = c->lg[1];
   k.pml_cz = c->pml_cz; k.pml_group = c->pml_group; k.pml_order = c->pml_order; k.brick_group = c->brick_group; k.whole_group = c->whole_group;
   k.dt = c->d.dt; k.dx = c->d.dx; k.dy = c->d.dy; k.dz = c->d.dz;
@@ -2050,6 +2066,7 @@ struct FusedSet {
   FusedTable<SlabDesc> p, pw;  // CPML: split for launches of their own, for whole half steps
   FusedTable<MemberIO> io;  // sources and receivers of the members
   bool whole = false;       // the half steps may run as one launch each
+  double cells = 0;
 };
 // The fused tables of a batch on the host.
 struct FusedHost {
@@ -2085,10 +2102,10 @@ static void fuse_host(std::vector<BatchMember> &ms, FusedHost &f) {
 }
 // The half steps of ms as one launch each: the split and order of their CPML
 // kernels, the blocks' number and the sources' cells allow it.
-static bool batch_whole(const std::vector<BatchMember> &ms) {
+static bool batch_whole(const std::vector<BatchMember> &ms, double &cells) {
+  cells = 0;
   if (ms.empty()) return false;
   const ddx_ctx *c0 = ms[0].c;
-  double cells = 0;
   bool ok = c0->pml_cz == kPmlPairs && !c0->pml_order;
   for (const BatchMember &m : ms) {
     ok = ok && source_owned(m.c, m.ishot);
@@ -2099,7 +2116,7 @@ static bool batch_whole(const std::vector<BatchMember> &ms) {
 static hipError_t fuse_members(std::vector<BatchMember> &ms, FusedSet &f) {
   FusedHost h;
   fuse_host(ms, h);
-  f.whole = batch_whole(ms);
+  f.whole = batch_whole(ms, f.cells);
   HostTable<SlabDesc> pw = h.p;
   if (f.whole) pw.nblk = split_pml(pw.d, pw.s, pml_whole(ms[0].c->fmt));
   hipError_t e = upload_owned(h.v, f.v);
@@ -2110,9 +2127,10 @@ static hipError_t fuse_members(std::vector<BatchMember> &ms, FusedSet &f) {
   return e;
 }
 
-static HalfStep half_of(const BatchKey &k, const FusedTable<PhyDesc> &p, const FusedTable<SlabDesc> &q, float sc) {
+static HalfStep half_of(const BatchKey &k, const FusedTable<PhyDesc> &p, const FusedTable<SlabDesc> &q, float sc,
+                        double cells) {
   return {p.d, p.starts, p.n, p.nblk, q.d, q.starts, q.n, q.nblk, k.dx, k.dy, k.dz, sc,
-          sc / k.dx, sc / k.dy, sc / k.dz, k.whole_group, k.pml_group};
+          sc / k.dx, sc / k.dy, sc / k.dz, k.whole_group, k.pml_group, cells <= k.cached_cells};
 }
 
 // One modelling time step of every member (each at its own time index, the
@@ -2120,7 +2138,7 @@ static HalfStep half_of(const BatchKey &k, const FusedTable<PhyDesc> &p, const F
 static bool fused_step(const BatchKey &k, const FusedSet &f, const std::vector<BatchMember> &ms, int gs,
                        hipStream_t st, const int *gsp = nullptr) {
   const float rvs = std::ldexp(1.0f, k.lg0 - k.lg1), rsv = std::ldexp(1.0f, k.lg1 - k.lg0);
-  if (!f.whole || !k.tv.whole || !launch_vel_all(k.tv, PURE_FORWARD, k.fmt, half_of(k, f.v, f.pw, rvs), st)) {
+  if (!f.whole || !k.tv.whole || !launch_vel_all(k.tv, PURE_FORWARD, k.fmt, half_of(k, f.v, f.pw, rvs, f.cells), st)) {
     if (!launch_vel_phy(k.tv, PURE_FORWARD, k.fmt, f.v.d, f.v.starts, f.v.n, f.v.nblk, k.dx, k.dy, k.dz, rvs,
                         k.brick_group, st))
       return false;
@@ -2135,7 +2153,7 @@ static bool fused_step(const BatchKey &k, const FusedSet &f, const std::vector<B
   io.nblk = f.io.nblk;
   io.gs = gs;
   io.gsp = gsp;
-  if (!f.whole || !k.ts.whole || !launch_stress_all(k.ts, PURE_FORWARD, k.fmt, half_of(k, f.s, f.pw, k.dt * rsv), io, st)) {
+  if (!f.whole || !k.ts.whole || !launch_stress_all(k.ts, PURE_FORWARD, k.fmt, half_of(k, f.s, f.pw, k.dt * rsv, f.cells), io, st)) {
     launch_source_batch(k.fmt, f.io.d, f.io.n, gs, gsp, st);
     if (!launch_stress_phy(k.ts, PURE_FORWARD, k.fmt, f.s.d, f.s.starts, f.s.n, f.s.nblk, k.dx, k.dy, k.dz,
                            k.dt * rsv, k.brick_group, st))
@@ -2290,7 +2308,7 @@ static int fuse_into_scratch(std::vector<BatchMember> &ms, FusedSet &f, unsigned
                              std::string &err) {
   FusedHost h;
   fuse_host(ms, h);
-  f.whole = batch_whole(ms);
+  f.whole = batch_whole(ms, f.cells);
   std::vector<PmlPiece> pieces;
   PmlOrder ord;
   pml_order_host(h.p.d, ms[0].c->pml_cz, pieces, ord);
@@ -2388,6 +2406,7 @@ struct RtmTables {  // the fused tables of one RTM batch
   FusedTable<ImgDesc> img;
   bool whole = false;  // the forward and reverse half steps may run as one launch each
   bool rev = false;    // and the halves of a reverse iteration
+  double cells = 0;    // of one wavefield set of the members
   Tiling sh[6];        // brick shapes of fv, fs, bv, bs, rv, rs
 };
 
@@ -2470,6 +2489,7 @@ static int rtm_batch_tables(const std::vector<ddx_ctx *> &cs, const std::vector<
   if (e == hipSuccess) e = upload_owned(m2, T.inj);
   if (e == hipSuccess) e = upload_owned(im, T.img);
   T.whole = T.whole && cells <= c0->whole_cells;
+  T.cells = cells;
   if (T.whole) {
     a.nblk = split_pml(a.d, a.s, pml_whole(c0->fmt));
     b.nblk = split_pml(b.d, b.s, pml_whole(c0->fmt));
@@ -2496,7 +2516,7 @@ static bool rtm_fused_forward(const BatchKey &k, const ddx_ctx *c0, const RtmTab
                               const std::vector<ddx_ctx *> &cs, const std::vector<int> &its, int gs, hipStream_t st) {
   const int F = RTM_FORWARD;
   const float rvs = std::ldexp(1.0f, k.lg0 - k.lg1), rsv = std::ldexp(1.0f, k.lg1 - k.lg0);
-  if (!T.whole || !T.sh[0].whole || !launch_vel_all(T.sh[0], F, k.fmt, half_of(k, T.fv, T.fpw, rvs), st)) {
+  if (!T.whole || !T.sh[0].whole || !launch_vel_all(T.sh[0], F, k.fmt, half_of(k, T.fv, T.fpw, rvs, T.cells), st)) {
     if (!launch_vel_phy(T.sh[0], F, k.fmt, T.fv.d, T.fv.starts, T.fv.n, T.fv.nblk, k.dx, k.dy, k.dz, rvs,
                         k.brick_group, st))
       return false;
@@ -2507,7 +2527,7 @@ static bool rtm_fused_forward(const BatchKey &k, const ddx_ctx *c0, const RtmTab
   StepIO io;
   io.io = T.src.d;
   io.gs = gs;
-  if (!T.whole || !T.sh[1].whole || !launch_stress_all(T.sh[1], F, k.fmt, half_of(k, T.fs, T.fpw, k.dt * rsv), io, st)) {
+  if (!T.whole || !T.sh[1].whole || !launch_stress_all(T.sh[1], F, k.fmt, half_of(k, T.fs, T.fpw, k.dt * rsv, T.cells), io, st)) {
     launch_source_batch(k.fmt, T.src.d, T.src.n, gs, nullptr, st, 1.f);
     if (!launch_stress_phy(T.sh[1], F, k.fmt, T.fs.d, T.fs.starts, T.fs.n, T.fs.nblk, k.dx, k.dy, k.dz,
                            k.dt * rsv, k.brick_group, st))
@@ -2549,11 +2569,11 @@ static bool rtm_fused_reverse(const BatchKey &k, const ddx_ctx *c0, const RtmTab
     const RingBoxes x[2] = {{T.box[0].d, T.box[0].starts, T.box[0].n, T.box[0].nblk},
                             {T.box[1].d, T.box[1].starts, T.box[1].n, T.box[1].nblk}};
     launch_inject_batch(k.fmt, T.inj.d, T.inj.starts, T.inj.n, T.inj.nblk, gs, st);
-    if (!launch_rev_vel(T.sh[4], k.fmt, half_of(k, T.rv, T.rpw, rvs), half(T.bsr, -dt * rsv), io, x[0], st) ||
-        !launch_rev_stress(T.sh[5], k.fmt, half_of(k, T.rs, T.rpw, dt * rsv), half(T.bvr, -1.f * rvs), io, x[1], st))
+    if (!launch_rev_vel(T.sh[4], k.fmt, half_of(k, T.rv, T.rpw, rvs, T.cells), half(T.bsr, -dt * rsv), io, x[0], st) ||
+        !launch_rev_stress(T.sh[5], k.fmt, half_of(k, T.rs, T.rpw, dt * rsv, T.cells), half(T.bvr, -1.f * rvs), io, x[1], st))
       return false;
     launch_image(c0->d.image_fp64, k.fmt, T.img.d, T.img.starts, T.img.n, T.img.nblk,
-                 1.0f / std::ldexp(1.0f, k.lg0), st);
+                 1.0f / std::ldexp(1.0f, k.lg0), T.cells <= k.cached_cells, st);
     return true;
   }
   launch_source_batch(k.fmt, T.src.d, T.src.n, gs, nullptr, st, -1.f);
@@ -2562,7 +2582,7 @@ static bool rtm_fused_reverse(const BatchKey &k, const ddx_ctx *c0, const RtmTab
   for (size_t q = 0; q < cs.size(); q++)
     if (its[q] >= 1) ring(cs[q], -1, 2, its[q] - 1, st);
   for (ddx_ctx *c : cs) exchange_on(c, 0, 2, st);
-  if (!T.whole || !T.sh[4].whole || !launch_vel_all(T.sh[4], R, k.fmt, half_of(k, T.rv, T.rpw, rvs), st)) {
+  if (!T.whole || !T.sh[4].whole || !launch_vel_all(T.sh[4], R, k.fmt, half_of(k, T.rv, T.rpw, rvs, T.cells), st)) {
     if (!vel(T.rv, R, 1.f)) return false;
     launch_vel_pml(k.pml_cz, k.fmt, T.rp.d, T.rp.starts, T.rp.n, T.rp.nblk, dx, dy, dz, rvs, k.pml_group,
                    k.pml_order ? &T.rp.ord : nullptr, st);
@@ -2572,14 +2592,14 @@ static bool rtm_fused_reverse(const BatchKey &k, const ddx_ctx *c0, const RtmTab
   for (size_t q = 0; q < cs.size(); q++)
     if (its[q] >= 1) ring(cs[q], -1, 1, its[q] - 1, st);
   for (ddx_ctx *c : cs) exchange_on(c, 0, 0, st);
-  if (!T.whole || !T.sh[5].whole || !launch_stress_all(T.sh[5], R, k.fmt, half_of(k, T.rs, T.rpw, dt * rsv), StepIO{}, st)) {
+  if (!T.whole || !T.sh[5].whole || !launch_stress_all(T.sh[5], R, k.fmt, half_of(k, T.rs, T.rpw, dt * rsv, T.cells), StepIO{}, st)) {
     if (!stress(T.rs, R, dt)) return false;
     launch_stress_pml(k.pml_cz, 1, k.fmt, T.rp.d, T.rp.starts, T.rp.n, T.rp.nblk, dx, dy, dz, dt * rsv, k.pml_group,
                       k.pml_order ? &T.rp.ord : nullptr, st);
   }
   for (ddx_ctx *c : cs) exchange_on(c, 1, 2, st);
   launch_image(c0->d.image_fp64, k.fmt, T.img.d, T.img.starts, T.img.n, T.img.nblk, 1.0f / std::ldexp(1.0f, k.lg0),
-               st);
+               T.cells <= k.cached_cells, st);
   return true;
 }
 
@@ -3065,7 +3085,7 @@ extern "C" int ddx_image_step(ddx_ctx *c) {
   if (!c) return DDX_EINVAL;
   ProfScope ps(c, 5, c->img.bytes);
   launch_image(c->d.image_fp64, c->fmt, c->img.d, c->img.starts, c->img.n, c->img.nblk, 1.0f / scale_of(c, 0),
-               c->st);
+               ext_cells(c) <= c->cached_cells, c->st);
   return DDX_OK;
 }
 
@@ -3239,7 +3259,7 @@ static int rtm_reverse_step(ddx_ctx *c, int ishot, int it) {
   {
     ProfScope ps(c, 5, c->img.bytes);
     launch_image(c->d.image_fp64, c->fmt, c->img.d, c->img.starts, c->img.n, c->img.nblk, 1.0f / scale_of(c, 0),
-                 c->st);
+                 ext_cells(c) <= c->cached_cells, c->st);
   }
   if (c->snap_every > 0 && it >= 1 && (nt - it) % c->snap_every == 0) snapshot(c, 1, (nt - it) / c->snap_every);
   return DDX_OK;

@@ -223,10 +223,22 @@ __device__ __forceinline__ void rmw_add(GT *p, long i, float v) {
   const float old = widen(__builtin_nontemporal_load(p + i));
   __builtin_nontemporal_store(narrow(old + v, p), p + i);
 }
-template <typename GT>
-__device__ __forceinline__ float ld_stream(const GT *p, long i) { return widen(__builtin_nontemporal_load(p + i)); }
-template <typename GT>
-__device__ __forceinline__ void st_stream(GT *p, long i, float v) { __builtin_nontemporal_store(narrow(v, p), p + i); }
+// NT false: ordinary accesses, for launches whose arrays stay in the last-level
+// cache from step to step (cached_limit in engine.cpp).
+template <bool NT = true, typename GT>
+__device__ __forceinline__ auto ld_raw(const GT *p) {
+  if constexpr (NT) return __builtin_nontemporal_load(p);
+  else return *p;
+}
+template <bool NT = true, typename T, typename GT>
+__device__ __forceinline__ void st_raw(T v, GT *p) {
+  if constexpr (NT) __builtin_nontemporal_store(v, p);
+  else *p = v;
+}
+template <bool NT = true, typename GT>
+__device__ __forceinline__ float ld_stream(const GT *p, long i) { return widen(ld_raw<NT>(p + i)); }
+template <bool NT = true, typename GT>
+__device__ __forceinline__ void st_stream(GT *p, long i, float v) { st_raw<NT>(narrow(v, p), p + i); }
 template <typename GT, typename T>
 __device__ __forceinline__ void rmw_add_t(GT *p, long i, T v) {
   const T old = __builtin_nontemporal_load(p + i);
@@ -540,7 +552,7 @@ __device__ __forceinline__ float ld_halo(const GT *p, const XLane &xl, long id_h
 // S: storage format of the fields; `sign` carries the velocity-over-stress
 // scale ratio of the 16-bit formats (a power of two, exact).  XL: x arm from
 // neighbouring lanes (tx = 64); `live`: the lane's cell is in gridphy.
-template <int MODE, int TX, int TY, int CY, int CZ, class S, bool XL = false>
+template <int MODE, int TX, int TY, int CY, int CZ, class S, bool XL = false, bool NT = true>
 __device__ __forceinline__ void vel_zb_body(const PhyDesc &D, int i, int j0, int k0, float dx, float dy, float dz,
                                             float sign, bool live = true) {
   typedef typename GPtr<S>::T gT;
@@ -583,10 +595,10 @@ __device__ __forceinline__ void vel_zb_body(const PhyDesc &D, int i, int j0, int
       const Coef4 cz = MODE == RTM_BACKWARD ? coef_row(vowr_order(k, D.nz, D.R)) : c4;
       const long id = base + (long)kk * sz;
       // the updated cells are read before the stencil taps (see stress_zb_body)
-      const float ovx = ld_stream(fvx, id), ovy = ld_stream(fvy, id), ovz = ld_stream(fvz, id);
-      const float ovxp = P ? ld_stream(fvxp, id) : 0.f, ovyp = P ? ld_stream(fvyp, id) : 0.f;
-      const float ovzp = P ? ld_stream(fvzp, id) : 0.f;
-      const float dtr = sign * ld_stream(fdtr, id);
+      const float ovx = ld_stream<NT>(fvx, id), ovy = ld_stream<NT>(fvy, id), ovz = ld_stream<NT>(fvz, id);
+      const float ovxp = P ? ld_stream<NT>(fvxp, id) : 0.f, ovyp = P ? ld_stream<NT>(fvyp, id) : 0.f;
+      const float ovzp = P ? ld_stream<NT>(fvzp, id) : 0.f;
+      const float dtr = sign * ld_stream<NT>(fdtr, id);
       const float a = dtr / dx, bb = dtr / dy, c = dtr / dz;
       // XL: each x row is expanded and reduced to its derivative at once,
       // so one row (9 values) is live at a time
@@ -638,39 +650,39 @@ __device__ __forceinline__ void vel_zb_body(const PhyDesc &D, int i, int j0, int
         // PHY/fdtd3d_phy_mpi_2_vel_kernel.hpp:70-78: u += dt v (after the
         // update), vrt = dt x the increment
         const float dt = D.dt;
-        const float oux = ld_stream(G(D.f[UX]), id), ouy = ld_stream(G(D.f[UY]), id), ouz = ld_stream(G(D.f[UZ]), id);
+        const float oux = ld_stream<NT>(G(D.f[UX]), id), ouy = ld_stream<NT>(G(D.f[UY]), id), ouz = ld_stream<NT>(G(D.f[UZ]), id);
         const float ix = a * sxx_x + bb * sxy_y + c * sxz_z;
         const float iy = a * syx_x + bb * syy_y + c * syz_z;
         const float iz = a * szx_x + bb * szy_y + c * szz_z;
         const float nvx = ovx + ix, nvy = ovy + iy, nvz = ovz + iz;
-        st_stream(fvx, id, nvx);
-        st_stream(fvy, id, nvy);
-        st_stream(fvz, id, nvz);
-        st_stream(G(D.f[UX]), id, oux + dt * nvx);
-        st_stream(G(D.f[UY]), id, ouy + dt * nvy);
-        st_stream(G(D.f[UZ]), id, ouz + dt * nvz);
-        __builtin_nontemporal_store(dt * ix, G(D.f[VXRT]) + id);
-        __builtin_nontemporal_store(dt * iy, G(D.f[VYRT]) + id);
-        __builtin_nontemporal_store(dt * iz, G(D.f[VZRT]) + id);
+        st_stream<NT>(fvx, id, nvx);
+        st_stream<NT>(fvy, id, nvy);
+        st_stream<NT>(fvz, id, nvz);
+        st_stream<NT>(G(D.f[UX]), id, oux + dt * nvx);
+        st_stream<NT>(G(D.f[UY]), id, ouy + dt * nvy);
+        st_stream<NT>(G(D.f[UZ]), id, ouz + dt * nvz);
+        st_raw<NT>(dt * ix, G(D.f[VXRT]) + id);
+        st_raw<NT>(dt * iy, G(D.f[VYRT]) + id);
+        st_raw<NT>(dt * iz, G(D.f[VZRT]) + id);
       } else {
         const float nvx = ovx + (a * sxx_x + bb * sxy_y + c * sxz_z);
         const float nvy = ovy + (a * syx_x + bb * syy_y + c * syz_z);
         const float nvz = ovz + (a * szx_x + bb * szy_y + c * szz_z);
-        st_stream(fvx, id, nvx);
-        st_stream(fvy, id, nvy);
-        st_stream(fvz, id, nvz);
+        st_stream<NT>(fvx, id, nvx);
+        st_stream<NT>(fvy, id, nvy);
+        st_stream<NT>(fvz, id, nvz);
       }
       if constexpr (P) {
-        st_stream(fvxp, id, ovxp + a * sx);
-        st_stream(fvyp, id, ovyp + bb * sy_);
-        st_stream(fvzp, id, ovzp + c * sz_);
+        st_stream<NT>(fvxp, id, ovxp + a * sx);
+        st_stream<NT>(fvyp, id, ovyp + bb * sy_);
+        st_stream<NT>(fvzp, id, ovzp + c * sz_);
       }
     }
   }
 }
 
 // `dt` carries the stress-over-velocity scale ratio of the 16-bit formats.
-template <int MODE, int TX, int TY, int CY, int CZ, class S, bool XL = false, bool SRC = false>
+template <int MODE, int TX, int TY, int CY, int CZ, class S, bool XL = false, bool SRC = false, bool NT = true>
 __device__ __forceinline__ void stress_zb_body(const PhyDesc &D, int i, int j0, int k0, float a, float bb, float c, bool live = true, const SrcCell &src = SrcCell{}) {
   typedef typename GPtr<S>::T gT;
   const long sy = D.sy, sz = D.sz;
@@ -710,11 +722,11 @@ __device__ __forceinline__ void stress_zb_body(const PhyDesc &D, int i, int j0, 
       // the updated cells are read before the stencil taps: on this target
       // the memory counter also tracks stores, so a read issued after a
       // store waits for that store, which would serialise the updates
-      float oxx = ld_stream(fsxx, id), oyy = ld_stream(fsyy, id), ozz = ld_stream(fszz, id);
+      float oxx = ld_stream<NT>(fsxx, id), oyy = ld_stream<NT>(fsyy, id), ozz = ld_stream<NT>(fszz, id);
       if constexpr (SRC) add_source<gT>(src, D.ox + i, D.oy + j, D.oz + k, oxx, oyy, ozz);
-      const float oxy = ld_stream(fsxy, id), oxz = ld_stream(fsxz, id), oyz = ld_stream(fsyz, id);
-      const float oau = rtm_mode(MODE) ? ld_stream(fsau, id) : 0.f;
-      const float lm = ld_stream(flam, id), mu = ld_stream(fmu, id);
+      const float oxy = ld_stream<NT>(fsxy, id), oxz = ld_stream<NT>(fsxz, id), oyz = ld_stream<NT>(fsyz, id);
+      const float oau = rtm_mode(MODE) ? ld_stream<NT>(fsau, id) : 0.f;
+      const float lm = ld_stream<NT>(flam, id), mu = ld_stream<NT>(fmu, id);
       const float l2m = lm + 2.0f * mu;
       float xl_x = 0.f, xl_y = 0.f, xl_z = 0.f;  // x derivatives of vx, vy, vz (XL)
       if constexpr (XL) {
@@ -753,13 +765,13 @@ __device__ __forceinline__ void stress_zb_body(const PhyDesc &D, int i, int j0, 
       const float nxz = oxz + (a * mu * vz_x + c * mu * vx_z);
       const float nyz = oyz + (bb * mu * vz_y + c * mu * vy_z);
       const float nau = rtm_mode(MODE) ? oau + (a * l2m * vx_x + bb * l2m * vy_y + c * l2m * vz_z) : 0.f;
-      st_stream(fsxx, id, nxx);
-      st_stream(fsyy, id, nyy);
-      st_stream(fszz, id, nzz);
-      st_stream(fsxy, id, nxy);
-      st_stream(fsxz, id, nxz);
-      st_stream(fsyz, id, nyz);
-      if constexpr (rtm_mode(MODE)) st_stream(fsau, id, nau);
+      st_stream<NT>(fsxx, id, nxx);
+      st_stream<NT>(fsyy, id, nyy);
+      st_stream<NT>(fszz, id, nzz);
+      st_stream<NT>(fsxy, id, nxy);
+      st_stream<NT>(fsxz, id, nxz);
+      st_stream<NT>(fsyz, id, nyz);
+      if constexpr (rtm_mode(MODE)) st_stream<NT>(fsau, id, nau);
     }
   }
 }
@@ -834,7 +846,7 @@ struct YlTile {
   float v[NF][CZ][TY + 8][64];  // field, plane, row (j0-4 ..), x
 };
 
-template <int MODE, int TY, int CZ, class S, bool SRC = false>
+template <int MODE, int TY, int CZ, class S, bool SRC = false, bool NT = true>
 __device__ __forceinline__ void stress_yl_body(YlTile<3, TY, CZ> &ly, const PhyDesc &D, int i, int j0, int k0,
                                                float a, float bb, float c, bool live, const SrcCell &src = SrcCell{}) {
   typedef typename GPtr<S>::T gT;
@@ -912,11 +924,11 @@ __device__ __forceinline__ void stress_yl_body(YlTile<3, TY, CZ> &ly, const PhyD
     if (k >= D.nz) break;
     const Coef4 cz = MODE == RTM_BACKWARD ? coef_row(vowr_order(k, D.nz, D.R)) : c4;
     const long id = base + (long)kk * sz;
-    float oxx = ld_stream(fsxx, id), oyy = ld_stream(fsyy, id), ozz = ld_stream(fszz, id);
+    float oxx = ld_stream<NT>(fsxx, id), oyy = ld_stream<NT>(fsyy, id), ozz = ld_stream<NT>(fszz, id);
     if constexpr (SRC) add_source<gT>(src, D.ox + i, D.oy + j, D.oz + k, oxx, oyy, ozz);
-    const float oxy = ld_stream(fsxy, id), oxz = ld_stream(fsxz, id), oyz = ld_stream(fsyz, id);
-    const float oau = rtm_mode(MODE) ? ld_stream(fsau, id) : 0.f;
-    const float lm = ld_stream(flam, id), mu = ld_stream(fmu, id);
+    const float oxy = ld_stream<NT>(fsxy, id), oxz = ld_stream<NT>(fsxz, id), oyz = ld_stream<NT>(fsyz, id);
+    const float oau = rtm_mode(MODE) ? ld_stream<NT>(fsau, id) : 0.f;
+    const float lm = ld_stream<NT>(flam, id), mu = ld_stream<NT>(fmu, id);
     const float l2m = lm + 2.0f * mu;
     const long hid = hbase + (long)kk * sz;
     const float gx = ld_halo(vx, xl, hid), gy = ld_halo(vy, xl, hid), gz = ld_halo(vz, xl, hid);
@@ -965,13 +977,13 @@ __device__ __forceinline__ void stress_yl_body(YlTile<3, TY, CZ> &ly, const PhyD
     const float nxz = oxz + (a * mu * vz_x + c * mu * vx_z);
     const float nyz = oyz + (bb * mu * vz_y + c * mu * vy_z);
     const float nau = rtm_mode(MODE) ? oau + (a * l2m * vx_x + bb * l2m * vy_y + c * l2m * vz_z) : 0.f;
-    st_stream(fsxx, id, nxx);
-    st_stream(fsyy, id, nyy);
-    st_stream(fszz, id, nzz);
-    st_stream(fsxy, id, nxy);
-    st_stream(fsxz, id, nxz);
-    st_stream(fsyz, id, nyz);
-    if constexpr (rtm_mode(MODE)) st_stream(fsau, id, nau);
+    st_stream<NT>(fsxx, id, nxx);
+    st_stream<NT>(fsyy, id, nyy);
+    st_stream<NT>(fszz, id, nzz);
+    st_stream<NT>(fsxy, id, nxy);
+    st_stream<NT>(fsxz, id, nxz);
+    st_stream<NT>(fsyz, id, nyz);
+    if constexpr (rtm_mode(MODE)) st_stream<NT>(fsau, id, nau);
   }
 }
 
@@ -993,7 +1005,7 @@ __global__ __launch_bounds__(64 * TY) DDX_BRICK_ATTR void k_stress_phy_yl(const 
 // Velocity update with the y arm from LDS: the tile holds syy, sxy, syz and,
 // in the backward and reverse modes, sau (the velocity update's y-arm
 // fields).  Same operands and order of operations as vel_zb_body.
-template <int MODE, int TY, int CZ, class S>
+template <int MODE, int TY, int CZ, class S, bool NT = true>
 __device__ __forceinline__ void vel_yl_body(YlTile<(MODE == RTM_BACKWARD || MODE == RTM_REVERSE) ? 4 : 3, TY, CZ> &ly,
                                             const PhyDesc &D, int i, int j0, int k0, float dx, float dy, float dz,
                                             float sign, bool live) {
@@ -1085,10 +1097,10 @@ __device__ __forceinline__ void vel_yl_body(YlTile<(MODE == RTM_BACKWARD || MODE
     if (k >= D.nz) break;
     const Coef4 cz = MODE == RTM_BACKWARD ? coef_row(vowr_order(k, D.nz, D.R)) : c4;
     const long id = base + (long)kk * sz;
-    const float ovx = ld_stream(fvx, id), ovy = ld_stream(fvy, id), ovz = ld_stream(fvz, id);
-    const float ovxp = P ? ld_stream(fvxp, id) : 0.f, ovyp = P ? ld_stream(fvyp, id) : 0.f;
-    const float ovzp = P ? ld_stream(fvzp, id) : 0.f;
-    const float dtr = sign * ld_stream(fdtr, id);
+    const float ovx = ld_stream<NT>(fvx, id), ovy = ld_stream<NT>(fvy, id), ovz = ld_stream<NT>(fvz, id);
+    const float ovxp = P ? ld_stream<NT>(fvxp, id) : 0.f, ovyp = P ? ld_stream<NT>(fvyp, id) : 0.f;
+    const float ovzp = P ? ld_stream<NT>(fvzp, id) : 0.f;
+    const float dtr = sign * ld_stream<NT>(fdtr, id);
     const float a = dtr / dx, bb = dtr / dy, c = dtr / dz;
     const long hid = hbase + (long)kk * sz;
     const float gxx = ld_halo(sxx, xl, hid), gxy = ld_halo(sxy, xl, hid), gxz = ld_halo(sxz, xl, hid);
@@ -1146,13 +1158,13 @@ __device__ __forceinline__ void vel_yl_body(YlTile<(MODE == RTM_BACKWARD || MODE
     const float nvx = ovx + (a * sxx_x + bb * sxy_y + c * sxz_z);
     const float nvy = ovy + (a * syx_x + bb * syy_y + c * syz_z);
     const float nvz = ovz + (a * szx_x + bb * szy_y + c * szz_z);
-    st_stream(fvx, id, nvx);
-    st_stream(fvy, id, nvy);
-    st_stream(fvz, id, nvz);
+    st_stream<NT>(fvx, id, nvx);
+    st_stream<NT>(fvy, id, nvy);
+    st_stream<NT>(fvz, id, nvz);
     if constexpr (P) {
-      st_stream(fvxp, id, ovxp + a * sx);
-      st_stream(fvyp, id, ovyp + bb * sy_);
-      st_stream(fvzp, id, ovzp + c * sz_);
+      st_stream<NT>(fvxp, id, ovxp + a * sx);
+      st_stream<NT>(fvyp, id, ovyp + bb * sy_);
+      st_stream<NT>(fvzp, id, ovzp + c * sz_);
     }
   }
 }
@@ -1208,50 +1220,48 @@ __device__ __forceinline__ F2 ld2(const gbf16 *p, long i) {
   const unsigned u = *(const gu32 *)(p + i);
   return {__uint_as_float(u << 16), __uint_as_float(u & 0xffff0000u)};
 }
-__device__ __forceinline__ F2 ld2_nt(const gfloat *p, long i) {
-  const f2v v = __builtin_nontemporal_load((const gf2v *)(p + i));
+template <bool NT>
+__device__ __forceinline__ F2 ld2_stream(const gfloat *p, long i) {
+  const f2v v = ld_raw<NT>((const gf2v *)(p + i));
   return {v.x, v.y};
 }
-__device__ __forceinline__ F2 ld2_nt(const ghalf *p, long i) {
-  const h2v v = __builtin_nontemporal_load((const gh2v *)(p + i));
+template <bool NT>
+__device__ __forceinline__ F2 ld2_stream(const ghalf *p, long i) {
+  const h2v v = ld_raw<NT>((const gh2v *)(p + i));
   return {(float)v.x, (float)v.y};
 }
-__device__ __forceinline__ F2 ld2_nt(const gbf16 *p, long i) {
-  const unsigned u = __builtin_nontemporal_load((const gu32 *)(p + i));
+template <bool NT>
+__device__ __forceinline__ F2 ld2_stream(const gbf16 *p, long i) {
+  const unsigned u = ld_raw<NT>((const gu32 *)(p + i));
   return {__uint_as_float(u << 16), __uint_as_float(u & 0xffff0000u)};
 }
 // store the pair (both) or its first element only
-__device__ __forceinline__ void st2_nt(gfloat *p, long i, float a, float b, bool both) {
+template <bool NT>
+__device__ __forceinline__ void st2_stream(gfloat *p, long i, float a, float b, bool both) {
   if (both) {
     f2v v;
     v.x = a;
     v.y = b;
-    __builtin_nontemporal_store(v, (gf2v *)(p + i));
+    st_raw<NT>(v, (gf2v *)(p + i));
   } else {
-    __builtin_nontemporal_store(a, p + i);
+    st_raw<NT>(a, p + i);
   }
 }
-__device__ __forceinline__ void st2_nt(ghalf *p, long i, float a, float b, bool both) {
+template <bool NT>
+__device__ __forceinline__ void st2_stream(ghalf *p, long i, float a, float b, bool both) {
   if (both) {
     h2v v;
     v.x = (_Float16)a;
     v.y = (_Float16)b;
-    __builtin_nontemporal_store(v, (gh2v *)(p + i));
+    st_raw<NT>(v, (gh2v *)(p + i));
   } else {
-    __builtin_nontemporal_store((_Float16)a, p + i);
+    st_raw<NT>((_Float16)a, p + i);
   }
 }
-__device__ __forceinline__ void st2_nt(gbf16 *p, long i, float a, float b, bool both) {
-  if (both) {
-    __builtin_nontemporal_store((unsigned)bf16_rne(a) | ((unsigned)bf16_rne(b) << 16), (gu32 *)(p + i));
-  } else {
-    __builtin_nontemporal_store(bf16_rne(a), p + i);
-  }
-}
-template <typename GT>
-__device__ __forceinline__ void rmw2(GT *p, long i, float va, float vb, bool both) {
-  const F2 o = ld2_nt(p, i);
-  st2_nt(p, i, o.a + va, o.b + vb, both);
+template <bool NT>
+__device__ __forceinline__ void st2_stream(gbf16 *p, long i, float a, float b, bool both) {
+  if (both) st_raw<NT>((unsigned)bf16_rne(a) | ((unsigned)bf16_rne(b) << 16), (gu32 *)(p + i));
+  else st_raw<NT>(bf16_rne(a), p + i);
 }
 
 // cells i-4 .. i+5 of a row (i even): v[k] = f(i - 4 + k)
@@ -1362,7 +1372,7 @@ __device__ __forceinline__ bool brick2_full_order(const PhyDesc &D, const TileAt
   return x0 >= 3 && x1 <= D.nx - 4 && y0 >= 3 && y1 <= D.ny - 4 && z0 >= 3 && z1 <= D.nz - 4;
 }
 
-template <int MODE, int TX, int TY, int CY, int CZ, class S>
+template <int MODE, int TX, int TY, int CY, int CZ, class S, bool NT = true>
 __device__ __forceinline__ void vel_zb2_body(const PhyDesc &D, int i, int j0, int k0, float dx, float dy, float dz,
                                              float sign) {
   static_assert(MODE != FWI, "the FWI mode runs on the one-cell bricks");
@@ -1405,14 +1415,14 @@ __device__ __forceinline__ void vel_zb2_body(const PhyDesc &D, int i, int j0, in
       if (k >= D.nz) break;
       const Coef4 cz = MODE == RTM_BACKWARD ? coef_row(vowr_order(k, D.nz, D.R)) : c4;
       const long id = base + (long)kk * sz;
-      const F2 ovx = ld2_nt(fvx, id), ovy = ld2_nt(fvy, id), ovz = ld2_nt(fvz, id);
+      const F2 ovx = ld2_stream<NT>(fvx, id), ovy = ld2_stream<NT>(fvy, id), ovz = ld2_stream<NT>(fvz, id);
       F2 ovxp{0.f, 0.f}, ovyp{0.f, 0.f}, ovzp{0.f, 0.f};
       if constexpr (P) {
-        ovxp = ld2_nt(fvxp, id);
-        ovyp = ld2_nt(fvyp, id);
-        ovzp = ld2_nt(fvzp, id);
+        ovxp = ld2_stream<NT>(fvxp, id);
+        ovyp = ld2_stream<NT>(fvyp, id);
+        ovzp = ld2_stream<NT>(fvzp, id);
       }
-      const F2 dr = ld2_nt(fdtr, id);
+      const F2 dr = ld2_stream<NT>(fdtr, id);
       const float dtra = sign * dr.a, dtrb = sign * dr.b;
       const float aa = dtra / dx, ba = dtra / dy, ca = dtra / dz;
       const float ab = dtrb / dx, bb = dtrb / dy, cb = dtrb / dz;
@@ -1444,19 +1454,19 @@ __device__ __forceinline__ void vel_zb2_body(const PhyDesc &D, int i, int j0, in
       const float nyb = ovy.b + (ab * syx_x.b + bb * syy_y.b + cb * syz_zb);
       const float nza = ovz.a + (aa * szx_x.a + ba * szy_y.a + ca * szz_za);
       const float nzb = ovz.b + (ab * szx_x.b + bb * szy_y.b + cb * szz_zb);
-      st2_nt(fvx, id, nxa, nxb, both);
-      st2_nt(fvy, id, nya, nyb, both);
-      st2_nt(fvz, id, nza, nzb, both);
+      st2_stream<NT>(fvx, id, nxa, nxb, both);
+      st2_stream<NT>(fvy, id, nya, nyb, both);
+      st2_stream<NT>(fvz, id, nza, nzb, both);
       if constexpr (P) {
-        st2_nt(fvxp, id, ovxp.a + aa * sx.a, ovxp.b + ab * sx.b, both);
-        st2_nt(fvyp, id, ovyp.a + ba * sy_.a, ovyp.b + bb * sy_.b, both);
-        st2_nt(fvzp, id, ovzp.a + ca * sza, ovzp.b + cb * szb, both);
+        st2_stream<NT>(fvxp, id, ovxp.a + aa * sx.a, ovxp.b + ab * sx.b, both);
+        st2_stream<NT>(fvyp, id, ovyp.a + ba * sy_.a, ovyp.b + bb * sy_.b, both);
+        st2_stream<NT>(fvzp, id, ovzp.a + ca * sza, ovzp.b + cb * szb, both);
       }
     }
   }
 }
 
-template <int MODE, int TX, int TY, int CY, int CZ, class S, bool SRC = false>
+template <int MODE, int TX, int TY, int CY, int CZ, class S, bool SRC = false, bool NT = true>
 __device__ __forceinline__ void stress_zb2_body(const PhyDesc &D, int i, int j0, int k0, float a, float bb, float c, const SrcCell &src = SrcCell{}) {
   static_assert(MODE != FWI, "the FWI mode runs on the one-cell bricks");
   typedef typename GPtr<S>::T gT;
@@ -1493,15 +1503,15 @@ __device__ __forceinline__ void stress_zb2_body(const PhyDesc &D, int i, int j0,
       if (k >= D.nz) break;
       const Coef4 cz = MODE == RTM_BACKWARD ? coef_row(vowr_order(k, D.nz, D.R)) : c4;
       const long id = base + (long)kk * sz;
-      F2 oxx = ld2_nt(fsxx, id), oyy = ld2_nt(fsyy, id), ozz = ld2_nt(fszz, id);
+      F2 oxx = ld2_stream<NT>(fsxx, id), oyy = ld2_stream<NT>(fsyy, id), ozz = ld2_stream<NT>(fszz, id);
       if constexpr (SRC) {
         add_source<gT>(src, D.ox + i, D.oy + j, D.oz + k, oxx.a, oyy.a, ozz.a);
         add_source<gT>(src, D.ox + i + 1, D.oy + j, D.oz + k, oxx.b, oyy.b, ozz.b);
       }
-      const F2 oxy = ld2_nt(fsxy, id), oxz = ld2_nt(fsxz, id), oyz = ld2_nt(fsyz, id);
+      const F2 oxy = ld2_stream<NT>(fsxy, id), oxz = ld2_stream<NT>(fsxz, id), oyz = ld2_stream<NT>(fsyz, id);
       F2 oau{0.f, 0.f};
-      if constexpr (rtm_mode(MODE)) oau = ld2_nt(fsau, id);
-      const F2 lm = ld2_nt(flam, id), mu = ld2_nt(fmu, id);
+      if constexpr (rtm_mode(MODE)) oau = ld2_stream<NT>(fsau, id);
+      const F2 lm = ld2_stream<NT>(flam, id), mu = ld2_stream<NT>(fmu, id);
       const float l2ma = lm.a + 2.0f * mu.a, l2mb = lm.b + 2.0f * mu.b;
       float w[10];
       ld_xwin(w, vx, id);
@@ -1530,13 +1540,13 @@ __device__ __forceinline__ void stress_zb2_body(const PhyDesc &D, int i, int j0,
       const float nyzb = oyz.b + (bb * mu.b * vz_y.b + c * mu.b * vy_zb);
       const float naua = rtm_mode(MODE) ? oau.a + (a * l2ma * vx_x.a + bb * l2ma * vy_y.a + c * l2ma * vz_za) : 0.f;
       const float naub = rtm_mode(MODE) ? oau.b + (a * l2mb * vx_x.b + bb * l2mb * vy_y.b + c * l2mb * vz_zb) : 0.f;
-      st2_nt(fsxx, id, nxxa, nxxb, both);
-      st2_nt(fsyy, id, nyya, nyyb, both);
-      st2_nt(fszz, id, nzza, nzzb, both);
-      st2_nt(fsxy, id, nxya, nxyb, both);
-      st2_nt(fsxz, id, nxza, nxzb, both);
-      st2_nt(fsyz, id, nyza, nyzb, both);
-      if constexpr (rtm_mode(MODE)) st2_nt(fsau, id, naua, naub, both);
+      st2_stream<NT>(fsxx, id, nxxa, nxxb, both);
+      st2_stream<NT>(fsyy, id, nyya, nyyb, both);
+      st2_stream<NT>(fszz, id, nzza, nzzb, both);
+      st2_stream<NT>(fsxy, id, nxya, nxyb, both);
+      st2_stream<NT>(fsxz, id, nxza, nxzb, both);
+      st2_stream<NT>(fsyz, id, nyza, nyzb, both);
+      if constexpr (rtm_mode(MODE)) st2_stream<NT>(fsau, id, naua, naub, both);
     }
   }
 }
@@ -3119,7 +3129,7 @@ enum { FORM_ONE = 0, FORM_PAIR = 2, FORM_YL = 4 };
 struct NoLds {};
 template <int FORM, int NF, int TY, int CZ>
 using YlLds = typename std::conditional<FORM == FORM_YL, YlTile<NF, TY, CZ>, NoLds>::type;
-template <int FORM, int MODE, int TX, int TY, int CZ, class S>
+template <int FORM, int MODE, int TX, int TY, int CZ, class S, bool NT>
 __device__ __forceinline__ void vel_all_block(const HalfStep &a, int blk, void *lds) {
   static_assert(TX * TY == kBlock, "the bricks and the CPML cells share a block size");
   if (blk >= a.nphy) {
@@ -3139,23 +3149,23 @@ __device__ __forceinline__ void vel_all_block(const HalfStep &a, int blk, void *
     auto &ly = *(YlTile<MODE == RTM_REVERSE ? 4 : 3, TY, CZ> *)lds;
     const TileAt at = tile_at<64, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp);
     const bool live = zbrick<64, TY, 1, CZ>(D, at, i, j0, k0);
-    vel_yl_body<MODE, TY, CZ, S>(ly, D, i, j0, k0, a.dx, a.dy, a.dz, a.sc, live);
+    vel_yl_body<MODE, TY, CZ, S, NT>(ly, D, i, j0, k0, a.dx, a.dy, a.dz, a.sc, live);
   } else if constexpr (FORM == FORM_PAIR) {
     if (zbrick2<TX, TY, 1, CZ>(D, tile_at<2 * TX, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp), i, j0, k0))
-      vel_zb2_body<MODE, TX, TY, 1, CZ, S>(D, i, j0, k0, a.dx, a.dy, a.dz, a.sc);
+      vel_zb2_body<MODE, TX, TY, 1, CZ, S, NT>(D, i, j0, k0, a.dx, a.dy, a.dz, a.sc);
   } else {
     if (zbrick<TX, TY, 1, CZ>(D, tile_at<TX, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp), i, j0, k0))
-      vel_zb_body<MODE, TX, TY, 1, CZ, S>(D, i, j0, k0, a.dx, a.dy, a.dz, a.sc);
+      vel_zb_body<MODE, TX, TY, 1, CZ, S, false, NT>(D, i, j0, k0, a.dx, a.dy, a.dz, a.sc);
   }
 }
 
-template <int FORM, int MODE, int TX, int TY, int CZ, class S>
+template <int FORM, int MODE, int TX, int TY, int CZ, class S, bool NT>
 __global__ __launch_bounds__(kBlock) void k_vel_all(HalfStep a) {
   __shared__ YlLds<FORM, MODE == RTM_REVERSE ? 4 : 3, TY, CZ> lds;
-  vel_all_block<FORM, MODE, TX, TY, CZ, S>(a, blockIdx.x, &lds);
+  vel_all_block<FORM, MODE, TX, TY, CZ, S, NT>(a, blockIdx.x, &lds);
 }
 
-template <int FORM, int MODE, int TX, int TY, int CZ, class S>
+template <int FORM, int MODE, int TX, int TY, int CZ, class S, bool NT>
 __device__ __forceinline__ void stress_all_block(const HalfStep &a, const StepIO &io, int blk, void *lds) {
   static_assert(TX * TY == kBlock, "the bricks and the CPML cells share a block size");
   if (blk >= a.nphy) {
@@ -3183,20 +3193,20 @@ __device__ __forceinline__ void stress_all_block(const HalfStep &a, const StepIO
     auto &ly = *(YlTile<3, TY, CZ> *)lds;
     const TileAt at = tile_at<64, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp);
     const bool live = zbrick<64, TY, 1, CZ>(D, at, i, j0, k0);
-    stress_yl_body<MODE, TY, CZ, S, true>(ly, D, i, j0, k0, a.sx, a.sy, a.sz, live, src);
+    stress_yl_body<MODE, TY, CZ, S, true, NT>(ly, D, i, j0, k0, a.sx, a.sy, a.sz, live, src);
   } else if constexpr (FORM == FORM_PAIR) {
     if (zbrick2<TX, TY, 1, CZ>(D, tile_at<2 * TX, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp), i, j0, k0))
-      stress_zb2_body<MODE, TX, TY, 1, CZ, S, true>(D, i, j0, k0, a.sx, a.sy, a.sz, src);
+      stress_zb2_body<MODE, TX, TY, 1, CZ, S, true, NT>(D, i, j0, k0, a.sx, a.sy, a.sz, src);
   } else {
     if (zbrick<TX, TY, 1, CZ>(D, tile_at<TX, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp), i, j0, k0))
-      stress_zb_body<MODE, TX, TY, 1, CZ, S, false, true>(D, i, j0, k0, a.sx, a.sy, a.sz, true, src);
+      stress_zb_body<MODE, TX, TY, 1, CZ, S, false, true, NT>(D, i, j0, k0, a.sx, a.sy, a.sz, true, src);
   }
 }
 
-template <int FORM, int MODE, int TX, int TY, int CZ, class S>
+template <int FORM, int MODE, int TX, int TY, int CZ, class S, bool NT>
 __global__ __launch_bounds__(kBlock) void k_stress_all(HalfStep a, StepIO io) {
   __shared__ YlLds<FORM, 3, TY, CZ> lds;
-  stress_all_block<FORM, MODE, TX, TY, CZ, S>(a, io, blockIdx.x, &lds);
+  stress_all_block<FORM, MODE, TX, TY, CZ, S, NT>(a, io, blockIdx.x, &lds);
 }
 
 typedef __attribute__((address_space(1))) short gshort;
@@ -3256,7 +3266,7 @@ __device__ __forceinline__ void ring_block(const StepIO &io, const RingBoxes &r,
   ring_cell(D, (b - D.blk0) * kBlock + (int)threadIdx.x, D.ni * D.nj * D.nk, m, slice);
 }
 
-template <int FORM, int TX, int TY, int CZ, class S>
+template <int FORM, int TX, int TY, int CZ, class S, bool NT>
 __global__ __launch_bounds__(kBlock, kF32<S> ? 4 : 2) void k_rev_vel(HalfStep a, BackBricks q, StepIO io, RingBoxes rb) {
   __shared__ YlLds<FORM, 4, TY, CZ> lds;
   int i, j0, k0;
@@ -3269,21 +3279,21 @@ __global__ __launch_bounds__(kBlock, kF32<S> ? 4 : 2) void k_rev_vel(HalfStep a,
       auto &ly = *(YlTile<3, TY, CZ> *)&lds;
       const TileAt at = tile_at<64, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp);
       const bool live = zbrick<64, TY, 1, CZ>(D, at, i, j0, k0);
-      stress_yl_body<RTM_BACKWARD, TY, CZ, S, true>(ly, D, i, j0, k0, q.sx, q.sy, q.sz, live, src);
+      stress_yl_body<RTM_BACKWARD, TY, CZ, S, true, NT>(ly, D, i, j0, k0, q.sx, q.sy, q.sz, live, src);
     } else if constexpr (FORM == FORM_PAIR) {
       if (zbrick2<TX, TY, 1, CZ>(D, tile_at<2 * TX, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp), i, j0, k0))
-        stress_zb2_body<RTM_BACKWARD, TX, TY, 1, CZ, S, true>(D, i, j0, k0, q.sx, q.sy, q.sz, src);
+        stress_zb2_body<RTM_BACKWARD, TX, TY, 1, CZ, S, true, NT>(D, i, j0, k0, q.sx, q.sy, q.sz, src);
     } else {
       if (zbrick<TX, TY, 1, CZ>(D, tile_at<TX, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp), i, j0, k0))
-        stress_zb_body<RTM_BACKWARD, TX, TY, 1, CZ, S, false, true>(D, i, j0, k0, q.sx, q.sy, q.sz, true, src);
+        stress_zb_body<RTM_BACKWARD, TX, TY, 1, CZ, S, false, true, NT>(D, i, j0, k0, q.sx, q.sy, q.sz, true, src);
     }
     return;
   }
   if (blk >= a.nphy + a.npml) return ring_block(io, rb, blk - a.nphy - a.npml);
-  vel_all_block<FORM, RTM_REVERSE, TX, TY, CZ, S>(a, blk, &lds);
+  vel_all_block<FORM, RTM_REVERSE, TX, TY, CZ, S, NT>(a, blk, &lds);
 }
 
-template <int FORM, int TX, int TY, int CZ, class S>
+template <int FORM, int TX, int TY, int CZ, class S, bool NT>
 __global__ __launch_bounds__(kBlock, kF32<S> ? 4 : 2) void k_rev_stress(HalfStep a, BackBricks q, StepIO io, RingBoxes rb) {
   __shared__ YlLds<FORM, 4, TY, CZ> lds;
   int i, j0, k0;
@@ -3295,18 +3305,18 @@ __global__ __launch_bounds__(kBlock, kF32<S> ? 4 : 2) void k_rev_stress(HalfStep
       auto &ly = *(YlTile<4, TY, CZ> *)&lds;
       const TileAt at = tile_at<64, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp);
       const bool live = zbrick<64, TY, 1, CZ>(D, at, i, j0, k0);
-      vel_yl_body<RTM_BACKWARD, TY, CZ, S>(ly, D, i, j0, k0, a.dx, a.dy, a.dz, q.sc, live);
+      vel_yl_body<RTM_BACKWARD, TY, CZ, S, NT>(ly, D, i, j0, k0, a.dx, a.dy, a.dz, q.sc, live);
     } else if constexpr (FORM == FORM_PAIR) {
       if (zbrick2<TX, TY, 1, CZ>(D, tile_at<2 * TX, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp), i, j0, k0))
-        vel_zb2_body<RTM_BACKWARD, TX, TY, 1, CZ, S>(D, i, j0, k0, a.dx, a.dy, a.dz, q.sc);
+        vel_zb2_body<RTM_BACKWARD, TX, TY, 1, CZ, S, NT>(D, i, j0, k0, a.dx, a.dy, a.dz, q.sc);
     } else {
       if (zbrick<TX, TY, 1, CZ>(D, tile_at<TX, TY>(D.nx, D.ny, D.nz, CZ, b - D.blk0, grp), i, j0, k0))
-        vel_zb_body<RTM_BACKWARD, TX, TY, 1, CZ, S>(D, i, j0, k0, a.dx, a.dy, a.dz, q.sc);
+        vel_zb_body<RTM_BACKWARD, TX, TY, 1, CZ, S, false, NT>(D, i, j0, k0, a.dx, a.dy, a.dz, q.sc);
     }
     return;
   }
   if (blk >= a.nphy + a.npml) return ring_block(io, rb, blk - a.nphy - a.npml);
-  stress_all_block<FORM, RTM_REVERSE, TX, TY, CZ, S>(a, StepIO{}, blk, &lds);
+  stress_all_block<FORM, RTM_REVERSE, TX, TY, CZ, S, NT>(a, StepIO{}, blk, &lds);
 }
 
 #if DDX_PART == 0
@@ -3654,12 +3664,12 @@ __device__ __forceinline__ void img_cell(const ImgDesc &D, int b, long &q, long 
 
 // S: storage format of the velocity fields; inv_sv: inverse velocity-class
 // scale (values are unscaled before the products, exactly).
-template <class S>
+template <class S, bool NT>
 __device__ __forceinline__ float ld_v(const void *p, long id, float inv_sv) {
-  const float v = ld_stream((const typename GPtr<S>::T *)p, id);
+  const float v = ld_stream<NT>((const typename GPtr<S>::T *)p, id);
   return std::is_same<S, F32>::value ? v : v * inv_sv;
 }
-template <typename T, class S>
+template <typename T, class S, bool NT>
 __global__ __launch_bounds__(kBlock) void k_image(const ImgDesc *__restrict__ descs,
                                                   const int *__restrict__ starts, int n, float inv_sv) {
   const int b = blockIdx.x;
@@ -3668,12 +3678,12 @@ __global__ __launch_bounds__(kBlock) void k_image(const ImgDesc *__restrict__ de
   bool ok;
   img_cell(D, b, q, id, ok);
   if (!ok) return;
-  const float pfx = ld_v<S>(D.b[3], id, inv_sv), pfy = ld_v<S>(D.b[4], id, inv_sv), pfz = ld_v<S>(D.b[5], id, inv_sv);
-  const float sfx = ld_v<S>(D.b[0], id, inv_sv) - pfx, sfy = ld_v<S>(D.b[1], id, inv_sv) - pfy,
-              sfz = ld_v<S>(D.b[2], id, inv_sv) - pfz;
-  const float prx = ld_v<S>(D.r[3], id, inv_sv), pry = ld_v<S>(D.r[4], id, inv_sv), prz = ld_v<S>(D.r[5], id, inv_sv);
-  const float srx = ld_v<S>(D.r[0], id, inv_sv) - prx, sry = ld_v<S>(D.r[1], id, inv_sv) - pry,
-              srz = ld_v<S>(D.r[2], id, inv_sv) - prz;
+  const float pfx = ld_v<S, NT>(D.b[3], id, inv_sv), pfy = ld_v<S, NT>(D.b[4], id, inv_sv), pfz = ld_v<S, NT>(D.b[5], id, inv_sv);
+  const float sfx = ld_v<S, NT>(D.b[0], id, inv_sv) - pfx, sfy = ld_v<S, NT>(D.b[1], id, inv_sv) - pfy,
+              sfz = ld_v<S, NT>(D.b[2], id, inv_sv) - pfz;
+  const float prx = ld_v<S, NT>(D.r[3], id, inv_sv), pry = ld_v<S, NT>(D.r[4], id, inv_sv), prz = ld_v<S, NT>(D.r[5], id, inv_sv);
+  const float srx = ld_v<S, NT>(D.r[0], id, inv_sv) - prx, sry = ld_v<S, NT>(D.r[1], id, inv_sv) - pry,
+              srz = ld_v<S, NT>(D.r[2], id, inv_sv) - prz;
   // (the images keep read-add-store per image: this kernel runs at high
   // occupancy, and reading the five images first measured slower)
   typedef __attribute__((address_space(1))) T gT;
@@ -3746,10 +3756,11 @@ __global__ __launch_bounds__(kBlock) void k_compensate(const ImgDesc *__restrict
   X(64, 4, 1, 2) X(64, 4, 1, 4) X(64, 4, 1, 8) X(128, 2, 1, 4) X(64, 8, 1, 4) X(32, 8, 1, 4) X(64, 4, 2, 4) \
   X(128, 4, 1, 2) X(64, 2, 1, 8)
 #define DDX_TILINGS16(X) X(64, 4, 1, 2) X(64, 4, 1, 4) X(64, 4, 1, 8) X(128, 2, 1, 4) X(64, 2, 1, 8)
-// paired bricks (px = 2), every storage format.  32 pairs per row where rows
-// of 64 pairs leave lanes idle: BF16, 161 cells wide (3.2 M cells), 87 + 92 us
-// with (64, 4, 1, 4), 70 + 76 with (32, 8, 1, 4)
-#define DDX_TILINGS2(X) X(64, 4, 1, 1) X(64, 4, 1, 2) X(64, 4, 1, 4) X(64, 2, 1, 4) X(32, 8, 1, 2) X(32, 8, 1, 4)
+// paired bricks (px = 2), every storage format; and those of the 16-bit formats
+// alone: 32 pairs per row where rows of 64 pairs leave lanes idle (BF16, 161
+// cells wide, 3.2 M cells: 87 + 92 us with (64, 4, 1, 4), 70 + 76 with (32, 8, 1, 4))
+#define DDX_TILINGS2(X) X(64, 4, 1, 1) X(64, 4, 1, 2) X(64, 4, 1, 4) X(64, 2, 1, 4)
+#define DDX_TILINGS2H(X) X(32, 8, 1, 2) X(32, 8, 1, 4)
 // bricks with the y arm from LDS (xl = 2: tx = 64, cy = 1), (ty, kz), FP32
 #define DDX_TILINGSY(X) X(4, 2) X(4, 4) X(8, 2) X(8, 4) X(16, 2) X(16, 4)
 // lane-exchange bricks (xl: x arm from neighbouring lanes, tx = 64), FP32
@@ -3774,6 +3785,7 @@ bool tiling_supported(const Tiling &t, int fmt) {
   if (t.px == 2) {
 #define DDX_T(TX, TY, CY, CZ) if (t.tx == TX && t.ty == TY && t.cy == CY && t.kz == CZ) return true;
     DDX_TILINGS2(DDX_T)
+    if (fmt != STORE_F32) { DDX_TILINGS2H(DDX_T) }
 #undef DDX_T
     return false;
   }
@@ -3808,6 +3820,7 @@ int tiling_list(int fmt, Tiling *out, int max) {
 #undef DDX_T
 #define DDX_T(TX, TY, CY, CZ) add(TX, TY, CY, CZ, 2);
   DDX_TILINGS2(DDX_T)
+  if (fmt != STORE_F32) { DDX_TILINGS2H(DDX_T) }
 #undef DDX_T
   if (fmt == STORE_F32) {
 #define DDX_T(TX, TY, CY, CZ) add(TX, TY, CY, CZ, 1, 1);
@@ -3963,10 +3976,25 @@ bool vel_all_16(const Tiling &t, int form, int mode, int fmt, const HalfStep &a,
 bool stress_all_32(const Tiling &t, int form, int mode, const HalfStep &a, const StepIO &io, int grid, hipStream_t st);
 bool stress_all_16(const Tiling &t, int form, int mode, int fmt, const HalfStep &a, const StepIO &io, int grid,
                    hipStream_t st);
-#define DDX_V(FORM, MODE, TX, TY, CZ, S) \
-  hipLaunchKernelGGL((k_vel_all<FORM, MODE, TX, TY, CZ, S>), dim3(a.nphy + a.npml), dim3(kBlock), 0, st, a)
-#define DDX_S(FORM, MODE, TX, TY, CZ, S) \
-  hipLaunchKernelGGL((k_stress_all<FORM, MODE, TX, TY, CZ, S>), dim3(grid), dim3(kBlock), 0, st, a, io)
+// (two kernels each: HalfStep::cached)
+#define DDX_V(FORM, MODE, TX, TY, CZ, S)                                                     \
+  do {                                                                                       \
+    const dim3 gv(a.nphy + a.npml), bv(kBlock);                                              \
+    if (a.cached) hipLaunchKernelGGL((k_vel_all<FORM, MODE, TX, TY, CZ, S, false>), gv, bv, 0, st, a); \
+    else hipLaunchKernelGGL((k_vel_all<FORM, MODE, TX, TY, CZ, S, true>), gv, bv, 0, st, a); \
+  } while (0)
+#define DDX_S(FORM, MODE, TX, TY, CZ, S)                                                     \
+  do {                                                                                       \
+    const dim3 gs(grid), bs(kBlock);                                                         \
+    if (a.cached) hipLaunchKernelGGL((k_stress_all<FORM, MODE, TX, TY, CZ, S, false>), gs, bs, 0, st, a, io); \
+    else hipLaunchKernelGGL((k_stress_all<FORM, MODE, TX, TY, CZ, S, true>), gs, bs, 0, st, a, io); \
+  } while (0)
+#define DDX_R(K, FORM, TX, TY, CZ, S)                                                        \
+  do {                                                                                       \
+    const dim3 gr(grid), br(kBlock);                                                         \
+    if (a.cached) hipLaunchKernelGGL((K<FORM, TX, TY, CZ, S, false>), gr, br, 0, st, a, q, io, rb); \
+    else hipLaunchKernelGGL((K<FORM, TX, TY, CZ, S, true>), gr, br, 0, st, a, q, io, rb);    \
+  } while (0)
 bool rev_vel_32(const Tiling &t, int form, const HalfStep &a, const BackBricks &q, const StepIO &io,
                 const RingBoxes &rb, int grid, hipStream_t st);
 bool rev_vel_16(const Tiling &t, int form, int fmt, const HalfStep &a, const BackBricks &q, const StepIO &io,
@@ -3975,8 +4003,6 @@ bool rev_stress_32(const Tiling &t, int form, const HalfStep &a, const BackBrick
                    const RingBoxes &rb, int grid, hipStream_t st);
 bool rev_stress_16(const Tiling &t, int form, int fmt, const HalfStep &a, const BackBricks &q, const StepIO &io,
                    const RingBoxes &rb, int grid, hipStream_t st);
-#define DDX_R(K, FORM, TX, TY, CZ, S) \
-  hipLaunchKernelGGL((K<FORM, TX, TY, CZ, S>), dim3(grid), dim3(kBlock), 0, st, a, q, io, rb)
 #if DDX_PART == 9
 bool vel_all_32(const Tiling &t, int form, int mode, const HalfStep &a, hipStream_t st) {
 #define DDX_T(FORM, TX, TY, CZ)                                               \
@@ -4092,10 +4118,10 @@ bool vel_half(DDX_SIG) { DDX_TILINGS16(DDX_T16) return false; }
 bool stress_half(DDX_SIG) { DDX_TILINGS16(DDX_T16) return false; }
 #elif DDX_PART == 5
 #define DDX_F vel_zb2
-bool vel_pair(DDX_SIG) { DDX_TILINGS2(DDX_T2) return false; }
+bool vel_pair(DDX_SIG) { DDX_TILINGS2(DDX_T2) DDX_TILINGS2H(DDX_T16) return false; }
 #elif DDX_PART == 6
 #define DDX_F stress_zb2
-bool stress_pair(DDX_SIG) { DDX_TILINGS2(DDX_T2) return false; }
+bool stress_pair(DDX_SIG) { DDX_TILINGS2(DDX_T2) DDX_TILINGS2H(DDX_T16) return false; }
 #elif DDX_PART == 7
 #define DDX_F vel_zb
 bool vel_lane(DDX_SIG) { DDX_TILINGSX(DDX_TX) return false; }
@@ -4461,19 +4487,24 @@ void launch_recv_residual(void *const *vptr, const int *rsub, const long *roff, 
                      obs, syn);
 }
 
-void launch_image(int fp64, int fmt, const ImgDesc *d, const int *starts, int n, int nblk, float inv_sv,
+#define DDX_I(T, S)                                                                             \
+  do {                                                                                          \
+    if (cached) hipLaunchKernelGGL((k_image<T, S, false>), g, b, 0, st, d, starts, n, inv_sv);  \
+    else hipLaunchKernelGGL((k_image<T, S, true>), g, b, 0, st, d, starts, n, inv_sv);          \
+  } while (0)
+void launch_image(int fp64, int fmt, const ImgDesc *d, const int *starts, int n, int nblk, float inv_sv, bool cached,
                   hipStream_t st) {
   if (nblk <= 0) return;
   const dim3 g(nblk), b(kBlock);
   if (fmt == STORE_F16) {
-    if (fp64) hipLaunchKernelGGL((k_image<double, F16>), g, b, 0, st, d, starts, n, inv_sv);
-    else hipLaunchKernelGGL((k_image<float, F16>), g, b, 0, st, d, starts, n, inv_sv);
+    if (fp64) DDX_I(double, F16);
+    else DDX_I(float, F16);
   } else if (fmt == STORE_BF16) {
-    if (fp64) hipLaunchKernelGGL((k_image<double, BF16>), g, b, 0, st, d, starts, n, inv_sv);
-    else hipLaunchKernelGGL((k_image<float, BF16>), g, b, 0, st, d, starts, n, inv_sv);
+    if (fp64) DDX_I(double, BF16);
+    else DDX_I(float, BF16);
   } else {
-    if (fp64) hipLaunchKernelGGL((k_image<double, F32>), g, b, 0, st, d, starts, n, inv_sv);
-    else hipLaunchKernelGGL((k_image<float, F32>), g, b, 0, st, d, starts, n, inv_sv);
+    if (fp64) DDX_I(double, F32);
+    else DDX_I(float, F32);
   }
 }
 

@@ -30,9 +30,12 @@ def engine(c, storage="fp32", shots=None, **kw):
 GRIDS = [(75, 21, 19, 6), (64, 9, 8, 4), (300, 37, 9, 5)]
 
 
-@pytest.mark.parametrize("grid", GRIDS)
+@pytest.mark.parametrize("grid,cached", [(GRIDS[0], 1), (GRIDS[0], 0), (GRIDS[1], 1), (GRIDS[2], 0)])
 @pytest.mark.parametrize("storage", list(SHAPES))
-def test_whole_half_steps_equal_separate_kernels(storage, grid, monkeypatch):
+def test_whole_half_steps_equal_separate_kernels(storage, grid, cached, monkeypatch):
+    """cached: ordinary accesses to the updated cells, else streaming ones."""
+    if not cached:
+        monkeypatch.setenv("DDX_CACHED_CELLS", "0")
     nx, ny, nz, pml = grid
     c = case(nx=nx, ny=ny, nz=nz, pml=pml, ntime=20, rec_width=2)
     dx = c["dx"]
