@@ -52,11 +52,11 @@ from ddx import synth  # noqa: E402
 HBM_PEAK_GBS = 8000.0
 METRIC = "Gcell-updates/s + shots/s, 1 MI355X, vs plain FP32; p50/p99 shot latency"
 KERNEL_NAMES = {0: "velocity update, physical region (k_vel_phy)", 1: "stress update, physical region (k_stress_phy)",
-                2: "CPML velocity (k_vel_pml)", 3: "CPML stress (k_stress_pml)", 4: "CMM halo exchange (k_halo)",
+                2: "CPML velocity (k_vel_pml)", 3: "CPML stress (k_stress_pml)", 4: "CMM halo exchange (k_copy, mode 1)",
                 5: "imaging (k_image)"}
 # kernel-name prefixes of each class, as rocprofv3 reports them
 KERNEL_PREFIX = {0: ("ddx::k_vel_phy", "ddx::k_vel_lds"), 1: ("ddx::k_stress_phy", "ddx::k_stress_lds"),
-                 2: ("ddx::k_vel_pml",), 3: ("ddx::k_stress_pml",), 4: ("ddx::k_halo",), 5: ("ddx::k_image",)}
+                 2: ("ddx::k_vel_pml",), 3: ("ddx::k_stress_pml",), 4: (), 5: ("ddx::k_image",)}
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic.json")
 KERNEL_SRC = os.path.join(ROOT, "domain-decomposition-release_amd", "csrc", "kernels.hip")
 
@@ -470,8 +470,8 @@ def main():
     ap.add_argument("--ring-storage", choices=["fp32", "fp16", "bf16", "bfp16"], default="fp32",
                     help="VOWR boundary store format over FP32 wavefields (fp32: as --storage)")
     ap.add_argument("--exchange", type=int, default=-1,
-                    help="CMM exchange mode (ddx_set_exchange): 0 direct copy (default), 1 contiguous message "
-                         "blocks, 2 pack on store (needs DDX_MIRROR=1 in the environment)")
+                    help="CMM exchange mode (ddx_set_exchange): 0 nothing to move (default), 1 contiguous message "
+                         "blocks, 2 as 0 (needs DDX_MIRROR=1 in the environment)")
     ap.add_argument("--no-autotune", action="store_true",
                     help="keep the default brick shapes instead of ddx_autotune's choice")
     ap.add_argument("--ntime", type=int, default=0, help="override the time steps (profiling runs only)")

@@ -268,7 +268,7 @@ bool launch_vel_phy(const Tiling &t, int mode, int fmt, const PhyDesc *d, const 
                     float dx, float dy, float dz, float sign, int grp, hipStream_t st);
 bool launch_stress_phy(const Tiling &t, int mode, int fmt, const PhyDesc *d, const int *starts, int n, int nblk,
                        float dx, float dy, float dz, float dt, int grp, hipStream_t st);
-// One launch for a half step (CPML split 1, group-interleaved orders); false,
+// One launch for a half step (CPML split pml_whole, group-interleaved orders); false,
 // launching nothing, when no such kernel exists for the brick shape, format
 // and mode (the backward mode has no CPML cells).  The stress step also adds
 // the members' sources and samples their receivers (io).

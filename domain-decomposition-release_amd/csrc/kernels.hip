@@ -214,15 +214,10 @@ struct DivGuard {
 // Cells that one thread alone reads and writes in a launch (the updated
 // fields and the per-cell model arrays of the physical-region bricks, the
 // imaging inputs and images) go through non-temporal loads and stores, so
-// they do not push the stencil halos of neighbouring bricks out of L2.  Same
-// arithmetic as `p[i] += v`.  (Measured: 2-4% faster bricks, imaging
+// they do not push the stencil halos of neighbouring bricks out of L2.
+// (Measured on large grids: 2-4% faster bricks, imaging
 // 259 -> 174 us per launch; slower in the CPML kernels,
 // which keep ordinary accesses.)
-template <typename GT>
-__device__ __forceinline__ void rmw_add(GT *p, long i, float v) {
-  const float old = widen(__builtin_nontemporal_load(p + i));
-  __builtin_nontemporal_store(narrow(old + v, p), p + i);
-}
 // NT false: ordinary accesses, for launches whose arrays stay in the last-level
 // cache from step to step (cached_limit in engine.cpp).
 template <bool NT = true, typename GT>
@@ -264,20 +259,6 @@ __device__ __forceinline__ float dm4(PT f, long i, long s, float c0, float c1, f
   a += c1 * (ld(f, i + s) - ld(f, i - 2 * s));
   a += c2 * (ld(f, i + 2 * s) - ld(f, i - 3 * s));
   a += c3 * (ld(f, i + 3 * s) - ld(f, i - 4 * s));
-  return a;
-}
-template <typename PT>
-__device__ __forceinline__ float dp2(PT f, long i, long s, float c0, float c1) {
-  float a = 0.f;
-  a += c0 * (ld(f, i + s) - ld(f, i));
-  a += c1 * (ld(f, i + 2 * s) - ld(f, i - s));
-  return a;
-}
-template <typename PT>
-__device__ __forceinline__ float dm2(PT f, long i, long s, float c0, float c1) {
-  float a = 0.f;
-  a += c0 * (ld(f, i) - ld(f, i - s));
-  a += c1 * (ld(f, i + s) - ld(f, i - 2 * s));
   return a;
 }
 
@@ -2713,7 +2694,7 @@ __device__ __forceinline__ TileSlot tile_slot(int t, bool xarm, int lo, int hi, 
   return s;
 }
 
-// 4th-order differences on an LDS tile, as dp2 / dm2.
+// 4th-order differences on an LDS tile, forward- and backward-staggered.
 __device__ __forceinline__ float tp2(const float *s, int i, int st, float c0, float c1) {
   float a = 0.f;
   a += c0 * (s[i + st] - s[i]);
@@ -3123,7 +3104,8 @@ __device__ __forceinline__ void recv_block(const StepIO &io, int b) {
 // gaps; what each block does is what the separate kernels do.  Where it pays
 // and where not: kWholeCells in engine.cpp.  A modelling step is two launches
 // instead of six: 32x28x24 cells 31.8 -> 15.2 us per step, 64^3 with 20
-// layers 66 -> 51 us, 100^3 with 10 layers 96 -> 75 us.
+// layers 66 -> 51 us, 100^3 with 10 layers 96 -> 75 us (67 with ordinary
+// accesses, NT false).
 // ---------------------------------------------------------------------------
 enum { FORM_ONE = 0, FORM_PAIR = 2, FORM_YL = 4 };
 struct NoLds {};

@@ -563,8 +563,8 @@ class Engine:
         self._check(lib().ddx_set_graphs(self.h, int(bool(on))), "ddx_set_graphs")
 
     def set_exchange(self, mode):
-        """CMM exchange mode: 0 direct copy into the ghosts, 1 contiguous
-        message blocks (pack, then unpack)."""
+        """CMM exchange mode: 0 nothing to move (subdomains share the fields'
+        arrays), 1 contiguous message blocks (pack, then unpack)."""
         self._check(lib().ddx_set_exchange(self.h, int(mode)), "ddx_set_exchange")
 
     def exchange(self):
