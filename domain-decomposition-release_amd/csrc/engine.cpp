@@ -238,6 +238,11 @@ struct DevTable {  // a descriptor table and its first-block index array on the 
   double cells = 0;      // cells covered by one launch (stencil tables)
   double psi_cells = 0;  // sum over cells of the damped axes in range (CPML tables)
   PmlOrder ord;          // XCD-partitioned block order (CPML tables; pieces owned by the context)
+  // what d and starts hold, for the tables of batches (read back from the
+  // device it cost a batch call a synchronous copy per table and member: three
+  // RTM shots of 80^3 or less, 40 steps, 12.3 / 11.2 ms)
+  std::vector<T> host;
+  std::vector<int> host_starts;
 };
 
 struct PhyTables {  // physical-region tables of one brick shape and model, per wavefield set
@@ -472,6 +477,8 @@ static int upload_table(ddx_ctx *c, DevTable<T> &t, std::vector<T> &h, const std
                         int nblk) {
   t.n = (int)h.size();
   t.nblk = nblk;
+  t.host = h;
+  t.host_starts = starts;
   if (t.n == 0) return DDX_OK;
   int rc = dalloc(c, (void **)&t.d, sizeof(T) * h.size());
   if (rc) return rc;
@@ -1917,15 +1924,7 @@ struct FusedTable {
 };
 
 template <class T>
-static hipError_t download_table(const DevTable<T> &t, HostTable<T> &h) {
-  h.d.resize(t.n);
-  h.s.resize(t.n);
-  h.nblk = t.nblk;
-  if (t.n == 0) return hipSuccess;
-  hipError_t e = hipMemcpy(h.d.data(), t.d, sizeof(T) * t.n, hipMemcpyDeviceToHost);
-  if (e == hipSuccess) e = hipMemcpy(h.s.data(), t.starts, sizeof(int) * t.n, hipMemcpyDeviceToHost);
-  return e;
-}
+static HostTable<T> host_table(const DevTable<T> &t) { return {t.host, t.host_starts, t.nblk}; }
 
 // Tables of several members concatenated, block offsets shifted (host).
 template <class T>
@@ -2041,10 +2040,10 @@ static int batch_prepare(ddx_ctx *c, int ishot, const BatchKey &k, BatchMember &
   if (!phy_tables(c, k.tv, 0) || !phy_tables(c, k.ts, 0)) return DDX_EHIP;
   const PhyTables *a = phy_tables(c, k.tv, 0);
   const PhyTables *b = phy_tables(c, k.ts, 0);
-  hipError_t e = download_table(a->set[0], m.hv);
-  if (e == hipSuccess) e = download_table(b->set[0], m.hs);
-  if (e == hipSuccess) e = download_table(c->pml[0][0], m.hp);
-  if (e == hipSuccess) e = hipStreamSynchronize(c->st);
+  m.hv = host_table(a->set[0]);
+  m.hs = host_table(b->set[0]);
+  m.hp = host_table(c->pml[0][0]);
+  const hipError_t e = hipStreamSynchronize(c->st);
   if (e != hipSuccess) {
     c->err = std::string("HIP error: ") + hipGetErrorString(e) + " preparing a batch member";
     return DDX_EHIP;
@@ -2434,11 +2433,11 @@ static int rtm_batch_tables(const std::vector<ddx_ctx *> &cs, const std::vector<
     // build every shape first: building one may move the others in the cache
     for (int k = 0; k < 6; k++)
       if (!phy_tables(c, sh[k], model_for(c, mode_of[k]))) { err = c->err; return DDX_EHIP; }
-    for (int k = 0; k < 6 && e == hipSuccess; k++)
-      e = download_table(phy_tables(c, sh[k], model_for(c, mode_of[k]))->set[set_of[k]], hp[k][q]);
-    if (e == hipSuccess) e = download_table(c->pml[model_for(c, F)][0], hf[q]);
-    if (e == hipSuccess) e = download_table(c->pml[model_for(c, R)][1], hr[q]);
-    if (e == hipSuccess) e = download_table(c->img, him[q]);
+    for (int k = 0; k < 6; k++)
+      hp[k][q] = host_table(phy_tables(c, sh[k], model_for(c, mode_of[k]))->set[set_of[k]]);
+    hf[q] = host_table(c->pml[model_for(c, F)][0]);
+    hr[q] = host_table(c->pml[model_for(c, R)][1]);
+    him[q] = host_table(c->img);
     MemberIO x = member_io(c, shots[q], 0);
     x.join = joins ? (*joins)[q] : 0;
     x.rev = rev;
@@ -2457,8 +2456,8 @@ static int rtm_batch_tables(const std::vector<ddx_ctx *> &cs, const std::vector<
     for (int k = 0; k < 2 && e == hipSuccess && T.rev; k++) {
       const PhyTables *pt = phy_tables(c, sh[4 + k], model_for(c, B));
       if (!pt) { err = c->err; return DDX_EHIP; }
-      e = download_table(pt->set[0], hb[k][q]);
-      if (e == hipSuccess) e = download_table(c->ring[2 - k], hx[k][q]);
+      hb[k][q] = host_table(pt->set[0]);
+      hx[k][q] = host_table(c->ring[2 - k]);
       set_member(hb[k][q], (int)q);
       set_member(hx[k][q], (int)q);
     }
