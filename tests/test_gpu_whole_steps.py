@@ -179,3 +179,43 @@ def test_cpml_division_is_exact_at_every_magnitude(spacing, monkeypatch):
             e.close()
         for f, (a, b) in enumerate(zip(*outs)):
             assert np.array_equal(a, b, equal_nan=True), (scale, ddx.FIELD_NAMES[f])
+
+
+# Values a (three spacings) whose first-tap difference 9/8 a, divided by the
+# spacing, lies just above 2^-90: the remainder of the short division is then
+# no FP32 number, and for these a rounding it changes the quotient.
+SMALL_SPACINGS = [
+    ("0x1.44f05ep-20", ["0x1.dedd5ep-110", "0x1.26dfdp-110", "0x1.33fad4p-110", "0x1.c423fap-110", "0x1.8fb7ecp-110",
+                        "0x1.4eb436p-110", "0x1.7581e6p-110", "0x1.9d564ap-110"]),
+    ("0x1.953dfap-17", ["0x1.54e12cp-106", "0x1.8b19e4p-106", "0x1.31fe6p-106"]),
+    ("0x1.204942p-15", ["0x1.4f1488p-104"]),
+]
+
+
+@pytest.mark.parametrize("whole,cz", [("1e9", "0"), ("0", "1"), ("0", "0")])
+@pytest.mark.parametrize("spacing,values", SMALL_SPACINGS)
+def test_cpml_division_by_small_spacings(spacing, values, whole, cz, monkeypatch):
+    """The z difference of one plane of szz in the x layers over a small dz,
+    in the whole half step, the one-cell and the paired CPML kernels, against
+    the correctly rounded quotient: dt / rho is a power of two, so a velocity
+    is the quotient's bits."""
+    monkeypatch.setenv("DDX_WHOLE_CELLS", whole)
+    monkeypatch.setenv("DDX_PML_CZ", cz)
+    nx, ny, nz, pml = 20, 18, 16, 6
+    dz = np.float32(float.fromhex(spacing))
+    a = np.array([float.fromhex(v) for v in values], np.float32)
+    e = ddx.Engine(ddx.make_desc(nx, ny, nz, 10.0, pml, 2.0 ** -10, 15.0, 10, dz=float(dz), cfl_policy=1))
+    e.set_model(np.full((nz, ny, nx), 2500, np.float32), np.full((nz, ny, nx), 1400, np.float32),
+                np.full((nz, ny, nx), 2048, np.float32))
+    szz = np.zeros(e.ext_shape, np.float32)
+    k = pml + nz // 2
+    szz[k] = np.resize(a, szz[k].shape)
+    e.set(0, ddx.SZZ, szz)
+    e.step_vel(0, po.PURE_FORWARD)
+    v = e.get(0, ddx.VZ)
+    e.close()
+    want = np.float32(2.0 ** -21) * ((np.float32(1.125) * szz[k]) / dz)
+    rows = slice(pml, pml + ny)
+    for cols in (slice(2, pml), slice(pml + nx, nx + 2 * pml - 2)):
+        assert np.array_equal(v[k - 1, rows, cols], want[rows, cols])
+        assert np.array_equal(v[k, rows, cols], -want[rows, cols])
