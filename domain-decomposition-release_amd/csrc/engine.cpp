@@ -861,7 +861,9 @@ static const PhyTables *phy_tables(ddx_ctx *c, const Tiling &t, int model) {
 // the time loop.
 static int prepare_phy_tables(ddx_ctx *c, int model) {
   for (int m = 0; m < kModes; m++)
-    if (!phy_tables(c, c->tiling_vel[m], model) || !phy_tables(c, c->tiling_stress[m], model)) return DDX_EHIP;
+    if (!phy_tables(c, c->tiling_vel[m], model) || !phy_tables(c, c->tiling_stress[m], model) ||
+        !phy_tables(c, c->apart[0][m], model) || !phy_tables(c, c->apart[1][m], model))
+      return DDX_EHIP;
   return DDX_OK;
 }
 
@@ -2345,7 +2347,14 @@ extern "C" int ddx_model_batch_noalloc(ddx_ctx *const *ctxs, const int *ishots, 
   for (int q = 0; q < n; q++)
     if (!ctxs[q]) return DDX_EINVAL;
   ddx_ctx *c0 = ctxs[0];
-  const BatchKey k = batch_key(c0, batch_cells(ctxs, n));
+  BatchKey k = batch_key(c0, batch_cells(ctxs, n));
+  // a shot of a member's own may not build the tables of the shapes for
+  // separate launches: then those of ctxs[0]'s own shots
+  for (int q = 0; q < n; q++)
+    if (!cached_phy_tables(ctxs[q], k.tv, 0) || !cached_phy_tables(ctxs[q], k.ts, 0)) {
+      k = batch_key(c0, 0);
+      break;
+    }
   HIPCHECK(c0, hipSetDevice(k.device));
   unsigned char *dev = nullptr;
   if (int rc = scratch_of(k.device, &dev, c0->err)) return rc;
@@ -3582,6 +3591,8 @@ extern "C" int ddx_autotune(ddx_ctx *c, int reps, int *timed) {
     return rc;
   }
   if (timed) *timed = count;
+  for (int m = 0; m < 2; m++)  // shapes taken from the cache have no tables yet
+    if (c->model[m] && (rc = prepare_phy_tables(c, m))) return rc;
   if ((rc = ddx_reset_wave(c, 0)) || (rc = ddx_reset_wave(c, 1))) return rc;
   HIPCHECK(c, hipStreamSynchronize(c->st));
   HIPCHECK(c, hipGetLastError());

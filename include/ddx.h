@@ -305,9 +305,11 @@ int ddx_model_batch(ddx_ctx *const *ctxs, const int *ishots, int n);
  * batch's tables need more).  Every member must be ready without
  * allocating: its shot's seismogram buffer exists (ddx_model_shot or
  * ddx_set_observed ran on it once) and its tables of ctxs[0]'s brick
- * shapes are built (one shot ran with them); DDX_ESTATE otherwise.  Runs
- * the time steps eagerly (no graph replay).  Seismograms equal those of
- * ddx_model_batch.  The array is shared by every call on one GPU and keeps
+ * shapes are built (one shot ran with them); DDX_ESTATE otherwise.  (A batch
+ * too large for half steps in one launch takes the shapes that ctxs[0]'s
+ * ddx_autotune found for separate launches where every member has their
+ * tables, as contexts tuned alike have.)  Runs the time steps eagerly (no
+ * graph replay).  Seismograms equal those of ddx_model_batch.  The array is shared by every call on one GPU and keeps
  * the last call's tables: calls that overlap on one GPU (from several host
  * threads) race and must be serialised by the caller. */
 int ddx_model_batch_noalloc(ddx_ctx *const *ctxs, const int *ishots, int n);

@@ -74,3 +74,35 @@ def test_noalloc_refuses_unprepared_context():
             noalloc([e])
     finally:
         e.close()
+
+
+def test_noalloc_batch_above_the_one_launch_limit(monkeypatch):
+    """Tuned members each small enough for half steps in one launch, the batch
+    too large for it: the first context's shapes for separate launches may
+    differ from those it runs shots with.  The batch needs no more than one
+    shot of each member with the latter, whether the first context timed its
+    shapes or took them from the cache, and of a member of another grid that
+    was given them."""
+    nt = 20
+    for q, n in enumerate([(36, 33, 30), (70, 24, 22), (100, 20, 18), (130, 18, 20)]):
+        sizes = [n, n, (n[0] - 9, n[1] + 5, n[2] + 3)]
+        cs = uneven(sizes, seed=20 + q)
+        cs[1] = cs[0]
+        monkeypatch.setenv("DDX_WHOLE_CELLS", str(int(1.6 * np.prod([v + 16 for v in n]))))
+        es = [engine(c, nt) for c in cs]
+        try:
+            for e in es[:2]:
+                e.autotune(reps=1)
+            for k in (0, 1):
+                es[2].set_brick(k, ddx.PURE_FORWARD, *es[0].brick(k, ddx.PURE_FORWARD))
+            ref = []
+            for e in es:
+                e.model_shot(0)
+                ref.append(e.seismograms(0))
+            for order in ([1, 0], [0, 1, 2], [1, 2]):
+                noalloc([es[i] for i in order])
+                for i in order:
+                    assert np.array_equal(es[i].seismograms(0), ref[i]), (n, order, i)
+        finally:
+            for e in es:
+                e.close()
