@@ -1986,7 +1986,7 @@ struct BatchMember {
   ddx_ctx *c = nullptr;
   int ishot = 0, it = 0;
   int join = 0;  // batch step of the shot's first time step
-  HostTable<PhyDesc> hv, hs;
+  HostTable<PhyDesc> h[2][2];  // of BatchKey::brick, once the batch has had that many cells
   HostTable<SlabDesc> hp;
 };
 
@@ -1994,22 +1994,27 @@ struct BatchMember {
 struct BatchKey {
   int device = 0, fmt = 0, lg0 = 0, lg1 = 0, pml_cz = kPmlPairs, pml_group = 0, pml_order = 1, brick_group = 0, whole_group = 0;
   float dt = 0.f, dx = 0.f, dy = 0.f, dz = 0.f;
-  Tiling tv{0, 0, 0, 0}, ts{0, 0, 0, 0};
-  double cached_cells = 0;
+  // [velocity, stress]: up to whole_cells, and in launches of more (brick_for);
+  // a continuous batch passes from one to the other as its members change
+  Tiling brick[2][2] = {{{0, 0, 0, 0}, {0, 0, 0, 0}}, {{0, 0, 0, 0}, {0, 0, 0, 0}}};
+  double whole_cells = 0, cached_cells = 0;
 };
 static double batch_cells(ddx_ctx *const *cs, int n) {
   double cells = 0;
   for (int q = 0; q < n; q++) cells += ext_cells(cs[q]);
   return cells;
 }
-static BatchKey batch_key(const ddx_ctx *c, double cells) {
+static BatchKey batch_key(const ddx_ctx *c) {
   BatchKey k;
+  k.whole_cells = c->whole_cells;
   k.cached_cells = c->cached_cells;
   k.device = c->d.device; k.fmt = c->fmt; k.lg0 = c->lg[0]; k.lg1 = c->lg[1];
   k.pml_cz = c->pml_cz; k.pml_group = c->pml_group; k.pml_order = c->pml_order; k.brick_group = c->brick_group; k.whole_group = c->whole_group;
   k.dt = c->d.dt; k.dx = c->d.dx; k.dy = c->d.dy; k.dz = c->d.dz;
-  k.tv = brick_for(c, 0, PURE_FORWARD, cells);
-  k.ts = brick_for(c, 1, PURE_FORWARD, cells);
+  for (int kernel = 0; kernel < 2; kernel++) {
+    k.brick[0][kernel] = brick_for(c, kernel, PURE_FORWARD, 0);
+    k.brick[1][kernel] = c->apart[kernel][PURE_FORWARD];
+  }
   return k;
 }
 static bool batch_compatible(const BatchKey &k, const ddx_ctx *c) {
@@ -2020,37 +2025,49 @@ static bool batch_compatible(const BatchKey &k, const ddx_ctx *c) {
 static const char *kBatchMismatch =
     "batch members need one device, equal dt, spacing, storage format and scales, and no CPML stream overlap";
 
+// Whether the tables of a [velocity, stress] pair of shapes exist on c.
+static bool has_tables(const ddx_ctx *c, const Tiling *brick) {
+  return cached_phy_tables(c, brick[0], 0) && cached_phy_tables(c, brick[1], 0);
+}
+
+// Host copies of m's tables for k.brick[large] (built when they do not exist).
+static bool member_tables(const BatchKey &k, int large, BatchMember &m) {
+  for (int kernel = 0; kernel < 2; kernel++) {
+    HostTable<PhyDesc> &h = m.h[large][kernel];
+    if (!h.d.empty()) continue;
+    const PhyTables *t = phy_tables(m.c, k.brick[large][kernel], 0);
+    if (!t) return false;
+    h = host_table(t->set[0]);
+  }
+  return true;
+}
+
 // Ready a context to join a batch: seismogram buffer, zeroed wavefields,
-// tables of the batch's brick shapes (host copies).
-// noalloc: allocate nothing -- the seismogram buffer and the tables of the
-// batch's brick shapes must exist already (DDX_ESTATE otherwise).
-static int batch_prepare(ddx_ctx *c, int ishot, const BatchKey &k, BatchMember &m, bool noalloc = false) {
+// tables of the batch's brick shapes k.brick[large] (host copies).
+// noalloc: allocate nothing -- the seismogram buffer and the tables must
+// exist already (DDX_ESTATE otherwise).
+static int batch_prepare(ddx_ctx *c, int ishot, const BatchKey &k, BatchMember &m, int large, bool noalloc = false) {
   if (int rc = check_ready(c, ishot)) return rc;
   if (noalloc) {
     if (!c->seis[ishot]) {
       c->err = "no seismogram buffer for this shot yet (run ddx_model_shot or ddx_set_observed on it once)";
       return DDX_ESTATE;
     }
-    if (!cached_phy_tables(c, k.tv, 0) || !cached_phy_tables(c, k.ts, 0)) {
+    if (!has_tables(c, k.brick[large])) {
       c->err = "the tables of the batch's brick shapes are not built on this context yet (run one shot with them)";
       return DDX_ESTATE;
     }
   }
   if (int rc = ensure_seis(c, ishot)) return rc;
   if (int rc = ddx_reset_wave(c, 0)) return rc;
-  // build both shapes first: building one may move the other in the cache
-  if (!phy_tables(c, k.tv, 0) || !phy_tables(c, k.ts, 0)) return DDX_EHIP;
-  const PhyTables *a = phy_tables(c, k.tv, 0);
-  const PhyTables *b = phy_tables(c, k.ts, 0);
-  m.hv = host_table(a->set[0]);
-  m.hs = host_table(b->set[0]);
+  m.c = c;
+  if (!member_tables(k, large, m)) return DDX_EHIP;
   m.hp = host_table(c->pml[0][0]);
   const hipError_t e = hipStreamSynchronize(c->st);
   if (e != hipSuccess) {
     c->err = std::string("HIP error: ") + hipGetErrorString(e) + " preparing a batch member";
     return DDX_EHIP;
   }
-  m.c = c;
   m.ishot = ishot;
   m.it = 0;
   return DDX_OK;
@@ -2066,6 +2083,7 @@ struct FusedSet {
   FusedTable<PhyDesc> v, s;
   FusedTable<SlabDesc> p, pw;  // CPML: split for launches of their own, for whole half steps
   FusedTable<MemberIO> io;  // sources and receivers of the members
+  Tiling tv, ts;            // brick shapes of v and s
   bool whole = false;       // the half steps may run as one launch each
   double cells = 0;
 };
@@ -2075,7 +2093,8 @@ struct FusedHost {
   HostTable<SlabDesc> p;
   HostTable<MemberIO> io;
 };
-static void fuse_host(std::vector<BatchMember> &ms, FusedHost &f) {
+// large: of the shapes BatchKey::brick[1].
+static void fuse_host(std::vector<BatchMember> &ms, int large, FusedHost &f) {
   std::vector<const HostTable<PhyDesc> *> pv, ps;
   std::vector<const HostTable<SlabDesc> *> pp;
   // one MemberIO part per member (its receiver blocks), so upload_fused
@@ -2084,10 +2103,10 @@ static void fuse_host(std::vector<BatchMember> &ms, FusedHost &f) {
   std::vector<const HostTable<MemberIO> *> pio;
   for (size_t q = 0; q < ms.size(); q++) {
     BatchMember &m = ms[q];
-    set_member(m.hs, (int)q);
+    set_member(m.h[large][1], (int)q);
     set_member(m.hp, (int)q);
-    pv.push_back(&m.hv);
-    ps.push_back(&m.hs);
+    pv.push_back(&m.h[large][0]);
+    ps.push_back(&m.h[large][1]);
     pp.push_back(&m.hp);
     MemberIO x = member_io(m.c, m.ishot, 0);
     x.join = m.join;
@@ -2114,10 +2133,20 @@ static bool batch_whole(const std::vector<BatchMember> &ms, double &cells) {
   }
   return ok && cells <= c0->whole_cells;
 }
-static hipError_t fuse_members(std::vector<BatchMember> &ms, FusedSet &f) {
-  FusedHost h;
-  fuse_host(ms, h);
+// The shapes, and whether the half steps run whole, by the members' cells.
+static int fused_shapes(const BatchKey &k, const std::vector<BatchMember> &ms, FusedSet &f) {
   f.whole = batch_whole(ms, f.cells);
+  const int large = f.cells > k.whole_cells;
+  f.tv = k.brick[large][0];
+  f.ts = k.brick[large][1];
+  return large;
+}
+static hipError_t fuse_members(const BatchKey &k, std::vector<BatchMember> &ms, FusedSet &f) {
+  FusedHost h;
+  const int large = fused_shapes(k, ms, f);
+  for (BatchMember &m : ms)
+    if (!member_tables(k, large, m)) return hipErrorOutOfMemory;
+  fuse_host(ms, large, h);
   HostTable<SlabDesc> pw = h.p;
   if (f.whole) pw.nblk = split_pml(pw.d, pw.s, pml_whole(ms[0].c->fmt));
   hipError_t e = upload_owned(h.v, f.v);
@@ -2139,8 +2168,8 @@ static HalfStep half_of(const BatchKey &k, const FusedTable<PhyDesc> &p, const F
 static bool fused_step(const BatchKey &k, const FusedSet &f, const std::vector<BatchMember> &ms, int gs,
                        hipStream_t st, const int *gsp = nullptr) {
   const float rvs = std::ldexp(1.0f, k.lg0 - k.lg1), rsv = std::ldexp(1.0f, k.lg1 - k.lg0);
-  if (!f.whole || !k.tv.whole || !launch_vel_all(k.tv, PURE_FORWARD, k.fmt, half_of(k, f.v, f.pw, rvs, f.cells), st)) {
-    if (!launch_vel_phy(k.tv, PURE_FORWARD, k.fmt, f.v.d, f.v.starts, f.v.n, f.v.nblk, k.dx, k.dy, k.dz, rvs,
+  if (!f.whole || !f.tv.whole || !launch_vel_all(f.tv, PURE_FORWARD, k.fmt, half_of(k, f.v, f.pw, rvs, f.cells), st)) {
+    if (!launch_vel_phy(f.tv, PURE_FORWARD, k.fmt, f.v.d, f.v.starts, f.v.n, f.v.nblk, k.dx, k.dy, k.dz, rvs,
                         k.brick_group, st))
       return false;
     launch_vel_pml(k.pml_cz, k.fmt, f.p.d, f.p.starts, f.p.n, f.p.nblk, k.dx, k.dy, k.dz, rvs, k.pml_group,
@@ -2154,9 +2183,9 @@ static bool fused_step(const BatchKey &k, const FusedSet &f, const std::vector<B
   io.nblk = f.io.nblk;
   io.gs = gs;
   io.gsp = gsp;
-  if (!f.whole || !k.ts.whole || !launch_stress_all(k.ts, PURE_FORWARD, k.fmt, half_of(k, f.s, f.pw, k.dt * rsv, f.cells), io, st)) {
+  if (!f.whole || !f.ts.whole || !launch_stress_all(f.ts, PURE_FORWARD, k.fmt, half_of(k, f.s, f.pw, k.dt * rsv, f.cells), io, st)) {
     launch_source_batch(k.fmt, f.io.d, f.io.n, gs, gsp, st);
-    if (!launch_stress_phy(k.ts, PURE_FORWARD, k.fmt, f.s.d, f.s.starts, f.s.n, f.s.nblk, k.dx, k.dy, k.dz,
+    if (!launch_stress_phy(f.ts, PURE_FORWARD, k.fmt, f.s.d, f.s.starts, f.s.n, f.s.nblk, k.dx, k.dy, k.dz,
                            k.dt * rsv, k.brick_group, st))
       return false;
     launch_stress_pml(k.pml_cz, 0, k.fmt, f.p.d, f.p.starts, f.p.n, f.p.nblk, k.dx, k.dy, k.dz, k.dt * rsv,
@@ -2229,7 +2258,8 @@ extern "C" int ddx_model_batch(ddx_ctx *const *ctxs, const int *ishots, int n) {
   for (int q = 0; q < n; q++)
     if (!ctxs[q]) return DDX_EINVAL;
   ddx_ctx *c0 = ctxs[0];
-  const BatchKey k = batch_key(c0, batch_cells(ctxs, n));
+  const BatchKey k = batch_key(c0);
+  const int large = batch_cells(ctxs, n) > k.whole_cells;
   HIPCHECK(c0, hipSetDevice(k.device));
   std::vector<BatchMember> ms(n);
   for (int q = 0; q < n; q++) {
@@ -2240,13 +2270,13 @@ extern "C" int ddx_model_batch(ddx_ctx *const *ctxs, const int *ishots, int n) {
       c0->err = std::string(kBatchMismatch) + ", and equal ntime";
       return DDX_EINVAL;
     }
-    if (int rc = batch_prepare(c, ishots[q], k, ms[q])) {
+    if (int rc = batch_prepare(c, ishots[q], k, ms[q], large)) {
       if (q) c0->err = "batch member " + std::to_string(q) + ": " + c->err;
       return rc;
     }
   }
   FusedSet f;
-  HIPCHECK(c0, fuse_members(ms, f));
+  HIPCHECK(c0, fuse_members(k, ms, f));
   const int nt = c0->d.ntime;
   if (int rc = run_fused(k, f, ms, 0, nt, c0->st, c0->d_it, c0->use_graph && c0->prof.mask == 0, c0->err)) return rc;
   for (BatchMember &m : ms) m.it = nt;
@@ -2305,11 +2335,10 @@ static void view(FusedTable<T> &t, const HostTable<T> &h, unsigned char *dev, si
 }
 
 // The fused tables of ms copied into scratch (dev) on stream st; f gets views.
-static int fuse_into_scratch(std::vector<BatchMember> &ms, FusedSet &f, unsigned char *dev, hipStream_t st,
-                             std::string &err) {
+static int fuse_into_scratch(const BatchKey &k, std::vector<BatchMember> &ms, FusedSet &f, unsigned char *dev,
+                             hipStream_t st, std::string &err) {
   FusedHost h;
-  fuse_host(ms, h);
-  f.whole = batch_whole(ms, f.cells);
+  fuse_host(ms, fused_shapes(k, ms, f), h);
   std::vector<PmlPiece> pieces;
   PmlOrder ord;
   pml_order_host(h.p.d, ms[0].c->pml_cz, pieces, ord);
@@ -2347,14 +2376,12 @@ extern "C" int ddx_model_batch_noalloc(ddx_ctx *const *ctxs, const int *ishots, 
   for (int q = 0; q < n; q++)
     if (!ctxs[q]) return DDX_EINVAL;
   ddx_ctx *c0 = ctxs[0];
-  BatchKey k = batch_key(c0, batch_cells(ctxs, n));
+  BatchKey k = batch_key(c0);
+  const int large = batch_cells(ctxs, n) > k.whole_cells;
   // a shot of a member's own may not build the tables of the shapes for
   // separate launches: then those of ctxs[0]'s own shots
   for (int q = 0; q < n; q++)
-    if (!cached_phy_tables(ctxs[q], k.tv, 0) || !cached_phy_tables(ctxs[q], k.ts, 0)) {
-      k = batch_key(c0, 0);
-      break;
-    }
+    if (!has_tables(ctxs[q], k.brick[1])) std::copy(k.brick[0], k.brick[0] + 2, k.brick[1]);
   HIPCHECK(c0, hipSetDevice(k.device));
   unsigned char *dev = nullptr;
   if (int rc = scratch_of(k.device, &dev, c0->err)) return rc;
@@ -2367,13 +2394,13 @@ extern "C" int ddx_model_batch_noalloc(ddx_ctx *const *ctxs, const int *ishots, 
       c0->err = std::string(kBatchMismatch) + ", and equal ntime";
       return DDX_EINVAL;
     }
-    if (int rc = batch_prepare(c, ishots[q], k, ms[q], true)) {
+    if (int rc = batch_prepare(c, ishots[q], k, ms[q], large, true)) {
       if (q) c0->err = "batch member " + std::to_string(q) + ": " + c->err;
       return rc;
     }
   }
   FusedSet f;
-  if (int rc = fuse_into_scratch(ms, f, dev, c0->st, c0->err)) return rc;
+  if (int rc = fuse_into_scratch(k, ms, f, dev, c0->st, c0->err)) return rc;
   const int nt = c0->d.ntime;
   if (int rc = run_fused(k, f, ms, 0, nt, c0->st, nullptr, false, c0->err)) return rc;
   HIPCHECK(c0, hipGetLastError());
@@ -2616,7 +2643,7 @@ extern "C" int ddx_rtm_batch(ddx_ctx *const *ctxs, const int *ishots, int n) {
   for (int q = 0; q < n; q++)
     if (!ctxs[q]) return DDX_EINVAL;
   ddx_ctx *c0 = ctxs[0];
-  const BatchKey k = batch_key(c0, batch_cells(ctxs, n));
+  const BatchKey k = batch_key(c0);
   HIPCHECK(c0, hipSetDevice(k.device));
   std::vector<ddx_ctx *> cs(ctxs, ctxs + n);
   std::vector<int> shots(ishots, ishots + n);
@@ -2721,7 +2748,7 @@ extern "C" int ddx_batch_add(ddx_batch *b, ddx_ctx *c, int ishot) {
     if (d == c) { b->err = "the context's finished shot has not been collected"; return DDX_EINVAL; }
   // the first member to join sets what the others must share
   const bool first = !b->keyed;
-  const BatchKey key = first ? batch_key(c, ext_cells(c)) : b->key;
+  const BatchKey key = first ? batch_key(c) : b->key;
   if (!batch_compatible(key, c)) {
     b->err = kBatchMismatch;
     return DDX_EINVAL;
@@ -2731,7 +2758,7 @@ extern "C" int ddx_batch_add(ddx_batch *b, ddx_ctx *c, int ishot) {
   if (e == hipSuccess && !b->d_step) e = hipMalloc((void **)&b->d_step, sizeof(int));
   if (e != hipSuccess) { b->err = std::string("HIP: ") + hipGetErrorString(e); return DDX_EHIP; }
   BatchMember m;
-  if (int rc = batch_prepare(c, ishot, key, m)) {
+  if (int rc = batch_prepare(c, ishot, key, m, 0)) {
     b->err = c->err;
     return rc;
   }
@@ -2756,7 +2783,7 @@ extern "C" int ddx_batch_add_rtm(ddx_batch *b, ddx_ctx *c, int ishot) {
   for (ddx_ctx *d : b->done)
     if (d == c) { b->err = "the context's finished shot has not been collected"; return DDX_EINVAL; }
   const bool first = !b->keyed;
-  const BatchKey key = first ? batch_key(c, ext_cells(c)) : b->key;
+  const BatchKey key = first ? batch_key(c) : b->key;
   if (!batch_compatible(key, c) || c->set_overlap || (b->image_fp64 >= 0 && c->d.image_fp64 != b->image_fp64)) {
     b->err = std::string(kBatchMismatch) + ", one image precision for the RTM members, and no reverse-set overlap";
     return DDX_EINVAL;
@@ -2848,7 +2875,7 @@ extern "C" int ddx_batch_run(ddx_batch *b, int max_steps, ddx_ctx **done, int ca
     if (b->dirty) {
       b->graph.reset();
       if (!b->members.empty()) {
-        const hipError_t e = fuse_members(b->members, b->fused);
+        const hipError_t e = fuse_members(b->key, b->members, b->fused);
         if (e != hipSuccess) { b->err = std::string("HIP: ") + hipGetErrorString(e); return DDX_EHIP; }
       }
       b->dirty = false;

@@ -219,3 +219,44 @@ def test_cpml_division_by_small_spacings(spacing, values, whole, cz, monkeypatch
     for cols in (slice(2, pml), slice(pml + nx, nx + 2 * pml - 2)):
         assert np.array_equal(v[k - 1, rows, cols], want[rows, cols])
         assert np.array_equal(v[k, rows, cols], -want[rows, cols])
+
+
+@pytest.mark.parametrize("storage", ["fp32", "bf16"])
+def test_continuous_batch_across_the_one_launch_limit(storage, monkeypatch):
+    """Members join and leave so that a continuous batch lies below, above and
+    again below the cells up to which half steps run as one launch: modelling
+    and RTM members equal their single shots."""
+    c = case(nx=70, ny=18, nz=20, pml=6, ntime=24, rec_width=2)
+    d = case(nx=41, ny=22, nz=20, pml=6, ntime=36, rec_width=2, seed=3)
+    monkeypatch.setenv("DDX_WHOLE_CELLS", str(int(1.5 * (70 + 12) * (18 + 12) * (20 + 12))))
+    es = [engine(x, storage) for x in (c, d, c, d)]
+    es[0].autotune(reps=1)
+    want = []
+    for e in es:
+        e.model_shot(0)
+        want.append(e.seismograms(0))
+    for e in es[2:]:
+        e.rtm_shot(0)
+    images = [[e.image(i, 0) for i in range(5)] for e in es[2:]]
+    for e in es[2:]:
+        e.reset_images()
+    b = ddx.Batch()
+    done = []
+    b.add(es[0])
+    done += b.run(5)
+    b.add(es[1])
+    done += b.run(5)
+    b.add(es[2], rtm=True)
+    done += b.run(5)
+    b.add(es[3], rtm=True)
+    while len(b):
+        done += b.run(50)
+    assert len(done) == 4
+    for e, w in zip(es[:2], want):
+        assert np.array_equal(e.seismograms(0), w)
+    for e, w in zip(es[2:], images):
+        for i in range(5):
+            assert np.array_equal(e.image(i, 0), w[i]), i
+    b.close()
+    for e in es:
+        e.close()
