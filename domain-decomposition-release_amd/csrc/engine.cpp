@@ -327,6 +327,7 @@ struct ddx_ctx {
   // and that of the physical region in a launch of its own, where it differs
   // (batches too large for whole half steps): [velocity, stress]
   Tiling apart[2][kModes];
+  bool own_back[2] = {false, false};  // the caller set the backward mode's shape
   // device memory
   std::vector<void *> allocs;
   std::vector<size_t> alloc_bytes;  // size of each allocation in allocs
@@ -2423,8 +2424,12 @@ static int rtm_begin(ddx_ctx *c, int ishot);
 static void ring(ddx_ctx *c, int dir, int which, int it, hipStream_t st = nullptr);
 static int ring_status(ddx_ctx *c, std::string &err);
 
-// Whether bricks of these shapes run the halves of a reverse iteration in one launch each.
+// Whether bricks of these shapes (the reverse mode's) run the halves of a
+// reverse iteration in one launch each, the backward stress in the velocity's
+// and the other way round; not against a backward shape that the caller set.
 static bool rev_shapes(const ddx_ctx *c, const Tiling &tv, const Tiling &ts) {
+  if (c->own_back[1] && !same_tiling(c->tiling_stress[RTM_BACKWARD], tv)) return false;
+  if (c->own_back[0] && !same_tiling(c->tiling_vel[RTM_BACKWARD], ts)) return false;
   return tv.whole && ts.whole && tv.cy == 1 && ts.cy == 1 && whole_shape(tv, c->fmt) && whole_shape(ts, c->fmt);
 }
 
@@ -3510,6 +3515,7 @@ extern "C" int ddx_set_tiling_mode(ddx_ctx *c, int kernel, int mode, int tx, int
   }
   HIPCHECK(c, hipStreamSynchronize(c->st));
   set_brick(c, kernel, mode, t);
+  if (mode == RTM_BACKWARD) c->own_back[kernel] = true;
   for (int m = 0; m < 2; m++)
     if (c->model[m] && !phy_tables(c, t, m)) return DDX_EHIP;
   return DDX_OK;
@@ -3568,6 +3574,7 @@ extern "C" int ddx_autotune(ddx_ctx *c, int reps, int *timed) {
   for (int kernel = 0; kernel < 2 && !rc; kernel++)
     for (int mode = 0; mode < kModes && !rc; mode++) {
       if (mode == FWI) continue;  // FWI keeps its one-cell brick
+      if (mode == RTM_BACKWARD) c->own_back[kernel] = false;
       Tiling &slot = (kernel == 0 ? c->tiling_vel : c->tiling_stress)[mode];
       const std::string key = tune_key(c, kernel, mode);
       {
@@ -3643,6 +3650,7 @@ extern "C" int ddx_set_brick(ddx_ctx *c, int kernel, int mode, int tx, int ty, i
   }
   HIPCHECK(c, hipStreamSynchronize(c->st));
   set_brick(c, kernel, mode, t);
+  if (mode == RTM_BACKWARD) c->own_back[kernel] = true;
   for (int m = 0; m < 2; m++)
     if (c->model[m] && !phy_tables(c, t, m)) return DDX_EHIP;
   return DDX_OK;

@@ -271,8 +271,10 @@ int ddx_set_tiling_mode(ddx_ctx *ctx, int kernel, int mode, int tx, int ty, int 
  * (64,2,1,8), FP32 storage; 4 form 3 with the y arm read from an LDS tile
  * of the block's rows, shapes (64,ty,1,kz) for ty in {4, 8, 16} and kz in
  * {2, 4}, FP32 storage.  Forms 2 to 4 do not run the FWI mode.
- * ddx_get_brick returns the shape in use as tx, ty, cy, kz, px.  No
- * reference counterpart. */
+ * ddx_get_brick returns the shape set, tuned or taken by default as tx, ty,
+ * cy, kz, px.  (RTM on small grids runs the backward bricks in the launches
+ * of the reverse half steps and in their shapes, unless the backward mode was
+ * given another shape by one of these calls.)  No reference counterpart. */
 int ddx_set_brick(ddx_ctx *ctx, int kernel, int mode, int tx, int ty, int cy, int kz, int px);
 int ddx_get_brick(const ddx_ctx *ctx, int kernel, int mode, int *out5);
 /* Brick autotuner (no reference counterpart): for each physical-region

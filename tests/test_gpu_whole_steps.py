@@ -260,3 +260,31 @@ def test_continuous_batch_across_the_one_launch_limit(storage, monkeypatch):
     b.close()
     for e in es:
         e.close()
+
+
+@pytest.mark.parametrize("storage", ["fp32", "bf16"])
+def test_backward_bricks_of_their_own(storage):
+    """RTM with a shape set for the backward mode that is not the reverse
+    mode's, alone and as a batch: the images of the default shapes."""
+    c = case(nx=70, ny=21, nz=19, pml=6, ntime=30, rec_width=2)
+    shapes = [None, ((64, 4, 1, 4, 1), (64, 2, 1, 8, 1)), ((64, 4, 1, 2, 2), (64, 2, 1, 4, 2))]
+    ref = None
+    for shape in shapes:
+        es = [engine(c, storage) for _ in range(2)]
+        for e in es:
+            if shape is not None:
+                for k in (0, 1):
+                    e.set_brick(k, po.RTM_BACKWARD, *shape[k])
+                    assert e.brick(k, po.RTM_BACKWARD) == shape[k]
+            e.model_shot(0)
+        es[0].rtm_shot(0)
+        out = [es[0].image(i, 0) for i in range(5)]
+        es[0].reset_images()
+        ddx.rtm_batch(es)
+        out += [e.image(i, 0) for e in es for i in range(5)]
+        for e in es:
+            e.close()
+        if ref is None:
+            ref = out
+        for a, b in zip(ref, out):
+            assert np.array_equal(a, b), shape
