@@ -658,9 +658,10 @@ static const Tiling &brick_for(const ddx_ctx *c, int kernel, int mode, double ce
 // paired bricks, rows of 64 pairs where they waste no more lanes than rows of
 // 32 by over 5% (161x150x131 in BF16, 60 steps, rows of 64 pairs against 32:
 // 17.1 / 14.9 ms).
+static bool narrow_rows(int nx) { return (nx + 63) / 64 * 64 > 1.05 * ((nx + 31) / 32 * 32); }
 static void default_bricks(ddx_ctx *c) {
-  const int nx = c->d.nx, w64 = (nx + 63) / 64 * 64, w32 = (nx + 31) / 32 * 32;
-  const bool narrow = w64 > 1.05 * w32;
+  const int nx = c->d.nx, w64 = (nx + 63) / 64 * 64;
+  const bool narrow = narrow_rows(nx);
   Tiling t{64, 4, 1, 2}, f{64, 4, 1, 2};
   if (c->fmt != STORE_F32) {
     // pairs: a row of 128 cells or of 64, by the lanes they leave idle
@@ -3560,9 +3561,12 @@ extern "C" int ddx_autotune(ddx_ctx *c, int reps, int *timed) {
   if (!c || reps < 1 || reps > 100) return DDX_EINVAL;
   if (!c->have_model) { c->err = "set the model before ddx_autotune"; return DDX_ESTATE; }
   HIPCHECK(c, hipStreamSynchronize(c->st));
-  // The velocity bricks' LDS y arm is ahead on large grids only (676x676x210:
-  // 80.2 ms of 20 steps with it, 82.0 without; RTM of 88^3: 21.6 and 21.7).
-  const bool small = ext_cells(c) <= kWholeCells;
+  // Whole half steps are offered the velocity bricks' LDS y arm by
+  // default_bricks' rule: where rows of 64 leave idle lanes, rows of 32 are
+  // ahead of it (192^3 with 15 layers, 40 modelling steps: 16.2 ms with it,
+  // 16.5 without; 64^3 1.60 either way).  Not in the reverse mode, whose shape
+  // the backward bricks share, which the timing does not see.
+  const bool narrow = narrow_rows(c->d.nx);
   Tiling cand[64];
   const int nc = std::min(tiling_list(c->fmt, cand, 64), 64);
   hipEvent_t e0, e1;
@@ -3586,14 +3590,16 @@ extern "C" int ddx_autotune(ddx_ctx *c, int reps, int *timed) {
           continue;
         }
       }
-      float best = 1e30f;
-      Tiling bt = slot;
+      const Tiling was = slot;
+      const auto offered = [&](const Tiling &t) { return kernel != 0 || t.xl != 2 || (!narrow && mode != RTM_REVERSE); };
+      float best = 1e30f, best_offered = 1e30f;
+      Tiling bt = slot, apart_offered = slot;
       for (int q = 0; q < nc && !rc; q++) {
-        if (kernel == 0 && cand[q].xl == 2 && small) continue;
         float ms = 0.f;
         if ((rc = time_launches(c, e0, e1, reps, ms, [&] { return phy_launch(c, kernel, 0, mode, cand[q]); }))) break;
         count++;
         if (ms < best) { best = ms; bt = cand[q]; }
+        if (ms < best_offered && offered(cand[q])) { best_offered = ms; apart_offered = cand[q]; }
       }
       const Tiling apart = bt;
       // the whole half step (CPML cells too): that brick and the CPML kernel
@@ -3601,9 +3607,9 @@ extern "C" int ddx_autotune(ddx_ctx *c, int reps, int *timed) {
       if (!rc && mode != RTM_BACKWARD && c->pml[model_for(c, mode)][0].cells + phy_cells(c) <= c->whole_cells) {
         float whole_best = 1e30f;
         for (int q = -1; q < nc && !rc; q++) {
-          Tiling t = q < 0 ? apart : cand[q];
+          Tiling t = q < 0 ? apart_offered : cand[q];
           t.whole = q >= 0;
-          if (q >= 0 && (!whole_shape(t, c->fmt) || (kernel == 0 && t.xl == 2))) continue;
+          if (q >= 0 && (!whole_shape(t, c->fmt) || !offered(t))) continue;
           slot = t;
           float ms = 0.f;
           rc = time_launches(c, e0, e1, reps, ms, [&] { return kernel == 0 ? vel_update(c, 0, mode) : stress_update(c, 0, mode); });
@@ -3611,8 +3617,8 @@ extern "C" int ddx_autotune(ddx_ctx *c, int reps, int *timed) {
           if (!rc && ms < whole_best) { whole_best = ms; bt = t; }
         }
       }
+      slot = rc ? was : bt;
       if (rc) break;
-      slot = bt;
       c->apart[kernel][mode] = apart;
       std::lock_guard<std::mutex> lk(g_tune_mu);
       g_tune_cache[key] = {apart, bt};

@@ -288,3 +288,20 @@ def test_backward_bricks_of_their_own(storage):
             ref = out
         for a, b in zip(ref, out):
             assert np.array_equal(a, b), shape
+
+
+def test_autotune_times_every_shape(monkeypatch):
+    """Every brick shape of the format is timed in launches of its own, on
+    small grids too."""
+    monkeypatch.setenv("DDX_WHOLE_CELLS", "0")
+    shapes = 9 + 4 + 5 + 6  # one-cell, paired, lane exchange, LDS y arm
+
+    def timed(c):
+        e = engine(c)
+        n = e.autotune(reps=1)
+        e.close()
+        return n
+
+    a = case(nx=44, ny=50, nz=47, pml=5, ntime=10)
+    assert timed(a) == 2 * 4 * shapes
+    assert timed(a) == 0
