@@ -328,6 +328,7 @@ struct ddx_ctx {
   // (batches too large for whole half steps): [velocity, stress]
   Tiling apart[2][kModes];
   bool own_back[2] = {false, false};  // the caller set the backward mode's shape
+  bool tuned = false;                 // ddx_autotune chose the shapes
   // device memory
   std::vector<void *> allocs;
   std::vector<size_t> alloc_bytes;  // size of each allocation in allocs
@@ -358,6 +359,7 @@ struct ddx_ctx {
   int brick_group = kBrickGroup;     // XCD group size of the bricks' block order
   int whole_group = -1;              // the same of the half steps that run as one launch (columns)
   double whole_cells = kWholeCells;  // half steps of at most so many cells run as one launch
+  double rev_cells = -1;             // and the halves of a reverse iteration (< 0: rev_limit)
   double cached_cells = 0;           // and of at most so many through ordinary accesses (cached_limit)
   int pml_cz = kPmlPairs;            // work split of the CPML kernels
   int pml_group = 32;                // XCD group size of the CPML block order (0: launch order)
@@ -763,6 +765,7 @@ extern "C" int ddx_create(const ddx_desc *desc, ddx_ctx **out) {
     if (v >= 0 && v <= 65536) c->brick_group = c->whole_group = v;
   }
   if (const char *e = getenv("DDX_WHOLE_CELLS")) c->whole_cells = atof(e);  // for sweeps
+  if (const char *e = getenv("DDX_REV_CELLS")) c->rev_cells = atof(e);      // for sweeps
   c->cached_cells = cached_limit(c->fmt);
   if (const char *e = getenv("DDX_CACHED_CELLS")) c->cached_cells = atof(e);  // for sweeps
   default_bricks(c);
@@ -2425,6 +2428,23 @@ static int rtm_begin(ddx_ctx *c, int ishot);
 static void ring(ddx_ctx *c, int dir, int which, int it, hipStream_t st = nullptr);
 static int ring_status(ddx_ctx *c, std::string &err);
 
+// The halves of a reverse iteration run as one launch each up to so many
+// cells; above, the backward bricks are better off alone, in a shape and with
+// registers of their own.  RTM of n^3 grids, 40 steps, halves / separate
+// launches (cells with the layers):
+//   FP32, rows of 64 (default_bricks): 64 (0.8 M) 4.25 / 4.82 ms, 112 (2.9 M)
+//   13.76 / 14.05, 128 with 8 layers (3.0 M) 15.2 / 14.6, 170 (8.0 M) 41.9 /
+//   39.5; tuned 64 4.16 / 4.77, 112 13.81 / 14.01, 128 (3.9 M) 18.65 / 18.64;
+//   rows of 32: 88 (1.6 M) 7.89 / 9.07, 150 (5.8 M) 32.4 / 33.7, 208 (13.5 M)
+//   71.8 / 71.4; tuned, with better backward bricks apart: 88 7.83 / 8.78, 140
+//   (4.9 M) 26.5 / 26.0, 208 71.2 / 67.0;
+//   BF16: 112 13.3 / 14.4, 128 17.9 / 17.9, 140 28.2 / 27.5, 208 85.8 / 79.0.
+static double rev_limit(const ddx_ctx *c, bool tuned) {
+  if (c->rev_cells >= 0) return c->rev_cells;
+  if (c->fmt != STORE_F32) return 4e6;
+  return !narrow_rows(c->d.nx) ? 2.9e6 : tuned ? 4e6 : 6e6;
+}
+
 // Whether bricks of these shapes (the reverse mode's) run the halves of a
 // reverse iteration in one launch each, the backward stress in the velocity's
 // and the other way round; not against a backward shape that the caller set.
@@ -2537,7 +2557,7 @@ static int rtm_batch_tables(const std::vector<ddx_ctx *> &cs, const std::vector<
     if (e == hipSuccess) e = upload_owned(a, T.fpw);
     if (e == hipSuccess) e = upload_owned(b, T.rpw);
   }
-  T.rev = T.rev && T.whole;
+  T.rev = T.rev && T.whole && cells <= rev_limit(c0, c0->tuned);
   for (int k = 0; k < 2 && e == hipSuccess && T.rev; k++) {
     HostTable<PhyDesc> h;
     HostTable<CopyDesc> x;
@@ -3226,25 +3246,33 @@ static int rtm_forward_step(ddx_ctx *c, int ishot, int it) {
   return DDX_OK;
 }
 
-// One reverse iteration it (RTM/rtm3d_blend_elastic_model_mpi_meat.hpp:64-113).
+// A half of a reverse iteration as one launch: the reverse half step of
+// `kernel` and, in its shape t, the backward bricks of the other one.
+struct RevHalf {
+  HalfStep a;
+  BackBricks q;
+};
+static bool rev_half(ddx_ctx *c, int kernel, const Tiling &t, RevHalf &h) {
+  const int model = model_for(c, RTM_REVERSE);  // of the backward modes too
+  const PhyTables *p = phy_tables(c, t, model);
+  const float sc = kernel == 0 ? ratio_vs(c) : c->d.dt * ratio_sv(c);
+  if (!p || !whole_half(c, t, p->set[1], c->pml_whole[model][1], sc, h.a)) return false;
+  const DevTable<PhyDesc> &b = p->set[0];
+  const float bc = kernel == 0 ? -c->d.dt * ratio_sv(c) : -ratio_vs(c);
+  h.q = {b.d, b.starts, b.n, b.nblk, bc, bc / c->d.dx, bc / c->d.dy, bc / c->d.dz};
+  return true;
+}
+
 // The halves of a reverse iteration in one launch each, where the reverse half
 // steps run as one launch anyway and the backward bricks own the source cell:
 // each saves two small launches (4.7 us) and a tail.  False: nothing launched.
 static bool reverse_halves(ddx_ctx *c, int ishot, int it) {
   const Tiling &tv = c->tiling_vel[RTM_REVERSE], &ts = c->tiling_stress[RTM_REVERSE];
-  const int model = model_for(c, RTM_REVERSE);  // of the backward modes too
-  if (!rev_shapes(c, tv, ts) || !source_in_phy(c, ishot) || c->exch_mode == 1 || it > c->store_slices) return false;
-  HalfStep v, s;
-  BackBricks bs, bv;
-  const auto back = [&](const DevTable<PhyDesc> &t, float sc) {
-    return BackBricks{t.d, t.starts, t.n, t.nblk, sc, sc / c->d.dx, sc / c->d.dy, sc / c->d.dz};
-  };
-  const PhyTables *p = phy_tables(c, tv, model);
-  if (!p || !whole_half(c, tv, p->set[1], c->pml_whole[model][1], ratio_vs(c), v)) return false;
-  bs = back(p->set[0], -c->d.dt * ratio_sv(c));
-  p = phy_tables(c, ts, model);
-  if (!p || !whole_half(c, ts, p->set[1], c->pml_whole[model][1], c->d.dt * ratio_sv(c), s)) return false;
-  bv = back(p->set[0], -ratio_vs(c));
+  if (ext_cells(c) > rev_limit(c, c->tuned) || !rev_shapes(c, tv, ts) || !source_in_phy(c, ishot) || c->exch_mode == 1 ||
+      it > c->store_slices)
+    return false;
+  RevHalf v, s;
+  if (!rev_half(c, 0, tv, v) || !rev_half(c, 1, ts, s)) return false;
   StepIO io;
   io.io = c->d_io;
   io.gs = it;
@@ -3252,11 +3280,12 @@ static bool reverse_halves(ddx_ctx *c, int ishot, int it) {
   const DevTable<CopyDesc> &x = c->ring[2], &y = c->ring[1];
   launch_recv_inject(c->fmt, c->d_vptr[1], c->d_rsub, c->d_roff, c->nrec, it, c->d.ntime, c->seis[ishot],
                      scale_of(c, 0), c->st);
-  launch_rev_vel(tv, c->fmt, v, bs, io, {x.d, x.starts, x.n, x.nblk}, c->st);
-  launch_rev_stress(ts, c->fmt, s, bv, io, {y.d, y.starts, y.n, y.nblk}, c->st);
+  launch_rev_vel(tv, c->fmt, v.a, v.q, io, {x.d, x.starts, x.n, x.nblk}, c->st);
+  launch_rev_stress(ts, c->fmt, s.a, s.q, io, {y.d, y.starts, y.n, y.nblk}, c->st);
   return true;
 }
 
+// One reverse iteration it (RTM/rtm3d_blend_elastic_model_mpi_meat.hpp:64-113).
 static int rtm_reverse_step(ddx_ctx *c, int ishot, int it) {
   const int nt = c->d.ntime;
   int rc;
@@ -3564,8 +3593,7 @@ extern "C" int ddx_autotune(ddx_ctx *c, int reps, int *timed) {
   // Whole half steps are offered the velocity bricks' LDS y arm by
   // default_bricks' rule: where rows of 64 leave idle lanes, rows of 32 are
   // ahead of it (192^3 with 15 layers, 40 modelling steps: 16.2 ms with it,
-  // 16.5 without; 64^3 1.60 either way).  Not in the reverse mode, whose shape
-  // the backward bricks share, which the timing does not see.
+  // 16.5 without; 64^3 1.60 either way).
   const bool narrow = narrow_rows(c->d.nx);
   Tiling cand[64];
   const int nc = std::min(tiling_list(c->fmt, cand, 64), 64);
@@ -3591,7 +3619,7 @@ extern "C" int ddx_autotune(ddx_ctx *c, int reps, int *timed) {
         }
       }
       const Tiling was = slot;
-      const auto offered = [&](const Tiling &t) { return kernel != 0 || t.xl != 2 || (!narrow && mode != RTM_REVERSE); };
+      const auto offered = [&](const Tiling &t) { return kernel != 0 || t.xl != 2 || !narrow; };
       float best = 1e30f, best_offered = 1e30f;
       Tiling bt = slot, apart_offered = slot;
       for (int q = 0; q < nc && !rc; q++) {
@@ -3606,13 +3634,22 @@ extern "C" int ddx_autotune(ddx_ctx *c, int reps, int *timed) {
       // apart, against every shape that runs them as one launch
       if (!rc && mode != RTM_BACKWARD && c->pml[model_for(c, mode)][0].cells + phy_cells(c) <= c->whole_cells) {
         float whole_best = 1e30f;
-        for (int q = -1; q < nc && !rc; q++) {
+        // a reverse half step runs with the backward bricks in its launch
+        const bool halves = mode == RTM_REVERSE && ext_cells(c) <= rev_limit(c, true) && c->exch_mode != 1 &&
+                            !c->set_overlap && !c->pml_overlap && c->pml_cz == kPmlPairs && !c->pml_order;
+        for (int q = halves ? 0 : -1; q < nc && !rc; q++) {
           Tiling t = q < 0 ? apart_offered : cand[q];
           t.whole = q >= 0;
           if (q >= 0 && (!whole_shape(t, c->fmt) || !offered(t))) continue;
           slot = t;
           float ms = 0.f;
-          rc = time_launches(c, e0, e1, reps, ms, [&] { return kernel == 0 ? vel_update(c, 0, mode) : stress_update(c, 0, mode); });
+          rc = time_launches(c, e0, e1, reps, ms, [&]() -> int {
+            if (!halves) return kernel == 0 ? vel_update(c, 0, mode) : stress_update(c, 0, mode);
+            RevHalf h;
+            const bool ok = rev_half(c, kernel, t, h) &&
+                            (kernel == 0 ? launch_rev_vel : launch_rev_stress)(t, c->fmt, h.a, h.q, StepIO{}, RingBoxes{}, c->st);
+            return ok ? DDX_OK : DDX_EHIP;
+          });
           count++;
           if (!rc && ms < whole_best) { whole_best = ms; bt = t; }
         }
@@ -3631,6 +3668,7 @@ extern "C" int ddx_autotune(ddx_ctx *c, int reps, int *timed) {
     return rc;
   }
   if (timed) *timed = count;
+  c->tuned = true;
   for (int m = 0; m < 2; m++)  // shapes taken from the cache have no tables yet
     if (c->model[m] && (rc = prepare_phy_tables(c, m))) return rc;
   if ((rc = ddx_reset_wave(c, 0)) || (rc = ddx_reset_wave(c, 1))) return rc;

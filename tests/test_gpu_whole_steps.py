@@ -305,3 +305,26 @@ def test_autotune_times_every_shape(monkeypatch):
     a = case(nx=44, ny=50, nz=47, pml=5, ntime=10)
     assert timed(a) == 2 * 4 * shapes
     assert timed(a) == 0
+
+
+@pytest.mark.parametrize("storage,tuned", [("fp32", False), ("fp32", True), ("bf16", False)])
+def test_reverse_halves_limit_changes_no_image(storage, tuned, monkeypatch):
+    """Whole half steps with the backward bricks in the reverse half steps'
+    launches and in their own, alone and as a batch."""
+    c = case(nx=70, ny=21, nz=19, pml=6, ntime=24, rec_width=2)
+    outs = []
+    for cells in ("0", "1e9"):
+        monkeypatch.setenv("DDX_REV_CELLS", cells)
+        es = [engine(c, storage) for _ in range(2)]
+        for e in es:
+            if tuned:
+                e.autotune(reps=1)
+            e.model_shot(0)
+        es[0].rtm_shot(0)
+        out = [es[0].image(i, 0) for i in range(5)]
+        ddx.rtm_batch(es)
+        outs.append(out + [e.image(i, 0) for e in es for i in range(5)])
+        for e in es:
+            e.close()
+    for a, b in zip(*outs):
+        assert np.array_equal(a, b)
