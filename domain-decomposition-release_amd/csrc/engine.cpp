@@ -3556,19 +3556,35 @@ extern "C" int ddx_set_tiling_mode(ddx_ctx *c, int kernel, int mode, int tx, int
 // propagation mode, time `reps` launches of every z-blocked shape of the
 // context's storage format (one-cell and paired bricks) with HIP events on
 // the context stream, and keep the fastest.  Results are cached per process
-// by storage format and grid size bucket (each gridphy axis rounded up to 32
-// cells), so contexts of similar size reuse them.  The
+// by storage format, grid size bucket (each gridphy axis rounded up to 32
+// cells) and the size limits that the grid is under, so that contexts of
+// similar size reuse them.  The
 // timing launches run on the current wavefields; both sets are reset
 // afterwards.
 static std::mutex g_tune_mu;
 static std::map<std::string, std::pair<Tiling, Tiling>> g_tune_cache;  // a launch of its own, and as used
 
+// Whether the mode's half steps are small enough for one launch (whole_half).
+static bool small_half(const ddx_ctx *c, int mode) {
+  return c->pml[model_for(c, mode)][0].cells + phy_cells(c) <= c->whole_cells;
+}
+// Whether the mode's half steps are timed as halves of a reverse iteration.
+static bool reverse_tuned(const ddx_ctx *c, int mode) {
+  return mode == RTM_REVERSE && ext_cells(c) <= rev_limit(c, true) && c->exch_mode != 1 && !c->set_overlap &&
+         !c->pml_overlap && c->pml_cz == kPmlPairs && !c->pml_order;
+}
+
+// What decides which launches are timed is in the key.  The layers' width is
+// not beyond the limits it brings the grid under or over: a server's requests
+// of uneven widths share their choices.
 static std::string tune_key(const ddx_ctx *c, int kernel, int mode) {
-  char b[160];
+  char b[200];
   int big[3];
   for (int a = 0; a < 3; a++) big[a] = (c->all.pn[a] + 31) / 32 * 32;
-  snprintf(b, sizeof b, "f%d k%d m%d R%d b%dx%dx%d mig%d", c->fmt, kernel, mode,
-           mode == RTM_BACKWARD ? c->d.rec_width : 0, big[0], big[1], big[2], (int)model_for(c, mode));
+  snprintf(b, sizeof b, "f%d k%d m%d R%d b%dx%dx%d mig%d p%d,%d,%d,%d w%d r%d c%d", c->fmt, kernel, mode,
+           mode == RTM_BACKWARD ? c->d.rec_width : 0, big[0], big[1], big[2], (int)model_for(c, mode), c->pml_cz,
+           c->pml_group, c->pml_order, (int)c->pml_overlap, small_half(c, mode), reverse_tuned(c, mode),
+           ext_cells(c) <= c->cached_cells);
   return b;
 }
 
@@ -3622,7 +3638,7 @@ extern "C" int ddx_autotune(ddx_ctx *c, int reps, int *timed) {
       const auto offered = [&](const Tiling &t) { return kernel != 0 || t.xl != 2 || !narrow; };
       float best = 1e30f, best_offered = 1e30f;
       Tiling bt = slot, apart_offered = slot;
-      const bool whole = c->pml[model_for(c, mode)][0].cells + phy_cells(c) <= c->whole_cells;
+      const bool whole = small_half(c, mode);
       for (int q = 0; q < nc && !rc; q++) {
         float ms = 0.f;
         // where shots run in these launches, with the CPML launch in between:
@@ -3645,8 +3661,7 @@ extern "C" int ddx_autotune(ddx_ctx *c, int reps, int *timed) {
       if (!rc && mode != RTM_BACKWARD && whole) {
         float whole_best = 1e30f;
         // a reverse half step runs with the backward bricks in its launch
-        const bool halves = mode == RTM_REVERSE && ext_cells(c) <= rev_limit(c, true) && c->exch_mode != 1 &&
-                            !c->set_overlap && !c->pml_overlap && c->pml_cz == kPmlPairs && !c->pml_order;
+        const bool halves = reverse_tuned(c, mode);
         for (int q = halves ? 0 : -1; q < nc && !rc; q++) {
           Tiling t = q < 0 ? apart_offered : cand[q];
           t.whole = q >= 0;

@@ -281,8 +281,8 @@ int ddx_get_brick(const ddx_ctx *ctx, int kernel, int mode, int *out5);
  * kernel and propagation mode, times `reps` launches of every z-blocked
  * brick shape of the storage format on this context and keeps the fastest,
  * on small grids together with the CPML cells (whole half steps in one
- * launch); cached per process by storage format and grid size (rounded up to
- * 32 cells per axis).  Needs the model; resets both
+ * launch); cached per process by storage format, grid size (rounded up to
+ * 32 cells per axis) and the size limits that the grid is under.  Needs the model; resets both
  * wavefield sets.  *timed (nullable): shapes timed (0 when all came from the
  * cache). */
 int ddx_autotune(ddx_ctx *ctx, int reps, int *timed);

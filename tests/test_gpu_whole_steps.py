@@ -328,3 +328,26 @@ def test_reverse_halves_limit_changes_no_image(storage, tuned, monkeypatch):
             e.close()
     for a, b in zip(*outs):
         assert np.array_equal(a, b)
+
+
+def test_autotune_cache_is_keyed_by_what_decides(monkeypatch):
+    """Contexts share a tuner's choice where the same launches were timed for
+    it only: not across the limits up to which half steps, and the halves of a
+    reverse iteration, run as one launch."""
+
+    def timed(**kw):
+        e = engine(case(nx=60, ny=50, nz=47, ntime=10, **kw))
+        n = e.autotune(reps=1)
+        e.close()
+        return n
+
+    monkeypatch.setenv("DDX_WHOLE_CELLS", str(65 * 55 * 52))  # of the cells that half steps update
+    monkeypatch.setenv("DDX_REV_CELLS", "0")
+    timed(pml=5)
+    assert timed(pml=5) == 0
+    assert timed(pml=4) > 0  # small enough for whole half steps
+    monkeypatch.setenv("DDX_WHOLE_CELLS", "1e9")
+    assert timed(pml=5) == 0  # as that one
+    monkeypatch.setenv("DDX_REV_CELLS", "1e9")
+    assert timed(pml=5) > 0
+    assert timed(pml=4) == 0
