@@ -375,6 +375,8 @@ struct ddx_ctx {
   bool have_mirror = false;  // mode 2 may be selected (DDX_MIRROR=1 at creation, and a neighbour)
   DevTable<CopyDesc> cmm_pack[2][3], cmm_unpack[2][3];  // [set][batch], built on first use of mode 1
   char *cmm_block[2][3] = {};                           // the blocks of a set and batch, link after link
+  bool cmm_check = false;    // DDX_CMM_CHECK=1 at creation: the ghosts are overwritten with NaN (from
+  char *cmm_nan = nullptr;   // a block of them) before each unpack, which then has to bring all of them
   // snapshots of one field of set 0 during ddx_rtm_shot (gridphy of every
   // subdomain, rank after rank): [pass][index] device blocks
   int snap_field = -1, snap_every = 0, snap_count = 0;
@@ -725,6 +727,7 @@ extern "C" int ddx_create(const ddx_desc *desc, ddx_ctx **out) {
   {  // exchange mode 2 is offered, and the default, with DDX_MIRROR=1 and a neighbour
     const char *e = getenv("DDX_MIRROR");
     c->have_mirror = c->nsub > 1 && e && atoi(e) == 1;
+    if (const char *k = getenv("DDX_CMM_CHECK")) c->cmm_check = atoi(k) == 1;
     if (c->have_mirror) c->exch_mode = 2;
   }
   hipError_t he = hipSetDevice(d.device);
@@ -1421,6 +1424,7 @@ static const int kBatchFields[3][8] = {{VX, VY, VZ, -1}, {SXX, SYY, SZZ, SXY, SX
 static int build_cmm(ddx_ctx *c) {
   if (c->cmm_pack[0][0].d || c->cmm_block[0][0]) return DDX_OK;
   const int S = c->nsub;
+  long most = 0;
   for (int batch = 0; batch < 3; batch++)
     for (int set = 0; set < 2; set++) {
       std::vector<CopyDesc> hp, hu;
@@ -1469,7 +1473,13 @@ static int build_cmm(ddx_ctx *c) {
       c->cmm_pack[set][batch].bytes = c->cmm_unpack[set][batch].bytes = 2.0 * c->esz * off;
       if (off > 0)
         if (int rc = dalloc(c, (void **)&c->cmm_block[set][batch], (size_t)c->esz * off)) return rc;
+      most = std::max(most, off);
     }
+  if (c->cmm_check && most > 0) {
+    if (int rc = dalloc(c, (void **)&c->cmm_nan, (size_t)c->esz * most)) return rc;
+    HIPCHECK(c, hipMemsetAsync(c->cmm_nan, 0xff, (size_t)c->esz * most, c->st));  // a NaN in every format
+    HIPCHECK(c, hipStreamSynchronize(c->st));
+  }
   return DDX_OK;
 }
 
@@ -1483,6 +1493,7 @@ static void exchange_on(ddx_ctx *c, int set, int batch, hipStream_t st) {
   if (p.nblk == 0) return;
   ProfScope ps(c, 4, p.bytes + u.bytes, st);
   launch_copy(+1, c->esz, p.d, p.starts, p.n, p.nblk, c->cmm_block[set][batch], st);
+  if (c->cmm_nan) launch_copy(-1, c->esz, u.d, u.starts, u.n, u.nblk, c->cmm_nan, st);
   launch_copy(-1, c->esz, u.d, u.starts, u.n, u.nblk, c->cmm_block[set][batch], st);
 }
 
@@ -3026,11 +3037,11 @@ extern "C" int ddx_set_graphs(ddx_ctx *c, int on) {
 extern "C" int ddx_set_exchange(ddx_ctx *c, int mode) {
   if (!c) return DDX_EINVAL;
   if (mode < 0 || mode > 2) {
-    c->err = "exchange mode must be 0 (direct copy), 1 (CMM message blocks) or 2 (pack on store)";
+    c->err = "exchange mode must be 0 (nothing to move), 1 (CMM message blocks) or 2 (as 0)";
     return DDX_EINVAL;
   }
   if (mode == 2 && !c->have_mirror) {
-    c->err = "pack on store needs neighbouring subdomains and the mirror tables (DDX_MIRROR=1 at creation)";
+    c->err = "exchange mode 2 needs neighbouring subdomains and DDX_MIRROR=1 in the environment at creation";
     return DDX_EINVAL;
   }
   if (mode == 1)
