@@ -53,10 +53,14 @@ HBM_PEAK_GBS = 8000.0
 METRIC = "Gcell-updates/s + shots/s, 1 MI355X, vs plain FP32; p50/p99 shot latency"
 KERNEL_NAMES = {0: "velocity update, physical region (k_vel_phy)", 1: "stress update, physical region (k_stress_phy)",
                 2: "CPML velocity (k_vel_pml)", 3: "CPML stress (k_stress_pml)", 4: "CMM halo exchange (k_copy, mode 1)",
-                5: "imaging (k_image)"}
+                5: "imaging (k_image)",
+                # grids of up to 14 M cells (the in-process classes time these half steps as separate launches)
+                6: "velocity half steps in one launch (k_vel_all, k_rev_vel)",
+                7: "stress half steps in one launch (k_stress_all, k_rev_stress)"}
 # kernel-name prefixes of each class, as rocprofv3 reports them
 KERNEL_PREFIX = {0: ("ddx::k_vel_phy", "ddx::k_vel_lds"), 1: ("ddx::k_stress_phy", "ddx::k_stress_lds"),
-                 2: ("ddx::k_vel_pml",), 3: ("ddx::k_stress_pml",), 4: (), 5: ("ddx::k_image",)}
+                 2: ("ddx::k_vel_pml",), 3: ("ddx::k_stress_pml",), 4: (), 5: ("ddx::k_image",),
+                 6: ("ddx::k_vel_all", "ddx::k_rev_vel"), 7: ("ddx::k_stress_all", "ddx::k_rev_stress")}
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic.json")
 KERNEL_SRC = os.path.join(ROOT, "domain-decomposition-release_amd", "csrc", "kernels.hip")
 
@@ -207,8 +211,11 @@ def pmc_summary(fetch_db, write_db, workload):
     per_class = defaultdict(lambda: [0, 0.0, 0.0])
     per_kernel = {}
     rows = []
+    ours = sum(sum(vs) for n, vs in f.items() if "ddx::" in n)
     for name in sorted(f, key=lambda n: -sum(f[n])):
         k = kernel_class(name)
+        if k is None and "ddx::" in name and sum(f[name]) > 0.01 * ours:
+            log(f"bench: {name.split('(')[0]} reads {sum(f[name]) / ours:.1%} of the bytes and is in no class")
         if name not in w or k is None:
             continue
         fa = sum(f[name]) / len(f[name]) * cf * 1024.0
@@ -244,7 +251,8 @@ def brick_kernel_names(e, kernel, modes, storage):
     names = []
     for m in modes:
         tx, ty, cy, kz, form = e.brick(kernel, m)
-        tm = 0 if (kernel == 0 and m == ddx.RTM_FORWARD) else m  # forward velocity shares the pure-forward kernel
+        # forward velocity shares the pure-forward kernel, forward stress (with sau) the reverse one
+        tm = (0 if kernel == 0 else ddx.RTM_REVERSE) if m == ddx.RTM_FORWARD else m
         base = "k_vel_phy_zb" if kernel == 0 else "k_stress_phy_zb"
         if form == 2:  # paired bricks
             names.append(f"ddx::{base}2<{tm}, {tx}, {ty}, {cy}, {kz}, {st}>")
