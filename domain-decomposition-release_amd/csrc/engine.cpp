@@ -298,7 +298,10 @@ static const double kWholeCells = 14e6;
 // which keep nothing there.  n^3 grids with 15 layers, 40 steps, streaming
 // against ordinary: FP32 n = 64 1.71 / 1.65 ms, 100 (2.2 M cells) 3.83 / 3.53,
 // 128 (3.9 M) 5.72 / 6.01, 200 19.1 / 19.6; BF16 100 3.89 / 3.33, 160 (6.9 M)
-// 11.0 / 10.1, 180 (9.3 M) 15.1 / 14.7, 200 (12.2 M) 21.46 / 21.45.  RTM of
+// 11.0 / 10.1, 180 (9.3 M) 15.1 / 14.7, 200 (12.2 M) 21.46 / 21.45.  RTM (two
+// sets and the images, a set at a time in a launch) of n^3 grids with 15
+// layers, 40 steps: FP32 64 (0.8 M) 4.42 / 4.25, 88 8.73 / 7.80, 112 (2.9 M)
+// 13.97 / 13.80; BF16 100 12.7 / 10.6, 150 (5.8 M) 36.5 / 34.9, 180 55.3 / 54.3;
 // 141x97x75 with 12 layers (2.0 M), 140 steps: 52.9 / 46.8 ms.
 static double cached_limit(int fmt) { return fmt == STORE_F32 ? 3e6 : 10e6; }
 

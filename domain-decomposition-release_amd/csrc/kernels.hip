@@ -2060,17 +2060,16 @@ __device__ __forceinline__ void psi_store(GT *psi, long ncell, unsigned c, float
   sto(psi + 2 * ncell, o, p2);
 }
 
-// One x cell per thread (FP32 storage).  The cells of block (zc, tile) of slab
-// D; rv: 1, as the pairs' ratio of scales.
+// One x cell per thread (FP32 storage): the CPML cells of half steps that run
+// as one launch, and DDX_PML_CZ's splits.  The cells of block (zc, tile) of
+// slab D; rv: 1, as the pairs' ratio of scales.
 //
-// What bounds it: the slab's own bytes (42-48 loads and 12-16 stores per
-// cell), moved at 4.6 TB/s on large grids, the rate of a plain copy; on small
-// ones, how many blocks fit the GPU and their vector instructions.  Hence one
+// What bounds it there (grids up to 14 M cells): how many blocks fit the GPU
+// next to the bricks, and their vector instructions.  Hence one
 // scalar base per array and nine 32-bit offsets (the cell, two rows either
 // way, two planes either way) shared by all arrays, the coefficients of an
 // axis as one 16-byte load, and div_u: the stress kernel needs 89 vector
-// registers instead of 102 (5 wavefronts per SIMD, 4 before).  256x256x200,
-// 20 layers (7.0 M cells): velocity 180 -> 177 us, stress 224 -> 214 us.  The
+// registers instead of 102 (5 wavefronts per SIMD, 4 before).  The
 // z slabs' shared model and coefficients and the row found by a product
 // instead of a division: 64^3 with 20 layers 52 -> 51 us per step (clamping
 // the model's row and column too costs vector instructions: 53.6).
@@ -3216,7 +3215,8 @@ __device__ __forceinline__ float bfp_value(short q, int s) {
 // 88^3 with 20 layers: 75 + 81 us as nine launches, 63 + 71 as two; 141x97x75
 // with 12: 84 + 90 and 77 + 80.  Four wavefronts per SIMD are asked for, as
 // the reverse half steps alone have; it costs the (32, 8, 4) and (64, 4, 2)
-// shapes 12 and 8 bytes of scratch.
+// shapes 12 and 8 bytes of scratch.  From 2.9 to 6 M cells on the backward
+// bricks are ahead in launches of their own (rev_limit in engine.cpp).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void ring_cell(const CopyDesc &D, int e, int cnt, const MemberIO &m, int slice) {
   if (e >= cnt) return;

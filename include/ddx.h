@@ -265,7 +265,8 @@ int ddx_set_tiling_mode(ddx_ctx *ctx, int kernel, int mode, int tx, int ty, int 
 /* Brick shape including its lane form px: 1 one cell per thread; 2 the
  * paired bricks (two neighbouring x cells per thread, one 2-element access
  * per field), shapes (tx,ty,cy,kz) (64,4,1,1) (64,4,1,2) (64,4,1,4)
- * (64,2,1,4) in every storage format; 3 one cell per thread with the x
+ * (64,2,1,4) in every storage format and (32,8,1,2) (32,8,1,4) in the 16-bit
+ * ones; 3 one cell per thread with the x
  * stencil arm taken from neighbouring lanes of the wavefront (DPP shifts
  * instead of loads), shapes (64,4,1,2) (64,4,1,4) (64,4,1,8) (64,8,1,4)
  * (64,2,1,8), FP32 storage; 4 form 3 with the y arm read from an LDS tile
@@ -373,9 +374,12 @@ int ddx_batch_destroy(ddx_batch *b);
 /* Graph replay (no reference counterpart): with on = 1, ddx_model_shot
  * captures one time step (velocity, source, stress, receivers, with the CMM
  * exchanges) in a HIP graph and replays it every step; the time index comes
- * from a device counter that the step advances.  Cuts the host launch cost
- * of small shots; results are identical.  Off by default, and skipped while
- * ddx_profile is timing a kernel class. */
+ * from a device counter that the step advances.  For a host thread that
+ * cannot keep up with the launches: one submission per step instead of two
+ * (whole half steps) or six.  Where it keeps up, the launch that advances the
+ * counter costs more than it saves (32x28x24 cells: 14.2 us per step eager,
+ * 20.3 replayed; 100^3 67.5, 73.8).  Results are identical.  Off by default,
+ * and skipped while ddx_profile is timing a kernel class. */
 int ddx_set_graphs(ddx_ctx *ctx, int on);
 
 /* ---- measurement ------------------------------------------------------------
@@ -385,7 +389,9 @@ int ddx_set_graphs(ddx_ctx *ctx, int on);
  * class at once; any other value stops timing.
  * ddx_kernel_time returns the summed milliseconds and the launch count since
  * the last ddx_profile call, and the algorithmic bytes moved by those
- * launches (every class's, summed, after ddx_profile(ctx, -1)). */
+ * launches (every class's, summed, after ddx_profile(ctx, -1)).  While classes
+ * are timed, every half step runs as separate launches, also on small grids,
+ * where it is one launch otherwise: the times are of those launches. */
 int ddx_profile(ddx_ctx *ctx, int kernel);
 int ddx_kernel_time(ddx_ctx *ctx, double *ms, long long *launches, double *bytes);
 /* With ddx_profile(ctx, -1) every class is timed at once; this returns one
