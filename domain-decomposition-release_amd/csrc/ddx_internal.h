@@ -39,7 +39,7 @@ constexpr int kBlock = 256;
 constexpr int kTileX = 64;
 constexpr int kTileY = 4;
 // Work split of the CPML kernels (a context's pml_cz):
-//   kPmlPairs (the default): kBlock consecutive pairs of x cells of a slab
+//   kPmlPairs: kBlock consecutive pairs of x cells of a slab
 //     plane per block;
 //   1, 2, 4, 8: kBlock consecutive cells of a slab plane per block, cz
 //     planes per thread, the x and y stencil taps read through the caches;

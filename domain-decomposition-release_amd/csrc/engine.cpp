@@ -305,6 +305,14 @@ static const double kWholeCells = 14e6;
 // 141x97x75 with 12 layers (2.0 M), 140 steps: 52.9 / 46.8 ms.
 static double cached_limit(int fmt) { return fmt == STORE_F32 ? 3e6 : 10e6; }
 
+// CPML cells in launches of their own: pairs of x cells per thread in the
+// 16-bit formats; in FP32 from 20 layers on, one cell per thread in thinner
+// ones, whose short rows pairs cut badly.  One cell over pairs, velocity and
+// stress per step, 240^3, 301x270x250, 400x300x200 cells: 4 layers 0.89, 0.82,
+// 0.81; 8 0.99, 0.95, 0.98; 12 0.99, 0.96, 1.00; 16 1.00, 0.95, 1.01; 18 0.97,
+// 0.95, 0.98; 20 1.01, 0.97, 1.02; 24 1.02, 1.00, 1.01; 676x676x210 with 20 1.01.
+static int pml_split(int fmt, int layers) { return fmt == STORE_F32 && layers < 20 ? 1 : kPmlPairs; }
+
 struct ddx_ctx {
   ddx_desc d;
   std::string err;
@@ -364,7 +372,8 @@ struct ddx_ctx {
   double whole_cells = kWholeCells;  // half steps of at most so many cells run as one launch
   double rev_cells = -1;             // and the halves of a reverse iteration (< 0: rev_limit)
   double cached_cells = 0;           // and of at most so many through ordinary accesses (cached_limit)
-  int pml_cz = kPmlPairs;            // work split of the CPML kernels
+  int pml_cz = kPmlPairs;            // work split of the CPML kernels (pml_split)
+  bool pml_swept = false;            // DDX_PML_CZ chose one for all launches
   int pml_group = 32;                // XCD group size of the CPML block order (0: launch order)
   int pml_order = 0;                 // 1: the XCD-partitioned CPML block order (PmlOrder); 0: pml_group
   DevTable<SlabDesc> pml[2][2];        // [model][set]
@@ -752,13 +761,17 @@ extern "C" int ddx_create(const ddx_desc *desc, ddx_ctx **out) {
     delete c;
     return DDX_EHIP;
   }
+  c->pml_cz = pml_split(c->fmt, d.pml_num);
   // CPML work split, for sweeps (FP32 storage; half steps then run as separate
   // launches unless it is 0): 0 pairs, 1, 2, 4, 8 planes per thread
   // with cached taps, or kPmlTiled + 2, 4, 8 (18, 20, 24) for LDS plane tiles
   if (const char *e = getenv("DDX_PML_CZ")) {
     const int v = atoi(e);
     const int p = pml_planes(v);
-    if (c->fmt == STORE_F32 && v >= 0 && (p == 1 || p == 2 || p == 4 || p == 8) && (v < kPmlTiled || p > 1)) c->pml_cz = v;
+    if (c->fmt == STORE_F32 && v >= 0 && (p == 1 || p == 2 || p == 4 || p == 8) && (v < kPmlTiled || p > 1)) {
+      c->pml_cz = v;
+      c->pml_swept = v != kPmlPairs;
+    }
   }
   if (const char *e = getenv("DDX_PML_GROUP")) {  // XCD group size of the CPML blocks, for sweeps
     const int v = atoi(e);
@@ -1559,7 +1572,7 @@ static int phy_launch(ddx_ctx *c, int kernel, int set, int mode, const Tiling &t
 // the parts apart) or the launch's size rule it out.
 static bool whole_half(const ddx_ctx *c, const Tiling &t, const DevTable<PhyDesc> &p, const DevTable<SlabDesc> &q,
                        float sc, HalfStep &a) {
-  if (!t.whole || c->prof.mask || c->pml_overlap || c->pml_cz != kPmlPairs || c->pml_order) return false;
+  if (!t.whole || c->prof.mask || c->pml_overlap || c->pml_swept || c->pml_order) return false;
   if (p.cells + q.cells > c->whole_cells) return false;
   a = {p.d, p.starts, p.n, p.nblk, q.d, q.starts, q.n, q.nblk, c->d.dx, c->d.dy, c->d.dz, sc,
        sc / c->d.dx, sc / c->d.dy, sc / c->d.dz, c->whole_group, c->pml_group,
@@ -1931,6 +1944,7 @@ struct FusedTable {
   int *starts = nullptr;
   int n = 0, nblk = 0;
   bool owned = true;  // false: a view into the fixed batch scratch
+  int cz = kPmlPairs; // work split (CPML tables)
   PmlOrder ord;       // XCD-partitioned block order (CPML tables; pieces owned here)
   void reset() {
     if (owned && d) (void)hipFree(d);
@@ -1980,8 +1994,11 @@ static hipError_t upload_owned(const HostTable<T> &h, FusedTable<T> &out) {
   return e;
 }
 
-// A fused CPML table with its XCD-partitioned block order.
-static hipError_t upload_owned_pml(const HostTable<SlabDesc> &h, int cz, FusedTable<SlabDesc> &out) {
+// A fused CPML table in the work split cz (the members' own may differ), with
+// its XCD-partitioned block order.
+static hipError_t upload_owned_pml(HostTable<SlabDesc> &h, int cz, FusedTable<SlabDesc> &out) {
+  h.nblk = split_pml(h.d, h.s, cz);
+  out.cz = cz;
   hipError_t e = upload_owned(h, out);
   if (e != hipSuccess || h.d.empty()) return e;
   std::vector<PmlPiece> pieces;
@@ -2011,7 +2028,7 @@ struct BatchMember {
 
 // What members of one fused launch must share.
 struct BatchKey {
-  int device = 0, fmt = 0, lg0 = 0, lg1 = 0, pml_cz = kPmlPairs, pml_group = 0, pml_order = 1, brick_group = 0, whole_group = 0;
+  int device = 0, fmt = 0, lg0 = 0, lg1 = 0, pml_swept = 0, pml_group = 0, pml_order = 1, brick_group = 0, whole_group = 0;
   float dt = 0.f, dx = 0.f, dy = 0.f, dz = 0.f;
   // [velocity, stress]: up to whole_cells, and in launches of more (brick_for);
   // a continuous batch passes from one to the other as its members change
@@ -2028,7 +2045,7 @@ static BatchKey batch_key(const ddx_ctx *c) {
   k.whole_cells = c->whole_cells;
   k.cached_cells = c->cached_cells;
   k.device = c->d.device; k.fmt = c->fmt; k.lg0 = c->lg[0]; k.lg1 = c->lg[1];
-  k.pml_cz = c->pml_cz; k.pml_group = c->pml_group; k.pml_order = c->pml_order; k.brick_group = c->brick_group; k.whole_group = c->whole_group;
+  k.pml_swept = c->pml_swept ? c->pml_cz : 0; k.pml_group = c->pml_group; k.pml_order = c->pml_order; k.brick_group = c->brick_group; k.whole_group = c->whole_group;
   k.dt = c->d.dt; k.dx = c->d.dx; k.dy = c->d.dy; k.dz = c->d.dz;
   for (int kernel = 0; kernel < 2; kernel++) {
     k.brick[0][kernel] = brick_for(c, kernel, PURE_FORWARD, 0);
@@ -2038,7 +2055,7 @@ static BatchKey batch_key(const ddx_ctx *c) {
 }
 static bool batch_compatible(const BatchKey &k, const ddx_ctx *c) {
   return c->d.device == k.device && c->fmt == k.fmt && c->lg[0] == k.lg0 && c->lg[1] == k.lg1 &&
-         c->pml_cz == k.pml_cz && c->d.dt == k.dt && c->d.dx == k.dx && c->d.dy == k.dy && c->d.dz == k.dz &&
+         (c->pml_swept ? c->pml_cz : 0) == k.pml_swept && c->d.dt == k.dt && c->d.dx == k.dx && c->d.dy == k.dy && c->d.dz == k.dz &&
          !c->pml_overlap;
 }
 static const char *kBatchMismatch =
@@ -2145,7 +2162,7 @@ static bool batch_whole(const std::vector<BatchMember> &ms, double &cells) {
   cells = 0;
   if (ms.empty()) return false;
   const ddx_ctx *c0 = ms[0].c;
-  bool ok = c0->pml_cz == kPmlPairs && !c0->pml_order;
+  bool ok = !c0->pml_swept && !c0->pml_order;
   for (const BatchMember &m : ms) {
     ok = ok && source_owned(m.c, m.ishot);
     cells += ext_cells(m.c);
@@ -2191,7 +2208,7 @@ static bool fused_step(const BatchKey &k, const FusedSet &f, const std::vector<B
     if (!launch_vel_phy(f.tv, PURE_FORWARD, k.fmt, f.v.d, f.v.starts, f.v.n, f.v.nblk, k.dx, k.dy, k.dz, rvs,
                         k.brick_group, st))
       return false;
-    launch_vel_pml(k.pml_cz, k.fmt, f.p.d, f.p.starts, f.p.n, f.p.nblk, k.dx, k.dy, k.dz, rvs, k.pml_group,
+    launch_vel_pml(f.p.cz, k.fmt, f.p.d, f.p.starts, f.p.n, f.p.nblk, k.dx, k.dy, k.dz, rvs, k.pml_group,
                    k.pml_order ? &f.p.ord : nullptr, st);
   }
   for (const BatchMember &m : ms) exchange_on(m.c, 0, 0, st);
@@ -2207,7 +2224,7 @@ static bool fused_step(const BatchKey &k, const FusedSet &f, const std::vector<B
     if (!launch_stress_phy(f.ts, PURE_FORWARD, k.fmt, f.s.d, f.s.starts, f.s.n, f.s.nblk, k.dx, k.dy, k.dz,
                            k.dt * rsv, k.brick_group, st))
       return false;
-    launch_stress_pml(k.pml_cz, 0, k.fmt, f.p.d, f.p.starts, f.p.n, f.p.nblk, k.dx, k.dy, k.dz, k.dt * rsv,
+    launch_stress_pml(f.p.cz, 0, k.fmt, f.p.d, f.p.starts, f.p.n, f.p.nblk, k.dx, k.dy, k.dz, k.dt * rsv,
                       k.pml_group, k.pml_order ? &f.p.ord : nullptr, st);
     launch_recv_batch(k.fmt, io, st);
   }
@@ -2360,7 +2377,9 @@ static int fuse_into_scratch(const BatchKey &k, std::vector<BatchMember> &ms, Fu
   fuse_host(ms, fused_shapes(k, ms, f), h);
   std::vector<PmlPiece> pieces;
   PmlOrder ord;
-  pml_order_host(h.p.d, ms[0].c->pml_cz, pieces, ord);
+  f.p.cz = ms[0].c->pml_cz;
+  h.p.nblk = split_pml(h.p.d, h.p.s, f.p.cz);
+  pml_order_host(h.p.d, f.p.cz, pieces, ord);
   std::vector<unsigned char> buf;
   const size_t vd = stage(buf, h.v.d), vs = stage(buf, h.v.s);
   const size_t sd = stage(buf, h.s.d), ss = stage(buf, h.s.s);
@@ -2527,7 +2546,7 @@ static int rtm_batch_tables(const std::vector<ddx_ctx *> &cs, const std::vector<
     hi[q].d.push_back(x);
     hi[q].s.push_back(0);
     hi[q].nblk = recv_blocks(c);
-    T.whole = (q ? T.whole : c0->pml_cz == kPmlPairs && !c0->pml_order) && source_owned(c, shots[q]);
+    T.whole = (q ? T.whole : !c0->pml_swept && !c0->pml_order) && source_owned(c, shots[q]);
     T.rev = (q ? T.rev : rev_shapes(c0, sh[4], sh[5])) && source_in_phy(c, shots[q]) && c->exch_mode != 1;
     for (int k = 0; k < 2 && e == hipSuccess && T.rev; k++) {
       const PhyTables *pt = phy_tables(c, sh[4 + k], model_for(c, B));
@@ -2595,7 +2614,7 @@ static bool rtm_fused_forward(const BatchKey &k, const ddx_ctx *c0, const RtmTab
     if (!launch_vel_phy(T.sh[0], F, k.fmt, T.fv.d, T.fv.starts, T.fv.n, T.fv.nblk, k.dx, k.dy, k.dz, rvs,
                         k.brick_group, st))
       return false;
-    launch_vel_pml(k.pml_cz, k.fmt, T.fp.d, T.fp.starts, T.fp.n, T.fp.nblk, k.dx, k.dy, k.dz, rvs, k.pml_group,
+    launch_vel_pml(T.fp.cz, k.fmt, T.fp.d, T.fp.starts, T.fp.n, T.fp.nblk, k.dx, k.dy, k.dz, rvs, k.pml_group,
                    k.pml_order ? &T.fp.ord : nullptr, st);
   }
   for (ddx_ctx *c : cs) exchange_on(c, 0, 0, st);
@@ -2607,7 +2626,7 @@ static bool rtm_fused_forward(const BatchKey &k, const ddx_ctx *c0, const RtmTab
     if (!launch_stress_phy(T.sh[1], F, k.fmt, T.fs.d, T.fs.starts, T.fs.n, T.fs.nblk, k.dx, k.dy, k.dz,
                            k.dt * rsv, k.brick_group, st))
       return false;
-    launch_stress_pml(k.pml_cz, 1, k.fmt, T.fp.d, T.fp.starts, T.fp.n, T.fp.nblk, k.dx, k.dy, k.dz, k.dt * rsv,
+    launch_stress_pml(T.fp.cz, 1, k.fmt, T.fp.d, T.fp.starts, T.fp.n, T.fp.nblk, k.dx, k.dy, k.dz, k.dt * rsv,
                       k.pml_group, k.pml_order ? &T.fp.ord : nullptr, st);
   }
   for (ddx_ctx *c : cs) exchange_on(c, 0, 1, st);
@@ -2659,7 +2678,7 @@ static bool rtm_fused_reverse(const BatchKey &k, const ddx_ctx *c0, const RtmTab
   for (ddx_ctx *c : cs) exchange_on(c, 0, 2, st);
   if (!T.whole || !T.sh[4].whole || !launch_vel_all(T.sh[4], R, k.fmt, half_of(k, T.rv, T.rpw, rvs, T.cells), st)) {
     if (!vel(T.rv, R, 1.f)) return false;
-    launch_vel_pml(k.pml_cz, k.fmt, T.rp.d, T.rp.starts, T.rp.n, T.rp.nblk, dx, dy, dz, rvs, k.pml_group,
+    launch_vel_pml(T.rp.cz, k.fmt, T.rp.d, T.rp.starts, T.rp.n, T.rp.nblk, dx, dy, dz, rvs, k.pml_group,
                    k.pml_order ? &T.rp.ord : nullptr, st);
   }
   for (ddx_ctx *c : cs) exchange_on(c, 1, 0, st);
@@ -2669,7 +2688,7 @@ static bool rtm_fused_reverse(const BatchKey &k, const ddx_ctx *c0, const RtmTab
   for (ddx_ctx *c : cs) exchange_on(c, 0, 0, st);
   if (!T.whole || !T.sh[5].whole || !launch_stress_all(T.sh[5], R, k.fmt, half_of(k, T.rs, T.rpw, dt * rsv, T.cells), StepIO{}, st)) {
     if (!stress(T.rs, R, dt)) return false;
-    launch_stress_pml(k.pml_cz, 1, k.fmt, T.rp.d, T.rp.starts, T.rp.n, T.rp.nblk, dx, dy, dz, dt * rsv, k.pml_group,
+    launch_stress_pml(T.rp.cz, 1, k.fmt, T.rp.d, T.rp.starts, T.rp.n, T.rp.nblk, dx, dy, dz, dt * rsv, k.pml_group,
                       k.pml_order ? &T.rp.ord : nullptr, st);
   }
   for (ddx_ctx *c : cs) exchange_on(c, 1, 2, st);
@@ -3585,7 +3604,7 @@ static bool small_half(const ddx_ctx *c, int mode) {
 // Whether the mode's half steps are timed as halves of a reverse iteration.
 static bool reverse_tuned(const ddx_ctx *c, int mode) {
   return mode == RTM_REVERSE && ext_cells(c) <= rev_limit(c, true) && c->exch_mode != 1 && !c->set_overlap &&
-         !c->pml_overlap && c->pml_cz == kPmlPairs && !c->pml_order;
+         !c->pml_overlap && !c->pml_swept && !c->pml_order;
 }
 
 // What decides which launches are timed is in the key.  The layers' width is
@@ -3596,8 +3615,8 @@ static std::string tune_key(const ddx_ctx *c, int kernel, int mode) {
   int big[3];
   for (int a = 0; a < 3; a++) big[a] = (c->all.pn[a] + 31) / 32 * 32;
   snprintf(b, sizeof b, "f%d k%d m%d R%d b%dx%dx%d mig%d p%d,%d,%d,%d w%d r%d c%d", c->fmt, kernel, mode,
-           mode == RTM_BACKWARD ? c->d.rec_width : 0, big[0], big[1], big[2], (int)model_for(c, mode), c->pml_cz,
-           c->pml_group, c->pml_order, (int)c->pml_overlap, small_half(c, mode), reverse_tuned(c, mode),
+           mode == RTM_BACKWARD ? c->d.rec_width : 0, big[0], big[1], big[2], (int)model_for(c, mode),
+           small_half(c, mode) && !c->pml_swept ? 0 : c->pml_cz, c->pml_group, c->pml_order, (int)c->pml_overlap, small_half(c, mode), reverse_tuned(c, mode),
            ext_cells(c) <= c->cached_cells);
   return b;
 }

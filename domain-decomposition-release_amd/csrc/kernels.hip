@@ -2061,11 +2061,13 @@ __device__ __forceinline__ void psi_store(GT *psi, long ncell, unsigned c, float
 }
 
 // One x cell per thread (FP32 storage): the CPML cells of half steps that run
-// as one launch, and DDX_PML_CZ's splits.  The cells of block (zc, tile) of
-// slab D; rv: 1, as the pairs' ratio of scales.
+// as one launch, those of thin layers in launches of their own (pml_split in
+// engine.cpp), and DDX_PML_CZ's splits.  The cells of block (zc, tile) of slab
+// D; rv: 1, as the pairs' ratio of scales.
 //
-// What bounds it there (grids up to 14 M cells): how many blocks fit the GPU
-// next to the bricks, and their vector instructions.  Hence one
+// What bounds it: on large grids the slab's own bytes (42-48 loads and 12-16
+// stores per cell); up to 14 M cells, how many blocks fit the GPU next to the
+// bricks, and their vector instructions.  Hence one
 // scalar base per array and nine 32-bit offsets (the cell, two rows either
 // way, two planes either way) shared by all arrays, the coefficients of an
 // axis as one 16-byte load, and div_u: the stress kernel needs 89 vector
@@ -2334,8 +2336,9 @@ __global__ __launch_bounds__(kBlock) DDX_PML_ATTR void k_stress_pml(const SlabDe
 
 
 // ---------------------------------------------------------------------------
-// CPML halves, two neighbouring x cells per thread (work split kPmlPairs, the
-// default).  A plane's rows are cut into pairs whose first cell lies on an
+// CPML halves, two neighbouring x cells per thread (work split kPmlPairs: the
+// 16-bit formats, and in launches of their own FP32 with thick layers,
+// pml_split in engine.cpp).  A plane's rows are cut into pairs whose first cell lies on an
 // even element of the storage (D.sh shifts a slab's rows; the memory variables
 // and coefficients have rows of D.ip elements in the same pairs), so every
 // access of a pair is one aligned 2-element load or store in every format.  A

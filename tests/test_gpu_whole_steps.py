@@ -351,3 +351,45 @@ def test_autotune_cache_is_keyed_by_what_decides(monkeypatch):
     monkeypatch.setenv("DDX_REV_CELLS", "1e9")
     assert timed(pml=5) > 0
     assert timed(pml=4) == 0
+
+
+@pytest.mark.parametrize("first", [0, 1])
+def test_batches_of_uneven_layers_in_separate_launches(first, monkeypatch):
+    """Members with layers on both sides of the width up to which the CPML
+    launches take one cell per thread, each side first: fused and continuous
+    batches equal single shots."""
+    monkeypatch.setenv("DDX_WHOLE_CELLS", "0")
+    cs = [case(nx=33, ny=22, nz=20, pml=20, ntime=24, rec_width=2),
+          case(nx=70, ny=18, nz=19, pml=6, ntime=24, rec_width=2, seed=3)]
+    es = [engine(c) for c in (cs if first == 0 else cs[::-1])]
+    want, images = [], []
+    for e in es:
+        e.model_shot(0)
+        want.append(e.seismograms(0))
+        e.rtm_shot(0)
+        images.append([e.image(i, 0) for i in range(5)])
+        e.reset_images()
+
+    def check():
+        for e, w in zip(es, want):
+            assert np.array_equal(e.seismograms(0), w)
+
+    ddx.model_batch(es)
+    check()
+    ddx.rtm_batch(es)
+    for e, w in zip(es, images):
+        assert all(np.array_equal(e.image(i, 0), w[i]) for i in range(5))
+        e.reset_images()
+    b = ddx.Batch()
+    for rtm in (False, True):
+        b.add(es[0], rtm=rtm)
+        b.run(5)
+        b.add(es[1], rtm=rtm)
+        while len(b):
+            b.run(50)
+        check()
+    for e, w in zip(es, images):
+        assert all(np.array_equal(e.image(i, 0), w[i]) for i in range(5))
+    b.close()
+    for e in es:
+        e.close()
