@@ -54,7 +54,7 @@ METRIC = "Gcell-updates/s + shots/s, 1 MI355X, vs plain FP32; p50/p99 shot laten
 KERNEL_NAMES = {0: "velocity update, physical region (k_vel_phy)", 1: "stress update, physical region (k_stress_phy)",
                 2: "CPML velocity (k_vel_pml)", 3: "CPML stress (k_stress_pml)", 4: "CMM halo exchange (k_copy, mode 1)",
                 5: "imaging (k_image)",
-                # grids of up to 14 M cells (the in-process classes time these half steps as separate launches)
+                # grids of up to 14 M cells, 10 M in 16 bits (the in-process classes time these half steps as separate launches)
                 6: "velocity half steps in one launch (k_vel_all, k_rev_vel)",
                 7: "stress half steps in one launch (k_stress_all, k_rev_stress)"}
 # kernel-name prefixes of each class, as rocprofv3 reports them

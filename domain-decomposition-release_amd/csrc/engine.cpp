@@ -289,8 +289,12 @@ static const int kBrickGroup = 8;
 // 12.1, 160 19.5 / 19.9, 192 (12.5 M cells) 28.2 / 28.4, 224 (18.4 M) 42.1 /
 // 41.7; the 256x256x200 RTM shot (20.1 M) is 1-2% slower in one launch: the
 // bricks then hold the CPML kernel's registers, and what one launch gains,
-// its last wave of blocks, is a small part of a large one.
-static const double kWholeCells = 14e6;
+// its last wave of blocks, is a small part of a large one.  8 layers: 190 (8.7
+// M) 13.7 / 14.5, 208 (11.2 M) 16.6 / 16.8 (40 steps).  BF16, 40 steps, whose
+// pairs take more registers still: 8 layers, 190 12.4 / 14.0, 208 19.3 / 18.8;
+// 12 layers, 190 (9.8 M) 10.9 / 11.3 (30 steps); 20 layers, 150 (6.9 M) 10.2 /
+// 11.0, 170 (9.3 M) 13.7 / 13.5, 190 (12.2 M) 17.8 / 17.2.
+static double whole_limit(int fmt) { return fmt == STORE_F32 ? 14e6 : 10e6; }
 
 // A wavefield set of at most so many cells stays in the 256 MB last-level cache
 // from one launch to the next; then the bricks read and write their own cells,
@@ -369,7 +373,7 @@ struct ddx_ctx {
   std::vector<PhyTables> phy_cache;  // physical-region tables per brick shape
   int brick_group = kBrickGroup;     // XCD group size of the bricks' block order
   int whole_group = -1;              // the same of the half steps that run as one launch (columns)
-  double whole_cells = kWholeCells;  // half steps of at most so many cells run as one launch
+  double whole_cells = 0;            // half steps of at most so many cells run as one launch (whole_limit)
   double rev_cells = -1;             // and the halves of a reverse iteration (< 0: rev_limit)
   double cached_cells = 0;           // and of at most so many through ordinary accesses (cached_limit)
   int pml_cz = kPmlPairs;            // work split of the CPML kernels (pml_split)
@@ -783,6 +787,7 @@ extern "C" int ddx_create(const ddx_desc *desc, ddx_ctx **out) {
     const int v = atoi(e);
     if (v >= 0 && v <= 65536) c->brick_group = c->whole_group = v;
   }
+  c->whole_cells = whole_limit(c->fmt);
   if (const char *e = getenv("DDX_WHOLE_CELLS")) c->whole_cells = atof(e);  // for sweeps
   if (const char *e = getenv("DDX_REV_CELLS")) c->rev_cells = atof(e);      // for sweeps
   c->cached_cells = cached_limit(c->fmt);

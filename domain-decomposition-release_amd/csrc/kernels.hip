@@ -3106,7 +3106,7 @@ __device__ __forceinline__ void recv_block(const StepIO &io, int b) {
 // step does not write, and the receivers read velocities.  One launch fills
 // the GPU's last wave of bricks with CPML blocks and drops the launches'
 // gaps; what each block does is what the separate kernels do.  Where it pays
-// and where not: kWholeCells in engine.cpp.  A modelling step is two launches
+// and where not: whole_limit in engine.cpp.  A modelling step is two launches
 // instead of six: 32x28x24 cells 31.8 -> 15.2 us per step, 64^3 with 20
 // layers 66 -> 51 us, 100^3 with 10 layers 96 -> 75 us (67 with ordinary
 // accesses, NT false).
