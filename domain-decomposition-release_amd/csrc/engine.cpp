@@ -374,7 +374,7 @@ struct ddx_ctx {
   int brick_group = kBrickGroup;     // XCD group size of the bricks' block order
   int whole_group = -1;              // the same of the half steps that run as one launch (columns)
   double whole_cells = 0;            // half steps of at most so many cells run as one launch (whole_limit)
-  double rev_cells = -1;             // and the halves of a reverse iteration (< 0: rev_limit)
+  double rev_cells = -1;             // and the halves of a reverse iteration (< 0: rev_fits)
   double cached_cells = 0;           // and of at most so many through ordinary accesses (cached_limit)
   int pml_cz = kPmlPairs;            // work split of the CPML kernels (pml_split)
   bool pml_swept = false;            // DDX_PML_CZ chose one for all launches
@@ -2477,10 +2477,18 @@ static int ring_status(ddx_ctx *c, std::string &err);
 //   71.8 / 71.4; tuned, with better backward bricks apart: 88 7.83 / 8.78, 140
 //   (4.9 M) 26.5 / 26.0, 208 71.2 / 67.0;
 //   BF16: 112 13.3 / 14.4, 128 17.9 / 17.9, 140 28.2 / 27.5, 208 85.8 / 79.0.
-static double rev_limit(const ddx_ctx *c, bool tuned) {
-  if (c->rev_cells >= 0) return c->rev_cells;
-  if (c->fmt != STORE_F32) return 4e6;
-  return !narrow_rows(c->d.nx) ? 2.9e6 : tuned ? 4e6 : 6e6;
+// Batches of small members gain at any size, since each member's launches are
+// short: 30 steps of 20 of 64^3 with 10 layers (11.9 M) 51.1 / 53.0 ms, tuned
+// 50.2 / 52.9, 14 in BF16 (8.3 M) 37.5 / 37.7, tuned 42.5 / 42.1; 9 of 80^3 40.1
+// / 42.4, tuned 40.4 / 40.2; 9 of 88^3 50.9 / 53.4, tuned 52.0 / 50.9, 7 in
+// BF16 48.1 / 45.5; 3 of 140^3 54.7 / 55.7, tuned 54.1 / 51.6; 5 of 112^3 48.5 /
+// 46.1.
+static bool rev_fits(const ddx_ctx *c, bool tuned, double cells, int members) {
+  if (c->rev_cells >= 0) return cells <= c->rev_cells;
+  const bool f32 = c->fmt == STORE_F32, slow_back = f32 && !tuned && narrow_rows(c->d.nx);
+  const double all = !f32 ? 4e6 : slow_back ? 6e6 : narrow_rows(c->d.nx) ? 4e6 : 2.9e6;
+  const double each = !f32 ? 0.65e6 : slow_back ? 6e6 : 1e6;
+  return cells <= all || cells <= each * members;
 }
 
 // Whether bricks of these shapes (the reverse mode's) run the halves of a
@@ -2595,7 +2603,7 @@ static int rtm_batch_tables(const std::vector<ddx_ctx *> &cs, const std::vector<
     if (e == hipSuccess) e = upload_owned(a, T.fpw);
     if (e == hipSuccess) e = upload_owned(b, T.rpw);
   }
-  T.rev = T.rev && T.whole && cells <= rev_limit(c0, c0->tuned);
+  T.rev = T.rev && T.whole && rev_fits(c0, c0->tuned, cells, (int)cs.size());
   for (int k = 0; k < 2 && e == hipSuccess && T.rev; k++) {
     HostTable<PhyDesc> h;
     HostTable<CopyDesc> x;
@@ -3306,7 +3314,7 @@ static bool rev_half(ddx_ctx *c, int kernel, const Tiling &t, RevHalf &h) {
 // each saves two small launches (4.7 us) and a tail.  False: nothing launched.
 static bool reverse_halves(ddx_ctx *c, int ishot, int it) {
   const Tiling &tv = c->tiling_vel[RTM_REVERSE], &ts = c->tiling_stress[RTM_REVERSE];
-  if (ext_cells(c) > rev_limit(c, c->tuned) || !rev_shapes(c, tv, ts) || !source_in_phy(c, ishot) || c->exch_mode == 1 ||
+  if (!rev_fits(c, c->tuned, ext_cells(c), 1) || !rev_shapes(c, tv, ts) || !source_in_phy(c, ishot) || c->exch_mode == 1 ||
       it > c->store_slices)
     return false;
   RevHalf v, s;
@@ -3608,7 +3616,7 @@ static bool small_half(const ddx_ctx *c, int mode) {
 }
 // Whether the mode's half steps are timed as halves of a reverse iteration.
 static bool reverse_tuned(const ddx_ctx *c, int mode) {
-  return mode == RTM_REVERSE && ext_cells(c) <= rev_limit(c, true) && c->exch_mode != 1 && !c->set_overlap &&
+  return mode == RTM_REVERSE && rev_fits(c, true, ext_cells(c), 1) && c->exch_mode != 1 && !c->set_overlap &&
          !c->pml_overlap && !c->pml_swept && !c->pml_order;
 }
 

@@ -3219,7 +3219,7 @@ __device__ __forceinline__ float bfp_value(short q, int s) {
 // with 12: 84 + 90 and 77 + 80.  Four wavefronts per SIMD are asked for, as
 // the reverse half steps alone have; it costs the (32, 8, 4) and (64, 4, 2)
 // shapes 12 and 8 bytes of scratch.  From 2.9 to 6 M cells on the backward
-// bricks are ahead in launches of their own (rev_limit in engine.cpp).
+// bricks are ahead in launches of their own (rev_fits in engine.cpp).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void ring_cell(const CopyDesc &D, int e, int cnt, const MemberIO &m, int slice) {
   if (e >= cnt) return;
