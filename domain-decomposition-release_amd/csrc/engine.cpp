@@ -670,6 +670,9 @@ static const Tiling &brick_for(const ddx_ctx *c, int kernel, int mode, double ce
   return (kernel == 0 ? c->tiling_vel : c->tiling_stress)[mode];
 }
 
+static double ext_cells(const ddx_ctx *c) { return (double)c->gext[0] * c->gext[1] * c->gext[2]; }
+static double phy_cells(const ddx_ctx *c) { return (double)c->d.nx * c->d.ny * c->d.nz; }
+
 // Brick shapes of a context that is not tuned.  FP32: rows of 64 cells with
 // the y arm from LDS where they waste no more lanes than rows of 32 by over
 // 5%, else one-cell bricks of rows of 32 (n^3 grids, 15 layers, 60 modelling
@@ -677,7 +680,10 @@ static const Tiling &brick_for(const ddx_ctx *c, int kernel, int mode, double ce
 // 5.59 / 5.65, 128 8.50 / 8.69, 160 16.1 / 15.8, 200 29.8 / 28.3).  16-bit:
 // paired bricks, rows of 64 pairs where they waste no more lanes than rows of
 // 32 by over 5% (161x150x131 in BF16, 60 steps, rows of 64 pairs against 32:
-// 17.1 / 14.9 ms).
+// 17.1 / 14.9 ms).  The FWI mode, which the tuner leaves alone, takes one-cell
+// bricks: (32, 8, 1, 4), or rows of 64, 2 planes deep where whole half steps
+// have them, else 4 (250^3, velocity and stress brick: 347 and 282 us with 2
+// planes, 325 and 266 with 4).
 static bool narrow_rows(int nx) { return (nx + 63) / 64 * 64 > 1.05 * ((nx + 31) / 32 * 32); }
 static void default_bricks(ddx_ctx *c) {
   const int nx = c->d.nx, w64 = (nx + 63) / 64 * 64;
@@ -692,6 +698,7 @@ static void default_bricks(ddx_ctx *c) {
     t = f = {32, 8, 1, 4};
   } else {
     t.xl = 2;
+    if (ext_cells(c) > c->whole_cells) f.kz = 4;
   }
   for (int m = 0; m < kModes; m++) set_brick(c, 0, m, m == FWI ? f : t), set_brick(c, 1, m, m == FWI ? f : t);
 }
@@ -1740,9 +1747,6 @@ extern "C" int ddx_reset_wave(ddx_ctx *c, int set) {
       HIPCHECK(c, hipMemsetAsync(sl.psi[set], 0, (size_t)c->esz * 6 * __builtin_popcount(sl.axes) * sl.nstore, c->st));
   return DDX_OK;
 }
-
-static double ext_cells(const ddx_ctx *c) { return (double)c->gext[0] * c->gext[1] * c->gext[2]; }
-static double phy_cells(const ddx_ctx *c) { return (double)c->d.nx * c->d.ny * c->d.nz; }
 
 static int check_ready(ddx_ctx *c, int ishot) {
   if (!c->have_model || !c->have_wavelet || !c->have_geometry) {
