@@ -2064,7 +2064,8 @@ static BatchKey batch_key(const ddx_ctx *c) {
 }
 static bool batch_compatible(const BatchKey &k, const ddx_ctx *c) {
   return c->d.device == k.device && c->fmt == k.fmt && c->lg[0] == k.lg0 && c->lg[1] == k.lg1 &&
-         (c->pml_swept ? c->pml_cz : 0) == k.pml_swept && c->d.dt == k.dt && c->d.dx == k.dx && c->d.dy == k.dy && c->d.dz == k.dz &&
+         (c->pml_swept ? c->pml_cz : 0) == k.pml_swept && c->d.dt == k.dt && c->d.dx == k.dx &&
+         c->d.dy == k.dy && c->d.dz == k.dz &&
          !c->pml_overlap;
 }
 static const char *kBatchMismatch =
@@ -3318,8 +3319,8 @@ static bool rev_half(ddx_ctx *c, int kernel, const Tiling &t, RevHalf &h) {
 // each saves two small launches (4.7 us) and a tail.  False: nothing launched.
 static bool reverse_halves(ddx_ctx *c, int ishot, int it) {
   const Tiling &tv = c->tiling_vel[RTM_REVERSE], &ts = c->tiling_stress[RTM_REVERSE];
-  if (!rev_fits(c, c->tuned, ext_cells(c), 1) || !rev_shapes(c, tv, ts) || !source_in_phy(c, ishot) || c->exch_mode == 1 ||
-      it > c->store_slices)
+  if (!rev_fits(c, c->tuned, ext_cells(c), 1) || !rev_shapes(c, tv, ts) || !source_in_phy(c, ishot) ||
+      c->exch_mode == 1 || it > c->store_slices)
     return false;
   RevHalf v, s;
   if (!rev_half(c, 0, tv, v) || !rev_half(c, 1, ts, s)) return false;
@@ -3633,8 +3634,8 @@ static std::string tune_key(const ddx_ctx *c, int kernel, int mode) {
   for (int a = 0; a < 3; a++) big[a] = (c->all.pn[a] + 31) / 32 * 32;
   snprintf(b, sizeof b, "f%d k%d m%d R%d b%dx%dx%d mig%d p%d,%d,%d,%d w%d r%d c%d", c->fmt, kernel, mode,
            mode == RTM_BACKWARD ? c->d.rec_width : 0, big[0], big[1], big[2], (int)model_for(c, mode),
-           small_half(c, mode) && !c->pml_swept ? 0 : c->pml_cz, c->pml_group, c->pml_order, (int)c->pml_overlap, small_half(c, mode), reverse_tuned(c, mode),
-           ext_cells(c) <= c->cached_cells);
+           small_half(c, mode) && !c->pml_swept ? 0 : c->pml_cz, c->pml_group, c->pml_order, (int)c->pml_overlap,
+           small_half(c, mode), reverse_tuned(c, mode), ext_cells(c) <= c->cached_cells);
   return b;
 }
 
@@ -3721,8 +3722,8 @@ extern "C" int ddx_autotune(ddx_ctx *c, int reps, int *timed) {
           rc = time_launches(c, e0, e1, reps, ms, [&]() -> int {
             if (!halves) return kernel == 0 ? vel_update(c, 0, mode) : stress_update(c, 0, mode);
             RevHalf h;
-            const bool ok = rev_half(c, kernel, t, h) &&
-                            (kernel == 0 ? launch_rev_vel : launch_rev_stress)(t, c->fmt, h.a, h.q, StepIO{}, RingBoxes{}, c->st);
+            const auto launch = kernel == 0 ? launch_rev_vel : launch_rev_stress;
+            const bool ok = rev_half(c, kernel, t, h) && launch(t, c->fmt, h.a, h.q, StepIO{}, RingBoxes{}, c->st);
             return ok ? DDX_OK : DDX_EHIP;
           });
           count++;
